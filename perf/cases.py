@@ -401,7 +401,8 @@ def _run_linear(state: dict):
     shared_activation_quantizer.clear()
     x, weight, bias = state["x"], state["weight"], state["bias"]
     if not state["backward"]:
-        return prequantized_linear(x, weight, bias)
+        with torch.no_grad():
+            return prequantized_linear(x, weight, bias)
     out = prequantized_linear(x, weight, bias)
     wanted = [x, weight] if bias is None else [x, weight, bias]
     return [out.detach(), *torch.autograd.grad(out, wanted, state["grad_out"])]
