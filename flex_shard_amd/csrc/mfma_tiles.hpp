@@ -48,17 +48,19 @@ struct GemmParams {
 #define FSH_STAMP(slot) do {} while (0)
 #endif
 
-// Several problems served by one launch of the large-tile kernel: problem i
+// Several problems served by one launch: problem i
 // owns the workgroup ids [first_workgroup[i], first_workgroup[i+1]), each run
 // a multiple of 8 long so that the id -> XCD mapping is the same for all.
 // Workgroups are dispatched in id order, so the host lists the problem with
 // the longest tiles first and the short ones fill the tail of the long ones.
-constexpr int kMaxGemmProblems = 4;
-struct GemmLaunch {
-  GemmParams problem[kMaxGemmProblems];
-  int32_t first_workgroup[kMaxGemmProblems];  // INT32_MAX past the last problem
+template <int N>
+struct GemmLaunchOf {
+  static constexpr int kMaxProblems = N;
+  GemmParams problem[N];
+  int32_t first_workgroup[N];  // INT32_MAX past the last problem
   int32_t total_workgroups;
 };
+using GemmLaunch = GemmLaunchOf<4>;  // the large-tile kernel (a longer lookup costs its resident form scalar registers)
 
 constexpr int kXcds = 8;         // accelerator dies, each with its own L2
 constexpr int kGroupTilesM = 4;  // tile rows walked together
@@ -103,33 +105,6 @@ __device__ inline bool tile_of_workgroup(const GemmParams& p, int64_t id, int64_
   tile_in_order(p, t, tm, tn);
   return true;
 }
-
-// Epilogue of the whole-tile kernels, staged through LDS (free once the last
-// k-tile's barrier has passed; every wave uses a private region, but the
-// phases are still separated by workgroup barriers).
-//
-// The accumulate is issued as mfma(B, A), so accumulator r of block (i, j)
-// belongs to output row m = lane%32 and column n = 8*(r/4) + 4*(lane/32) + r%4
-// of the block.  In that layout a store instruction would touch 32 rows with
-// 16 bytes each, and the transposed output would leave as 2-byte stores.
-// Instead:
-//   1. D is loaded row-wise (16 bytes per lane) into the staging region; the
-//      finals = bf16(alpha*acc + beta*D) are computed in registers and written
-//      to LDS as [row][col], each over the D value it used;
-//   2. the wave reads its region back row-wise and stores C as 16 bytes per
-//      lane, 256 contiguous bytes per row;
-//   3. for a transposed (or mirrored) output the finals are read back in
-//      accumulator layout, written again as [col][row] and leave the same way.
-// The LDS row pitch is the row plus 8 bytes: 8-byte writes of 16 lanes then
-// cover all 32 banks, and so do the row-wise 8-byte reads of a half-wave.
-template <typename Cfg>
-struct WholeTileEpilogue {
-  static constexpr int kPitch = Cfg::kWaveN * 2 + 8;   // bytes, [row][col] staging
-  static constexpr int kPitchT = Cfg::kWaveM * 2 + 8;  // bytes, [col][row] staging
-  static constexpr int kRegion =
-      (Cfg::kWaveM * kPitch > Cfg::kWaveN * kPitchT) ? Cfg::kWaveM * kPitch : Cfg::kWaveN * kPitchT;
-  static constexpr int kLdsBytes = Cfg::WM * Cfg::WN * kRegion;
-};
 
 // Values that are the same in every lane but that the compiler cannot prove
 // so: moved to scalar registers.
@@ -203,129 +178,6 @@ __device__ __forceinline__ void load_d_rows_from(const uint16_t* d, int64_t ldd,
   for (int q = 0; q < R::kPasses; ++q) rows.t[q] = *reinterpret_cast<const u32x4*>(base + q * pass_bytes + lane_off);
 }
 
-template <typename Cfg>
-__device__ __forceinline__ void load_d_rows(const GemmParams& p, int64_t batch, int64_t m0, int64_t n0, int wm, int wn,
-                                            int lane, int half, DRows<Cfg>& rows) {
-  load_d_rows_from<Cfg>(p.D + batch * p.sD, p.ldd, m0, n0, wm, wn, lane, half, rows);
-}
-
-template <typename Cfg, int kPitch>
-__device__ __forceinline__ void stage_d_rows(uint8_t* region, int lane, int half, const DRows<Cfg>& rows) {
-  using R = DRows<Cfg>;
-  const int r0 = half * (Cfg::kWaveM / 2) + lane / R::kLanesPerRow, chunk = lane % R::kLanesPerRow;
-  uint8_t* ddst = region + r0 * kPitch + chunk * 16;
-#pragma unroll
-  for (int q = 0; q < R::kPasses; ++q) {
-    uint8_t* d = ddst + q * R::kRowsPerPass * kPitch;
-    *reinterpret_cast<u32x2*>(d) = u32x2{rows.t[q].x, rows.t[q].y};
-    *reinterpret_cast<u32x2*>(d + 8) = u32x2{rows.t[q].z, rows.t[q].w};
-  }
-}
-
-template <typename Cfg>
-__device__ inline void store_whole_tile(const GemmParams& p, int64_t batch, int64_t m0, int64_t n0, int wm, int wn,
-                                        int lane, bool mirror, const f32x16 (&acc)[Cfg::TM][Cfg::TN],
-                                        uint8_t* lds) {
-  using Epi = WholeTileEpilogue<Cfg>;
-  constexpr int TM = Cfg::TM, TN = Cfg::TN;
-  static_assert(TM % 2 == 0, "the D tile is handled in two halves of TM/2 blocks");
-  const bool has_d = p.D != nullptr;
-  uint16_t* C = p.C + batch * p.sC;
-  // A symmetric product mirrors its off-diagonal tiles into the lower triangle.
-  uint16_t* Ct = mirror ? C : (p.Ct ? p.Ct + batch * p.sCt : nullptr);
-  const int64_t ldct = mirror ? p.ldc : p.ldct;
-  const int64_t wave_row = m0 + wm * Cfg::kWaveM, wave_col = n0 + wn * Cfg::kWaveN;
-  uint8_t* region = lds + (wm * Cfg::WN + wn) * Epi::kRegion;
-  const int r_lane = lane & 31, h = lane >> 5;
-
-  // D goes to the wave's staging region row-wise and is read back in
-  // accumulator layout; each final then replaces the D value it used.
-  DRows<Cfg> upper, lower;
-  if (has_d) {
-    load_d_rows<Cfg>(p, batch, m0, n0, wm, wn, lane, 0, upper);
-    load_d_rows<Cfg>(p, batch, m0, n0, wm, wn, lane, 1, lower);
-    stage_d_rows<Cfg, Epi::kPitch>(region, lane, 0, upper);
-  }
-  FSH_STAMP(8);
-
-  // finals = bf16(fma(beta, D, alpha*acc)): one rounding of the scaled
-  // accumulator, one of the sum, as a BLAS epilogue does.
-  const bool unit_alpha = p.alpha == 1.0f;
-  // Block tiles and wave sub-tiles are square, so C's diagonal runs through
-  // the (i, i) blocks of the diagonal sub-tiles of the diagonal tiles.
-  const bool on_diagonal = p.diag_add != 0.0f && m0 == n0 && wm == wn;
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    if (has_d && i == TM / 2) stage_d_rows<Cfg, Epi::kPitch>(region, lane, 1, lower);
-    // All of a 32-row block's D reads are issued before its first write: the
-    // compiler cannot move a read above a write to the same region.
-    u32x2 dv[TN][4];
-    if (has_d) {
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-          dv[j][b] = *reinterpret_cast<const u32x2*>(region + (i * 32 + r_lane) * Epi::kPitch +
-                                                     (j * 32 + 8 * b + 4 * h) * 2);
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        float v[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) v[t] = unit_alpha ? acc[i][j][4 * b + t] : p.alpha * acc[i][j][4 * b + t];
-        if (has_d) {
-          v[0] = __builtin_fmaf(p.beta, u32_as_f32(dv[j][b].x << 16), v[0]);
-          v[1] = __builtin_fmaf(p.beta, u32_as_f32(dv[j][b].x & 0xFFFF0000u), v[1]);
-          v[2] = __builtin_fmaf(p.beta, u32_as_f32(dv[j][b].y << 16), v[2]);
-          v[3] = __builtin_fmaf(p.beta, u32_as_f32(dv[j][b].y & 0xFFFF0000u), v[3]);
-        }
-        if (on_diagonal && i == j) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-            if (r_lane == 8 * b + 4 * h + t) v[t] += p.diag_add;
-        }
-        *reinterpret_cast<u32x2*>(region + (i * 32 + r_lane) * Epi::kPitch + (j * 32 + 8 * b + 4 * h) * 2) =
-            u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-      }
-  }
-  FSH_STAMP(9);
-  __syncthreads();
-  store_staged_rows<Cfg::kWaveM, Cfg::kWaveN * 2, Epi::kPitch>(region, C + wave_row * p.ldc + wave_col, p.ldc, lane);
-  FSH_STAMP(10);
-  if (Ct == nullptr) return;  // uniform over the workgroup
-  __syncthreads();
-  FSH_STAMP(11);
-  // The finals come back from the [row][col] image in accumulator layout
-  // (all reads before the first write: the transposed image reuses the
-  // region) and are written again as [col][row].
-  u32x2 fin[TM][TN][4];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        fin[i][j][b] = *reinterpret_cast<const u32x2*>(region + (i * 32 + r_lane) * Epi::kPitch +
-                                                       (j * 32 + 8 * b + 4 * h) * 2);
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const uint32_t pair = (t >> 1) ? fin[i][j][b].y : fin[i][j][b].x;
-          *reinterpret_cast<uint16_t*>(region + (j * 32 + 8 * b + 4 * h + t) * Epi::kPitchT + (i * 32 + r_lane) * 2) =
-              static_cast<uint16_t>((t & 1) ? (pair >> 16) : pair);
-        }
-  FSH_STAMP(12);
-  __syncthreads();
-  store_staged_rows<Cfg::kWaveN, Cfg::kWaveM * 2, Epi::kPitchT>(region, Ct + wave_col * ldct + wave_row, ldct, lane);
-}
-
 // Orders the LDS traffic of one wave: lanes exchange data through the wave's
 // private staging region, which the hardware serves in program order; this
 // only keeps the compiler from moving a lane's reads above other lanes'
@@ -336,12 +188,29 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Epilogue of the large-tile kernel: the same steps as store_whole_tile, but
-// on the upper and then the lower 64 rows of the wave's 128x128 sub-tile, in a
-// staging region of 17 KB per wave that only the wave itself touches.  The
-// region then fits beside one k-loop stage, which leaves the other stage free
-// to receive the next tile's first operands while this runs, and no step
-// needs a workgroup barrier (whose memory fence would wait for those loads).
+// Epilogue of the large-tile kernel, staged through LDS.
+//
+// The accumulate is issued as mfma(B, A), so accumulator r of block (i, j)
+// belongs to output row m = lane%32 and column n = 8*(r/4) + 4*(lane/32) + r%4
+// of the block.  In that layout a store instruction would touch 32 rows with
+// 16 bytes each, and the transposed output would leave as 2-byte stores.
+// Instead:
+//   1. D is loaded row-wise (16 bytes per lane) into the staging region; the
+//      finals = bf16(fma(beta, D, alpha*acc)) are computed in registers and
+//      written to LDS as [row][col], each over the D value it used;
+//   2. the wave reads its region back row-wise and stores C as 16 bytes per
+//      lane, 256 contiguous bytes per row;
+//   3. for a transposed (or mirrored) output the finals are read back in
+//      accumulator layout, written again as [col][row] and leave the same way.
+// The LDS row pitch is the row plus 8 bytes: 8-byte writes of 16 lanes then
+// cover all banks, and so do the row-wise 8-byte reads of a half-wave.
+//
+// The upper and then the lower 64 rows of the wave's 128x128 sub-tile are
+// taken in turn, in a staging region of 17 KB per wave that only the wave
+// itself touches.  The region then fits beside one k-loop stage, which leaves
+// the other stage free to receive the next tile's first operands while this
+// runs, and no step needs a workgroup barrier (whose memory fence would wait
+// for those loads).
 template <typename Cfg>
 struct HalfTileEpilogue {
   static constexpr int kRows = Cfg::kWaveM / 2;                 // 64
@@ -536,6 +405,12 @@ constexpr int kSchedValu = 0x002, kSchedMfma = 0x008, kSchedVmemRead = 0x020, kS
 __device__ inline void dma_load_16(uint32_t voffset, const uint8_t* base, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voffset), "s"(base), "s"(lds_addr) : "memory");
 }
+// The same with a per-lane 64-bit address.
+__device__ inline void dma_load_16_at(const uint8_t* src, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory");
+}
+template <int kInFlight>
+__device__ inline void wait_for_dma_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kInFlight) : "memory"); }
 __device__ inline void wait_for_dma_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // The 4-byte form: lane l writes LDS bytes [M0 + 4 l, M0 + 4 l + 4).
 __device__ inline void dma_touch_4(uint32_t voffset, const uint8_t* base, uint32_t lds_addr) {

@@ -12,336 +12,16 @@
 // A tall input is its own X^T, so no transpose kernel is needed in either
 // case, and the result lands in the caller's buffer without a copy.
 //
-// GEMM kernels: 256 threads (2x2 wavefronts) on v_mfma_f32_32x32x16_bf16, in
-// two tile configurations (256x256x64 for large problems, 128x128x32 when
-// there are too few tiles to fill the chip) and two bodies: a predicated one
-// for any shape, and a predicate-free, software-pipelined one for problems
-// whose dimensions are multiples of the tile.  Global->register->LDS double
-// buffering with one barrier per k-tile; LDS rows padded by 16 bytes so the
-// 64 lanes of a ds_read_b128 hit distinct banks.
-#include "mfma_tiles.hpp"
+// GEMM kernels: 256 threads (2x2 wavefronts) on v_mfma_f32_32x32x16_bf16,
+// operands global -> LDS directly: 256x256x64 tiles for large problems of
+// whole tiles (below), smaller tiles for everything else (gemm_tiles.hpp).
+#include "gemm_tiles.hpp"
 #include "muon_elementwise.hpp"
+
+#include <cmath>
 
 namespace fsh {
 namespace {
-
-// Tile configuration of one GEMM kernel instantiation.
-//   BM x BN block tile, BK k-tile, WM x WN wavefronts, each wave owns a
-//   (BM/WM) x (BN/WN) sub-tile made of 32x32 MFMA tiles.
-template <int BM_, int BN_, int BK_, int WM_, int WN_>
-struct GemmCfg {
-  static constexpr int BM = BM_, BN = BN_, BK = BK_, WM = WM_, WN = WN_;
-  static constexpr int kThreads = WM * WN * 64;
-  static constexpr int kWaveM = BM / WM, kWaveN = BN / WN;
-  static constexpr int TM = kWaveM / 32, TN = kWaveN / 32;
-  static constexpr int kLdsStride = BK + 8;  // bf16 per LDS row: 16 bytes of padding
-  static constexpr int kStageElems = (BM + BN) * kLdsStride;
-  static constexpr int kLdsBytes = 2 * kStageElems * 2;  // double buffered
-  static constexpr int kChunksPerRow = BK / 8;
-  static constexpr int kChunksA = BM * kChunksPerRow / kThreads;
-  static constexpr int kChunksB = BN * kChunksPerRow / kThreads;
-  static_assert(BM * kChunksPerRow % kThreads == 0 && BN * kChunksPerRow % kThreads == 0, "chunk split");
-};
-
-// Large problems: 256x256x64, four waves of 128x128 (256 fp32 accumulators per
-// lane).  Per 16-wide k step a wave issues 8 ds_read_b128 for 16 MFMAs, so LDS
-// traffic is half of what 64x64 wave tiles need, and a k-tile lasts ~2000
-// cycles, long enough for the next tile's global loads to land.
-using BigCfg = GemmCfg<256, 256, 64, 2, 2>;
-// Small problems (few tiles): 128x128x32, four waves of 64x64.
-using SmallCfg = GemmCfg<128, 128, 32, 2, 2>;
-
-template <typename Cfg>
-__global__ __launch_bounds__(Cfg::kThreads) void gemm_nt_kernel(const GemmParams p) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
-  constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, TM = Cfg::TM, TN = Cfg::TN;
-  constexpr int kLdsStride = Cfg::kLdsStride;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
-  int64_t batch;
-  int tm, tn;
-  if (!tile_of_workgroup(p, blockIdx.x, &batch, &tm, &tn)) return;  // whole workgroup, before any barrier
-  const int64_t m0 = static_cast<int64_t>(tm) * BM;
-  const int64_t n0 = static_cast<int64_t>(tn) * BN;
-
-  const uint16_t* A = p.A + batch * p.sA;
-  const uint16_t* B = p.B + batch * p.sB;
-
-  // Global -> register staging in 16-byte chunks.
-  u32x4 ra[Cfg::kChunksA], rb[Cfg::kChunksB];
-  auto load_global = [&](int64_t k0) {
-#pragma unroll
-    for (int i = 0; i < Cfg::kChunksA; ++i) {
-      const int c = tid + i * Cfg::kThreads;
-      const int64_t row = m0 + c / Cfg::kChunksPerRow, gk = k0 + (c % Cfg::kChunksPerRow) * 8;
-      ra[i] = u32x4{0, 0, 0, 0};
-      if (row < p.M && gk < p.K) ra[i] = *reinterpret_cast<const u32x4*>(A + row * p.lda + gk);
-    }
-#pragma unroll
-    for (int i = 0; i < Cfg::kChunksB; ++i) {
-      const int c = tid + i * Cfg::kThreads;
-      const int64_t row = n0 + c / Cfg::kChunksPerRow, gk = k0 + (c % Cfg::kChunksPerRow) * 8;
-      rb[i] = u32x4{0, 0, 0, 0};
-      if (row < p.N && gk < p.K) rb[i] = *reinterpret_cast<const u32x4*>(B + row * p.ldb + gk);
-    }
-  };
-  auto store_lds = [&](int buf) {
-    uint16_t* base = smem + buf * Cfg::kStageElems;
-#pragma unroll
-    for (int i = 0; i < Cfg::kChunksA; ++i) {
-      const int c = tid + i * Cfg::kThreads;
-      *reinterpret_cast<u32x4*>(&base[(c / Cfg::kChunksPerRow) * kLdsStride + (c % Cfg::kChunksPerRow) * 8]) = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < Cfg::kChunksB; ++i) {
-      const int c = tid + i * Cfg::kThreads;
-      *reinterpret_cast<u32x4*>(&base[(BM + c / Cfg::kChunksPerRow) * kLdsStride + (c % Cfg::kChunksPerRow) * 8]) = rb[i];
-    }
-  };
-
-  // acc[i][j] accumulates (B sub-tile j) x (A sub-tile i)^T, i.e. the
-  // transposed 32x32 block: a lane then owns one output row (m) and runs of
-  // four consecutive columns (n), which makes the epilogue's C stores 8 bytes
-  // wide.
-  f32x16 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-  const int frag_row = lane & 31;
-  const int frag_k = (lane >> 5) * 8;
-  const int64_t ktiles = (p.K + BK - 1) / BK;
-
-  load_global(0);
-  store_lds(0);
-  __syncthreads();
-
-  for (int64_t kt = 0; kt < ktiles; ++kt) {
-    const int buf = static_cast<int>(kt & 1);
-    if (kt + 1 < ktiles) load_global((kt + 1) * BK);
-    const uint16_t* As = smem + buf * Cfg::kStageElems;
-    const uint16_t* Bs = As + BM * kLdsStride;
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      bf16x8 af[TM], bf[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        af[i] = *reinterpret_cast<const bf16x8*>(
-            &As[(wm * Cfg::kWaveM + i * 32 + frag_row) * kLdsStride + ks * 16 + frag_k]);
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        bf[j] = *reinterpret_cast<const bf16x8*>(
-            &Bs[(wn * Cfg::kWaveN + j * 32 + frag_row) * kLdsStride + ks * 16 + frag_k]);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
-    }
-    if (kt + 1 < ktiles) store_lds(buf ^ 1);
-    __syncthreads();
-  }
-
-  // Epilogue.  Accumulator r of block (i, j) belongs to output row
-  // m = lane%32 and column n = 8*(r/4) + 4*(lane/32) + r%4 of the block.
-  const uint16_t* D = p.D ? p.D + batch * p.sD : nullptr;
-  uint16_t* C = p.C + batch * p.sC;
-  // A symmetric product mirrors its off-diagonal tiles into the lower triangle.
-  const bool mirror = p.symmetric && tm != tn;
-  uint16_t* Ct = mirror ? C : (p.Ct ? p.Ct + batch * p.sCt : nullptr);
-  const int64_t ldct = mirror ? p.ldc : p.ldct;
-  const bool c_vec = (p.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(C) & 7) == 0);
-  const bool d_vec = D != nullptr && (p.ldd % 4 == 0) && ((reinterpret_cast<uintptr_t>(D) & 7) == 0);
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int64_t row = m0 + wm * Cfg::kWaveM + i * 32 + (lane & 31);
-    if (row >= p.M) continue;
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int64_t col = n0 + wn * Cfg::kWaveN + j * 32 + 8 * b + 4 * (lane >> 5);
-        if (col >= p.N) continue;
-        const bool full = col + 3 < p.N;
-        float dv[4] = {0.f, 0.f, 0.f, 0.f};
-        if (D != nullptr) {
-          if (full && d_vec) {
-            const u32x2 raw = *reinterpret_cast<const u32x2*>(&D[row * p.ldd + col]);
-            dv[0] = u32_as_f32(raw.x << 16);
-            dv[1] = u32_as_f32(raw.x & 0xFFFF0000u);
-            dv[2] = u32_as_f32(raw.y << 16);
-            dv[3] = u32_as_f32(raw.y & 0xFFFF0000u);
-          } else {
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-              if (col + t < p.N) dv[t] = bf16_bits_to_f32(D[row * p.ldd + col + t]);
-          }
-        }
-        uint32_t packed[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          float v = p.alpha * acc[i][j][4 * b + t];
-          if (D != nullptr) v += p.beta * dv[t];
-          if (row == col + t) v += p.diag_add;
-          packed[t] = f32_to_bf16_bits(v);
-        }
-        if (full && c_vec) {
-          *reinterpret_cast<u32x2*>(&C[row * p.ldc + col]) =
-              u32x2{packed[0] | (packed[1] << 16), packed[2] | (packed[3] << 16)};
-        } else {
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-            if (col + t < p.N) C[row * p.ldc + col + t] = static_cast<uint16_t>(packed[t]);
-        }
-        if (Ct != nullptr) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-            if (col + t < p.N) Ct[(col + t) * ldct + row] = static_cast<uint16_t>(packed[t]);
-        }
-      }
-  }
-}
-
-
-// Interior fast path: M, N multiples of the block tile and K of BK, so there
-// are no predicates, addresses are one per-thread 32-bit offset plus uniform
-// terms, and the k loop is software pipelined by hand.  With 256 accumulators
-// a SIMD holds a single wave, so nothing else hides latency: the fragments of
-// k step s+1 are read from LDS while the MFMAs of step s issue, the next
-// tile's global loads are spread over the first k step, and their LDS writes
-// are interleaved with the MFMAs of the last one.
-template <typename Cfg>
-__global__ __launch_bounds__(Cfg::kThreads) void gemm_nt_interior_kernel(const GemmParams p) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
-  constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, TM = Cfg::TM, TN = Cfg::TN;
-  constexpr int kLdsStride = Cfg::kLdsStride, KS = BK / 16, CPR = Cfg::kChunksPerRow;
-  constexpr int kRowsPerPass = Cfg::kThreads / CPR;  // tile rows covered by one chunk pass
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
-  int64_t batch;
-  int tm, tn;
-  if (!tile_of_workgroup(p, blockIdx.x, &batch, &tm, &tn)) return;  // whole workgroup, before any barrier
-  const int64_t m0 = static_cast<int64_t>(tm) * BM;
-  const int64_t n0 = static_cast<int64_t>(tn) * BN;
-
-  // Uniform tile bases and one per-thread byte offset each for A and B.
-  const uint8_t* Ab = reinterpret_cast<const uint8_t*>(p.A + batch * p.sA + m0 * p.lda);
-  const uint8_t* Bb = reinterpret_cast<const uint8_t*>(p.B + batch * p.sB + n0 * p.ldb);
-  const int trow = tid / CPR, tkc = tid % CPR;
-  const uint32_t a_toff = static_cast<uint32_t>((trow * p.lda + tkc * 8) * 2);
-  const uint32_t b_toff = static_cast<uint32_t>((trow * p.ldb + tkc * 8) * 2);
-  const int64_t a_pass = static_cast<int64_t>(kRowsPerPass) * p.lda * 2;
-  const int64_t b_pass = static_cast<int64_t>(kRowsPerPass) * p.ldb * 2;
-  const int lds_toff = trow * kLdsStride + tkc * 8;  // elements
-
-  u32x4 ra[Cfg::kChunksA], rb[Cfg::kChunksB];
-  auto load_global = [&](int64_t kt) {
-    const int64_t koff = kt * BK * 2;
-#pragma unroll
-    for (int i = 0; i < Cfg::kChunksA; ++i)
-      ra[i] = *reinterpret_cast<const u32x4*>(Ab + (koff + i * a_pass) + a_toff);
-#pragma unroll
-    for (int i = 0; i < Cfg::kChunksB; ++i)
-      rb[i] = *reinterpret_cast<const u32x4*>(Bb + (koff + i * b_pass) + b_toff);
-  };
-  auto store_lds = [&](int buf) {
-    uint16_t* base = smem + buf * Cfg::kStageElems + lds_toff;
-#pragma unroll
-    for (int i = 0; i < Cfg::kChunksA; ++i)
-      *reinterpret_cast<u32x4*>(&base[i * kRowsPerPass * kLdsStride]) = ra[i];
-#pragma unroll
-    for (int i = 0; i < Cfg::kChunksB; ++i)
-      *reinterpret_cast<u32x4*>(&base[(BM + i * kRowsPerPass) * kLdsStride]) = rb[i];
-  };
-
-  f32x16 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-  const int a_frag = (wm * Cfg::kWaveM + (lane & 31)) * kLdsStride + (lane >> 5) * 8;
-  const int b_frag = (BM + wn * Cfg::kWaveN + (lane & 31)) * kLdsStride + (lane >> 5) * 8;
-  bf16x8 af[2][TM], bf[2][TN];
-  auto load_frags = [&](int set, const uint16_t* stage, int ks) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-      af[set][i] = *reinterpret_cast<const bf16x8*>(&stage[a_frag + i * 32 * kLdsStride + ks * 16]);
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-      bf[set][j] = *reinterpret_cast<const bf16x8*>(&stage[b_frag + j * 32 * kLdsStride + ks * 16]);
-  };
-  auto mfma_step = [&](int set) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[set][j], af[set][i], acc[i][j], 0, 0, 0);
-  };
-
-  const int64_t ktiles = p.K / BK;
-  load_global(0);
-  store_lds(0);
-  __syncthreads();
-  load_frags(0, smem, 0);
-
-  constexpr int kMfmaPerStep = TM * TN;
-  constexpr int kFragReads = TM + TN;
-  constexpr int kGlobalLoads = Cfg::kChunksA + Cfg::kChunksB;
-  // One k-tile.  `more` (a compile-time tag) says whether a next tile exists:
-  // the last tile is peeled so that each variant is straight-line code the
-  // scheduling hints can reorder freely.
-  auto k_tile = [&](int64_t kt, auto more_tag) {
-    constexpr bool more = decltype(more_tag)::value;
-    const int buf = static_cast<int>(kt & 1);
-    const uint16_t* stage = smem + buf * Cfg::kStageElems;
-    if (more) load_global(kt + 1);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      if (ks + 1 < KS) load_frags((ks + 1) & 1, stage, ks + 1);
-      if (ks == KS - 1 && more) store_lds(buf ^ 1);
-      mfma_step(ks & 1);
-      if (ks == 0 && more) {
-#pragma unroll
-        for (int g = 0; g < kGlobalLoads; ++g) {
-          __builtin_amdgcn_sched_group_barrier(kSchedVmemRead, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
-          if (g < kFragReads) __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
-        }
-      } else if (ks + 1 < KS) {
-#pragma unroll
-        for (int g = 0; g < kFragReads; ++g) {
-          __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(kSchedMfma, kMfmaPerStep / kFragReads, 0);
-        }
-      } else if (more) {
-#pragma unroll
-        for (int g = 0; g < kGlobalLoads; ++g) {
-          __builtin_amdgcn_sched_group_barrier(kSchedDsWrite, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
-        }
-      }
-    }
-    __syncthreads();
-    if (more) load_frags(0, smem + (buf ^ 1) * Cfg::kStageElems, 0);
-  };
-  for (int64_t kt = 0; kt + 1 < ktiles; ++kt) k_tile(kt, std::true_type{});
-  k_tile(ktiles - 1, std::false_type{});
-
-  store_whole_tile<Cfg>(p, batch, m0, n0, wm, wn, lane, p.symmetric && tm != tn, acc,
-                        reinterpret_cast<uint8_t*>(smem));
-}
 
 // ---------------------------------------------------------------------------
 // Large whole-tile problems: 256x256x64 tiles with global->LDS loads.
@@ -423,7 +103,7 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   auto locate = [&](int64_t id, int& which, int64_t& batch, int& tm, int& tn) -> bool {
     int w = 0;
 #pragma unroll
-    for (int i = 1; i < kMaxGemmProblems; ++i) w += id >= launch.first_workgroup[i] ? 1 : 0;
+    for (int i = 1; i < GemmLaunch::kMaxProblems; ++i) w += id >= launch.first_workgroup[i] ? 1 : 0;
     w = uniform_i32(w);
     int64_t b;
     int r, c;
@@ -772,44 +452,69 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   }
 }
 
-// A validated problem with its kernel chosen and its tile schedule filled in.
-enum GemmKernelKind { kKernelDma, kKernelInteriorBig, kKernelInteriorSmall, kKernelEdgeBig, kKernelEdgeSmall };
+// A validated problem and whether it takes the large-tile kernel.
 struct PlannedGemm {
   GemmParams p;
-  GemmKernelKind kind;
-  int64_t workgroups;
+  int64_t batch;
+  bool large;
 };
 
-template <typename Cfg>
-int plan_gemm_cfg(PlannedGemm* plan, int64_t batch) {
-  GemmParams& p = plan->p;
-  p.tiles_m = static_cast<int32_t>(ceil_div(p.M, Cfg::BM));
-  p.tiles_n = static_cast<int32_t>(ceil_div(p.N, Cfg::BN));
-  const int64_t tiles = p.symmetric ? static_cast<int64_t>(p.tiles_n) * (p.tiles_n + 1) / 2
-                                    : static_cast<int64_t>(p.tiles_m) * p.tiles_n;
-  p.tiles_per_matrix = static_cast<int32_t>(tiles);
-  p.work_items = tiles * batch;
-  p.items_per_xcd = ceil_div(p.work_items, static_cast<int64_t>(kXcds));
-  if (tiles > 0x3FFFFFFFLL || p.items_per_xcd * kXcds > 0x3FFFFFFFLL)
-    return fail(FSH_ENOTSUP, "gemm: too many tiles");
-  plan->workgroups = p.items_per_xcd * kXcds;
-  constexpr bool big = std::is_same<Cfg, BigCfg>::value;
-  // Interior path: whole tiles, 16-byte accesses in the epilogue, 32-bit tile spans.
-  const bool interior =
-      p.M % Cfg::BM == 0 && p.N % Cfg::BN == 0 && p.K % Cfg::BK == 0 && p.ldc % 8 == 0 &&
-      (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && p.sC % 8 == 0 &&
-      (p.Ct == nullptr || (p.ldct % 8 == 0 && (reinterpret_cast<uintptr_t>(p.Ct) & 15) == 0 && p.sCt % 8 == 0)) &&
-      (p.D == nullptr || (p.ldd % 8 == 0 && (reinterpret_cast<uintptr_t>(p.D) & 15) == 0 && p.sD % 8 == 0)) &&
-      static_cast<int64_t>(Cfg::BM) * p.lda * 2 < (1LL << 31) && static_cast<int64_t>(Cfg::BN) * p.ldb * 2 < (1LL << 31);
-  if (interior)
-    plan->kind = big ? kKernelDma : kKernelInteriorSmall;
-  else
-    plan->kind = big ? kKernelEdgeBig : kKernelEdgeSmall;
-  if (p.k_major && plan->kind != kKernelDma)
-    return fail(FSH_ENOTSUP,
-                "gemm: k-major operands need whole 256 x 256 x 64 tiles and at least 192 of them (m %lld, n %lld, "
-                "k %lld, batch %lld)", (long long)p.M, (long long)p.N, (long long)p.K, (long long)batch);
-  return FSH_OK;
+// ---- Which tiles a launch takes.
+// What a launch of these kernels was measured to take, from the number of its
+// tiles (of its longest k; shorter ones count by their share of it) and that
+// k: a start and end of 5 us (10 us with 256 x 256 tiles, whose output is 128
+// KB per workgroup), and per k-tile of 64 what the chip takes for one round of
+// resident workgroups.  A 256 x 256 tile computes four times what a 128 x 128
+// one does in 1.8 (half the chip busy) to 1.6 times its time, and that less
+// and less, since with the whole chip busy the clock falls from 2.3 to 1.6
+// GHz; but it leaves compute units idle in a launch of few tiles, and so do
+// 128 x 128 tiles against 64 x 64 ones.  Measured on 4096^3: 106 us with
+// 256 x 256, 135 with 128 x 128, 202 with 64 x 64 tiles; on 1024^3: 23.5, 12.4
+// and 8.0 us.
+enum TileKind { kTiles64, kTiles128, kTiles256 };
+struct TileWork {
+  double tile_ktiles = 0.0;  // k-tiles of all tiles together
+  double max_ktiles = 0.0;
+  void add(int64_t tiles, int64_t k) {
+    const double kt = static_cast<double>(ceil_div(k, (int64_t)64));
+    tile_ktiles += static_cast<double>(tiles) * kt;
+    if (kt > max_ktiles) max_ktiles = kt;
+  }
+};
+double launch_us(TileKind kind, const TileWork& w) {
+  if (w.tile_ktiles == 0.0) return 0.0;
+  const double n = w.tile_ktiles / w.max_ktiles / 256.0;  // in tiles per compute unit
+  double per_ktile;
+  if (kind == kTiles256) {
+    const double full = floor(n), r = n - full;
+    per_ktile = 1.57 * full + (r == 0.0 ? 0.0 : r <= 0.5 ? 1.13 : 1.13 + 0.88 * (r - 0.5));
+  } else if (kind == kTiles128) {
+    const double full = floor(n / 2), r = n - 2 * full;
+    per_ktile = full + (r == 0.0 ? 0.0 : r <= 1.0 ? 0.62 : 1.0);
+  } else {
+    const double full = floor(n / 3), r = n - 3 * full;
+    per_ktile = 0.59 * full + (r == 0.0 ? 0.0 : r <= 1.0 ? 0.27 : r <= 2.0 ? 0.40 : 0.59);
+  }
+  return (kind == kTiles256 ? 10.0 : 5.0) + per_ktile * w.max_ktiles;
+}
+int64_t count_tiles(int64_t m, int64_t n, bool symmetric, int64_t tile) {
+  const int64_t tn = ceil_div(n, tile);
+  return symmetric ? tn * (tn + 1) / 2 : ceil_div(m, tile) * tn;
+}
+TileKind small_tile_kind(const TileWork& w64, const TileWork& w128) {
+  return launch_us(kTiles64, w64) < launch_us(kTiles128, w128) ? kTiles64 : kTiles128;
+}
+double small_tiles_us(const TileWork& w64, const TileWork& w128) {
+  return fmin(launch_us(kTiles64, w64), launch_us(kTiles128, w128));
+}
+
+// The 256 x 256 kernel takes whole tiles with 16-byte accesses in the epilogue and 32-bit tile spans.
+bool fits_large_tiles(const GemmParams& p) {
+  return p.M % DmaGemm::BM == 0 && p.N % DmaGemm::BN == 0 && p.K % DmaGemm::BK == 0 && p.ldc % 8 == 0 &&
+         (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && p.sC % 8 == 0 &&
+         (p.Ct == nullptr || (p.ldct % 8 == 0 && (reinterpret_cast<uintptr_t>(p.Ct) & 15) == 0 && p.sCt % 8 == 0)) &&
+         (p.D == nullptr || (p.ldd % 8 == 0 && (reinterpret_cast<uintptr_t>(p.D) & 15) == 0 && p.sD % 8 == 0)) &&
+         static_cast<int64_t>(DmaGemm::BM) * p.lda * 2 < (1LL << 31) && static_cast<int64_t>(DmaGemm::BN) * p.ldb * 2 < (1LL << 31);
 }
 
 // The Muon update an epilogue applies instead of storing its product (see
@@ -858,117 +563,190 @@ int plan_gemm(const fsh_gemm_desc& d, PlannedGemm* plan, const GemmUpdate* updat
 #ifdef FSH_TRACE
   if (const char* e = getenv("FSH_GEMM_TRACE")) p.trace = reinterpret_cast<uint64_t*>(strtoull(e, nullptr, 0));
 #endif
-  // The big tile pays off once it fills the chip at least once.
-  const int64_t big_n = ceil_div(d.n, BigCfg::BN);
-  const int64_t big_tiles = (d.symmetric ? big_n * (big_n + 1) / 2 : ceil_div(d.m, BigCfg::BM) * big_n) * d.batch;
-  const int rc = big_tiles >= 192 ? plan_gemm_cfg<BigCfg>(plan, d.batch) : plan_gemm_cfg<SmallCfg>(plan, d.batch);
-  if (rc == FSH_OK && p.update_ptrs != nullptr && plan->kind != kKernelDma)
-    return fail(FSH_ENOTSUP, "gemm: only the large-tile kernel applies a fused update");
-  return rc;
+  plan->batch = d.batch;
+  plan->large = fits_large_tiles(p);  // may take the large-tile kernel; choose_kernels decides whether it does
+  return FSH_OK;
 }
 
-// Whether `d` would run on the large-tile kernel (whose epilogue can apply a fused update).
-bool takes_large_tile_kernel(const fsh_gemm_desc& d) {
-  PlannedGemm plan;
-  return plan_gemm(d, &plan) == FSH_OK && plan.kind == kKernelDma;
-}
 
-template <typename Kernel>
-int launch_single(Kernel kernel, LdsReservation* reserved, int lds_bytes, int threads, const PlannedGemm& plan,
-                  hipStream_t stream, const char* name) {
-  if (int rc = reserve_lds_once(*reserved, kernel, lds_bytes)) return rc;
-  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(plan.workgroups)), dim3(threads), lds_bytes, stream, plan.p);
-  return check_launch(name);
-}
-
-// Launches the planned problems in order.  Runs of problems that take the
-// large-tile kernel share launches (up to kMaxGemmProblems each, longest k
-// first): the short tiles of one problem then fill the partly empty last
-// round of another instead of each launch paying its own tail.  The problems
-// of one call must not depend on each other.
-int launch_planned(PlannedGemm* plans, int count, hipStream_t stream) {
-  static LdsReservation reserved_dma, reserved_persistent, reserved_dma_km, reserved_persistent_km, reserved_small,
-      reserved_edge_big, reserved_edge_small;
-  constexpr int kDmaLds = kDmaGemmLdsBytes;
-  int i = 0;
-  while (i < count) {
-    if (plans[i].kind != kKernelDma) {
-      int rc;
-      if (plans[i].kind == kKernelInteriorSmall)
-        rc = launch_single(&gemm_nt_interior_kernel<SmallCfg>, &reserved_small,
-                           max_int(SmallCfg::kLdsBytes, WholeTileEpilogue<SmallCfg>::kLdsBytes), SmallCfg::kThreads,
-                           plans[i], stream, "gemm_nt_interior_kernel");
-      else if (plans[i].kind == kKernelEdgeBig)
-        rc = launch_single(&gemm_nt_kernel<BigCfg>, &reserved_edge_big, BigCfg::kLdsBytes, BigCfg::kThreads, plans[i],
-                           stream, "gemm_nt_kernel");
-      else
-        rc = launch_single(&gemm_nt_kernel<SmallCfg>, &reserved_edge_small, SmallCfg::kLdsBytes, SmallCfg::kThreads,
-                           plans[i], stream, "gemm_nt_kernel");
-      if (rc) return rc;
-      ++i;
-      continue;
-    }
-    int order[kMaxGemmProblems];
-    int n = 0;
-    int64_t total = 0;
-    const int k_major = plans[i].p.k_major;  // one operand layout per launch
-    while (i < count && n < kMaxGemmProblems && plans[i].kind == kKernelDma && plans[i].p.k_major == k_major &&
-           total + plans[i].workgroups <= 0x3FFFFFFFLL) {
-      total += plans[i].workgroups;
-      order[n++] = i++;
-    }
-    for (int a = 1; a < n; ++a)  // insertion sort, longest k first, stable
-      for (int b = a; b > 0 && plans[order[b]].p.K > plans[order[b - 1]].p.K; --b) {
-        const int t = order[b];
-        order[b] = order[b - 1];
-        order[b - 1] = t;
-      }
-    GemmLaunch launch;
-    memset(&launch, 0, sizeof(launch));
-    int64_t first = 0;
-    for (int k = 0; k < kMaxGemmProblems; ++k) {
-      launch.first_workgroup[k] = k < n ? static_cast<int32_t>(first) : INT32_MAX;
-      if (k < n) {
-        launch.problem[k] = plans[order[k]].p;
-        first += plans[order[k]].workgroups;
-      }
-    }
-    launch.total_workgroups = static_cast<int32_t>(total);
-    // Equally long tiles and more of them than compute units: one resident
-    // workgroup per compute unit walks a static schedule.
-    bool equal_k = true;
-    for (int k = 1; k < n; ++k) equal_k = equal_k && plans[order[k]].p.K == plans[order[0]].p.K;
-    const int64_t units = compute_units();
-    const bool resident = equal_k && units >= kXcds && units % kXcds == 0 && total > units;
-    const dim3 grid(static_cast<uint32_t>(resident ? units : total)), block(DmaGemm::kThreads);
-    if (resident && k_major) {
-      if (int rc = reserve_lds_once(reserved_persistent_km, &gemm_nt_dma_kernel<true, true>, kDmaLds)) return rc;
-      hipLaunchKernelGGL((gemm_nt_dma_kernel<true, true>), grid, block, kDmaLds, stream, launch);
-    } else if (resident) {
-      if (int rc = reserve_lds_once(reserved_persistent, &gemm_nt_dma_kernel<true, false>, kDmaLds)) return rc;
-      hipLaunchKernelGGL((gemm_nt_dma_kernel<true, false>), grid, block, kDmaLds, stream, launch);
-    } else if (k_major) {
-      if (int rc = reserve_lds_once(reserved_dma_km, &gemm_nt_dma_kernel<false, true>, kDmaLds)) return rc;
-      hipLaunchKernelGGL((gemm_nt_dma_kernel<false, true>), grid, block, kDmaLds, stream, launch);
+// Which of the problems that may take the large-tile kernel do: all of them
+// (together they fill its launch) or none, whichever is estimated to take
+// less time with the rest of the call.  Operands given k-major and fused
+// updates exist in the large-tile kernel only.
+int choose_kernels(PlannedGemm* plans, int count) {
+  TileWork large, small64, small128, all64, all128;
+  bool bound = false;
+  for (int i = 0; i < count; ++i) {
+    const GemmParams& p = plans[i].p;
+    const bool must = p.k_major || p.update_ptrs != nullptr;
+    if (must && !plans[i].large)
+      return fail(FSH_ENOTSUP, "gemm: k-major operands and fused updates need whole 256 x 256 x 64 tiles (m %lld, n %lld, k %lld)",
+                  (long long)p.M, (long long)p.N, (long long)p.K);
+    bound = bound || must;
+    const bool sym = p.symmetric != 0;
+    const int64_t n64 = count_tiles(p.M, p.N, sym, 64) * plans[i].batch, n128 = count_tiles(p.M, p.N, sym, 128) * plans[i].batch;
+    all64.add(n64, p.K);
+    all128.add(n128, p.K);
+    if (plans[i].large) {
+      large.add(count_tiles(p.M, p.N, sym, 256) * plans[i].batch, p.K);
     } else {
-      if (int rc = reserve_lds_once(reserved_dma, &gemm_nt_dma_kernel<false, false>, kDmaLds)) return rc;
-      hipLaunchKernelGGL((gemm_nt_dma_kernel<false, false>), grid, block, kDmaLds, stream, launch);
+      small64.add(n64, p.K);
+      small128.add(n128, p.K);
     }
-    if (int rc = check_launch("gemm_nt_dma_kernel")) return rc;
+  }
+  if (!bound && small_tiles_us(all64, all128) <= launch_us(kTiles256, large) + small_tiles_us(small64, small128))
+    for (int i = 0; i < count; ++i) plans[i].large = false;
+  return FSH_OK;
+}
+
+// Fills in a problem's schedule of `tile` x `tile` tiles.
+int schedule_tiles(PlannedGemm* plan, int64_t tile, int64_t* workgroups) {
+  GemmParams& p = plan->p;
+  const int64_t tiles_m = ceil_div(p.M, tile), tiles_n = ceil_div(p.N, tile);
+  const int64_t tiles = count_tiles(p.M, p.N, p.symmetric != 0, tile);
+  p.work_items = tiles * plan->batch;
+  p.items_per_xcd = ceil_div(p.work_items, static_cast<int64_t>(kXcds));
+  if (tiles > 0x3FFFFFFFLL || p.items_per_xcd * kXcds > 0x3FFFFFFFLL) return fail(FSH_ENOTSUP, "gemm: too many tiles");
+  p.tiles_m = static_cast<int32_t>(tiles_m);
+  p.tiles_n = static_cast<int32_t>(tiles_n);
+  p.tiles_per_matrix = static_cast<int32_t>(tiles);
+  *workgroups = p.items_per_xcd * kXcds;
+  return FSH_OK;
+}
+
+// The problems `members` (indices into plans, longest k first) as one launch of `tile` x `tile` tiles.
+template <typename Launch>
+int fill_launch(PlannedGemm* plans, const int* members, int n, int64_t tile, Launch* launch) {
+  memset(launch, 0, sizeof(*launch));
+  int64_t first = 0;
+  for (int k = 0; k < Launch::kMaxProblems; ++k) {
+    launch->first_workgroup[k] = INT32_MAX;
+    if (k >= n) continue;
+    int64_t workgroups = 0;
+    if (int rc = schedule_tiles(&plans[members[k]], tile, &workgroups)) return rc;
+    launch->first_workgroup[k] = static_cast<int32_t>(first);
+    launch->problem[k] = plans[members[k]].p;
+    first += workgroups;
+    if (first > 0x3FFFFFFFLL) return fail(FSH_ENOTSUP, "gemm: too many tiles in one launch");
+  }
+  launch->total_workgroups = static_cast<int32_t>(first);
+  return FSH_OK;
+}
+
+int launch_large_tiles(const GemmLaunch& launch, bool k_major, hipStream_t stream) {
+  static LdsReservation reserved_dma, reserved_persistent, reserved_dma_km, reserved_persistent_km;
+  constexpr int kLds = kDmaGemmLdsBytes;
+  // Equally long tiles and more of them than compute units: one resident
+  // workgroup per compute unit walks a static schedule.
+  bool equal_k = true;
+  for (int k = 1; k < GemmLaunch::kMaxProblems; ++k)
+    equal_k = equal_k && (launch.first_workgroup[k] == INT32_MAX || launch.problem[k].K == launch.problem[0].K);
+  const int64_t units = compute_units(), total = launch.total_workgroups;
+  const bool resident = equal_k && units >= kXcds && units % kXcds == 0 && total > units;
+  const dim3 grid(static_cast<uint32_t>(resident ? units : total)), block(DmaGemm::kThreads);
+  if (resident && k_major) {
+    if (int rc = reserve_lds_once(reserved_persistent_km, &gemm_nt_dma_kernel<true, true>, kLds)) return rc;
+    hipLaunchKernelGGL((gemm_nt_dma_kernel<true, true>), grid, block, kLds, stream, launch);
+  } else if (resident) {
+    if (int rc = reserve_lds_once(reserved_persistent, &gemm_nt_dma_kernel<true, false>, kLds)) return rc;
+    hipLaunchKernelGGL((gemm_nt_dma_kernel<true, false>), grid, block, kLds, stream, launch);
+  } else if (k_major) {
+    if (int rc = reserve_lds_once(reserved_dma_km, &gemm_nt_dma_kernel<false, true>, kLds)) return rc;
+    hipLaunchKernelGGL((gemm_nt_dma_kernel<false, true>), grid, block, kLds, stream, launch);
+  } else {
+    if (int rc = reserve_lds_once(reserved_dma, &gemm_nt_dma_kernel<false, false>, kLds)) return rc;
+    hipLaunchKernelGGL((gemm_nt_dma_kernel<false, false>), grid, block, kLds, stream, launch);
+  }
+  return check_launch("gemm_nt_dma_kernel");
+}
+
+template <typename Cfg, int kBlocksPerUnit>
+int launch_tiles_as(const TileLaunch& launch, hipStream_t stream) {
+  static LdsReservation reserved;
+  if (int rc = reserve_lds_once(reserved, &gemm_nt_tiles_kernel<Cfg, kBlocksPerUnit>, Cfg::kLdsBytes)) return rc;
+  hipLaunchKernelGGL((gemm_nt_tiles_kernel<Cfg, kBlocksPerUnit>), dim3(static_cast<uint32_t>(launch.total_workgroups)),
+                     dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, launch);
+  return check_launch("gemm_nt_tiles_kernel");
+}
+
+// Small tiles: 64 x 64 (three workgroups per compute unit) or 128 x 128 (two;
+// one with its operands requested three k-tiles ahead when the launch has no
+// more tiles than units).
+int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stream) {
+  TileWork w64, w128;
+  for (int k = 0; k < n; ++k) {
+    const PlannedGemm& q = plans[members[k]];
+    w64.add(count_tiles(q.p.M, q.p.N, q.p.symmetric != 0, 64) * q.batch, q.p.K);
+    w128.add(count_tiles(q.p.M, q.p.N, q.p.symmetric != 0, 128) * q.batch, q.p.K);
+  }
+  TileLaunch launch;
+  if (small_tile_kind(w64, w128) == kTiles64) {
+    if (int rc = fill_launch(plans, members, n, 64, &launch)) return rc;
+    return launch_tiles_as<GemmTiles<2, 2, 1, 1, 3>, 3>(launch, stream);
+  }
+  if (int rc = fill_launch(plans, members, n, 128, &launch)) return rc;
+  if (launch.total_workgroups <= compute_units()) return launch_tiles_as<GemmTiles<2, 2, 2, 2, 4>, 1>(launch, stream);
+  return launch_tiles_as<GemmTiles<2, 2, 2, 2, 2>, 2>(launch, stream);
+}
+
+// Launches the planned problems.  Problems that take the same kernel share
+// launches: the short tiles of one problem then fill the partly empty last
+// round of another instead of each launch paying its own start and tail.  The
+// problems of one call must not depend on each other.
+int launch_planned(PlannedGemm* plans, int count, hipStream_t stream) {
+  for (int group = 0; group < 3; ++group) {  // large tiles, large tiles with k-major operands, small tiles
+    const int limit = group < 2 ? GemmLaunch::kMaxProblems : TileLaunch::kMaxProblems;
+    for (int next = 0; next < count;) {
+      int members[TileLaunch::kMaxProblems];
+      int n = 0;
+      for (; next < count && n < limit; ++next)
+        if (plans[next].large == (group < 2) && (group == 2 || plans[next].p.k_major == group)) members[n++] = next;
+      if (n == 0) break;
+      for (int a = 1; a < n; ++a)  // insertion sort, longest k first, stable
+        for (int b = a; b > 0 && plans[members[b]].p.K > plans[members[b - 1]].p.K; --b) {
+          const int t = members[b];
+          members[b] = members[b - 1];
+          members[b - 1] = t;
+        }
+      if (group == 2) {
+        if (int rc = launch_tiles(plans, members, n, stream)) return rc;
+      } else {
+        GemmLaunch launch;
+        if (int rc = fill_launch(plans, members, n, 256, &launch)) return rc;
+        if (int rc = launch_large_tiles(launch, group == 1, stream)) return rc;
+      }
+    }
   }
   return FSH_OK;
 }
 
-int launch_gemms(const fsh_gemm_desc* descs, int count, hipStream_t stream, const GemmUpdate* updates = nullptr) {
+// `large` (null: decided here): the problems that take the large-tile kernel.
+int launch_gemms(const fsh_gemm_desc* descs, int count, hipStream_t stream, const GemmUpdate* updates = nullptr,
+                 const bool* large = nullptr) {
   constexpr int kChunk = 16;
   PlannedGemm plans[kChunk];
   for (int begin = 0; begin < count; begin += kChunk) {
     const int n = count - begin < kChunk ? count - begin : kChunk;
-    for (int i = 0; i < n; ++i)
+    for (int i = 0; i < n; ++i) {
       if (int rc = plan_gemm(descs[begin + i], &plans[i], updates ? &updates[begin + i] : nullptr)) return rc;
+      if (large != nullptr && !large[begin + i]) plans[i].large = false;
+    }
+    if (large == nullptr)
+      if (int rc = choose_kernels(plans, n)) return rc;
     if (int rc = launch_planned(plans, n, stream)) return rc;
   }
   return FSH_OK;
+}
+
+// A caller's k-major product: refused below 192 large tiles, where a
+// transposed copy and the small tiles are faster.
+int check_k_major(const fsh_gemm_desc& d) {
+  if (!d.k_major || d.m <= 0 || d.n <= 0) return FSH_OK;
+  if (count_tiles(d.m, d.n, d.symmetric != 0, 256) * d.batch >= 192 && d.m % 256 == 0 && d.n % 256 == 0 && d.k % 64 == 0)
+    return FSH_OK;
+  return fail(FSH_ENOTSUP,
+              "gemm: k-major operands need whole 256 x 256 x 64 tiles and at least 192 of them (m %lld, n %lld, "
+              "k %lld, batch %lld)", (long long)d.m, (long long)d.n, (long long)d.k, (long long)d.batch);
 }
 
 // ------------------------------------------------------- Frobenius normalize
@@ -1289,12 +1067,15 @@ int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
 
 FSH_API int fsh_gemm_bf16_nt(const fsh_gemm_desc* desc, void* stream) {
   if (desc == nullptr) return fsh::fail(FSH_EINVAL, "fsh_gemm_bf16_nt: null descriptor");
+  if (int rc = fsh::check_k_major(*desc)) return rc;
   return fsh::launch_gemms(desc, 1, static_cast<hipStream_t>(stream));
 }
 
 FSH_API int fsh_gemm_bf16_nt_group(const fsh_gemm_desc* descs, int32_t count, void* stream) {
   if (count < 0 || (count > 0 && descs == nullptr))
     return fsh::fail(FSH_EINVAL, "fsh_gemm_bf16_nt_group: bad descriptor list");
+  for (int i = 0; i < count; ++i)
+    if (int rc = fsh::check_k_major(descs[i])) return rc;
   return fsh::launch_gemms(descs, count, static_cast<hipStream_t>(stream));
 }
 
@@ -1336,9 +1117,38 @@ int64_t ns_partial_offset(int64_t batch, int64_t rows, int64_t cols) {
   return 2 * align256(batch * s * l * 2) + 2 * align256(batch * s * s * 2);
 }
 
+// Which problems run on the large-tile kernel: all that consist of its whole
+// tiles or none, whichever is estimated to take less time over an iteration's
+// three products together with the other problems of the call.
+void ns_choose_large(const fsh_ns_problem* problems, int count, int32_t steps, bool* large) {
+  double with_large_us = 0.0, without_us = 0.0;
+  for (int which = 0; which < 3; ++which) {
+    TileWork w256, small64, small128, all64, all128;
+    for (int i = 0; i < count; ++i) {
+      const fsh_ns_problem& q = problems[i];
+      const int64_t s = q.rows < q.cols ? q.rows : q.cols, l = q.rows < q.cols ? q.cols : q.rows;
+      large[i] = steps > 0 && s > 0 && s % 256 == 0 && l % 256 == 0 && l < (1LL << 22);
+      const int64_t m = which == 2 ? l : s, k = which == 0 ? l : s;
+      const bool sym = which != 2;
+      const int64_t n64 = count_tiles(m, s, sym, 64) * q.batch, n128 = count_tiles(m, s, sym, 128) * q.batch;
+      all64.add(n64, k);
+      all128.add(n128, k);
+      if (large[i]) {
+        w256.add(count_tiles(m, s, sym, 256) * q.batch, k);
+      } else {
+        small64.add(n64, k);
+        small128.add(n128, k);
+      }
+    }
+    with_large_us += launch_us(kTiles256, w256) + small_tiles_us(small64, small128);
+    without_us += small_tiles_us(all64, all128);
+  }
+  for (int i = 0; i < count; ++i) large[i] = large[i] && with_large_us < without_us;
+}
+
 // `partials_ready`: the norm partials of x are in the workspace already (the
 // fused momentum kernel wrote them), so x is not read for its norm.
-int ns_begin(const fsh_ns_problem& q, int32_t steps, float eps, hipStream_t stream, NsState* st,
+int ns_begin(const fsh_ns_problem& q, bool large, float eps, int32_t steps, hipStream_t stream, NsState* st,
              bool partials_ready = false) {
   const int64_t batch = q.batch, rows = q.rows, cols = q.cols;
   if (batch <= 0 || rows <= 0 || cols <= 0)
@@ -1368,12 +1178,11 @@ int ns_begin(const fsh_ns_problem& q, int32_t steps, float eps, hipStream_t stre
   st->G = reinterpret_cast<uint16_t*>(ws + 2 * align256(batch * sl * 2));
   st->P = reinterpret_cast<uint16_t*>(ws + 2 * align256(batch * sl * 2) + align256(batch * ss * 2));
   float* partial = reinterpret_cast<float*>(ws + 2 * align256(batch * sl * 2) + 2 * align256(batch * ss * 2));
-  // With whole 256 x 256 x 64 tiles, and enough of them for the large-tile
-  // kernel, G = X X^T is computed from X^T as it lies (k-major operands), so
+  // On the large-tile kernel G = X X^T is computed from X^T as it lies (k-major operands), so
   // X itself is never written: a tall input alternates between the caller's
   // buffer and one workspace buffer, a wide one between the two workspace
   // buffers and its last step writes X' = P X into the caller's buffer.
-  st->single = steps > 0 && s % 256 == 0 && l % 64 == 0 && (s / 256) * (s / 256 + 1) / 2 * batch >= 192;
+  st->single = large;
   st->X = tall ? w0 : x;
   st->XT[0] = tall ? x : w0;
   st->XT[1] = (st->single && tall) ? w0 : w1;
@@ -1455,13 +1264,15 @@ fsh_gemm_desc ns_product(const NsState& st, int which, float a, float b, float c
 int ns_iterate(NsState* st, int count, float a, float b, float c, int32_t steps, hipStream_t stream,
                const GemmUpdate* last_updates = nullptr) {
   fsh_gemm_desc descs[FSH_MAX_NS_PROBLEMS];
+  bool large[FSH_MAX_NS_PROBLEMS];
+  for (int i = 0; i < count; ++i) large[i] = st[i].single;
   for (int step = 0; step < steps; ++step) {
     // The same product of every problem goes out together: problems are
     // independent of each other, the three products of one are not.
     for (int which = 0; which < 3; ++which) {
       const bool last = step + 1 == steps;
       for (int i = 0; i < count; ++i) descs[i] = ns_product(st[i], which, a, b, c, last);
-      if (int rc = launch_gemms(descs, count, stream, last && which == 2 ? last_updates : nullptr)) return rc;
+      if (int rc = launch_gemms(descs, count, stream, last && which == 2 ? last_updates : nullptr, large)) return rc;
     }
     for (int i = 0; i < count; ++i) st[i].cur ^= 1;
   }
@@ -1482,8 +1293,10 @@ FSH_API int fsh_newton_schulz_multi(const fsh_ns_problem* problems, int32_t coun
   if (steps < 0) return fail(FSH_EINVAL, "fsh_newton_schulz_multi: negative step count %d", steps);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   NsState st[FSH_MAX_NS_PROBLEMS];
+  bool large[FSH_MAX_NS_PROBLEMS];
+  ns_choose_large(problems, count, steps, large);
   for (int i = 0; i < count; ++i)
-    if (int rc = ns_begin(problems[i], steps, eps, stream, &st[i])) return rc;
+    if (int rc = ns_begin(problems[i], large[i], eps, steps, stream, &st[i])) return rc;
   return ns_iterate(st, count, a, b, c, steps, stream);
 }
 
@@ -1554,8 +1367,10 @@ FSH_API int fsh_muon_step(const fsh_muon_group* groups, int32_t count, float ler
     if (int rc = check_launch("muon_prepare_sumsq_kernel")) return rc;
   }
   NsState st[FSH_MAX_NS_PROBLEMS];
+  bool large[FSH_MAX_NS_PROBLEMS];
+  ns_choose_large(problems, count, steps, large);
   for (int i = 0; i < count; ++i)
-    if (int rc = ns_begin(problems[i], steps, eps, stream, &st[i], /*partials_ready=*/true)) return rc;
+    if (int rc = ns_begin(problems[i], large[i], eps, steps, stream, &st[i], /*partials_ready=*/true)) return rc;
   // A group whose last product runs on the large-tile kernel gets its update
   // from that product's epilogue: the direction is never written and read
   // back.  The other groups' directions land in their batch buffers and a
@@ -1563,8 +1378,7 @@ FSH_API int fsh_muon_step(const fsh_muon_group* groups, int32_t count, float ler
   GemmUpdate updates[FSH_MAX_NS_PROBLEMS];
   for (int i = 0; i < count; ++i) {
     // (the epilogue writes bf16 parameters; fp32 masters take the separate launch)
-    const bool fused = steps > 0 && groups[i].master_dtype == FSH_DT_BF16 &&
-                       takes_large_tile_kernel(ns_product(st[i], 2, a, b, c, true));
+    const bool fused = st[i].single && groups[i].master_dtype == FSH_DT_BF16;
     updates[i].ptrs = fused ? groups[i].param_ptrs_dev : nullptr;
     updates[i].decay = decay_factor;
     updates[i].neg_lr = groups[i].neg_adjusted_lr;

@@ -1,0 +1,71 @@
+"""The tile kernels of the bf16 NT product at the sizes where they can go
+wrong: ragged rows and columns, contractions that end inside a k-tile or hold
+fewer k-tiles than the pipeline is deep, every tile size the launch rule
+chooses between, and several problems in one launch."""
+
+import pytest
+import torch
+
+from flex_shard_amd import hip_ops
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # 64 x 64 tiles
+    (1, 1, 1, 8), (1, 64, 64, 64), (1, 65, 63, 72), (2, 130, 257, 136), (1, 129, 127, 520), (3, 33, 300, 248),
+    # 128 x 128 tiles, operands requested three k-tiles ahead (240 tiles)
+    (1, 1920, 1928, 264), (1, 1923, 1837, 392), (1, 1920, 1920, 576),
+    # 128 x 128 tiles, two workgroups per compute unit (640 tiles)
+    (32, 520, 500, 456), (32, 512, 512, 512), (32, 513, 511, 520),
+    # 256 x 256 tiles, resident workgroups
+    (20, 1024, 1280, 1024),
+]
+
+
+def _operands(batch, m, n, k, device, seed):
+    gen = torch.Generator(device=device)
+    gen.manual_seed(seed)
+    a = torch.randn(batch, m, k, generator=gen, device=device).bfloat16()
+    b = torch.randn(batch, n, k, generator=gen, device=device).bfloat16()
+    d = torch.randn(batch, m, n, generator=gen, device=device).bfloat16()
+    return a, b, d
+
+
+def _close(got, ref):
+    # one rounding to bf16 (half an ulp, 2^-9 of the value) of an fp32 sum whose own error, k 2^-24 of the
+    # sum of magnitudes (about k for these operands), stays below 2e-2 up to k = 1024
+    return torch.allclose(got.double(), ref, rtol=2.0**-8, atol=2e-2)
+
+
+@pytest.mark.parametrize("batch,m,n,k", CASES)
+def test_ragged_products_with_addend_and_transposed_output(device, batch, m, n, k):
+    a, b, d = _operands(batch, m, n, k, device, m + n + k)
+    pad = 512
+    bufs = [torch.full((batch * m * n + 2 * pad,), 7.0, dtype=torch.bfloat16, device=device) for _ in range(2)]
+    c, ct = bufs[0][pad:-pad].view(batch, m, n), bufs[1][pad:-pad].view(batch, n, m)
+    hip_ops.gemm_nt(a, b, d=d, alpha=0.5, beta=2.0, out=c, out_t=ct)
+    ref = 0.5 * torch.bmm(a.double(), b.double().transpose(1, 2).contiguous()) + 2.0 * d.double()
+    assert _close(c, ref)
+    assert torch.equal(ct, c.transpose(1, 2).contiguous())
+    for buf in bufs:
+        assert (buf[:pad] == 7).all() and (buf[-pad:] == 7).all()
+
+
+@pytest.mark.parametrize("batch,n,k", [(1, 70, 40), (4, 300, 200), (40, 648, 328), (1, 1928, 136)])
+def test_ragged_symmetric_products_with_a_diagonal_term(device, batch, n, k):
+    a, _, _ = _operands(batch, n, n, k, device, n + k)
+    got = hip_ops.gemm_nt(a, a, symmetric=True, diag_add=1.5)
+    assert torch.equal(got, got.transpose(1, 2).contiguous())
+    ref = torch.bmm(a.double(), a.double().transpose(1, 2).contiguous()) + 1.5 * torch.eye(n, device=device, dtype=torch.float64)
+    assert _close(got, ref)
+    assert torch.equal(got, hip_ops.gemm_nt(a, a, diag_add=1.5))  # the same sums, every tile computed
+
+
+def test_more_problems_than_one_launch_holds(device):
+    problems = []
+    for i in range(11):
+        a, b, _ = _operands(1 + i % 3, 40 + 37 * i, 250 - 19 * i, 8 * (1 + 3 * i), device, i)
+        problems.append({"a": a, "b": b})
+    for q, out in zip(problems, hip_ops.gemm_nt_group(problems)):
+        assert torch.equal(out, hip_ops.gemm_nt(q["a"], q["b"]))
+        assert _close(out, torch.bmm(q["a"].double(), q["b"].double().transpose(1, 2).contiguous()))
