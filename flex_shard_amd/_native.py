@@ -116,11 +116,12 @@ class MuonGroup(Structure):
         ("neg_adjusted_lr", c_float),
         ("direction_scale", c_float),
         ("master_dtype", c_int32),
-        ("reserved", c_int32),
+        ("layout", c_int32),
     ]
 
 
 MAX_NS_PROBLEMS = 16
+MUON_PADDED = 1
 NS_STATIC_SCRATCH_BYTES = 128 << 20
 
 

@@ -16,7 +16,7 @@
 // operands global -> LDS directly: 256x256x64 tiles for large problems of
 // whole tiles (below), smaller tiles for everything else (gemm_tiles.hpp).
 #include "gemm_tiles.hpp"
-#include "muon_elementwise.hpp"
+#include "muon_groups.hpp"
 
 #include <cmath>
 
@@ -749,309 +749,6 @@ int check_k_major(const fsh_gemm_desc& d) {
               "k %lld, batch %lld)", (long long)d.m, (long long)d.n, (long long)d.k, (long long)d.batch);
 }
 
-// ------------------------------------------------------- Frobenius normalize
-constexpr int kNormThreads = 256;
-constexpr int kNormBlocksPerMatrix = 64;
-
-// s plus the squares of the eight bf16 values of v, added one after the
-// other in element order.
-__device__ __forceinline__ float add_squares8(float s, const u32x4 v) {
-  const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float lo = u32_as_f32(d[j] << 16), hi = u32_as_f32(d[j] & 0xFFFF0000u);
-    s += lo * lo;
-    s += hi * hi;
-  }
-  return s;
-}
-// The workgroup's total in a fixed order: lanes by the wave reduction, then
-// the four waves as (0 + 1) + (2 + 3).  All threads call it.
-__device__ __forceinline__ void store_block_partial(float s, float* lds, float* slot) {
-  s = wave_sum_f32(s);
-  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) *slot = (lds[0] + lds[1]) + (lds[2] + lds[3]);
-}
-
-// partial[b][j] = sum of squares of slice j of matrix b in fp32.  The order
-// is fixed: a thread walks its 8-element groups front to back, lanes are
-// folded by the wave reduction, waves left to right.  numel is a multiple of
-// 8 and every matrix starts 16-byte aligned.
-__global__ __launch_bounds__(kNormThreads) void sumsq_partial_kernel(const uint16_t* __restrict__ x,
-                                                                    int64_t numel, float* __restrict__ partial) {
-  __shared__ float lds[kNormThreads / 64];
-  const int64_t b = blockIdx.y;
-  const uint16_t* m = x + b * numel;
-  const int64_t groups = numel / 8;
-  const int64_t per = ceil_div(groups, (int64_t)kNormBlocksPerMatrix);
-  const int64_t begin = blockIdx.x * per;
-  const int64_t end = (begin + per) < groups ? (begin + per) : groups;
-  float s = 0.0f;
-  for (int64_t g = begin + threadIdx.x; g < end; g += kNormThreads) s = add_squares8(s, load_stream_u32x4(m + g * 8));
-  store_block_partial(s, lds, &partial[b * kNormBlocksPerMatrix + blockIdx.x]);
-}
-
-// The momentum step of Muon for a batch of separately allocated matrices,
-// fused with the sum of squares of its output: for matrix b (blockIdx.y)
-//   m = bf16(lerp(m, g, 1 - mu));  u = nesterov ? bf16(lerp(g, m, mu)) : m
-// with u written to slot b of the contiguous batch buffer, and partial[b][j]
-// = the sum of squares of slice j of u.  Slices, the walk of a thread through
-// its slice and the order of the additions are those of sumsq_partial_kernel
-// on the stored u, so the partials are the same bits and the orthogonalization
-// that follows need not read u again to find its norm.
-struct MuonPrepareBatch {
-  const int64_t* momentum_ptrs;  // device table [batch]
-  const int64_t* grad_ptrs;      // device table [batch]
-  uint16_t* out;                 // [batch, numel]
-  float* partial;                // [batch, kNormBlocksPerMatrix]
-  int64_t numel;
-  float one_minus_mu, mu;
-  int32_t nesterov;
-};
-__global__ __launch_bounds__(kNormThreads) void muon_prepare_sumsq_kernel(const MuonPrepareBatch q) {
-  __shared__ float lds[kNormThreads / 64];
-  const int64_t b = blockIdx.y;
-  uint16_t* mom = reinterpret_cast<uint16_t*>(q.momentum_ptrs[b]);
-  const uint16_t* grad = reinterpret_cast<const uint16_t*>(q.grad_ptrs[b]);
-  uint16_t* out = q.out + b * q.numel;
-  const int64_t groups = q.numel / 8;
-  const int64_t per = ceil_div(groups, (int64_t)kNormBlocksPerMatrix);
-  const int64_t begin = blockIdx.x * per;
-  const int64_t end = (begin + per) < groups ? (begin + per) : groups;
-  float s = 0.0f;
-  // Four 16-byte groups per pass, all eight loads issued before the first
-  // store: the tables give the compiler no aliasing information, so a plain
-  // loop would hold every load back behind the previous group's stores.  The
-  // squares are still added group by group in walk order.
-  constexpr int kUnroll = 4;
-  int64_t g = begin + threadIdx.x;
-  for (; g + (kUnroll - 1) * kNormThreads < end; g += kUnroll * kNormThreads) {
-    u32x4 mraw[kUnroll], graw[kUnroll];
-#pragma unroll
-    for (int k = 0; k < kUnroll; ++k) {
-      mraw[k] = load_stream_u32x4(mom + (g + k * kNormThreads) * 8);
-      graw[k] = load_stream_u32x4(grad + (g + k * kNormThreads) * 8);
-    }
-#pragma unroll
-    for (int k = 0; k < kUnroll; ++k) {
-      float mv[8], gv[8];
-      unpack8(mraw[k], mv);
-      unpack8(graw[k], gv);
-      uint32_t mb[8], ob[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) muon_prepare_one(mv[j], gv[j], q.one_minus_mu, q.mu, q.nesterov, &mb[j], &ob[j]);
-      store_stream_u32x4(mom + (g + k * kNormThreads) * 8, pack8(mb));
-      const u32x4 u = pack8(ob);
-      store_stream_u32x4(out + (g + k * kNormThreads) * 8, u);
-      s = add_squares8(s, u);
-    }
-  }
-  for (; g < end; g += kNormThreads) {
-    float mv[8], gv[8];
-    unpack8(load_stream_u32x4(mom + g * 8), mv);
-    unpack8(load_stream_u32x4(grad + g * 8), gv);
-    uint32_t mb[8], ob[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) muon_prepare_one(mv[j], gv[j], q.one_minus_mu, q.mu, q.nesterov, &mb[j], &ob[j]);
-    store_stream_u32x4(mom + g * 8, pack8(mb));
-    const u32x4 u = pack8(ob);
-    store_stream_u32x4(out + g * 8, u);
-    s = add_squares8(s, u);
-  }
-  store_block_partial(s, lds, &q.partial[b * kNormBlocksPerMatrix + blockIdx.x]);
-}
-
-// The same for fp32 master state: momentum buffers and gradients are fp32,
-//   m = lerp(m, g, 1 - mu) (fp32);  u = bf16(nesterov ? lerp(g, m, mu) : m).
-__global__ __launch_bounds__(kNormThreads) void muon_prepare_sumsq_f32_kernel(const MuonPrepareBatch q) {
-  __shared__ float lds[kNormThreads / 64];
-  const int64_t b = blockIdx.y;
-  float* mom = reinterpret_cast<float*>(q.momentum_ptrs[b]);
-  const float* grad = reinterpret_cast<const float*>(q.grad_ptrs[b]);
-  uint16_t* out = q.out + b * q.numel;
-  const int64_t groups = q.numel / 8;
-  const int64_t per = ceil_div(groups, (int64_t)kNormBlocksPerMatrix);
-  const int64_t begin = blockIdx.x * per;
-  const int64_t end = (begin + per) < groups ? (begin + per) : groups;
-  float s = 0.0f;
-  constexpr int kUnroll = 2;  // 2 x (32 + 32) bytes of loads per thread before the first store
-  int64_t g = begin + threadIdx.x;
-  for (; g + (kUnroll - 1) * kNormThreads < end; g += kUnroll * kNormThreads) {
-    float mv[kUnroll][8], gv[kUnroll][8];
-#pragma unroll
-    for (int k = 0; k < kUnroll; ++k) {
-      load8_f32(mom + (g + k * kNormThreads) * 8, mv[k]);
-      load8_f32(grad + (g + k * kNormThreads) * 8, gv[k]);
-    }
-#pragma unroll
-    for (int k = 0; k < kUnroll; ++k) {
-      uint32_t ob[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        muon_prepare_one_f32(mv[k][j], gv[k][j], q.one_minus_mu, q.mu, q.nesterov, &mv[k][j], &ob[j]);
-      store8_f32(mom + (g + k * kNormThreads) * 8, mv[k]);
-      const u32x4 u = pack8(ob);
-      store_stream_u32x4(out + (g + k * kNormThreads) * 8, u);
-      s = add_squares8(s, u);
-    }
-  }
-  for (; g < end; g += kNormThreads) {
-    float mv[8], gv[8];
-    load8_f32(mom + g * 8, mv);
-    load8_f32(grad + g * 8, gv);
-    uint32_t ob[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) muon_prepare_one_f32(mv[j], gv[j], q.one_minus_mu, q.mu, q.nesterov, &mv[j], &ob[j]);
-    store8_f32(mom + g * 8, mv);
-    const u32x4 u = pack8(ob);
-    store_stream_u32x4(out + g * 8, u);
-    s = add_squares8(s, u);
-  }
-  store_block_partial(s, lds, &q.partial[b * kNormBlocksPerMatrix + blockIdx.x]);
-}
-
-// The update of Muon for the same batch: parameter b (a separate allocation)
-// takes the direction in slot b of the batch buffer,
-//   p = bf16(p * decay);  p = bf16(p + neg_lr * d)   (d first scaled and rounded if scale != 1).
-struct MuonApplyBatch {
-  const int64_t* param_ptrs;  // device table [batch]
-  const uint16_t* direction;  // [batch, numel]
-  int64_t numel;
-  float decay, neg_lr, dir_scale;
-};
-__global__ __launch_bounds__(kNormThreads) void muon_apply_batch_kernel(const MuonApplyBatch q) {
-  const int64_t b = blockIdx.y;
-  uint16_t* param = reinterpret_cast<uint16_t*>(q.param_ptrs[b]);
-  const uint16_t* dir = q.direction + b * q.numel;
-  const int64_t groups = q.numel / 8;
-  // A block owns runs of four consecutive 4 KiB pieces; a thread's four
-  // loads of the parameter and of the direction go out before its stores.
-  constexpr int kUnroll = 4;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kNormThreads * kUnroll;
-  for (int64_t g0 = static_cast<int64_t>(blockIdx.x) * kNormThreads * kUnroll + threadIdx.x; g0 < groups; g0 += stride) {
-    u32x4 praw[kUnroll], draw[kUnroll];
-#pragma unroll
-    for (int k = 0; k < kUnroll; ++k) {
-      const int64_t g = g0 + k * kNormThreads;
-      if (g < groups) {
-        praw[k] = load_stream_u32x4(param + g * 8);
-        draw[k] = load_stream_u32x4(dir + g * 8);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kUnroll; ++k) {
-      const int64_t g = g0 + k * kNormThreads;
-      if (g < groups) {
-        float pv[8], dv[8];
-        unpack8(praw[k], pv);
-        unpack8(draw[k], dv);
-        uint32_t pb[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pb[j] = muon_apply_one(pv[j], dv[j], q.decay, q.neg_lr, q.dir_scale);
-        store_stream_u32x4(param + g * 8, pack8(pb));
-      }
-    }
-  }
-}
-
-// The update on fp32 parameters: p = p * decay; p = p + neg_lr * d, d the bf16
-// direction (times scale in fp32 if scale != 1).
-__global__ __launch_bounds__(kNormThreads) void muon_apply_batch_f32_kernel(const MuonApplyBatch q) {
-  const int64_t b = blockIdx.y;
-  float* param = reinterpret_cast<float*>(q.param_ptrs[b]);
-  const uint16_t* dir = q.direction + b * q.numel;
-  const int64_t groups = q.numel / 8;
-  constexpr int kUnroll = 2;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kNormThreads * kUnroll;
-  for (int64_t g0 = static_cast<int64_t>(blockIdx.x) * kNormThreads * kUnroll + threadIdx.x; g0 < groups; g0 += stride) {
-    float pv[kUnroll][8];
-    u32x4 draw[kUnroll];
-#pragma unroll
-    for (int k = 0; k < kUnroll; ++k) {
-      const int64_t g = g0 + k * kNormThreads;
-      if (g < groups) {
-        load8_f32(param + g * 8, pv[k]);
-        draw[k] = load_stream_u32x4(dir + g * 8);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kUnroll; ++k) {
-      const int64_t g = g0 + k * kNormThreads;
-      if (g < groups) {
-        float dv[8];
-        unpack8(draw[k], dv);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pv[k][j] = muon_apply_one_f32(pv[k][j], dv[j], q.decay, q.neg_lr, q.dir_scale);
-        store8_f32(param + g * 8, pv[k]);
-      }
-    }
-  }
-}
-
-// Reads matrix b of `in` ([rows, cols]), divides by max(||.||_F, eps) as bf16
-// tensor ops would (norm rounded to bf16, fp32 division, bf16 result), and
-// writes the result to `out_same` ([rows, cols]) and `out_t` ([cols, rows]);
-// either output may be null.
-// A workgroup owns a 64x64 tile: 16-byte loads and stores of 8 elements along
-// the rows, and for the transposed copy the tile goes through LDS and leaves
-// as 16-byte stores of 8 elements along the columns.  rows and cols are
-// multiples of 8, so an 8-element group is either whole or absent.
-constexpr int kNormTile = 64;
-constexpr int kNormPitch = kNormTile + 2;  // u16 per LDS row
-__global__ __launch_bounds__(kNormThreads) void normalize_dual_kernel(const uint16_t* __restrict__ in,
-                                                                     uint16_t* __restrict__ out_same,
-                                                                     uint16_t* __restrict__ out_t, int64_t rows,
-                                                                     int64_t cols, const float* __restrict__ partial,
-                                                                     float eps_bf16) {
-  __shared__ uint16_t tile[kNormTile * kNormPitch];
-  const int64_t b = blockIdx.z;
-  float total = 0.0f;
-  for (int j = 0; j < kNormBlocksPerMatrix; ++j) total += partial[b * kNormBlocksPerMatrix + j];
-  float norm = bf16_bits_to_f32(f32_to_bf16_bits(sqrtf(total)));
-  norm = norm < eps_bf16 ? eps_bf16 : norm;
-  const int64_t r0 = static_cast<int64_t>(blockIdx.y) * kNormTile, c0 = static_cast<int64_t>(blockIdx.x) * kNormTile;
-  const uint16_t* m = in + b * rows * cols;
-  uint16_t* o = out_same ? out_same + b * rows * cols : nullptr;
-  uint16_t* ot = out_t ? out_t + b * rows * cols : nullptr;
-  const int q = threadIdx.x & 7, line = threadIdx.x >> 3;  // 8 groups of 8 elements per line, 32 lines per pass
-#pragma unroll
-  for (int pass = 0; pass < 2; ++pass) {
-    const int lr = line + 32 * pass;
-    const int64_t r = r0 + lr, c = c0 + 8 * q;
-    if (r < rows && c < cols) {
-      const u32x4 v = load_stream_u32x4(m + r * cols + c);
-      const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-      uint32_t bits[8];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        bits[2 * j] = f32_to_bf16_bits(u32_as_f32(d[j] << 16) / norm);
-        bits[2 * j + 1] = f32_to_bf16_bits(u32_as_f32(d[j] & 0xFFFF0000u) / norm);
-      }
-      if (o != nullptr)
-        store_stream_u32x4(o + r * cols + c, u32x4{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16),
-                                                     bits[4] | (bits[5] << 16), bits[6] | (bits[7] << 16)});
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        *reinterpret_cast<uint32_t*>(&tile[lr * kNormPitch + 8 * q + 2 * j]) = bits[2 * j] | (bits[2 * j + 1] << 16);
-    }
-  }
-  if (ot == nullptr) return;  // the same for the whole workgroup
-  __syncthreads();
-#pragma unroll
-  for (int pass = 0; pass < 2; ++pass) {
-    const int lc = line + 32 * pass;  // tile column = row of the transposed output
-    const int64_t c = c0 + lc, r = r0 + 8 * q;
-    if (c < cols && r < rows) {
-      uint32_t bits[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) bits[j] = tile[(8 * q + j) * kNormPitch + lc];
-      store_stream_u32x4(ot + c * rows + r, u32x4{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16),
-                                                    bits[4] | (bits[5] << 16), bits[6] | (bits[7] << 16)});
-    }
-  }
-}
-
 float bf16_round_host(float f) {
   uint32_t u;
   memcpy(&u, &f, 4);
@@ -1084,13 +781,13 @@ FSH_API int fsh_gemm_bf16_nt_group(const fsh_gemm_desc* descs, int32_t count, vo
 //   second X^T buffer                [batch, s*l] bf16
 //   G                                [batch, s*s] bf16
 //   P                                [batch, s*s] bf16
-//   norm partials                    [batch, 64] fp32
+//   norm partials                    [batch, slices_of(s*l / 8)] fp32
 FSH_API int64_t fsh_newton_schulz_workspace_bytes(int64_t batch, int64_t rows, int64_t cols) {
   using namespace fsh;
   if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
   const int64_t s = rows < cols ? rows : cols, l = rows < cols ? cols : rows;
   return 2 * align256(batch * s * l * 2) + 2 * align256(batch * s * s * 2) +
-         align256(batch * kNormBlocksPerMatrix * 4);
+         align256(batch * slices_of(ceil_div(s * l, (int64_t)8)) * 4);
 }
 
 namespace fsh {
@@ -1146,10 +843,9 @@ void ns_choose_large(const fsh_ns_problem* problems, int count, int32_t steps, b
   for (int i = 0; i < count; ++i) large[i] = large[i] && with_large_us < without_us;
 }
 
-// `partials_ready`: the norm partials of x are in the workspace already (the
-// fused momentum kernel wrote them), so x is not read for its norm.
-int ns_begin(const fsh_ns_problem& q, bool large, float eps, int32_t steps, hipStream_t stream, NsState* st,
-             bool partials_ready = false) {
+// Checks a problem and lays out its buffers; `normalize` receives its part of
+// the normalization launch.
+int ns_begin(const fsh_ns_problem& q, bool large, int32_t steps, NsState* st, NormalizeGroup* normalize) {
   const int64_t batch = q.batch, rows = q.rows, cols = q.cols;
   if (batch <= 0 || rows <= 0 || cols <= 0)
     return fail(FSH_EINVAL, "newton_schulz: bad sizes (batch %lld, rows %lld, cols %lld)", (long long)batch,
@@ -1189,22 +885,52 @@ int ns_begin(const fsh_ns_problem& q, bool large, float eps, int32_t steps, hipS
   st->cur = steps & 1;
   st->tall = tall;
 
-  if (!partials_ready) {
-    hipLaunchKernelGGL(sumsq_partial_kernel, dim3(kNormBlocksPerMatrix, static_cast<uint32_t>(batch)),
-                       dim3(kNormThreads), 0, stream, x, rows * cols, partial);
-    if (int rc = check_launch("sumsq_partial_kernel")) return rc;
-  }
   // Input is [rows, cols]; "same orientation" output is X for a wide input
   // and X^T for a tall one.
   uint16_t* same = tall ? st->XT[st->cur] : st->X;
   uint16_t* transposed = tall ? st->X : st->XT[st->cur];
   if (st->single) (tall ? transposed : same) = nullptr;
-  const dim3 grid(static_cast<uint32_t>(ceil_div(cols, (int64_t)kNormTile)),
-                  static_cast<uint32_t>(ceil_div(rows, (int64_t)kNormTile)), static_cast<uint32_t>(batch));
-  if (grid.y > 65535) return fail(FSH_ENOTSUP, "newton_schulz: more than %d row tiles", 65535 * kNormTile);
-  hipLaunchKernelGGL(normalize_dual_kernel, grid, dim3(kNormThreads), 0, stream, x, same, transposed, rows, cols,
-                     partial, bf16_round_host(eps));
-  return check_launch("normalize_dual_kernel");
+  normalize->in = x;
+  normalize->out_same = same;
+  normalize->out_t = transposed;
+  normalize->partial = partial;
+  normalize->rows = rows;
+  normalize->cols = cols;
+  normalize->tiles_c = ceil_div(cols, (int64_t)kNormTile);
+  normalize->tiles = normalize->tiles_c * ceil_div(rows, (int64_t)kNormTile);
+  normalize->slices = static_cast<int32_t>(slices_of(rows * cols / 8));
+  return FSH_OK;
+}
+
+// Gives every group its block range: `blocks` per matrix of the group, `batch` matrices.
+template <typename Group>
+int add_blocks(Group* group, int64_t blocks, int64_t batch, int64_t* total) {
+  group->first_block = static_cast<int32_t>(*total);
+  *total += blocks * batch;
+  if (*total >= INT32_MAX) return fail(FSH_ENOTSUP, "newton_schulz: more than %d blocks in one launch", INT32_MAX);
+  return FSH_OK;
+}
+
+int launch_normalize(NormalizeLaunch& launch, const NsState* st, int count, float eps, hipStream_t stream) {
+  int64_t blocks = 0;
+  for (int i = 0; i < count; ++i)
+    if (int rc = add_blocks(&launch.group[i], launch.group[i].tiles, st[i].batch, &blocks)) return rc;
+  for (int i = count; i < kMaxMuonGroups; ++i) launch.group[i].first_block = INT32_MAX;
+  launch.eps_bf16 = bf16_round_host(eps);
+  hipLaunchKernelGGL(normalize_groups_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kNormThreads), 0, stream, launch);
+  return check_launch("normalize_groups_kernel");
+}
+
+// One block per slice of every matrix of the groups for which `take` holds.
+// Returns the number of blocks, or a negative error.
+template <typename Take>
+int64_t assign_slices(MuonLaunch& launch, const int64_t* batch, int count, Take take) {
+  int64_t blocks = 0;
+  // (groups left out get an empty range)
+  for (int i = 0; i < count; ++i)
+    if (int rc = add_blocks(&launch.group[i], take(i) ? launch.group[i].slices : 0, batch[i], &blocks)) return rc;
+  for (int i = count; i < kMaxMuonGroups; ++i) launch.group[i].first_block = INT32_MAX;
+  return blocks;
 }
 
 // The three products of one iteration; `which` = 0: G = X X^T, 1: P = a I +
@@ -1292,11 +1018,28 @@ FSH_API int fsh_newton_schulz_multi(const fsh_ns_problem* problems, int32_t coun
                 FSH_MAX_NS_PROBLEMS);
   if (steps < 0) return fail(FSH_EINVAL, "fsh_newton_schulz_multi: negative step count %d", steps);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
+  if (count == 0) return FSH_OK;
   NsState st[FSH_MAX_NS_PROBLEMS];
   bool large[FSH_MAX_NS_PROBLEMS];
   ns_choose_large(problems, count, steps, large);
-  for (int i = 0; i < count; ++i)
-    if (int rc = ns_begin(problems[i], large[i], eps, steps, stream, &st[i])) return rc;
+  NormalizeLaunch normalize;
+  MuonLaunch sums;
+  memset(&sums, 0, sizeof(sums));
+  int64_t batch[FSH_MAX_NS_PROBLEMS];
+  for (int i = 0; i < count; ++i) {
+    if (int rc = ns_begin(problems[i], large[i], steps, &st[i], &normalize.group[i])) return rc;
+    batch[i] = problems[i].batch;
+    MuonGroupDev& g = sums.group[i];
+    g.batch = static_cast<uint16_t*>(problems[i].x_dev);
+    g.partial = const_cast<float*>(normalize.group[i].partial);
+    g.vectors = problems[i].rows * problems[i].cols / 8;
+    g.slices = normalize.group[i].slices;
+  }
+  const int64_t blocks = assign_slices(sums, batch, count, [](int) { return true; });
+  if (blocks < 0) return static_cast<int>(blocks);
+  hipLaunchKernelGGL(sumsq_groups_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kNormThreads), 0, stream, sums);
+  if (int rc = check_launch("sumsq_groups_kernel")) return rc;
+  if (int rc = launch_normalize(normalize, st, count, eps, stream)) return rc;
   return ns_iterate(st, count, a, b, c, steps, stream);
 }
 
@@ -1326,9 +1069,11 @@ FSH_API int fsh_muon_step(const fsh_muon_group* groups, int32_t count, float ler
   fsh_ns_problem problems[FSH_MAX_NS_PROBLEMS];
   for (int i = 0; i < count; ++i) {
     const fsh_muon_group& g = groups[i];
-    if (g.batch <= 0 || g.batch > 65535 || g.rows <= 0 || g.cols <= 0 || g.rows % 8 || g.cols % 8)
+    if (g.batch <= 0 || g.batch > 65535 || g.rows <= 0 || g.cols <= 0 ||
+        ((g.rows % 8 || g.cols % 8) && g.layout != FSH_MUON_PADDED))
       return fail(FSH_EINVAL, "fsh_muon_step: group %d has bad sizes (batch %lld, rows %lld, cols %lld; rows and cols "
-                  "must be multiples of 8)", i, (long long)g.batch, (long long)g.rows, (long long)g.cols);
+                  "must be multiples of 8 unless the layout is FSH_MUON_PADDED)", i, (long long)g.batch, (long long)g.rows,
+                  (long long)g.cols);
     if (!g.param_ptrs_dev || !g.grad_ptrs_dev || !g.momentum_ptrs_dev || !g.batch_dev || !g.workspace_dev)
       return fail(FSH_EINVAL, "fsh_muon_step: group %d has a null pointer", i);
     if (!aligned(g.batch_dev, 16) || !aligned(g.workspace_dev, 256))
@@ -1336,41 +1081,56 @@ FSH_API int fsh_muon_step(const fsh_muon_group* groups, int32_t count, float ler
     if (g.master_dtype != FSH_DT_BF16 && g.master_dtype != FSH_DT_F32)
       return fail(FSH_EINVAL, "fsh_muon_step: group %d: master_dtype %d is neither FSH_DT_BF16 nor FSH_DT_F32", i,
                   g.master_dtype);
-    if (g.workspace_nbytes < fsh_newton_schulz_workspace_bytes(g.batch, g.rows, g.cols))
+    if (g.layout != 0 && g.layout != FSH_MUON_PADDED)
+      return fail(FSH_EINVAL, "fsh_muon_step: group %d: unknown layout %d", i, g.layout);
+    const int64_t rows = ceil_div(g.rows, (int64_t)8) * 8, cols = ceil_div(g.cols, (int64_t)8) * 8;
+    if (g.workspace_nbytes < fsh_newton_schulz_workspace_bytes(g.batch, rows, cols))
       return fail(FSH_EINVAL, "fsh_muon_step: group %d: workspace of %lld bytes, need %lld", i,
-                  (long long)g.workspace_nbytes, (long long)fsh_newton_schulz_workspace_bytes(g.batch, g.rows, g.cols));
+                  (long long)g.workspace_nbytes, (long long)fsh_newton_schulz_workspace_bytes(g.batch, rows, cols));
     problems[i].x_dev = g.batch_dev;
     problems[i].batch = g.batch;
-    problems[i].rows = g.rows;
-    problems[i].cols = g.cols;
+    problems[i].rows = rows;
+    problems[i].cols = cols;
     problems[i].workspace_dev = g.workspace_dev;
     problems[i].workspace_nbytes = g.workspace_nbytes;
   }
-  for (int i = 0; i < count; ++i) {
-    const fsh_muon_group& g = groups[i];
-    MuonPrepareBatch q;
-    q.momentum_ptrs = g.momentum_ptrs_dev;
-    q.grad_ptrs = g.grad_ptrs_dev;
-    q.out = static_cast<uint16_t*>(g.batch_dev);
-    q.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(g.workspace_dev) +
-                                         ns_partial_offset(g.batch, g.rows, g.cols));
-    q.numel = g.rows * g.cols;
-    q.one_minus_mu = lerp_weight;
-    q.mu = nesterov_weight;
-    q.nesterov = nesterov;
-    if (g.master_dtype == FSH_DT_F32)
-      hipLaunchKernelGGL(muon_prepare_sumsq_f32_kernel, dim3(kNormBlocksPerMatrix, static_cast<uint32_t>(g.batch)),
-                         dim3(kNormThreads), 0, stream, q);
-    else
-      hipLaunchKernelGGL(muon_prepare_sumsq_kernel, dim3(kNormBlocksPerMatrix, static_cast<uint32_t>(g.batch)),
-                         dim3(kNormThreads), 0, stream, q);
-    if (int rc = check_launch("muon_prepare_sumsq_kernel")) return rc;
-  }
+  if (count == 0) return FSH_OK;
   NsState st[FSH_MAX_NS_PROBLEMS];
   bool large[FSH_MAX_NS_PROBLEMS];
   ns_choose_large(problems, count, steps, large);
-  for (int i = 0; i < count; ++i)
-    if (int rc = ns_begin(problems[i], large[i], eps, steps, stream, &st[i], /*partials_ready=*/true)) return rc;
+  NormalizeLaunch normalize;
+  MuonLaunch launch;
+  memset(&launch, 0, sizeof(launch));
+  launch.one_minus_mu = lerp_weight;
+  launch.mu = nesterov_weight;
+  launch.nesterov = nesterov;
+  launch.decay = decay_factor;
+  int64_t batch[FSH_MAX_NS_PROBLEMS];
+  for (int i = 0; i < count; ++i) {
+    if (int rc = ns_begin(problems[i], large[i], steps, &st[i], &normalize.group[i])) return rc;
+    const fsh_muon_group& g = groups[i];
+    batch[i] = g.batch;
+    MuonGroupDev& q = launch.group[i];
+    q.param_ptrs = g.param_ptrs_dev;
+    q.momentum_ptrs = g.momentum_ptrs_dev;
+    q.grad_ptrs = g.grad_ptrs_dev;
+    q.batch = static_cast<uint16_t*>(g.batch_dev);
+    q.partial = const_cast<float*>(normalize.group[i].partial);
+    q.vectors = problems[i].rows * problems[i].cols / 8;
+    q.rows = g.rows;
+    q.cols = g.cols;
+    q.row_vectors = problems[i].cols / 8;
+    q.slices = normalize.group[i].slices;
+    q.f32 = g.master_dtype == FSH_DT_F32 ? 1 : 0;
+    q.padded = g.rows % 8 || g.cols % 8 ? 1 : 0;
+    q.neg_lr = g.neg_adjusted_lr;
+    q.dir_scale = g.direction_scale;
+  }
+  int64_t blocks = assign_slices(launch, batch, count, [](int) { return true; });
+  if (blocks < 0) return static_cast<int>(blocks);
+  hipLaunchKernelGGL(muon_prepare_groups_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kNormThreads), 0, stream, launch);
+  if (int rc = check_launch("muon_prepare_groups_kernel")) return rc;
+  if (int rc = launch_normalize(normalize, st, count, eps, stream)) return rc;
   // A group whose last product runs on the large-tile kernel gets its update
   // from that product's epilogue: the direction is never written and read
   // back.  The other groups' directions land in their batch buffers and a
@@ -1385,27 +1145,11 @@ FSH_API int fsh_muon_step(const fsh_muon_group* groups, int32_t count, float ler
     updates[i].dir_scale = groups[i].direction_scale;
   }
   if (int rc = ns_iterate(st, count, a, b, c, steps, stream, updates)) return rc;
-  for (int i = 0; i < count; ++i) {
-    if (updates[i].ptrs != nullptr) continue;
-    const fsh_muon_group& g = groups[i];
-    MuonApplyBatch q;
-    q.param_ptrs = g.param_ptrs_dev;
-    q.direction = static_cast<const uint16_t*>(g.batch_dev);
-    q.numel = g.rows * g.cols;
-    q.decay = decay_factor;
-    q.neg_lr = g.neg_adjusted_lr;
-    q.dir_scale = g.direction_scale;
-    const int64_t groups8 = q.numel / 8;
-    const int64_t blocks = ceil_div(groups8, (int64_t)kNormThreads * 4);  // four 16-byte groups per thread
-    const dim3 grid(static_cast<uint32_t>(blocks < 1 ? 1 : (blocks > 4096 ? 4096 : blocks)),
-                    static_cast<uint32_t>(g.batch));
-    if (g.master_dtype == FSH_DT_F32)
-      hipLaunchKernelGGL(muon_apply_batch_f32_kernel, grid, dim3(kNormThreads), 0, stream, q);
-    else
-      hipLaunchKernelGGL(muon_apply_batch_kernel, grid, dim3(kNormThreads), 0, stream, q);
-    if (int rc = check_launch("muon_apply_batch_kernel")) return rc;
-  }
-  return FSH_OK;
+  blocks = assign_slices(launch, batch, count, [&](int i) { return updates[i].ptrs == nullptr; });
+  if (blocks < 0) return static_cast<int>(blocks);
+  if (blocks == 0) return FSH_OK;
+  hipLaunchKernelGGL(muon_apply_groups_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kNormThreads), 0, stream, launch);
+  return check_launch("muon_apply_groups_kernel");
 }
 
 // ------------------------------------------------------------------------
@@ -1418,7 +1162,10 @@ FSH_API int fsh_muon_step(const fsh_muon_group* groups, int32_t count, float ler
 namespace fsh {
 namespace {
 
-static __device__ __align__(256) uint8_t scratch[FSH_NS_STATIC_SCRATCH_BYTES];
+// The norm partials of a batch that otherwise fills the scratch: 4 bytes per
+// 8192 elements or per matrix, and at most a quarter of the bytes are elements.
+constexpr int64_t kScratchPartials = 1 << 20;
+static __device__ __align__(256) uint8_t scratch[FSH_NS_STATIC_SCRATCH_BYTES + kScratchPartials];
 
 constexpr int kMaxDevices = 64;
 std::atomic<void*> g_scratch_ptr[kMaxDevices];
@@ -1458,8 +1205,9 @@ FSH_API int fsh_newton_schulz_noalloc(void* x_dev, int64_t batch, int64_t rows, 
                 "fsh_newton_schulz_noalloc: batch %lld of %lld x %lld exceeds the %lld-byte static scratch; call "
                 "fsh_newton_schulz with a workspace of fsh_newton_schulz_workspace_bytes()",
                 (long long)batch, (long long)rows, (long long)cols, (long long)FSH_NS_STATIC_SCRATCH_BYTES);
-  const int64_t need = fsh_newton_schulz_workspace_bytes(batch, rows, cols);
-  if (need > FSH_NS_STATIC_SCRATCH_BYTES)
+  // (everything but the norm partials, which have room of their own behind the advertised size)
+  const int64_t need = ns_partial_offset(batch, rows, cols) + align256(batch * 64 * 4);
+  if (need > FSH_NS_STATIC_SCRATCH_BYTES || fsh_newton_schulz_workspace_bytes(batch, rows, cols) > FSH_NS_STATIC_SCRATCH_BYTES + kScratchPartials)
     return fail(FSH_ENOTSUP,
                 "fsh_newton_schulz_noalloc: batch %lld of %lld x %lld needs %lld bytes of scratch, the static scratch "
                 "holds %lld; call fsh_newton_schulz with a workspace of that size",
@@ -1470,6 +1218,7 @@ FSH_API int fsh_newton_schulz_noalloc(void* x_dev, int64_t batch, int64_t rows, 
   // Every region of the workspace is written before it is read (norm
   // partials, both iterate buffers, G and P), so nothing has to be cleared
   // between calls.
-  return fsh_newton_schulz(x_dev, batch, rows, cols, a, b, c, steps, eps, ptr, FSH_NS_STATIC_SCRATCH_BYTES, stream_);
+  return fsh_newton_schulz(x_dev, batch, rows, cols, a, b, c, steps, eps, ptr,
+                           FSH_NS_STATIC_SCRATCH_BYTES + kScratchPartials, stream_);
 }
 

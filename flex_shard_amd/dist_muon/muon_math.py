@@ -194,30 +194,30 @@ class OwnedMuon:
         self._stacked = any(p.ndim > 2 for p in self.params)
         self._matrices = self._as_matrices(self.params)
         self._momentum_matrices = self._as_matrices(self.momentum_buffers)
-        # Matrices of one shape and dtype are orthogonalized as one batch; the step's
-        # launch tables (address tables, batch buffers, workspaces) are built once.
+        # Matrices of one shape and dtype are orthogonalized as one batch (of matrices
+        # padded to whole 16-byte rows where rows or columns are not multiples of 8);
+        # the step's launch tables (address tables, batch buffers, workspaces) are built once.
         self._groups: dict[tuple[int, int, torch.dtype], list[int]] = {}  # (rows, cols, dtype) -> matrix indices
-        # Matrices whose rows or columns are not multiples of 8 (the batched
-        # step's 16-byte rows) take the per-matrix kernels, padded inside
-        # the orthogonalization.
-        self._odd: list[int] = []
         for index, m in enumerate(self._matrices):
-            if m.shape[0] % 8 or m.shape[1] % 8:
-                self._odd.append(index)
-            else:
-                self._groups.setdefault((*m.shape, m.dtype), []).append(index)
-        self._plan = None
-        if self._groups:
-            self._plan = hip_ops.MuonStepPlan(
+            self._groups.setdefault((*m.shape, m.dtype), []).append(index)
+        # One C call takes a bounded number of shape groups: as many plans as that needs.
+        self._plans: list[tuple[list[tuple], hip_ops.MuonStepPlan]] = []
+        self._batch: dict[tuple, torch.Tensor] = {}
+        self._workspace: dict[tuple, torch.Tensor] = {}
+        keys = list(self._groups)
+        for begin in range(0, len(keys), hip_ops.MuonStepPlan.MAX_GROUPS):
+            chunk = keys[begin : begin + hip_ops.MuonStepPlan.MAX_GROUPS]
+            plan = hip_ops.MuonStepPlan(
                 [
                     # whole parameters are their own learning-rate reference shape: direction scale 1
-                    (key[:2], len(members), -_adjust_muon_learning_rate(lr, adjust_lr_fn, key[:2]), 1.0, key[2])
-                    for key, members in self._groups.items()
+                    (key[:2], len(self._groups[key]), -_adjust_muon_learning_rate(lr, adjust_lr_fn, key[:2]), 1.0, key[2])
+                    for key in chunk
                 ],
                 self.params[0].device,
             )
-            self._batch = dict(zip(self._groups, self._plan.batches))
-            self._workspace = dict(zip(self._groups, self._plan.workspaces))
+            self._plans.append((chunk, plan))
+            self._batch.update(zip(chunk, plan.batches))
+            self._workspace.update(zip(chunk, plan.workspaces))
 
     @staticmethod
     def _as_matrices(tensors: Sequence[torch.Tensor]) -> list[torch.Tensor]:
@@ -243,39 +243,26 @@ class OwnedMuon:
                     f"gradient {tuple(g.shape)} {g.dtype} does not match parameter {tuple(p.shape)} {p.dtype}"
                 )
         _require_master_gpu(*grads)
-        # One C call: per shape group a momentum launch over all its matrices
-        # (which also leaves the sums of squares the normalization needs),
-        # Newton-Schulz with every product issued for all groups together, and
-        # an update launch per group.  Same bits as _prepare_muon_input ->
+        # One C call: a momentum launch over all matrices (which also leaves
+        # the sums of squares the normalization needs), Newton-Schulz with
+        # every product issued for all groups together, and an update launch.  Same bits as _prepare_muon_input ->
         # _compute_muon_direction -> _apply_muon_update per matrix.
         grad_matrices = self._as_matrices(grads)
         if self._stacked:
             # views of a stacked parameter are taken per step: they follow a
             # parameter whose storage was replaced (``p.data = ...``) since
             self._matrices = self._as_matrices(self.params)
-        for index in self._odd:
-            p, g = self._matrices[index], grad_matrices[index]
-            direction = _prepare_muon_input(
-                g, self._momentum_matrices[index], momentum=self.momentum, nesterov=self.nesterov,
-                out=torch.empty(p.shape, dtype=torch.bfloat16, device=p.device),
+        for keys, plan in self._plans:
+            members = [self._groups[key] for key in keys]
+            plan.step(
+                [[self._matrices[i] for i in group] for group in members],
+                [[self._momentum_matrices[i] for i in group] for group in members],
+                [[grad_matrices[i] for i in group] for group in members],
+                lerp_weight=1 - self.momentum, nesterov_weight=self.momentum, nesterov=self.nesterov,
+                decay_factor=1 - self.lr * self.weight_decay, coefficients=self.ns_coefficients, steps=self.ns_steps,
+                eps=self.eps,
+                # lr and adjust_lr_fn are read on every step, like the weight decay
+                # beside them: a scheduler that changes opt.lr moves both halves of
+                # the update together.
+                neg_adjusted_lrs=[-_adjust_muon_learning_rate(self.lr, self.adjust_lr_fn, key[:2]) for key in keys],
             )
-            _compute_muon_direction(direction, ns_coefficients=self.ns_coefficients, ns_steps=self.ns_steps, eps=self.eps)
-            _apply_muon_update(
-                p, direction, lr=self.lr, weight_decay=self.weight_decay, adjust_lr_fn=self.adjust_lr_fn,
-                compute_matrix_shape=p.shape,
-            )
-        if self._plan is None:
-            return
-        members = list(self._groups.values())
-        self._plan.step(
-            [[self._matrices[i] for i in group] for group in members],
-            [[self._momentum_matrices[i] for i in group] for group in members],
-            [[grad_matrices[i] for i in group] for group in members],
-            lerp_weight=1 - self.momentum, nesterov_weight=self.momentum, nesterov=self.nesterov,
-            decay_factor=1 - self.lr * self.weight_decay, coefficients=self.ns_coefficients, steps=self.ns_steps,
-            eps=self.eps,
-            # lr and adjust_lr_fn are read on every step, like the weight decay
-            # beside them: a scheduler that changes opt.lr moves both halves of
-            # the update together.
-            neg_adjusted_lrs=[-_adjust_muon_learning_rate(self.lr, self.adjust_lr_fn, key[:2]) for key in self._groups],
-        )

@@ -745,14 +745,16 @@ class MuonStepPlan:
     re-uploaded only when a tensor moved (gradients usually do, parameters and
     momentum buffers usually do not)."""
 
+    MAX_GROUPS = _native.MAX_NS_PROBLEMS
+
     def __init__(self, groups: Sequence[tuple], device: torch.device) -> None:
         """``groups``: per group (shape, matrix count, neg_adjusted_lr,
         direction_scale[, master dtype]); the master dtype (of parameters,
         gradients and momentum buffers) is bf16 when left out, or fp32."""
         if not groups:
             raise ValueError("a Muon step needs at least one group")
-        if len(groups) > _native.MAX_NS_PROBLEMS:
-            raise NotImplementedError(f"at most {_native.MAX_NS_PROBLEMS} shape groups per step")
+        if len(groups) > self.MAX_GROUPS:
+            raise NotImplementedError(f"at most {self.MAX_GROUPS} shape groups per step")
         if device.type != "cuda":
             raise RuntimeError("flex_shard_amd kernels run on the GPU only; there is no CPU path.")
         self._device = device
@@ -766,9 +768,12 @@ class MuonStepPlan:
             master = rest[0] if rest else torch.bfloat16
             if master not in (torch.bfloat16, torch.float32):
                 raise NotImplementedError(f"Muon master tensors are bf16 or fp32, got {master}")
-            if len(shape) != 2 or shape[0] % 8 or shape[1] % 8 or n <= 0:
-                raise NotImplementedError(f"whole matrices with rows and cols multiples of 8, got {n} x {tuple(shape)}")
-            batch = torch.empty((n, *shape), dtype=torch.bfloat16, device=device)
+            if len(shape) != 2 or shape[0] <= 0 or shape[1] <= 0 or n <= 0:
+                raise NotImplementedError(f"whole, non-empty matrices, got {n} x {tuple(shape)}")
+            # Matrices whose rows are not whole 16-byte vectors are orthogonalized zero-padded to multiples of 8.
+            padded = (-(-shape[0] // 8) * 8, -(-shape[1] // 8) * 8)
+            slot.layout = 0 if padded == tuple(shape) else _native.MUON_PADDED
+            batch = torch.empty((n, *padded), dtype=torch.bfloat16, device=device)
             workspace = torch.empty(newton_schulz_workspace_bytes(n, *shape), dtype=torch.uint8, device=device)
             tables = [(torch.zeros(n, dtype=torch.int64, device=device), [0] * n) for _ in range(3)]
             self.batches.append(batch)
@@ -791,7 +796,7 @@ class MuonStepPlan:
                 raise ValueError(f"all matrices of a Muon step must live on {self._device}, got {t.device}")
             if t.dtype != dtype or not t.is_contiguous() or tuple(t.shape) != shape:
                 raise ValueError(f"the Muon step kernels need contiguous {dtype} matrices of shape {shape}")
-            if t.data_ptr() % 16:
+            if t.data_ptr() % 16 and not (shape[0] % 8 or shape[1] % 8):
                 raise ValueError("the Muon step kernels need 16-byte aligned matrices")
             addresses.append(t.data_ptr())
         if addresses != current:

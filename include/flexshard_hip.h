@@ -415,6 +415,11 @@ int fsh_fp8_gemm_1x128_128x1(const void* aq_dev, const float* as_dev, const void
  * are updated in fp32 (fsh_muon_prepare_f32 / fsh_muon_apply_f32, same bits),
  * only the Newton-Schulz input is rounded to bf16, and the update is always a
  * separate launch.
+ * Rows and columns that are not multiples of 8 need layout = FSH_MUON_PADDED:
+ * the orthogonalization then works on matrices padded with zero rows and
+ * columns to multiples of 8 (which change nothing: the norm is the same and
+ * they stay zero), batch_dev and the workspace are sized for those, and the
+ * addresses of such a group need only the master's own alignment.
  * batch_dev is scratch of batch*rows*cols bf16: it holds the momentum
  * output and, for groups updated by a separate launch, the orthogonalized
  * direction afterwards (its contents after the call are otherwise unspecified).
@@ -425,18 +430,19 @@ int fsh_fp8_gemm_1x128_128x1(const void* aq_dev, const float* as_dev, const void
  * some, updated.  Treat it as fatal for the optimizer state; do not retry
  * the step.
  * ---------------------------------------------------------------------- */
+#define FSH_MUON_PADDED 1
 typedef struct fsh_muon_group {
   const int64_t* param_ptrs_dev;    /* [batch] addresses of the parameters, updated in place   */
   const int64_t* grad_ptrs_dev;     /* [batch] addresses of the gradients                      */
   const int64_t* momentum_ptrs_dev; /* [batch] addresses of the momentum buffers, updated      */
   void* batch_dev;                  /* [batch, rows, cols] bf16 scratch                        */
-  int64_t batch, rows, cols;        /* rows, cols multiples of 8                               */
+  int64_t batch, rows, cols;        /* rows, cols multiples of 8 (any with FSH_MUON_PADDED)    */
   void* workspace_dev;              /* >= fsh_newton_schulz_workspace_bytes(batch, rows, cols) */
   int64_t workspace_nbytes;
   float neg_adjusted_lr;            /* -lr * shape factor of dist_muon/optimizer.py:2031-2046  */
   float direction_scale;            /* 1, or ratio / reference_ratio of :2082-2097             */
   int32_t master_dtype;             /* FSH_DT_BF16 or FSH_DT_F32: parameters, gradients, momentum */
-  int32_t reserved;
+  int32_t layout;                   /* 0, or FSH_MUON_PADDED: rows and cols may be of any size     */
 } fsh_muon_group;
 int fsh_muon_step(const fsh_muon_group* groups, int32_t count, float lerp_weight /* 1 - mu */,
                   float nesterov_weight /* mu */, int32_t nesterov, float decay_factor /* 1 - lr*wd */, float a,

@@ -69,3 +69,33 @@ def test_more_problems_than_one_launch_holds(device):
     for q, out in zip(problems, hip_ops.gemm_nt_group(problems)):
         assert torch.equal(out, hip_ops.gemm_nt(q["a"], q["b"]))
         assert _close(out, torch.bmm(q["a"].double(), q["b"].double().transpose(1, 2).contiguous()))
+
+
+@pytest.mark.parametrize("master", [torch.bfloat16, torch.float32])
+def test_muon_step_on_odd_shapes_equals_the_per_matrix_kernels(device, master):
+    """Matrices whose rows are not whole 16-byte vectors, beside ones whose
+    are, in the batched step: more shape groups than one call takes, one
+    matrix larger than a block's slice, odd addresses."""
+    from flex_shard_amd.dist_muon import OwnedMuon
+    from flex_shard_amd.dist_muon.muon_math import _apply_muon_update, _compute_muon_direction, _prepare_muon_input
+
+    gen = torch.Generator(device=device)
+    gen.manual_seed(5)
+    shapes = [(1, 1), (7, 9), (64, 72), (130, 257), (257, 130), (33, 8), (8, 33)] + [(20 + i, 40) for i in range(12)]
+
+    def odd_view(shape):  # starts one element into its storage where the shape allows it
+        off = 0 if shape[0] % 8 == 0 and shape[1] % 8 == 0 else 1
+        return torch.randn(shape[0] * shape[1] + off, generator=gen, device=device).to(master)[off:].view(shape)
+
+    params, grads = [odd_view(s) for s in shapes], [odd_view(s) for s in shapes]
+    want, momenta = [p.clone() for p in params], [torch.zeros_like(p) for p in params]
+    opt = OwnedMuon(params, lr=0.02)
+    for _ in range(2):
+        opt.step(grads)
+        for p, m, g in zip(want, momenta, grads):
+            d = _prepare_muon_input(g, m, momentum=0.95, nesterov=True, out=torch.empty(p.shape, dtype=torch.bfloat16, device=device))
+            _compute_muon_direction(d)
+            _apply_muon_update(p, d, lr=0.02, weight_decay=0.1, adjust_lr_fn=None, compute_matrix_shape=p.shape)
+    for shape, p, w, m, n in zip(shapes, params, want, opt.momentum_buffers, momenta):
+        assert torch.equal(p, w), shape
+        assert torch.equal(m, n), shape
