@@ -25,10 +25,10 @@ struct GemmTiles {
   static constexpr int kAhead = TM * TN >= 4 ? 1 : 3, kSets = TM * TN >= 4 ? 2 : 4;
   // Epilogue: one [kWaveM][kWaveN] bf16 image per wave, rows 8 bytes off a
   // multiple of the bank window.
-  static constexpr int kPitch = kWaveN * 2 + 8;
-  static constexpr int kRegion = kWaveM * kPitch;
+  static constexpr int kPitch = kWaveN * 2 + 8;   // [row][col]
+  static constexpr int kPitchT = kWaveM * 2 + 8;  // [col][row]
+  static constexpr int kRegion = max_int(kWaveM * kPitch, kWaveN * kPitchT);
   static constexpr int kLdsBytes = kStages * kStageBytes;
-  static_assert(kWaveM == kWaveN, "the transposed image reuses the region, and the diagonal runs through (i, i) blocks");
   static_assert(kWaves * kRegion <= kLdsBytes, "the images fit the loop's LDS");
   static_assert(BM % kFillRows == 0 && BN % kFillRows == 0, "whole requests");
 };
@@ -56,21 +56,21 @@ __device__ __forceinline__ bool rows_are_16_byte(const uint16_t* p, int64_t ld) 
   return (ld & 7) == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
 
-// A wave's image in LDS to `out` rows [row0, +) x columns [col0, +), cut at
-// rows x cols, whole row segments per store instruction.
-template <typename Cfg>
+// A wave's [kRows][kCols] image in LDS to `out` rows [row0, +) x columns
+// [col0, +), cut at rows x cols, whole row segments per store instruction.
+template <int kRows, int kCols, int kPitch>
 __device__ __forceinline__ void store_wave_image(const uint8_t* region, uint16_t* out, int64_t ld, int64_t row0,
                                                  int64_t col0, int64_t rows, int64_t cols, int lane) {
-  constexpr int kLanesPerRow = Cfg::kWaveN / 8, kRowsPerPass = 64 / kLanesPerRow;
+  constexpr int kLanesPerRow = kCols / 8, kRowsPerPass = 64 / kLanesPerRow;
   const bool vec = rows_are_16_byte(out, ld);
   const int r0 = lane / kLanesPerRow, chunk = lane % kLanesPerRow;
   const int64_t col = col0 + chunk * 8;
   if (col >= cols) return;
 #pragma unroll
-  for (int pass = 0; pass < Cfg::kWaveM / kRowsPerPass; ++pass) {
+  for (int pass = 0; pass < kRows / kRowsPerPass; ++pass) {
     const int r = pass * kRowsPerPass + r0;
     if (row0 + r >= rows) break;
-    const uint8_t* src = region + r * Cfg::kPitch + chunk * 16;
+    const uint8_t* src = region + r * kPitch + chunk * 16;
     const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
     const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
     store_row_piece(out + (row0 + r) * ld, col, cols, vec, u32x4{lo.x, lo.y, hi.x, hi.y});
@@ -122,7 +122,6 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams& p, int64_t bat
 #pragma unroll
         for (int b = 0; b < 4; ++b) dv[i][j][b] = *slot(i, j, b);
   }
-  const bool on_diagonal = p.diag_add != 0.0f && row0 == col0;
   u32x2 fin[TM][TN][4];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -139,7 +138,7 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams& p, int64_t bat
           v[2] = __builtin_fmaf(p.beta, u32_as_f32(dv[i][j][b].y << 16), v[2]);
           v[3] = __builtin_fmaf(p.beta, u32_as_f32(dv[i][j][b].y & 0xFFFF0000u), v[3]);
         }
-        if (i == j && on_diagonal) {
+        if (p.diag_add != 0.0f && row0 + 32 * i == col0 + 32 * j) {  // (sub-tiles start at multiples of 32)
 #pragma unroll
           for (int t = 0; t < 4; ++t) v[t] = r_lane == 8 * b + 4 * h + t ? v[t] + p.diag_add : v[t];
         }
@@ -152,7 +151,7 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams& p, int64_t bat
 #pragma unroll
       for (int b = 0; b < 4; ++b) *slot(i, j, b) = fin[i][j][b];
   wave_lds_sync();
-  store_wave_image<Cfg>(region, C, p.ldc, row0, col0, p.M, p.N, lane);
+  store_wave_image<Cfg::kWaveM, Cfg::kWaveN, Cfg::kPitch>(region, C, p.ldc, row0, col0, p.M, p.N, lane);
   if (Ct == nullptr) return;  // uniform over the workgroup
   wave_lds_sync();  // the row reads are done before the image is written again as [col][row]
 #pragma unroll
@@ -164,24 +163,26 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams& p, int64_t bat
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const uint32_t pair = (t >> 1) ? fin[i][j][b].y : fin[i][j][b].x;
-          *reinterpret_cast<uint16_t*>(region + (j * 32 + 8 * b + 4 * h + t) * Cfg::kPitch + (i * 32 + r_lane) * 2) =
+          *reinterpret_cast<uint16_t*>(region + (j * 32 + 8 * b + 4 * h + t) * Cfg::kPitchT + (i * 32 + r_lane) * 2) =
               static_cast<uint16_t>((t & 1) ? (pair >> 16) : pair);
         }
   wave_lds_sync();
-  store_wave_image<Cfg>(region, Ct, ldct, col0, row0, p.N, p.M, lane);
+  store_wave_image<Cfg::kWaveN, Cfg::kWaveM, Cfg::kPitchT>(region, Ct, ldct, col0, row0, p.N, p.M, lane);
 }
 
 // What bounds it: the request path of a compute unit takes a 1 KB request per
 // 16 cycles, so the 32 requests of a 128 x 128 x 64 k-tile last as long as its
 // MFMAs (512 cycles), and a request holds up the wave that issues it; each is
-// therefore issued behind an MFMA, and two workgroups per compute unit cover
-// each other's waits.  Requested in one go at the top of a k-tile (with the
-// barrier in front of the fragment reads), 6592^3 ran at 843 TFLOP/s instead
-// of 998 and 84 tiles of k = 3072 took 46.5 us instead of 33; the kernels this
-// one replaced (register-staged 128 x 128 x 32, and 256 x 256 x 64 with
-// predicated accesses for ragged shapes) took 690 us for 6592^3 against 576
-// here, 45 us against 23 for 768 x 768 x 3072 (batch 4, symmetric, 64 x 64
-// tiles here) and 15-18 us against 6-8 for a single small matrix's products.
+// therefore issued behind an MFMA, fragments are read a k step ahead (three
+// for 32 x 32 waves), and workgroups that share a compute unit cover each
+// other's barriers.  6592^3 with 128 x 128 tiles: 843 TFLOP/s with the requests
+// in one go at the top of a k-tile and the fragment reads behind the barrier,
+// 988 rotated as below, 1054 with the loop split so that no request sits
+// behind a branch of its own, 1130 with 256 x 128 tiles of eight waves.
+// Against the kernels this one replaced (register-staged 128 x 128 x 32, and
+// 256 x 256 x 64 with predicated accesses for ragged shapes): 6592^3 690 ->
+// 532 us, 768 x 768 x 3072 (batch 4, symmetric) 45 -> 19 us, one 304 x 304 x
+// 704 product 17.7 -> 5.7 us.
 //
 // Operands travel global -> LDS directly into swizzled 128-byte rows, as in
 // the 256 x 256 kernel.  Rows past the matrix are read from its last row and
@@ -228,11 +229,14 @@ __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) vo
   const uint32_t fill_lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_address)lds_bytes)) + wave * 1024;
   const int ktiles = static_cast<int>((p.K + Cfg::BK - 1) / Cfg::BK);
   const int tail_chunks = static_cast<int>((p.K / 8) & 7);  // 0: the last k-tile is whole
-  auto issue_one = [&](int kt, uint32_t stage, int idx) {
-    int64_t off = static_cast<int64_t>(kt) * Cfg::kRowBytes;
-    if (tail_chunks != 0 && kt == ktiles - 1 && fill_chunk >= tail_chunks) off -= (fill_chunk - (tail_chunks - 1)) * 16;
+  // Byte offset of k-tile kt along the rows; chunks past K read the row's last chunk instead.
+  const int64_t tail_back = tail_chunks != 0 && fill_chunk >= tail_chunks ? (fill_chunk - (tail_chunks - 1)) * 16 : 0;
+  auto k_offset = [&](int kt) -> int64_t {
+    return static_cast<int64_t>(kt) * Cfg::kRowBytes - (kt == ktiles - 1 ? tail_back : 0);
+  };
+  auto issue_one = [&](int64_t k_off, uint32_t stage, int idx) {
     // (operand B's rows follow operand A's in the stage)
-    dma_load_16_at(src[idx] + off, fill_lds + stage * Cfg::kStageBytes + idx * (Cfg::kFillRows * Cfg::kRowBytes));
+    dma_load_16_at(src[idx] + k_off, fill_lds + stage * Cfg::kStageBytes + idx * (Cfg::kFillRows * Cfg::kRowBytes));
   };
 
   // Fragment side: lane l reads row l & 31 of a 32-row block, chunk 2 ks + (l >> 5).
@@ -274,21 +278,25 @@ __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) vo
   // kt + 1 are read, and which releases kt's own stage (every wave holds its
   // last fragments in registers) to the requests for kt + kStages: half of
   // them behind the MFMAs there, half in the first k step of kt + 1.
+  //   second / first: the second half of the requests for kt + kStages - 1
+  //   and the first half of those for kt + kStages go out
   constexpr int kFirst = (Cfg::kLoads + 1) / 2, kSecond = Cfg::kLoads - kFirst;
   uint32_t stage = 0;  // of kt
-  auto k_tile = [&](int kt, auto masked_tag, auto last_tag) {
+  auto k_tile = [&](int kt, auto second_tag, auto first_tag, auto masked_tag, auto last_tag) {
+    constexpr bool second = decltype(second_tag)::value, first = decltype(first_tag)::value;
     constexpr bool masked = decltype(masked_tag)::value, last = decltype(last_tag)::value;
     const uint32_t before = stage == 0 ? kStages - 1 : stage - 1, after = stage + 1 == kStages ? 0 : stage + 1;
 #pragma unroll
     for (int ks = 0; ks + 1 < KS; ++ks) {
       if (ks + Cfg::kAhead < KS) read_frags(stage, ks + Cfg::kAhead, masked);
+      __builtin_amdgcn_sched_barrier(0);
+      const int64_t k_off = second && ks == 0 ? k_offset(kt + kStages - 1) : 0;
 #pragma unroll
       for (int g = 0; g < kMfmas; ++g) {
         mfma(ks, g);
-        if (ks == 0 && kt > 0 && kt - 1 + kStages < ktiles) {
+        if (second && ks == 0) {
 #pragma unroll
-          for (int idx = g * kSecond / kMfmas; idx < (g + 1) * kSecond / kMfmas; ++idx)
-            issue_one(kt - 1 + kStages, before, kFirst + idx);
+          for (int idx = g * kSecond / kMfmas; idx < (g + 1) * kSecond / kMfmas; ++idx) issue_one(k_off, before, kFirst + idx);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -296,56 +304,70 @@ __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) vo
     if (!last) {
       // k-tile kt + 1 has landed (this wave's part); those behind it stay in flight.
       const int behind = ktiles - 2 - kt;
-      if (kStages >= 4 && behind >= 2)
+      if (kStages >= 4 && (first || behind >= 2))
         wait_for_dma_loads_but<2 * Cfg::kLoads>();
-      else if (kStages >= 3 && behind >= 1)
+      else if (kStages >= 3 && (first || behind >= 1))
         wait_for_dma_loads_but<Cfg::kLoads>();
       else
         wait_for_dma_loads();
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
       for (int ks = 0; ks < Cfg::kAhead; ++ks) read_frags(after, ks, false);
+      __builtin_amdgcn_sched_barrier(0);
     }
+    const int64_t k_off = first ? k_offset(kt + kStages) : 0;
 #pragma unroll
     for (int g = 0; g < kMfmas; ++g) {
       mfma(KS - 1, g);
-      if (!last && kt + kStages < ktiles) {
+      if (first) {
 #pragma unroll
-        for (int idx = g * kFirst / kMfmas; idx < (g + 1) * kFirst / kMfmas; ++idx) issue_one(kt + kStages, stage, idx);
+        for (int idx = g * kFirst / kMfmas; idx < (g + 1) * kFirst / kMfmas; ++idx) issue_one(k_off, stage, idx);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
     stage = after;
   };
 
+  // Fill the pipeline: the first kStages - 1 k-tiles and half of the next.
 #pragma unroll
   for (int kt = 0; kt < kStages; ++kt)
     if (kt < ktiles) {
+      const int64_t k_off = k_offset(kt);
 #pragma unroll
-      for (int idx = 0; idx < Cfg::kLoads; ++idx) issue_one(kt, kt, idx);
+      for (int idx = 0; idx < (kt + 1 < kStages ? Cfg::kLoads : kFirst); ++idx) issue_one(k_off, kt, idx);
     }
-  if (kStages >= 4 && ktiles >= 4)
-    wait_for_dma_loads_but<3 * Cfg::kLoads>();
-  else if (kStages >= 3 && ktiles >= 3)
+  if (ktiles >= kStages)
+    wait_for_dma_loads_but<(kStages - 2) * Cfg::kLoads + kFirst>();
+  else if (kStages >= 4 && ktiles == 3)
     wait_for_dma_loads_but<2 * Cfg::kLoads>();
-  else if (ktiles >= 2)
+  else if (kStages >= 3 && ktiles == 2)
     wait_for_dma_loads_but<Cfg::kLoads>();
   else
     wait_for_dma_loads();
   asm volatile("s_barrier" ::: "memory");
 #pragma unroll
   for (int ks = 0; ks < Cfg::kAhead; ++ks) read_frags(0, ks, false);
-  for (int kt = 0; kt + 1 < ktiles; ++kt) k_tile(kt, std::false_type{}, std::false_type{});
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  int kt = 0;
+  for (; kt + kStages < ktiles; ++kt) k_tile(kt, yes, yes, no, no);
+  // Drain: nothing more to request but the half that is still due.
+  bool due = ktiles >= kStages;
+  for (; kt + 1 < ktiles; ++kt) {
+    if (due) k_tile(kt, yes, no, no, no);
+    else k_tile(kt, no, no, no, no);
+    due = false;
+  }
   if (tail_chunks != 0) {
     // the fragments read ahead were read unmasked
 #pragma unroll
     for (int ks = 0; ks < Cfg::kAhead; ++ks) read_frags(stage, ks, true);
-    k_tile(ktiles - 1, std::true_type{}, std::true_type{});
+    k_tile(ktiles - 1, no, no, yes, yes);
   } else {
-    k_tile(ktiles - 1, std::false_type{}, std::true_type{});
+    k_tile(ktiles - 1, no, no, no, yes);
   }
   __syncthreads();  // the images overlay the stages
-  store_wave_tile<Cfg>(p, batch, m0 + wm * Cfg::kWaveM, n0 + wn * Cfg::kWaveN, lane, p.symmetric && tm != tn, acc,
+  store_wave_tile<Cfg>(p, batch, m0 + wm * Cfg::kWaveM, n0 + wn * Cfg::kWaveN, lane, p.symmetric && tn >= p.symmetric * (tm + 1), acc,
                        lds_bytes + wave * Cfg::kRegion);
 }
 

@@ -25,7 +25,9 @@ struct GemmParams {
   float alpha, beta;
   float diag_add;         // added to C[i][i] before the rounding
   int32_t tiles_m, tiles_n;
-  int32_t symmetric;      // only tiles with tm <= tn are computed; the others are mirrored
+  // Not 0: the product is symmetric.  Tile rows are `symmetric` tile columns high; only the tiles from a tile row's
+  // diagonal on are computed, those right of the diagonal's tile row are mirrored.
+  int32_t symmetric;
   int32_t k_major;        // A is [K, M] and B is [K, N]: the product is A^T B (large-tile kernel only)
   int32_t tiles_per_matrix;
   int64_t work_items;     // tiles_per_matrix * batch
@@ -90,16 +92,17 @@ __device__ inline bool tile_of_workgroup(const GemmParams& p, int64_t id, int64_
   *batch = item / tiles;
   int t = static_cast<int>(item % tiles);
   if (p.symmetric) {
-    // Upper triangle row by row: row r holds columns r .. tiles_n-1.  One
-    // matrix's triangle (36 tiles of a 2048^2 result) is about what an XCD
-    // holds at a time, and it needs only the 8 row panels of the operand.
+    // Upper triangle row by row: row r holds columns symmetric * r ..
+    // tiles_n-1.  One matrix's triangle (36 tiles of a 2048^2 result) is about
+    // what an XCD holds at a time, and it needs only the 8 row panels of the
+    // operand.
     int r = 0;
-    for (int len = p.tiles_n; t >= len; --len) {
+    for (int len = p.tiles_n; t >= len; len -= p.symmetric) {
       t -= len;
       ++r;
     }
     *tm = r;
-    *tn = r + t;
+    *tn = p.symmetric * r + t;
     return true;
   }
   tile_in_order(p, t, tm, tn);

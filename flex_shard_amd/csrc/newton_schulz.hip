@@ -460,53 +460,70 @@ struct PlannedGemm {
 };
 
 // ---- Which tiles a launch takes.
-// What a launch of these kernels was measured to take, from the number of its
-// tiles (of its longest k; shorter ones count by their share of it) and that
-// k: a start and end of 5 us (10 us with 256 x 256 tiles, whose output is 128
-// KB per workgroup), and per k-tile of 64 what the chip takes for one round of
-// resident workgroups.  A 256 x 256 tile computes four times what a 128 x 128
-// one does in 1.8 (half the chip busy) to 1.6 times its time, and that less
-// and less, since with the whole chip busy the clock falls from 2.3 to 1.6
-// GHz; but it leaves compute units idle in a launch of few tiles, and so do
-// 128 x 128 tiles against 64 x 64 ones.  Measured on 4096^3: 106 us with
-// 256 x 256, 135 with 128 x 128, 202 with 64 x 64 tiles; on 1024^3: 23.5, 12.4
-// and 8.0 us.
-enum TileKind { kTiles64, kTiles128, kTiles256 };
-struct TileWork {
-  double tile_ktiles = 0.0;  // k-tiles of all tiles together
-  double max_ktiles = 0.0;
-  void add(int64_t tiles, int64_t k) {
-    const double kt = static_cast<double>(ceil_div(k, (int64_t)64));
-    tile_ktiles += static_cast<double>(tiles) * kt;
-    if (kt > max_ktiles) max_ktiles = kt;
-  }
+// The kernels differ in how many tiles the chip holds at once (a round) and in
+// what a k-tile of 64 of such a round takes; a round also starts and ends, its
+// output being written by all workgroups at the same time.  Both were measured
+// over 13 shapes from 512^2 to 8192 x 6144 at k = 512 and 2048 (us for k = 512
+// / 2048, tiles of 64 x 64, 128 x 128, 256 x 128, 256 x 256):
+//   1024 x 1024     5.5 / 10.4    8.1 / 17.4   10.2 / 25.4   15.5 / 38.7
+//   2048 x 2048    11.5 / 30.6    9.7 / 22.7   11.6 / 28.0   16.8 / 42.8
+//   4096 x 2048    18.8 / 55.6   15.5 / 40.0   14.9 / 36.5   19.3 / 45.8
+//   4096 x 4096    35.9 / 108.5  27.3 / 80.5   28.0 / 74.6   22.9 / 61.7
+// A partly filled round is faster: fewer workgroups share a compute unit, and
+// with half the chip busy the clock stays at 2.3 instead of 1.6 GHz.
+enum TileKind { kTiles64, kTiles128, kTiles128Deep, kTiles256x128, kTiles256 };
+struct TileShape {
+  int64_t m, n;
+  double round;                // tiles the chip holds at once
+  double empty, half, full;    // us per k-tile of a round that is nearly empty, half full, full
+  double ends;                 // us a round spends starting and ending
 };
-double launch_us(TileKind kind, const TileWork& w) {
-  if (w.tile_ktiles == 0.0) return 0.0;
-  const double n = w.tile_ktiles / w.max_ktiles / 256.0;  // in tiles per compute unit
-  double per_ktile;
-  if (kind == kTiles256) {
-    const double full = floor(n), r = n - full;
-    per_ktile = 1.57 * full + (r == 0.0 ? 0.0 : r <= 0.5 ? 1.13 : 1.13 + 0.88 * (r - 0.5));
-  } else if (kind == kTiles128) {
-    const double full = floor(n / 2), r = n - 2 * full;
-    per_ktile = full + (r == 0.0 ? 0.0 : r <= 1.0 ? 0.62 : 1.0);
-  } else {
-    const double full = floor(n / 3), r = n - 3 * full;
-    per_ktile = 0.59 * full + (r == 0.0 ? 0.0 : r <= 1.0 ? 0.27 : r <= 2.0 ? 0.40 : 0.59);
+constexpr TileShape kTileShapes[] = {
+    {64, 64, 768.0, 0.17, 0.40, 0.55, 1.7},       // three workgroups per compute unit
+    {128, 128, 512.0, 0.37, 0.71, 1.02, 4.2},     // two
+    {128, 128, 256.0, 0.35, 0.43, 0.52, 3.2},     // one, its operands requested three k-tiles ahead
+    {256, 128, 256.0, 0.54, 0.68, 0.91, 5.5},     // one of eight waves
+    {256, 256, 256.0, 0.96, 1.10, 1.58, 8.0},     // one
+};
+// The products of one launch, as the tiles of every kind see them.
+struct LaunchWork {
+  double tiles[5] = {0, 0, 0, 0, 0}, tile_ktiles[5] = {0, 0, 0, 0, 0};
+  double max_ktiles = 0.0;
+  void add(int64_t m, int64_t n, int64_t k, bool symmetric, int64_t batch);
+};
+int64_t count_tiles(int64_t m, int64_t n, bool symmetric, int64_t tile_m, int64_t tile_n) {
+  const int64_t tm = ceil_div(m, tile_m), tn = ceil_div(n, tile_n), step = tile_m / tile_n;
+  return symmetric ? tm * tn - step * (tm * (tm - 1) / 2) : tm * tn;
+}
+void LaunchWork::add(int64_t m, int64_t n, int64_t k, bool symmetric, int64_t batch) {
+  const double kt = static_cast<double>(ceil_div(k, (int64_t)64));
+  for (int i = 0; i < 5; ++i) {
+    const double count = static_cast<double>(count_tiles(m, n, symmetric, kTileShapes[i].m, kTileShapes[i].n)) * static_cast<double>(batch);
+    tiles[i] += count;
+    tile_ktiles[i] += count * kt;
   }
-  return (kind == kTiles256 ? 10.0 : 5.0) + per_ktile * w.max_ktiles;
+  max_ktiles = fmax(max_ktiles, kt);
 }
-int64_t count_tiles(int64_t m, int64_t n, bool symmetric, int64_t tile) {
-  const int64_t tn = ceil_div(n, tile);
-  return symmetric ? tn * (tn + 1) / 2 : ceil_div(m, tile) * tn;
+// Tiles of a shorter contraction count by their share of the longest one.
+double launch_us(TileKind kind, const LaunchWork& w) {
+  if (w.max_ktiles == 0.0) return 0.0;
+  const TileShape& shape = kTileShapes[kind];
+  const double rounds = w.tile_ktiles[kind] / w.max_ktiles / shape.round, whole = floor(rounds), part = rounds - whole;
+  double per_ktile = whole * shape.full;
+  if (part > 0.0)
+    per_ktile += part <= 0.5 ? shape.empty + (shape.half - shape.empty) * 2.0 * part
+                             : shape.half + (shape.full - shape.half) * (2.0 * part - 1.0);
+  return 3.0 + per_ktile * w.max_ktiles + shape.ends * fmax(1.0, ceil(w.tiles[kind] / shape.round));
 }
-TileKind small_tile_kind(const TileWork& w64, const TileWork& w128) {
-  return launch_us(kTiles64, w64) < launch_us(kTiles128, w128) ? kTiles64 : kTiles128;
+TileKind small_tile_kind(const LaunchWork& w) {
+  TileKind best = kTiles64;
+  for (const TileKind kind : {kTiles128, kTiles128Deep, kTiles256x128}) {
+    if (kind == kTiles128Deep && w.tiles[kind] > kTileShapes[kind].round) continue;  // one round or none
+    if (launch_us(kind, w) < launch_us(best, w)) best = kind;
+  }
+  return best;
 }
-double small_tiles_us(const TileWork& w64, const TileWork& w128) {
-  return fmin(launch_us(kTiles64, w64), launch_us(kTiles128, w128));
-}
+double small_tiles_us(const LaunchWork& w) { return launch_us(small_tile_kind(w), w); }
 
 // The 256 x 256 kernel takes whole tiles with 16-byte accesses in the epilogue and 32-bit tile spans.
 bool fits_large_tiles(const GemmParams& p) {
@@ -574,7 +591,7 @@ int plan_gemm(const fsh_gemm_desc& d, PlannedGemm* plan, const GemmUpdate* updat
 // less time with the rest of the call.  Operands given k-major and fused
 // updates exist in the large-tile kernel only.
 int choose_kernels(PlannedGemm* plans, int count) {
-  TileWork large, small64, small128, all64, all128;
+  LaunchWork large, small, all;
   bool bound = false;
   for (int i = 0; i < count; ++i) {
     const GemmParams& p = plans[i].p;
@@ -583,27 +600,20 @@ int choose_kernels(PlannedGemm* plans, int count) {
       return fail(FSH_ENOTSUP, "gemm: k-major operands and fused updates need whole 256 x 256 x 64 tiles (m %lld, n %lld, k %lld)",
                   (long long)p.M, (long long)p.N, (long long)p.K);
     bound = bound || must;
-    const bool sym = p.symmetric != 0;
-    const int64_t n64 = count_tiles(p.M, p.N, sym, 64) * plans[i].batch, n128 = count_tiles(p.M, p.N, sym, 128) * plans[i].batch;
-    all64.add(n64, p.K);
-    all128.add(n128, p.K);
-    if (plans[i].large) {
-      large.add(count_tiles(p.M, p.N, sym, 256) * plans[i].batch, p.K);
-    } else {
-      small64.add(n64, p.K);
-      small128.add(n128, p.K);
-    }
+    all.add(p.M, p.N, p.K, p.symmetric != 0, plans[i].batch);
+    (plans[i].large ? large : small).add(p.M, p.N, p.K, p.symmetric != 0, plans[i].batch);
   }
-  if (!bound && small_tiles_us(all64, all128) <= launch_us(kTiles256, large) + small_tiles_us(small64, small128))
+  if (!bound && small_tiles_us(all) <= launch_us(kTiles256, large) + small_tiles_us(small))
     for (int i = 0; i < count; ++i) plans[i].large = false;
   return FSH_OK;
 }
 
-// Fills in a problem's schedule of `tile` x `tile` tiles.
-int schedule_tiles(PlannedGemm* plan, int64_t tile, int64_t* workgroups) {
+// Fills in a problem's schedule of tile_m x tile_n tiles.
+int schedule_tiles(PlannedGemm* plan, int64_t tile_m, int64_t tile_n, int64_t* workgroups) {
   GemmParams& p = plan->p;
-  const int64_t tiles_m = ceil_div(p.M, tile), tiles_n = ceil_div(p.N, tile);
-  const int64_t tiles = count_tiles(p.M, p.N, p.symmetric != 0, tile);
+  const int64_t tiles_m = ceil_div(p.M, tile_m), tiles_n = ceil_div(p.N, tile_n);
+  const int64_t tiles = count_tiles(p.M, p.N, p.symmetric != 0, tile_m, tile_n);
+  if (p.symmetric) p.symmetric = static_cast<int32_t>(tile_m / tile_n);
   p.work_items = tiles * plan->batch;
   p.items_per_xcd = ceil_div(p.work_items, static_cast<int64_t>(kXcds));
   if (tiles > 0x3FFFFFFFLL || p.items_per_xcd * kXcds > 0x3FFFFFFFLL) return fail(FSH_ENOTSUP, "gemm: too many tiles");
@@ -614,16 +624,16 @@ int schedule_tiles(PlannedGemm* plan, int64_t tile, int64_t* workgroups) {
   return FSH_OK;
 }
 
-// The problems `members` (indices into plans, longest k first) as one launch of `tile` x `tile` tiles.
+// The problems `members` (indices into plans, longest k first) as one launch of tile_m x tile_n tiles.
 template <typename Launch>
-int fill_launch(PlannedGemm* plans, const int* members, int n, int64_t tile, Launch* launch) {
+int fill_launch(PlannedGemm* plans, const int* members, int n, int64_t tile_m, int64_t tile_n, Launch* launch) {
   memset(launch, 0, sizeof(*launch));
   int64_t first = 0;
   for (int k = 0; k < Launch::kMaxProblems; ++k) {
     launch->first_workgroup[k] = INT32_MAX;
     if (k >= n) continue;
     int64_t workgroups = 0;
-    if (int rc = schedule_tiles(&plans[members[k]], tile, &workgroups)) return rc;
+    if (int rc = schedule_tiles(&plans[members[k]], tile_m, tile_n, &workgroups)) return rc;
     launch->first_workgroup[k] = static_cast<int32_t>(first);
     launch->problem[k] = plans[members[k]].p;
     first += workgroups;
@@ -669,24 +679,21 @@ int launch_tiles_as(const TileLaunch& launch, hipStream_t stream) {
   return check_launch("gemm_nt_tiles_kernel");
 }
 
-// Small tiles: 64 x 64 (three workgroups per compute unit) or 128 x 128 (two;
-// one with its operands requested three k-tiles ahead when the launch has no
-// more tiles than units).
 int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stream) {
-  TileWork w64, w128;
+  LaunchWork work;
   for (int k = 0; k < n; ++k) {
-    const PlannedGemm& q = plans[members[k]];
-    w64.add(count_tiles(q.p.M, q.p.N, q.p.symmetric != 0, 64) * q.batch, q.p.K);
-    w128.add(count_tiles(q.p.M, q.p.N, q.p.symmetric != 0, 128) * q.batch, q.p.K);
+    const GemmParams& p = plans[members[k]].p;
+    work.add(p.M, p.N, p.K, p.symmetric != 0, plans[members[k]].batch);
   }
+  const TileKind kind = small_tile_kind(work);
   TileLaunch launch;
-  if (small_tile_kind(w64, w128) == kTiles64) {
-    if (int rc = fill_launch(plans, members, n, 64, &launch)) return rc;
-    return launch_tiles_as<GemmTiles<2, 2, 1, 1, 3>, 3>(launch, stream);
+  if (int rc = fill_launch(plans, members, n, kTileShapes[kind].m, kTileShapes[kind].n, &launch)) return rc;
+  switch (kind) {
+    case kTiles64: return launch_tiles_as<GemmTiles<2, 2, 1, 1, 3>, 3>(launch, stream);
+    case kTiles128: return launch_tiles_as<GemmTiles<2, 2, 2, 2, 2>, 2>(launch, stream);
+    case kTiles128Deep: return launch_tiles_as<GemmTiles<2, 2, 2, 2, 4>, 1>(launch, stream);
+    default: return launch_tiles_as<GemmTiles<4, 2, 2, 2, 3>, 1>(launch, stream);
   }
-  if (int rc = fill_launch(plans, members, n, 128, &launch)) return rc;
-  if (launch.total_workgroups <= compute_units()) return launch_tiles_as<GemmTiles<2, 2, 2, 2, 4>, 1>(launch, stream);
-  return launch_tiles_as<GemmTiles<2, 2, 2, 2, 2>, 2>(launch, stream);
 }
 
 // Launches the planned problems.  Problems that take the same kernel share
@@ -712,7 +719,7 @@ int launch_planned(PlannedGemm* plans, int count, hipStream_t stream) {
         if (int rc = launch_tiles(plans, members, n, stream)) return rc;
       } else {
         GemmLaunch launch;
-        if (int rc = fill_launch(plans, members, n, 256, &launch)) return rc;
+        if (int rc = fill_launch(plans, members, n, 256, 256, &launch)) return rc;
         if (int rc = launch_large_tiles(launch, group == 1, stream)) return rc;
       }
     }
@@ -742,7 +749,7 @@ int launch_gemms(const fsh_gemm_desc* descs, int count, hipStream_t stream, cons
 // transposed copy and the small tiles are faster.
 int check_k_major(const fsh_gemm_desc& d) {
   if (!d.k_major || d.m <= 0 || d.n <= 0) return FSH_OK;
-  if (count_tiles(d.m, d.n, d.symmetric != 0, 256) * d.batch >= 192 && d.m % 256 == 0 && d.n % 256 == 0 && d.k % 64 == 0)
+  if (count_tiles(d.m, d.n, d.symmetric != 0, 256, 256) * d.batch >= 192 && d.m % 256 == 0 && d.n % 256 == 0 && d.k % 64 == 0)
     return FSH_OK;
   return fail(FSH_ENOTSUP,
               "gemm: k-major operands need whole 256 x 256 x 64 tiles and at least 192 of them (m %lld, n %lld, "
@@ -820,25 +827,17 @@ int64_t ns_partial_offset(int64_t batch, int64_t rows, int64_t cols) {
 void ns_choose_large(const fsh_ns_problem* problems, int count, int32_t steps, bool* large) {
   double with_large_us = 0.0, without_us = 0.0;
   for (int which = 0; which < 3; ++which) {
-    TileWork w256, small64, small128, all64, all128;
+    LaunchWork in_large, small, all;
     for (int i = 0; i < count; ++i) {
       const fsh_ns_problem& q = problems[i];
       const int64_t s = q.rows < q.cols ? q.rows : q.cols, l = q.rows < q.cols ? q.cols : q.rows;
       large[i] = steps > 0 && s > 0 && s % 256 == 0 && l % 256 == 0 && l < (1LL << 22);
       const int64_t m = which == 2 ? l : s, k = which == 0 ? l : s;
-      const bool sym = which != 2;
-      const int64_t n64 = count_tiles(m, s, sym, 64) * q.batch, n128 = count_tiles(m, s, sym, 128) * q.batch;
-      all64.add(n64, k);
-      all128.add(n128, k);
-      if (large[i]) {
-        w256.add(count_tiles(m, s, sym, 256) * q.batch, k);
-      } else {
-        small64.add(n64, k);
-        small128.add(n128, k);
-      }
+      all.add(m, s, k, which != 2, q.batch);
+      (large[i] ? in_large : small).add(m, s, k, which != 2, q.batch);
     }
-    with_large_us += launch_us(kTiles256, w256) + small_tiles_us(small64, small128);
-    without_us += small_tiles_us(all64, all128);
+    with_large_us += launch_us(kTiles256, in_large) + small_tiles_us(small);
+    without_us += small_tiles_us(all);
   }
   for (int i = 0; i < count; ++i) large[i] = large[i] && with_large_us < without_us;
 }
