@@ -14,7 +14,7 @@
 // accumulated from zero in a scratch accumulator and folded into the result
 // with one fused multiply-add per element; the folds of one 32x32 block run
 // on the vector ALU while the matrix core works on the next.
-#include "mfma_tiles.hpp"
+#include "fp8_tiles.hpp"
 
 namespace fsh {
 namespace {
@@ -125,41 +125,6 @@ struct Fp8GemmCfg {
 };
 using Fp8Gemm = Fp8GemmCfg<2>;
 static_assert(Fp8GemmCfg<1>::kLdsBytes <= Fp8Gemm::kLdsBytes, "the half tile lives in the whole tile's LDS");
-
-struct Fp8GemmParams {
-  const uint8_t* xq;
-  const float* xs;   // [k / 128][m]
-  const uint8_t* wq;
-  const float* ws;   // block scales: element (output-column block cb, k-block kb) at ws[cb * ws_cb + kb * ws_kb]
-  const float* cs;   // per-column scales [k / 128][n] (the other kernel variant)
-  uint16_t* out;
-  int64_t m, n, k;
-  int64_t ldxq, ldwq, ldo, ws_cb, ws_kb;
-  GemmParams schedule;  // tile order; its work items are the tiles computed whole
-  // Workgroups [whole_grid, ...) take the remaining tiles (in the same order)
-  // as two half tiles each, half_items in all.
-  int64_t whole_grid, half_items, half_items_per_xcd;
-};
-
-typedef int v8i32 __attribute__((ext_vector_type(8)));
-
-// acc[n] += (product[n] * row_scale) * (column_scales of lane n of this lane's row of 16).
-// The broadcast is the multiply-add's own operand modifier (the compiler keeps
-// a separate move per element when given the builtin).  column_scales comes
-// from LDS, not from the vector ALU, so the modifier's read needs no wait states.
-template <int N = 0>
-__device__ __forceinline__ void fold_with_row_broadcast(f32x16& acc, const f32x16& product, float row_scale,
-                                                        float column_scales) {
-  if constexpr (N < 16) {
-    const float scaled = product[N] * row_scale;
-    float sum = acc[N];
-    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-        : "+v"(sum)
-        : "v"(column_scales), "v"(scaled), "n"(N));
-    acc[N] = sum;
-    fold_with_row_broadcast<N + 1>(acc, product, row_scale, column_scales);
-  }
-}
 
 // One output tile (TM_ = 2) or half tile (TM_ = 1, rows [128 half, +128) of the tile).
 // kLongK: the contraction is longer than one window of weight block scales
@@ -612,7 +577,56 @@ FSH_API int fsh_act_quant_1x128(const void* x_dev, int64_t rows, int64_t cols, i
 namespace fsh {
 namespace {
 
-// Shared checks and launch of the two FP8 GEMM variants.  `p` arrives with
+// Which tiles a product takes: the ones with the lowest estimated time.
+// Measured (us with 64 x 64, 128 x 128, 256 x 256 tiles; block scales, the
+// column-scale variant runs 5-10 % longer on all three):
+//   48 x 14336, k 4096     14.5   24.9   35.5      48 x 4096, k 14336  34.6  69.8  112
+//   256 x 4096, k 4096     13.0   23.4   27.6      1000 x 2048, k 5120 22.1  31.4  46.3
+//   1024 x 4096, k 4096    30.7   26.9   38.3      2048 x 4096, k 4096 55.1  39.4  42.0
+//   1024 x 14336, k 4096   95.6   71.4   54.3      4096 x 4096, k 4096 112   73.0  58.8
+enum Fp8TileKind { kFp8Tiles64, kFp8Tiles128, kFp8Tiles256 };
+Fp8TileKind fp8_tile_kind(int64_t m, int64_t n, int64_t k) {
+  static constexpr TileShape kShapes[] = {
+      {64, 64, 768.0, 0.22, 0.34, 0.61, 2.0},    // three workgroups per compute unit
+      {128, 128, 512.0, 0.56, 0.69, 1.07, 4.0},  // two
+      {256, 256, 256.0, 0.75, 1.06, 1.59, 5.0},  // one; a round of at most half as many is cut into half tiles
+  };
+  const double ktiles = static_cast<double>(k / 128);
+  int best = 0;
+  double best_us = 0.0;
+  for (int i = 0; i < 3; ++i) {
+    const double tiles = static_cast<double>(ceil_div(m, kShapes[i].m)) * static_cast<double>(ceil_div(n, kShapes[i].n));
+    const double us = rounds_us(kShapes[i], tiles, tiles * ktiles, ktiles);
+    if (i == 0 || us < best_us) {
+      best = i;
+      best_us = us;
+    }
+  }
+  return static_cast<Fp8TileKind>(best);
+}
+
+template <typename Cfg, int kBlocksPerUnit>
+int launch_fp8_tiles(Fp8GemmParams& p, bool column_scales, hipStream_t stream) {
+  GemmParams& s = p.schedule;
+  s.tiles_m = static_cast<int32_t>(ceil_div(p.m, static_cast<int64_t>(Cfg::BM)));
+  s.tiles_n = static_cast<int32_t>(ceil_div(p.n, static_cast<int64_t>(Cfg::BN)));
+  const int64_t tiles = static_cast<int64_t>(s.tiles_m) * s.tiles_n;
+  s.tiles_per_matrix = static_cast<int32_t>(tiles);  // (few: the rule above prefers large tiles from a few thousand on)
+  s.work_items = tiles;
+  s.items_per_xcd = ceil_div(tiles, static_cast<int64_t>(kXcds));
+  const dim3 grid(static_cast<uint32_t>(s.items_per_xcd * kXcds)), block(Cfg::kThreads);
+  static LdsReservation reserved_block_scales, reserved_column_scales;
+  if (column_scales) {
+    if (int rc = reserve_lds_once(reserved_column_scales, &fp8_gemm_tiles_kernel<Cfg, true, kBlocksPerUnit>, Cfg::kLdsBytes)) return rc;
+    hipLaunchKernelGGL((fp8_gemm_tiles_kernel<Cfg, true, kBlocksPerUnit>), grid, block, Cfg::kLdsBytes, stream, p);
+  } else {
+    if (int rc = reserve_lds_once(reserved_block_scales, &fp8_gemm_tiles_kernel<Cfg, false, kBlocksPerUnit>, Cfg::kLdsBytes)) return rc;
+    hipLaunchKernelGGL((fp8_gemm_tiles_kernel<Cfg, false, kBlocksPerUnit>), grid, block, Cfg::kLdsBytes, stream, p);
+  }
+  return check_launch("fp8_gemm_tiles_kernel");
+}
+
+// Shared checks and launch of the FP8 GEMM variants.  `p` arrives with
 // the operands, sizes and scale tables filled in.
 int launch_fp8_gemm(Fp8GemmParams& p, bool column_scales, const char* who, void* stream) {
   if (p.m < 0 || p.n < 0 || p.k < 0) return fail(FSH_EINVAL, "%s: negative size", who);
@@ -644,6 +658,9 @@ int launch_fp8_gemm(Fp8GemmParams& p, bool column_scales, const char* who, void*
   // rounds of one per CU.  A last round that is at most half full is cut into
   // half tiles, twice as many workgroups of half the length: e.g. the 896
   // tiles of a [14336, 4096] result take 3.5 rounds instead of 4.
+  const Fp8TileKind kind = fp8_tile_kind(p.m, p.n, p.k);
+  if (kind == kFp8Tiles64) return launch_fp8_tiles<Fp8Tiles<2, 2, 1, 1, 3>, 3>(p, column_scales, static_cast<hipStream_t>(stream));
+  if (kind == kFp8Tiles128) return launch_fp8_tiles<Fp8Tiles<2, 2, 2, 2, 2>, 2>(p, column_scales, static_cast<hipStream_t>(stream));
   const int64_t units = compute_units();
   const int64_t tail = units > 0 ? tiles % units : 0;
   const int64_t cut = (tail > 0 && 2 * tail <= units) ? tail : 0;

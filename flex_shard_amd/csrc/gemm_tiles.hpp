@@ -33,50 +33,6 @@ struct GemmTiles {
   static_assert(BM % kFillRows == 0 && BN % kFillRows == 0, "whole requests");
 };
 
-// Eight bf16 of a row that ends at column `cols`, starting at column `col`
-// (< cols); 16-byte access when `vec` allows it, columns past the end as zero.
-__device__ __forceinline__ u32x4 load_row_piece(const uint16_t* row, int64_t col, int64_t cols, bool vec) {
-  if (vec && col + 8 <= cols) return *reinterpret_cast<const u32x4*>(row + col);
-  uint32_t e[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) e[t] = col + t < cols ? row[col + t] : 0u;
-  return u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-}
-__device__ __forceinline__ void store_row_piece(uint16_t* row, int64_t col, int64_t cols, bool vec, u32x4 v) {
-  if (vec && col + 8 <= cols) {
-    *reinterpret_cast<u32x4*>(row + col) = v;
-    return;
-  }
-  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-  for (int t = 0; t < 8; ++t)
-    if (col + t < cols) row[col + t] = static_cast<uint16_t>(w[t >> 1] >> (16 * (t & 1)));
-}
-__device__ __forceinline__ bool rows_are_16_byte(const uint16_t* p, int64_t ld) {
-  return (ld & 7) == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
-}
-
-// A wave's [kRows][kCols] image in LDS to `out` rows [row0, +) x columns
-// [col0, +), cut at rows x cols, whole row segments per store instruction.
-template <int kRows, int kCols, int kPitch>
-__device__ __forceinline__ void store_wave_image(const uint8_t* region, uint16_t* out, int64_t ld, int64_t row0,
-                                                 int64_t col0, int64_t rows, int64_t cols, int lane) {
-  constexpr int kLanesPerRow = kCols / 8, kRowsPerPass = 64 / kLanesPerRow;
-  const bool vec = rows_are_16_byte(out, ld);
-  const int r0 = lane / kLanesPerRow, chunk = lane % kLanesPerRow;
-  const int64_t col = col0 + chunk * 8;
-  if (col >= cols) return;
-#pragma unroll
-  for (int pass = 0; pass < kRows / kRowsPerPass; ++pass) {
-    const int r = pass * kRowsPerPass + r0;
-    if (row0 + r >= rows) break;
-    const uint8_t* src = region + r * kPitch + chunk * 16;
-    const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
-    const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
-    store_row_piece(out + (row0 + r) * ld, col, cols, vec, u32x4{lo.x, lo.y, hi.x, hi.y});
-  }
-}
-
 // Finals bf16(fma(beta, D, alpha * acc) + diagonal term) of a wave's sub-tile
 // at (row0, col0), through its LDS image: D arrives row-wise, C and the
 // transposed (or mirrored) output leave row-wise.  Only the wave itself

@@ -5,6 +5,7 @@
 #include "common.hpp"
 
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 
 namespace fsh {
@@ -412,6 +413,10 @@ __device__ inline void dma_load_16(uint32_t voffset, const uint8_t* base, uint32
 __device__ inline void dma_load_16_at(const uint8_t* src, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory");
 }
+// The 4-byte form: lane l writes LDS bytes [M0 + 4 l, M0 + 4 l + 4).
+__device__ inline void dma_load_4_at(const uint8_t* src, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds_addr) : "memory");
+}
 template <int kInFlight>
 __device__ inline void wait_for_dma_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kInFlight) : "memory"); }
 __device__ inline void wait_for_dma_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
@@ -421,6 +426,70 @@ __device__ inline void dma_touch_4(uint32_t voffset, const uint8_t* base, uint32
 }
 
 constexpr int max_int(int a, int b) { return a > b ? a : b; }
+
+// Eight bf16 of a row that ends at column `cols`, starting at column `col`
+// (< cols); 16-byte access when `vec` allows it, columns past the end as zero.
+__device__ __forceinline__ u32x4 load_row_piece(const uint16_t* row, int64_t col, int64_t cols, bool vec) {
+  if (vec && col + 8 <= cols) return *reinterpret_cast<const u32x4*>(row + col);
+  uint32_t e[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) e[t] = col + t < cols ? row[col + t] : 0u;
+  return u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
+}
+__device__ __forceinline__ void store_row_piece(uint16_t* row, int64_t col, int64_t cols, bool vec, u32x4 v) {
+  if (vec && col + 8 <= cols) {
+    *reinterpret_cast<u32x4*>(row + col) = v;
+    return;
+  }
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int t = 0; t < 8; ++t)
+    if (col + t < cols) row[col + t] = static_cast<uint16_t>(w[t >> 1] >> (16 * (t & 1)));
+}
+__device__ __forceinline__ bool rows_are_16_byte(const uint16_t* p, int64_t ld) {
+  return (ld & 7) == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
+}
+
+// A wave's [kRows][kCols] image in LDS to `out` rows [row0, +) x columns
+// [col0, +), cut at rows x cols, whole row segments per store instruction.
+template <int kRows, int kCols, int kPitch>
+__device__ __forceinline__ void store_wave_image(const uint8_t* region, uint16_t* out, int64_t ld, int64_t row0,
+                                                 int64_t col0, int64_t rows, int64_t cols, int lane) {
+  constexpr int kLanesPerRow = kCols / 8, kRowsPerPass = 64 / kLanesPerRow;
+  const bool vec = rows_are_16_byte(out, ld);
+  const int r0 = lane / kLanesPerRow, chunk = lane % kLanesPerRow;
+  const int64_t col = col0 + chunk * 8;
+  if (col >= cols) return;
+#pragma unroll
+  for (int pass = 0; pass < kRows / kRowsPerPass; ++pass) {
+    const int r = pass * kRowsPerPass + r0;
+    if (row0 + r >= rows) break;
+    const uint8_t* src = region + r * kPitch + chunk * 16;
+    const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
+    const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
+    store_row_piece(out + (row0 + r) * ld, col, cols, vec, u32x4{lo.x, lo.y, hi.x, hi.y});
+  }
+}
+
+
+// What a launch of a tile kernel takes, from measurements: tiles of the chip's
+// one round at a time, per k-tile the less the emptier the round is (fewer
+// workgroups share a compute unit, and with half the chip busy the clock stays
+// at 2.3 instead of 1.6 GHz), and a start and end per round.
+struct TileShape {
+  int64_t m, n;
+  double round;              // tiles the chip holds at once
+  double empty, half, full;  // us per k-tile of a round that is nearly empty, half full, full
+  double ends;               // us a round spends starting and ending
+};
+inline double rounds_us(const TileShape& shape, double tiles, double tile_ktiles, double max_ktiles) {
+  const double rounds = tile_ktiles / max_ktiles / shape.round, whole = floor(rounds), part = rounds - whole;
+  double per_ktile = whole * shape.full;
+  if (part > 0.0)
+    per_ktile += part <= 0.5 ? shape.empty + (shape.half - shape.empty) * 2.0 * part
+                             : shape.half + (shape.full - shape.half) * (2.0 * part - 1.0);
+  return 3.0 + per_ktile * max_ktiles + shape.ends * fmax(1.0, ceil(tiles / shape.round));
+}
 
 template <typename Kernel>
 int reserve_lds(Kernel kernel, int bytes) {

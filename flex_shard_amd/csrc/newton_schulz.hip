@@ -18,7 +18,6 @@
 #include "gemm_tiles.hpp"
 #include "muon_groups.hpp"
 
-#include <cmath>
 
 namespace fsh {
 namespace {
@@ -460,24 +459,13 @@ struct PlannedGemm {
 };
 
 // ---- Which tiles a launch takes.
-// The kernels differ in how many tiles the chip holds at once (a round) and in
-// what a k-tile of 64 of such a round takes; a round also starts and ends, its
-// output being written by all workgroups at the same time.  Both were measured
-// over 13 shapes from 512^2 to 8192 x 6144 at k = 512 and 2048 (us for k = 512
-// / 2048, tiles of 64 x 64, 128 x 128, 256 x 128, 256 x 256):
+// Measured over 13 shapes from 512^2 to 8192 x 6144 at k = 512 and 2048 (us for
+// k = 512 / 2048, tiles of 64 x 64, 128 x 128, 256 x 128, 256 x 256; k-tiles of 64):
 //   1024 x 1024     5.5 / 10.4    8.1 / 17.4   10.2 / 25.4   15.5 / 38.7
 //   2048 x 2048    11.5 / 30.6    9.7 / 22.7   11.6 / 28.0   16.8 / 42.8
 //   4096 x 2048    18.8 / 55.6   15.5 / 40.0   14.9 / 36.5   19.3 / 45.8
 //   4096 x 4096    35.9 / 108.5  27.3 / 80.5   28.0 / 74.6   22.9 / 61.7
-// A partly filled round is faster: fewer workgroups share a compute unit, and
-// with half the chip busy the clock stays at 2.3 instead of 1.6 GHz.
 enum TileKind { kTiles64, kTiles128, kTiles128Deep, kTiles256x128, kTiles256 };
-struct TileShape {
-  int64_t m, n;
-  double round;                // tiles the chip holds at once
-  double empty, half, full;    // us per k-tile of a round that is nearly empty, half full, full
-  double ends;                 // us a round spends starting and ending
-};
 constexpr TileShape kTileShapes[] = {
     {64, 64, 768.0, 0.17, 0.40, 0.55, 1.7},       // three workgroups per compute unit
     {128, 128, 512.0, 0.37, 0.71, 1.02, 4.2},     // two
@@ -507,13 +495,7 @@ void LaunchWork::add(int64_t m, int64_t n, int64_t k, bool symmetric, int64_t ba
 // Tiles of a shorter contraction count by their share of the longest one.
 double launch_us(TileKind kind, const LaunchWork& w) {
   if (w.max_ktiles == 0.0) return 0.0;
-  const TileShape& shape = kTileShapes[kind];
-  const double rounds = w.tile_ktiles[kind] / w.max_ktiles / shape.round, whole = floor(rounds), part = rounds - whole;
-  double per_ktile = whole * shape.full;
-  if (part > 0.0)
-    per_ktile += part <= 0.5 ? shape.empty + (shape.half - shape.empty) * 2.0 * part
-                             : shape.half + (shape.full - shape.half) * (2.0 * part - 1.0);
-  return 3.0 + per_ktile * w.max_ktiles + shape.ends * fmax(1.0, ceil(w.tiles[kind] / shape.round));
+  return rounds_us(kTileShapes[kind], w.tiles[kind], w.tile_ktiles[kind], w.max_ktiles);
 }
 TileKind small_tile_kind(const LaunchWork& w) {
   TileKind best = kTiles64;
