@@ -122,6 +122,7 @@ class MuonGroup(Structure):
 
 MAX_NS_PROBLEMS = 16
 MUON_PADDED = 1
+MAX_COPY_ROWS = 32
 NS_STATIC_SCRATCH_BYTES = 128 << 20
 
 
@@ -140,6 +141,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "fsh_quant_pack_plan_launch": (c_int, [c_void_p, c_void_p, c_void_p]),
     "fsh_quant_pack_plan_destroy": (None, [c_void_p]),
     "fsh_copy_segments": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int32, c_void_p]),
+    "fsh_copy_row_segments": (c_int, [c_void_p, c_int32, c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "fsh_zero_segments": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int32, c_void_p]),
     "fsh_pack_segments": (
         c_int,
@@ -152,6 +154,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "fsh_accumulate_grad": (c_int, [c_void_p, c_void_p, c_int32, c_int64, c_int32, c_void_p]),
     "fsh_reduce_rows_f32": (c_int, [c_void_p, c_void_p, c_int64, c_int32, c_int64, c_int64, c_int32, c_float, c_void_p]),
     "fsh_reduce_rows_bf16": (c_int, [c_void_p, c_void_p, c_int64, c_int32, c_int64, c_int64, c_int32, c_float, c_void_p]),
+    "fsh_reduce_rows_own": (
+        c_int,
+        [c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int64, c_int64, c_int32, c_int32, c_float, c_void_p],
+    ),
     "fsh_newton_schulz_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64]),
     "fsh_newton_schulz": (
         c_int,

@@ -81,9 +81,22 @@ __device__ __forceinline__ float fold_finish(float s, float factor) {
   return s;
 }
 
+// Row r of the contributions: row `own` (-1: none) lies somewhere else, at
+// own_src -- this rank's own gradients, which need not be copied into the
+// contributions first (a copy of the whole row, `world` times what the fold
+// reads of it: 360 us beside a 169 us fold of a layer's gradients).
+template <typename T>
+struct ContributionRows {
+  const T* src;
+  int64_t stride;
+  const T* own_src;
+  int own;
+  __device__ __forceinline__ const T* operator()(int r) const { return r == own ? own_src : src + r * stride; }
+};
+
 template <int MODE>
 __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(float* __restrict__ out,
-                                                              const float* __restrict__ src, int64_t stride,
+                                                              const ContributionRows<float> rows,
                                                               int world, int64_t n, float factor, int vec_ok) {
   const int64_t tid = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   const int64_t nthreads = static_cast<int64_t>(gridDim.x) * kThreads;
@@ -91,11 +104,11 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(float* __restrict
   if (vec_ok) {
     const int64_t groups = n / 4;
     for (int64_t gidx = tid; gidx < groups; gidx += nthreads) {
-      f32x4 s = load_stream_f32x4(src + gidx * 4);
+      f32x4 s = load_stream_f32x4(rows(0) + gidx * 4);
       s = f32x4{fold_term<MODE>(s.x, factor), fold_term<MODE>(s.y, factor), fold_term<MODE>(s.z, factor),
                 fold_term<MODE>(s.w, factor)};
       for (int r = 1; r < world; ++r) {
-        const f32x4 v = load_stream_f32x4(src + r * stride + gidx * 4);
+        const f32x4 v = load_stream_f32x4(rows(r) + gidx * 4);
         s.x = s.x + fold_term<MODE>(v.x, factor);
         s.y = s.y + fold_term<MODE>(v.y, factor);
         s.z = s.z + fold_term<MODE>(v.z, factor);
@@ -108,8 +121,8 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(float* __restrict
     done = groups * 4;
   }
   for (int64_t i = done + tid; i < n; i += nthreads) {
-    float s = fold_term<MODE>(src[i], factor);
-    for (int r = 1; r < world; ++r) s = s + fold_term<MODE>(src[r * stride + i], factor);
+    float s = fold_term<MODE>(rows(0)[i], factor);
+    for (int r = 1; r < world; ++r) s = s + fold_term<MODE>(rows(r)[i], factor);
     out[i] = fold_finish<MODE>(s, factor);
   }
 }
@@ -119,9 +132,8 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(float* __restrict
 // result is rounded to bf16 once.
 template <int MODE>
 __global__ __launch_bounds__(kThreads) void reduce_rows_bf16_kernel(uint16_t* __restrict__ out,
-                                                                   const uint16_t* __restrict__ src,
-                                                                   int64_t stride, int world, int64_t n,
-                                                                   float factor, int vec_ok) {
+                                                                   const ContributionRows<uint16_t> rows, int world,
+                                                                   int64_t n, float factor, int vec_ok) {
   const int64_t tid = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   const int64_t nthreads = static_cast<int64_t>(gridDim.x) * kThreads;
   int64_t done = 0;
@@ -129,11 +141,11 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_bf16_kernel(uint16_t* __
     const int64_t groups = n / 8;
     for (int64_t gidx = tid; gidx < groups; gidx += nthreads) {
       float s[8], v[8];
-      unpack8(load_stream_u32x4(src + gidx * 8), s);
+      unpack8(load_stream_u32x4(rows(0) + gidx * 8), s);
 #pragma unroll
       for (int j = 0; j < 8; ++j) s[j] = fold_term<MODE>(s[j], factor);
       for (int r = 1; r < world; ++r) {
-        unpack8(load_stream_u32x4(src + r * stride + gidx * 8), v);
+        unpack8(load_stream_u32x4(rows(r) + gidx * 8), v);
 #pragma unroll
         for (int j = 0; j < 8; ++j) s[j] = s[j] + fold_term<MODE>(v[j], factor);
       }
@@ -145,8 +157,8 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_bf16_kernel(uint16_t* __
     done = groups * 8;
   }
   for (int64_t i = done + tid; i < n; i += nthreads) {
-    float s = fold_term<MODE>(bf16_bits_to_f32(src[i]), factor);
-    for (int r = 1; r < world; ++r) s = s + fold_term<MODE>(bf16_bits_to_f32(src[r * stride + i]), factor);
+    float s = fold_term<MODE>(bf16_bits_to_f32(rows(0)[i]), factor);
+    for (int r = 1; r < world; ++r) s = s + fold_term<MODE>(bf16_bits_to_f32(rows(r)[i]), factor);
     out[i] = static_cast<uint16_t>(f32_to_bf16_bits(fold_finish<MODE>(s, factor)));
   }
 }
@@ -298,36 +310,76 @@ FSH_API int fsh_accumulate_grad(float* acc_dev, const void* grad_dev, int32_t gr
   return check_launch("fsh_accumulate_grad");
 }
 
+namespace fsh {
+namespace {
+
+template <int MODE>
+void launch_fold(float* out, const ContributionRows<float>& rows, int world, int64_t n, float factor, int vec_ok, hipStream_t s) {
+  hipLaunchKernelGGL((reduce_rows_kernel<MODE>), dim3(grid_for(ceil_div(n, 4))), dim3(kThreads), 0, s, out, rows, world, n, factor, vec_ok);
+}
+template <int MODE>
+void launch_fold(uint16_t* out, const ContributionRows<uint16_t>& rows, int world, int64_t n, float factor, int vec_ok, hipStream_t s) {
+  hipLaunchKernelGGL((reduce_rows_bf16_kernel<MODE>), dim3(grid_for(ceil_div(n, 8))), dim3(kThreads), 0, s, out, rows, world, n, factor, vec_ok);
+}
+
+// own < 0: every row is read from src.
+template <typename T>
+int reduce_rows(const char* who, void* out_dev, const void* src_dev, int64_t contribution_stride, int32_t world,
+                int32_t own, const void* own_dev, int64_t column_offset, int64_t numel, int32_t mode, float factor,
+                void* stream) {
+  if (numel < 0 || world <= 0 || column_offset < 0 || contribution_stride < 0 || own >= world)
+    return fail(FSH_EINVAL, "%s: bad sizes (world %d, own rank %d, numel %lld)", who, world, own, (long long)numel);
+  if (numel == 0) return FSH_OK;
+  const bool needs_src = own < 0 || world > 1;
+  if (!out_dev || (needs_src && !src_dev) || (own >= 0 && !own_dev)) return fail(FSH_EINVAL, "%s: null pointer", who);
+  if (!aligned(out_dev, sizeof(T)) || !aligned(src_dev, sizeof(T)) || !aligned(own_dev, sizeof(T)))
+    return fail(FSH_EINVAL, "%s: misaligned", who);
+  if (mode < FSH_REDUCE_SUM || mode > FSH_REDUCE_POSTDIV) return fail(FSH_EINVAL, "%s: unknown mode %d", who, mode);
+  ContributionRows<T> rows;
+  rows.own = own < 0 ? -1 : own;
+  rows.own_src = own < 0 ? nullptr : static_cast<const T*>(own_dev) + column_offset;
+  rows.src = needs_src ? static_cast<const T*>(src_dev) + column_offset : rows.own_src;
+  rows.stride = contribution_stride;
+  const int vec_ok = aligned(out_dev, 16) && aligned(rows.src, 16) && aligned(rows.own_src, 16) &&
+                     contribution_stride % static_cast<int64_t>(16 / sizeof(T)) == 0;
+  T* out = static_cast<T*>(out_dev);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (mode) {
+    case FSH_REDUCE_SUM: launch_fold<FSH_REDUCE_SUM>(out, rows, world, numel, factor, vec_ok, s); break;
+    case FSH_REDUCE_PREMUL: launch_fold<FSH_REDUCE_PREMUL>(out, rows, world, numel, factor, vec_ok, s); break;
+    case FSH_REDUCE_POSTMUL: launch_fold<FSH_REDUCE_POSTMUL>(out, rows, world, numel, factor, vec_ok, s); break;
+    default: launch_fold<FSH_REDUCE_POSTDIV>(out, rows, world, numel, factor, vec_ok, s); break;
+  }
+  return check_launch(who);
+}
+
+}  // namespace
+}  // namespace fsh
+
 FSH_API int fsh_reduce_rows_f32(float* out_dev, const float* src_dev, int64_t contribution_stride,
                                 int32_t world, int64_t column_offset, int64_t numel, int32_t mode,
                                 float factor, void* stream) {
+  return fsh::reduce_rows<float>("fsh_reduce_rows_f32", out_dev, src_dev, contribution_stride, world, -1, nullptr,
+                                 column_offset, numel, mode, factor, stream);
+}
+
+FSH_API int fsh_reduce_rows_bf16(void* out_dev, const void* src_dev, int64_t contribution_stride, int32_t world,
+                                 int64_t column_offset, int64_t numel, int32_t mode, float factor, void* stream) {
+  return fsh::reduce_rows<uint16_t>("fsh_reduce_rows_bf16", out_dev, src_dev, contribution_stride, world, -1, nullptr,
+                                    column_offset, numel, mode, factor, stream);
+}
+
+FSH_API int fsh_reduce_rows_own(void* out_dev, const void* src_dev, int64_t contribution_stride, int32_t world,
+                                int32_t own_rank, const void* own_dev, int64_t column_offset, int64_t numel,
+                                int32_t dtype, int32_t mode, float factor, void* stream) {
   using namespace fsh;
-  if (numel < 0 || world <= 0 || column_offset < 0 || contribution_stride < 0)
-    return fail(FSH_EINVAL, "fsh_reduce_rows_f32: bad sizes (world %d, numel %lld)", world, (long long)numel);
-  if (numel == 0) return FSH_OK;
-  if (!out_dev || !src_dev) return fail(FSH_EINVAL, "fsh_reduce_rows_f32: null pointer");
-  if (!aligned(out_dev, 4) || !aligned(src_dev, 4)) return fail(FSH_EINVAL, "fsh_reduce_rows_f32: misaligned");
-  if (mode < FSH_REDUCE_SUM || mode > FSH_REDUCE_POSTDIV)
-    return fail(FSH_EINVAL, "fsh_reduce_rows_f32: unknown mode %d", mode);
-  const float* src = src_dev + column_offset;
-  const int vec_ok = aligned(out_dev, 16) && aligned(src, 16) && (contribution_stride % 4 == 0);
-  const dim3 g(grid_for(ceil_div(numel, 4))), b(kThreads);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (mode) {
-    case FSH_REDUCE_SUM:
-      hipLaunchKernelGGL((reduce_rows_kernel<FSH_REDUCE_SUM>), g, b, 0, s, out_dev, src, contribution_stride, world, numel, factor, vec_ok);
-      break;
-    case FSH_REDUCE_PREMUL:
-      hipLaunchKernelGGL((reduce_rows_kernel<FSH_REDUCE_PREMUL>), g, b, 0, s, out_dev, src, contribution_stride, world, numel, factor, vec_ok);
-      break;
-    case FSH_REDUCE_POSTMUL:
-      hipLaunchKernelGGL((reduce_rows_kernel<FSH_REDUCE_POSTMUL>), g, b, 0, s, out_dev, src, contribution_stride, world, numel, factor, vec_ok);
-      break;
-    default:
-      hipLaunchKernelGGL((reduce_rows_kernel<FSH_REDUCE_POSTDIV>), g, b, 0, s, out_dev, src, contribution_stride, world, numel, factor, vec_ok);
-      break;
-  }
-  return check_launch("fsh_reduce_rows_f32");
+  if (own_rank < 0) return fail(FSH_EINVAL, "fsh_reduce_rows_own: negative rank %d", own_rank);
+  if (dtype != FSH_DT_F32 && dtype != FSH_DT_BF16) return fail(FSH_EINVAL, "fsh_reduce_rows_own: unsupported dtype %d", dtype);
+  return dtype == FSH_DT_F32
+             ? reduce_rows<float>("fsh_reduce_rows_own", out_dev, src_dev, contribution_stride, world, own_rank, own_dev,
+                                  column_offset, numel, mode, factor, stream)
+             : reduce_rows<uint16_t>("fsh_reduce_rows_own", out_dev, src_dev, contribution_stride, world, own_rank,
+                                     own_dev, column_offset, numel, mode, factor, stream);
 }
 
 FSH_API int fsh_muon_prepare(void* momentum_dev, const void* grad_dev, void* out_dev, int64_t numel,
@@ -392,34 +444,3 @@ FSH_API int fsh_muon_apply_f32(float* param_dev, const void* direction_dev, int6
   return check_launch("fsh_muon_apply_f32");
 }
 
-FSH_API int fsh_reduce_rows_bf16(void* out_dev, const void* src_dev, int64_t contribution_stride, int32_t world,
-                                 int64_t column_offset, int64_t numel, int32_t mode, float factor, void* stream) {
-  using namespace fsh;
-  if (numel < 0 || world <= 0 || column_offset < 0 || contribution_stride < 0)
-    return fail(FSH_EINVAL, "fsh_reduce_rows_bf16: bad sizes (world %d, numel %lld)", world, (long long)numel);
-  if (numel == 0) return FSH_OK;
-  if (!out_dev || !src_dev) return fail(FSH_EINVAL, "fsh_reduce_rows_bf16: null pointer");
-  if (!aligned(out_dev, 2) || !aligned(src_dev, 2)) return fail(FSH_EINVAL, "fsh_reduce_rows_bf16: misaligned");
-  if (mode < FSH_REDUCE_SUM || mode > FSH_REDUCE_POSTDIV)
-    return fail(FSH_EINVAL, "fsh_reduce_rows_bf16: unknown mode %d", mode);
-  const uint16_t* src = static_cast<const uint16_t*>(src_dev) + column_offset;
-  uint16_t* out = static_cast<uint16_t*>(out_dev);
-  const int vec_ok = aligned(out, 16) && aligned(src, 16) && (contribution_stride % 8 == 0);
-  const dim3 g(grid_for(ceil_div(numel, 8))), b(kThreads);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (mode) {
-    case FSH_REDUCE_SUM:
-      hipLaunchKernelGGL((reduce_rows_bf16_kernel<FSH_REDUCE_SUM>), g, b, 0, s, out, src, contribution_stride, world, numel, factor, vec_ok);
-      break;
-    case FSH_REDUCE_PREMUL:
-      hipLaunchKernelGGL((reduce_rows_bf16_kernel<FSH_REDUCE_PREMUL>), g, b, 0, s, out, src, contribution_stride, world, numel, factor, vec_ok);
-      break;
-    case FSH_REDUCE_POSTMUL:
-      hipLaunchKernelGGL((reduce_rows_bf16_kernel<FSH_REDUCE_POSTMUL>), g, b, 0, s, out, src, contribution_stride, world, numel, factor, vec_ok);
-      break;
-    default:
-      hipLaunchKernelGGL((reduce_rows_bf16_kernel<FSH_REDUCE_POSTDIV>), g, b, 0, s, out, src, contribution_stride, world, numel, factor, vec_ok);
-      break;
-  }
-  return check_launch("fsh_reduce_rows_bf16");
-}

@@ -28,6 +28,25 @@ __global__ __launch_bounds__(kThreads) void copy_segments_kernel(
              kThreads);
 }
 
+// Segments of several separately allocated source rows, whose addresses come
+// with the launch: the tables then depend on the layout alone, and new rows
+// need neither an upload nor a table of their own.
+struct RowPointers {
+  const uint8_t* row[FSH_MAX_COPY_ROWS];
+};
+__global__ __launch_bounds__(kThreads) void copy_row_segments_kernel(const RowPointers rows, uint8_t* __restrict__ dst,
+                                                                    const int64_t* __restrict__ table, int64_t nsegments,
+                                                                    int64_t slices_per_segment) {
+  const int64_t seg = blockIdx.x / slices_per_segment;
+  const int64_t slice = blockIdx.x - seg * slices_per_segment;
+  const int64_t nbytes = table[2 * nsegments + seg];
+  const int64_t begin = slice * kSliceBytes;
+  if (begin >= nbytes) return;
+  const int64_t len = (nbytes - begin) < kSliceBytes ? (nbytes - begin) : kSliceBytes;
+  copy_bytes(rows.row[table[seg]] + table[nsegments + seg] + begin, dst + table[3 * nsegments + seg] + begin, len,
+             threadIdx.x, kThreads);
+}
+
 __global__ __launch_bounds__(kThreads) void zero_segments_kernel(uint8_t* __restrict__ dst,
                                                                 const int64_t* __restrict__ numels,
                                                                 const int64_t* __restrict__ dst_offsets,
@@ -148,6 +167,27 @@ FSH_API int fsh_copy_segments(const void* src_dev, void* dst_dev, const int64_t*
                      static_cast<uint8_t*>(dst_dev), src_offsets_dev, numels_dev, dst_offsets_dev, slices,
                      static_cast<int64_t>(unit_nbytes));
   return check_launch("fsh_copy_segments");
+}
+
+FSH_API int fsh_copy_row_segments(const void* const* rows, int32_t nrows, void* dst_dev, const int64_t* table_dev,
+                                  int64_t nsegments, int64_t max_segment_nbytes, void* stream) {
+  using namespace fsh;
+  if (nsegments < 0 || max_segment_nbytes < 0 || nrows < 0) return fail(FSH_EINVAL, "fsh_copy_row_segments: negative size");
+  if (nsegments == 0 || max_segment_nbytes == 0) return FSH_OK;
+  if (nrows == 0 || nrows > FSH_MAX_COPY_ROWS)
+    return fail(FSH_EINVAL, "fsh_copy_row_segments: %d rows, not 1 to %d", nrows, FSH_MAX_COPY_ROWS);
+  if (!rows || !dst_dev || !table_dev) return fail(FSH_EINVAL, "fsh_copy_row_segments: null pointer");
+  RowPointers p;
+  for (int i = 0; i < FSH_MAX_COPY_ROWS; ++i) {
+    p.row[i] = static_cast<const uint8_t*>(rows[i < nrows ? i : nrows - 1]);
+    if (!p.row[i]) return fail(FSH_EINVAL, "fsh_copy_row_segments: row %d is null", i);
+  }
+  const int64_t slices = ceil_div(max_segment_nbytes, kSliceBytes);
+  const int64_t grid = nsegments * slices;
+  if (grid > 0x7FFFFFFFLL) return fail(FSH_ENOTSUP, "fsh_copy_row_segments: %lld workgroups exceed the grid limit", (long long)grid);
+  hipLaunchKernelGGL(copy_row_segments_kernel, dim3(static_cast<uint32_t>(grid)), dim3(kThreads), 0,
+                     static_cast<hipStream_t>(stream), p, static_cast<uint8_t*>(dst_dev), table_dev, nsegments, slices);
+  return check_launch("fsh_copy_row_segments");
 }
 
 FSH_API int fsh_zero_segments(void* dst_dev, const int64_t* numels_dev, const int64_t* dst_offsets_dev,

@@ -97,6 +97,40 @@ def copy_segments(source: torch.Tensor, output: torch.Tensor, descriptor: Segmen
     )
 
 
+@dataclass
+class RowCopyDescriptor:
+    """Byte segments ``(row, source offset, nbytes, destination offset)`` of
+    separately allocated source rows, on the device: the layout alone, since
+    the rows' addresses come with every launch."""
+
+    table: torch.Tensor
+    max_nbytes: int
+    _staged_host: torch.Tensor
+
+    @classmethod
+    def create(
+        cls, segments: Sequence[tuple[int, int, int, int]], device: torch.device, max_piece_nbytes: int = 131072
+    ) -> "RowCopyDescriptor":
+        # Long segments are cut so that a launch sized by the longest piece does not idle on the short ones.
+        piece = max_piece_nbytes
+        while sum(-(-n // piece) for _, _, n, _ in segments) > _MAX_SEGMENTS:
+            piece *= 2
+        columns: list[list[int]] = [[], [], [], []]
+        for row, src, nbytes, dst in segments:
+            for done in range(0, nbytes, piece):
+                step = min(piece, nbytes - done)
+                for column, value in zip(columns, (row, src + done, step, dst + done)):
+                    column.append(value)
+        table, host = _upload_i64([v for column in columns for v in column], device)
+        return cls(table.view(4, -1), max(columns[2], default=0), host)
+
+
+def copy_row_segments(rows: Sequence[torch.Tensor], output: torch.Tensor, descriptor: RowCopyDescriptor) -> None:
+    """Copy every segment of ``descriptor`` from ``rows`` to ``output`` in one launch."""
+    if descriptor.max_nbytes:
+        hip_ops.copy_row_segments(rows, output, descriptor.table, descriptor.max_nbytes)
+
+
 def zero_segments(output: torch.Tensor, descriptor: SegmentCopyDescriptor) -> None:
     """Zero the destination segments of ``descriptor`` in one launch."""
     if descriptor.nsegments == 0 or descriptor.max_segment_numel == 0:
@@ -230,8 +264,10 @@ def pack_segments_into_flat_buffer(
 
 
 __all__ = [
+    "RowCopyDescriptor",
     "SegmentCopyDescriptor",
     "SegmentPackDescriptor",
+    "copy_row_segments",
     "copy_segments",
     "pack_segments_into_flat_buffer",
     "zero_segments",

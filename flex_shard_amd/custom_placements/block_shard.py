@@ -33,12 +33,20 @@ from ..placement_contract import (
 )
 from .. import hip_ops
 from ..profiling import record_comm, record_copy_in, record_copy_out, record_range
-from ._copy_kernels import SegmentCopyDescriptor, SegmentPackDescriptor, copy_segments, pack_segments_into_flat_buffer
+from ._copy_kernels import (
+    RowCopyDescriptor,
+    SegmentCopyDescriptor,
+    SegmentPackDescriptor,
+    copy_row_segments,
+    copy_segments,
+    pack_segments_into_flat_buffer,
+)
 from .utils import (
     all_gather_rows,
     copy_tensor_to_dtype,
     foreach_copy_,
     group_size,
+    local_exchange_rows,
     pack_segments_into_flat_buffer_if_supported,
     pack_tensors_into_flat_buffer_with_scratch,
     reduce_scatter_grads,
@@ -515,7 +523,10 @@ class BucketedBlockShard(Placement):
             bucket = send.new_empty(layout.global_numel)
             prepared.buffers.insert(1, bucket)
         world_size = group_size(state.pg)
-        target = bucket if world_size * send.numel() == bucket.numel() else bucket.new_empty(world_size * send.numel())
+        even = world_size * send.numel() == bucket.numel()
+        if not even and self._copy_local_rows_into_bucket(bucket, send, state.pg, layout):
+            return None
+        target = bucket if even else bucket.new_empty(world_size * send.numel())
         with record_comm("FlexShard::all_gather", state.debug_fqn):
             work = all_gather_rows(target, send, state.pg, async_op=async_op)
         if target is not bucket:
@@ -524,6 +535,35 @@ class BucketedBlockShard(Placement):
                 work = None
             self._scatter_padded_rows_into_bucket(bucket, target.view(world_size, -1), layout)
         return work
+
+    def _copy_local_rows_into_bucket(
+        self, bucket: torch.Tensor, send: torch.Tensor, group: Any, layout: "BucketLayout"
+    ) -> bool:
+        """The exchange and the copy-out of uneven ranges in one launch, where
+        the exchange is local and every rank's row can be read where it lies:
+        no padded gathered rows in between."""
+        rows = local_exchange_rows(group, send)
+        if rows is None or len(rows) != len(layout.rank_numels) or bucket.dtype != send.dtype or not bucket.is_contiguous():
+            return False
+        # (a table is uploaded on the stream it is first used on: one per stream)
+        key = ("rows", id(layout), send.numel(), bucket.dtype, bucket.device, hip_ops.stream_ptr(bucket.device))
+        cached = self._scatter_descriptors.get(key)
+        if cached is None or cached[0] is not layout:
+            size = bucket.element_size()
+            descriptor = RowCopyDescriptor.create(
+                [
+                    (rank, 0, count * size, start * size)
+                    for rank, (start, count) in enumerate(zip(layout.rank_offsets, layout.rank_numels, strict=True))
+                    if count
+                ],
+                bucket.device,
+            )
+            if len(self._scatter_descriptors) >= 16:
+                self._scatter_descriptors.clear()
+            self._scatter_descriptors[key] = cached = (layout, descriptor)
+        with record_copy_out():
+            copy_row_segments(rows, bucket, cached[1])
+        return True
 
     def _scatter_padded_rows_into_bucket(self, bucket: torch.Tensor, rows: torch.Tensor, layout: "BucketLayout") -> None:
         """Copy each rank's valid prefix of its padded gathered row into its

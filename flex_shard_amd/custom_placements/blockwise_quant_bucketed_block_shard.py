@@ -35,13 +35,13 @@ from ..placement_contract import (
 )
 from ..profiling import record_comm, record_copy_in, record_copy_out
 from . import quant_plan
-from ._copy_kernels import SegmentCopyDescriptor, copy_segments
+from ._copy_kernels import RowCopyDescriptor, SegmentCopyDescriptor, copy_row_segments, copy_segments
 from .block_shard import BucketedBlockShard
 from .quant_plan import ScaleRegion as _ScaleRegion
 from .quant_plan import align_up as _align_up
 from .quant_plan import ceil_div as _ceil_div
 from .quant_plan import matrix_shape as _matrix_shape
-from .utils import all_gather_rows
+from .utils import all_gather_rows, local_exchange_rows
 
 if TYPE_CHECKING:
     from ..bucket_storage import ParamInfo
@@ -849,19 +849,44 @@ class BlockwiseQuantBucketedBlockShard(BucketedBlockShard):
         copy-out to finish."""
         state = self._unshard_state(prepared)
         local, gathered = prepared.buffers
+        refills = (
+            self.refill_behind_exchange and prepared.persistent_buffers is not None and not torch.compiler.is_compiling()
+        )
+        if refills and self._refill_from_local_rows(state, local, prepared.persistent_buffers[0]):
+            return None
         with record_comm("FlexShard::all_gather", state.debug_fqn):
             work = all_gather_rows(gathered, local, state.pg, async_op=async_op)
-        if (
-            self.refill_behind_exchange
-            and work is None
-            and prepared.persistent_buffers is not None
-            and not torch.compiler.is_compiling()
-        ):
+        if refills and work is None:
             rows = gathered.view(len(state.metadata.rank_qdata_numels), local.numel())
             self._check_rank_rows(state, rows)
             with record_copy_out():
                 state.copied_out = self._copy_out_rank_rows_fused(state.metadata, rows, prepared.persistent_buffers[0])
         return work
+
+    def _refill_from_local_rows(self, state: "_QuantUnshardState", local: torch.Tensor, compact: torch.Tensor) -> bool:
+        """The exchange and the copy-out of a refill in one launch, where the
+        exchange is local and every rank's row can be read where it lies: the
+        gathered rows, which nothing reads behind the copy-out, are then
+        neither written nor read back (half of the 290 us the two copies of a
+        Llama-3-8B layer's 218 MB took together)."""
+        rows = local_exchange_rows(state.pg, local)
+        metadata = state.metadata
+        if (
+            rows is None
+            or len(rows) != len(metadata.rank_qdata_numels)
+            or local.dtype != torch.uint8
+            or local.numel() != metadata.packed_send_nbytes_per_rank
+        ):
+            return False
+        plan = self._copy_out_plan(metadata, data_elem_nbytes=1, with_scales=True)
+        key = ("rows", compact.device, hip_ops.stream_ptr(compact.device))  # a table is uploaded on the stream it is first used on
+        descriptor = plan.descriptors.get(key)
+        if descriptor is None:
+            descriptor = plan.descriptors[key] = RowCopyDescriptor.create(plan.regions, compact.device)
+        with record_copy_out():
+            copy_row_segments(rows, compact, descriptor)
+        state.copied_out = True
+        return True
 
     def finish_prepared_unshard(self, prepared: PlacementPreparedUnshard) -> PlacementUnshardResult:
         state = self._unshard_state(prepared)

@@ -17,10 +17,11 @@ import torch
 import torch.distributed as dist
 
 from .. import hip_ops
+from .._native import MAX_COPY_ROWS
 from ._copy_kernels import (
-    SegmentCopyDescriptor,
+    RowCopyDescriptor,
     SegmentPackDescriptor,
-    copy_segments,
+    copy_row_segments,
     pack_segments_into_flat_buffer,
 )
 
@@ -248,7 +249,7 @@ def all_gather_rows(output: torch.Tensor, input: torch.Tensor, group: Any, *, as
         missing = sorted(set(range(world)) - {rank} - set(group.gather_rows))
         if missing:
             raise ValueError(f"LocalReduceGroup is missing the all-gather rows of ranks {missing}.")
-        if _gather_rows_in_one_launch(group, rows, input, rank):
+        if _gather_rows_in_one_launch(group, rows, input):
             return None
         rows[rank].copy_(input.reshape(-1))
         for other, row in group.gather_rows.items():
@@ -260,44 +261,57 @@ def all_gather_rows(output: torch.Tensor, input: torch.Tensor, group: Any, *, as
     return dist.all_gather_into_tensor(output, input, group=group, async_op=async_op)
 
 
-def _gather_rows_in_one_launch(group: LocalReduceGroup, rows: torch.Tensor, input: torch.Tensor, rank: int) -> bool:
-    """The local all-gather as one segment-copy launch (a device copy per row
-    through the runtime's copy engine path runs at a sixth of the memory
-    rate): every row is a segment whose source offset counts from this rank's
-    ``input``.  The descriptor tables are kept per set of addresses, which
-    repeat from step to step.  False when the rows do not qualify."""
-    if torch.compiler.is_compiling() or rows.device.type != "cuda" or not rows.is_contiguous():
-        return False
-    world, n = rows.shape
-    size = rows.element_size()
-    sources = {rank: input.reshape(-1), **{r: row.reshape(-1) for r, row in group.gather_rows.items() if r != rank}}
-    base = sources[rank].data_ptr()
+def local_exchange_rows(group: Any, input: torch.Tensor) -> list[torch.Tensor] | None:
+    """The rows a local all-gather of ``input`` consists of, in rank order,
+    when one launch can read them all where they lie (a
+    :class:`LocalReduceGroup` whose rows are contiguous GPU tensors of
+    ``input``'s dtype and length); None otherwise."""
+    if not isinstance(group, LocalReduceGroup) or group.local_row_only or torch.compiler.is_compiling():
+        return None
+    world, rank = group.size(), group.rank()
+    if world > MAX_COPY_ROWS or input.device.type != "cuda":
+        return None
+    dtype, numel, device = input.dtype, input.numel(), input.device
+    rows = []
     for r in range(world):
-        src = sources[r]
-        if src.device != rows.device or src.dtype != rows.dtype or src.numel() != n or not src.is_contiguous():
-            return False
-        if (src.data_ptr() - base) % size:
-            return False
-    key = (rows.data_ptr(), tuple(sources[r].data_ptr() for r in range(world)), n, size)
+        row = input if r == rank else group.gather_rows.get(r)
+        if row is None or row.dtype != dtype or row.numel() != numel or row.device != device or not row.is_contiguous():
+            return None
+        rows.append(row)
+    return rows
+
+
+def _gather_rows_in_one_launch(group: LocalReduceGroup, rows: torch.Tensor, input: torch.Tensor) -> bool:
+    """The local all-gather as one launch (a device copy per row through the
+    runtime's copy engine path runs at a sixth of the memory rate).  False
+    when the rows do not qualify."""
+    sources = local_exchange_rows(group, input)
+    if sources is None or not rows.is_contiguous() or rows.dtype != input.dtype or rows.device != input.device:
+        return False
+    nbytes = input.numel() * input.element_size()
+    # (a table is uploaded on the stream it is first used on: one per stream)
+    key = (nbytes, rows.device, hip_ops.stream_ptr(rows.device))
     descriptor = group._gather_descriptors.get(key)
     if descriptor is None:
         if len(group._gather_descriptors) >= 64:
             group._gather_descriptors.clear()
-        descriptor = group._gather_descriptors[key] = SegmentCopyDescriptor.create(
-            src_offsets=[(sources[r].data_ptr() - base) // size for r in range(world)],
-            numels=[n] * world,
-            dst_offsets=[r * n for r in range(world)],
-            device=rows.device,
+        descriptor = group._gather_descriptors[key] = RowCopyDescriptor.create(
+            [(r, 0, nbytes, r * nbytes) for r in range(len(sources))], rows.device
         )
-    copy_segments(sources[rank], rows.view(-1), descriptor)
+    copy_row_segments(sources, rows, descriptor)
     return True
 
 
-def _local_reduce(output: torch.Tensor, group: LocalReduceGroup, reduction: "GradientReduction") -> None:
+def _local_reduce(
+    output: torch.Tensor, group: LocalReduceGroup, reduction: "GradientReduction", own: torch.Tensor | None = None
+) -> None:
+    """``own``: this rank's contribution, read where it lies instead of from its row of the deposited ones."""
     contributions = group.contributions
+    world = group.size()
+    if contributions is None and own is not None and world == 1:
+        contributions = own.view(1, -1)
     if contributions is None:
         raise ValueError("LocalReduceGroup has no contributions; deposit every rank's send buffer first.")
-    world = group.size()
     segment = output.numel()
     if contributions.shape != (world, world * segment):
         raise ValueError(
@@ -313,7 +327,10 @@ def _local_reduce(output: torch.Tensor, group: LocalReduceGroup, reduction: "Gra
         mode, factor = hip_ops.REDUCE_PREMUL, 1.0 / pre
     else:
         mode, factor = hip_ops.REDUCE_SUM, 1.0
-    hip_ops.reduce_rows(output, contributions, group.rank() * segment, mode=mode, factor=factor)
+    hip_ops.reduce_rows(
+        output, contributions, group.rank() * segment, mode=mode, factor=factor,
+        own_row=None if own is None else (group.rank(), own),
+    )
     if post is not None:
         output.div_(post)
 
@@ -322,16 +339,24 @@ def reduce_scatter_grads(output: torch.Tensor, input: torch.Tensor, reduction: "
     """Reduce-scatter packed gradients into ``output`` as ``reduction`` asks.
 
     With a :class:`LocalReduceGroup` the reduction runs on this GPU (``input``
-    is deposited as this rank's contribution unless already present) and
-    consumes the deposits; with a
+    is this rank's contribution, read where it lies, unless one was deposited)
+    and consumes the deposits; with a
     ``torch.distributed`` group it is one collective, as in the reference."""
     if isinstance(group, LocalReduceGroup):
+        own = None
         if group.rank() not in group.deposited:
-            group.deposit(group.rank(), input)
+            held = group.contributions
+            if input.is_contiguous() and input.device.type == "cuda" and input.dtype == output.dtype and (
+                held is None or (held.dtype == input.dtype and held.device == input.device)
+            ):
+                own = input.view(-1)
+                group.mark_deposited(group.rank())
+            else:
+                group.deposit(group.rank(), input)
         missing = sorted(set(range(group.size())) - group.deposited)
         if missing:
             raise ValueError(f"LocalReduceGroup is missing the contributions of ranks {missing}.")
-        _local_reduce(output, group, reduction)
+        _local_reduce(output, group, reduction, own)
         group.deposited.clear()  # consumed: the next reduction needs fresh contributions
         return
     if group is None:
@@ -377,6 +402,7 @@ __all__ = [
     "foreach_copy_",
     "gradient_reduce_plan",
     "group_size",
+    "local_exchange_rows",
     "make_segment_pack_descriptor_if_supported",
     "pack_segments_into_flat_buffer_if_supported",
     "pack_tensors_into_flat_buffer",

@@ -35,7 +35,7 @@ __all__ = [
     "DT_BF16", "DT_F16", "DT_F32", "EPS_FP32", "EPS_INPUT_DTYPE", "REDUCE_POSTDIV", "REDUCE_POSTMUL",
     "REDUCE_PREMUL", "REDUCE_SUM", "SRC_BF16", "SRC_F16", "SRC_F32", "SRC_F32_AS_BF16", "SRC_F32_AS_F16",
     "MuonStepPlan", "QuantChunkSpec", "QuantPackPlan", "accumulate_grad", "act_quant_128x1_transposed", "act_quant_1x128", "act_quant_both",
-    "copy_segments", "fp8_gemm_1x128_128x1", "fp8_gemm_1x128_128x128", "fp8_gemm_1x128_128x128_dgrad",
+    "copy_row_segments", "copy_segments", "fp8_gemm_1x128_128x1", "fp8_gemm_1x128_128x128", "fp8_gemm_1x128_128x128_dgrad",
     "fp8_transpose", "gemm_nt", "gemm_nt_group", "muon_apply", "muon_prepare", "newton_schulz_multi",
     "newton_schulz", "newton_schulz_noalloc", "newton_schulz_workspace_bytes", "pack_segments", "quantize_pack",
     "reduce_rows", "stream_ptr", "unpack_dequant", "zero_segments",
@@ -212,6 +212,27 @@ def copy_segments(
     _native.check(status, "fsh_copy_segments")
 
 
+def copy_row_segments(
+    rows: Sequence[torch.Tensor], output: torch.Tensor, table: torch.Tensor, max_segment_nbytes: int
+) -> None:
+    """Copy byte segments of separately allocated source rows into ``output``:
+    ``table`` is int64 [4, n] (row index, byte offset in the row, bytes, byte
+    offset in the output).  The rows' addresses are taken from the tensors on
+    every call; the caller guarantees that the table stays inside rows and
+    output."""
+    _require_gpu(output, table, *rows)
+    if table.dtype != torch.int64 or table.ndim != 2 or table.shape[0] != 4 or not table.is_contiguous():
+        raise ValueError("the segment table must be a contiguous int64 tensor [4, n]")
+    if not 0 < len(rows) <= _native.MAX_COPY_ROWS:
+        raise ValueError(f"1 to {_native.MAX_COPY_ROWS} rows, got {len(rows)}")
+    addresses = (ctypes.c_void_p * len(rows))(*[row.data_ptr() for row in rows])
+    status = _native.lib().fsh_copy_row_segments(
+        addresses, len(rows), output.data_ptr(), table.data_ptr(), table.shape[1], max_segment_nbytes,
+        stream_ptr(output.device),
+    )
+    _native.check(status, "fsh_copy_row_segments")
+
+
 def zero_segments(output: torch.Tensor, numels: torch.Tensor, dst_offsets: torch.Tensor, max_segment_numel: int) -> None:
     _require_gpu(output, numels, dst_offsets)
     n = _check_i64_table(numels, dst_offsets)
@@ -289,11 +310,14 @@ def accumulate_grad(acc: torch.Tensor, grad: torch.Tensor, *, overwrite: bool = 
 
 
 def reduce_rows(
-    out: torch.Tensor, contributions: torch.Tensor, column_offset: int, *, mode: int = REDUCE_SUM, factor: float = 1.0
+    out: torch.Tensor, contributions: torch.Tensor, column_offset: int, *, mode: int = REDUCE_SUM, factor: float = 1.0,
+    own_row: tuple[int, torch.Tensor] | None = None,
 ) -> None:
     """``out[i] = fold_r contributions[r, column_offset + i]`` in rank order;
     ``contributions`` is [W, row] with unit column stride, fp32 or bf16 like
-    ``out`` (bf16 terms are added in fp32 and the sum rounded once)."""
+    ``out`` (bf16 terms are added in fp32 and the sum rounded once).
+    ``own_row`` ``(r, tensor)``: row ``r`` is read from that contiguous tensor
+    of ``row`` elements instead of from ``contributions``."""
     _require_gpu(out, contributions)
     if out.dtype != contributions.dtype or out.dtype not in (torch.float32, torch.bfloat16):
         raise NotImplementedError(
@@ -306,6 +330,17 @@ def reduce_rows(
     if column_offset < 0 or column_offset + out.numel() > row:
         raise ValueError(f"range [{column_offset}, {column_offset + out.numel()}) outside rows of {row} elements")
     stride = contributions.stride(0) if world > 1 else row
+    if own_row is not None:
+        own_rank, own = own_row
+        _require_gpu(out, own)
+        if not 0 <= own_rank < world or own.dtype != out.dtype or not own.is_contiguous() or own.numel() != row:
+            raise ValueError(f"own row {own_rank} must be one of {world} and a contiguous {out.dtype} tensor of {row} elements")
+        status = _native.lib().fsh_reduce_rows_own(
+            out.data_ptr(), contributions.data_ptr(), stride, world, own_rank, own.data_ptr(), column_offset, out.numel(),
+            _dt(out.dtype), mode, factor, stream_ptr(out.device),
+        )
+        _native.check(status, "fsh_reduce_rows_own")
+        return
     entry = "fsh_reduce_rows_f32" if out.dtype == torch.float32 else "fsh_reduce_rows_bf16"
     status = getattr(_native.lib(), entry)(
         out.data_ptr(), contributions.data_ptr(), stride, world, column_offset, out.numel(), mode, factor,

@@ -123,6 +123,14 @@ int fsh_copy_segments(const void* src_dev, void* dst_dev, const int64_t* src_off
                       int64_t nsegments, int64_t max_segment_numel, int32_t unit_nbytes,
                       void* stream);
 
+/* Segments of up to FSH_MAX_COPY_ROWS separately allocated rows (the rows of
+ * an exchange on one GPU), whose addresses are given on the host with every
+ * call.  table_dev: [4, nsegments] int64 -- row index, source byte offset
+ * within the row, bytes, destination byte offset. */
+#define FSH_MAX_COPY_ROWS 32
+int fsh_copy_row_segments(const void* const* rows, int32_t nrows, void* dst_dev, const int64_t* table_dev,
+                          int64_t nsegments, int64_t max_segment_nbytes, void* stream);
+
 int fsh_zero_segments(void* dst_dev, const int64_t* numels_dev, const int64_t* dst_offsets_dev,
                       int64_t nsegments, int64_t max_segment_numel, int32_t unit_nbytes,
                       void* stream);
@@ -200,6 +208,12 @@ int fsh_reduce_rows_f32(float* out_dev, const float* src_dev, int64_t contributi
  * stand-in does not imitate that.) */
 int fsh_reduce_rows_bf16(void* out_dev, const void* src_dev, int64_t contribution_stride, int32_t world,
                          int64_t column_offset, int64_t numel, int32_t mode, float factor, void* stream);
+/* The same fold with row `own_rank` read at own_dev (a row of its own,
+ * column_offset counting from its start) instead of src_dev; dtype FSH_DT_F32
+ * or FSH_DT_BF16.  src_dev may be null when world is 1. */
+int fsh_reduce_rows_own(void* out_dev, const void* src_dev, int64_t contribution_stride, int32_t world, int32_t own_rank,
+                        const void* own_dev, int64_t column_offset, int64_t numel, int32_t dtype, int32_t mode,
+                        float factor, void* stream);
 
 /* ------------------------------------------------------------------------
  * 6. Newton-Schulz orthogonalization on MFMA.
