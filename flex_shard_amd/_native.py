@@ -177,6 +177,17 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
          c_void_p],
     ),
+    "fsh_fp8_gemm_1x128_128x128_bias": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
+         c_int64, c_void_p],
+    ),
+    "fsh_fp8_linear_backward_scratch_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int32, c_int32, c_int32]),
+    "fsh_fp8_linear_backward": (
+        c_int,
+        [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p,
+         c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p],
+    ),
     "fsh_fp8_transpose": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p]),
     "fsh_act_quant_128x1_transposed": (
         c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_int32, c_void_p],

@@ -473,30 +473,7 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
             u32x2{pack_bf16x2(acc[i][j][4 * b], acc[i][j][4 * b + 1]),
                   pack_bf16x2(acc[i][j][4 * b + 2], acc[i][j][4 * b + 3])};
   wave_lds_sync();
-  {
-    constexpr int kLanesPerRow = Cfg::kWaveN * 2 / 16, kRowsPerPass = 64 / kLanesPerRow;
-    const int r0 = lane / kLanesPerRow, chunk = lane % kLanesPerRow;
-    const int64_t wave_row = m0 + wm * Cfg::kWaveM, col = n0 + wn * Cfg::kWaveN + chunk * 8;
-    const bool vec_ok = (p.ldo % 8 == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 15) == 0);
-#pragma unroll
-    for (int pass = 0; pass < Cfg::kWaveM / kRowsPerPass; ++pass) {
-      const int r = pass * kRowsPerPass + r0;
-      const int64_t row = wave_row + r;
-      if (row >= p.m || col >= p.n) continue;
-      const uint8_t* src = region + r * Cfg::kPitch + chunk * 16;
-      const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
-      const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
-      uint16_t* dst = p.out + row * p.ldo + col;
-      if (vec_ok && col + 8 <= p.n) {
-        *reinterpret_cast<u32x4*>(dst) = u32x4{lo.x, lo.y, hi.x, hi.y};
-      } else {
-        const uint32_t w[4] = {lo.x, lo.y, hi.x, hi.y};
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (col + e < p.n) dst[e] = static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1)));
-      }
-    }
-  }
+  store_fp8_product<Cfg::kWaveM, Cfg::kWaveN, Cfg::kPitch>(region, p, m0 + wm * Cfg::kWaveM, n0 + wn * Cfg::kWaveN, lane);
 #ifdef FSH_TRACE
   if (p.schedule.trace && lane == 0) {
     __builtin_amdgcn_s_waitcnt(0);
@@ -693,13 +670,15 @@ int launch_fp8_gemm(Fp8GemmParams& p, bool column_scales, const char* who, void*
 }  // namespace
 }  // namespace fsh
 
-FSH_API int fsh_fp8_gemm_1x128_128x128(const void* xq_dev, const float* xs_dev, const void* wq_dev,
-                                       const float* ws_dev, void* out_dev, int64_t m, int64_t n, int64_t k,
-                                       int64_t ldxq, int64_t ldwq, int64_t ldo, int64_t ws_cols, void* stream) {
+FSH_API int fsh_fp8_gemm_1x128_128x128_bias(const void* xq_dev, const float* xs_dev, const void* wq_dev,
+                                            const float* ws_dev, const void* bias_dev, void* out_dev, int64_t m,
+                                            int64_t n, int64_t k, int64_t ldxq, int64_t ldwq, int64_t ldo,
+                                            int64_t ws_cols, void* stream) {
   using namespace fsh;
   if (k > 0 && ws_cols < k / 128)
     return fail(FSH_EINVAL, "fsh_fp8_gemm_1x128_128x128: the weight scale table has %lld columns, k / 128 = %lld",
                 (long long)ws_cols, (long long)(k / 128));
+  if (!aligned(bias_dev, 2)) return fail(FSH_ENOTSUP, "fsh_fp8_gemm_1x128_128x128: the bias must be 2-byte aligned");
   Fp8GemmParams p;
   memset(&p, 0, sizeof(p));
   p.xq = static_cast<const uint8_t*>(xq_dev);
@@ -707,10 +686,18 @@ FSH_API int fsh_fp8_gemm_1x128_128x128(const void* xq_dev, const float* xs_dev, 
   p.wq = static_cast<const uint8_t*>(wq_dev);
   p.ws = ws_dev;
   p.out = static_cast<uint16_t*>(out_dev);
+  p.bias = static_cast<const uint16_t*>(bias_dev);
   p.m = m; p.n = n; p.k = k;
   p.ldxq = ldxq; p.ldwq = ldwq; p.ldo = ldo;
   p.ws_cb = ws_cols; p.ws_kb = 1;
   return launch_fp8_gemm(p, false, "fsh_fp8_gemm_1x128_128x128", stream);
+}
+
+FSH_API int fsh_fp8_gemm_1x128_128x128(const void* xq_dev, const float* xs_dev, const void* wq_dev,
+                                       const float* ws_dev, void* out_dev, int64_t m, int64_t n, int64_t k,
+                                       int64_t ldxq, int64_t ldwq, int64_t ldo, int64_t ws_cols, void* stream) {
+  return fsh_fp8_gemm_1x128_128x128_bias(xq_dev, xs_dev, wq_dev, ws_dev, nullptr, out_dev, m, n, k, ldxq, ldwq, ldo,
+                                         ws_cols, stream);
 }
 
 FSH_API int fsh_fp8_gemm_1x128_128x128_dgrad(const void* gq_dev, const float* gs_dev, const void* wtq_dev,

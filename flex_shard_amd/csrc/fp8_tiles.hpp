@@ -15,6 +15,7 @@ struct Fp8GemmParams {
   const float* ws;   // block scales: element (output-column block cb, k-block kb) at ws[cb * ws_cb + kb * ws_kb]
   const float* cs;   // per-column scales [k / 128][n] (the other kernel variant)
   uint16_t* out;
+  const uint16_t* bias;  // [n] added to the rounded product, or null
   int64_t m, n, k;
   int64_t ldxq, ldwq, ldo, ws_cb, ws_kb;
   GemmParams schedule;  // tile order; its work items are the tiles computed whole
@@ -22,6 +23,36 @@ struct Fp8GemmParams {
   // as two half tiles each, half_items in all (256 x 256 kernel only).
   int64_t whole_grid, half_items, half_items_per_xcd;
 };
+
+// The bias of eight output columns of a lane, added to the product's bf16
+// values where they are stored: bf16(fp32(bf16(product)) + fp32(bias)), the
+// bits of a separate addition of bf16 tensors without its pass over the output
+// (read and write again: 7.3 us at 1000 x 5120, and a launch).
+struct BiasOfLane {
+  float value[8];
+  __device__ __forceinline__ BiasOfLane(const uint16_t* bias, int64_t col, int64_t n) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) value[e] = col + e < n ? bf16_bits_to_f32(bias[col + e]) : 0.0f;
+  }
+  __device__ __forceinline__ u32x4 operator()(const u32x4& v) const {
+    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      w[j] = pack_bf16x2(u32_as_f32(d[j] << 16) + value[2 * j], u32_as_f32(d[j] & 0xFFFF0000u) + value[2 * j + 1]);
+    return u32x4{w[0], w[1], w[2], w[3]};
+  }
+};
+
+// A wave's finished image to the output, with the bias if there is one.
+template <int kRows, int kCols, int kPitch>
+__device__ __forceinline__ void store_fp8_product(const uint8_t* region, const Fp8GemmParams& p, int64_t row0, int64_t col0, int lane) {
+  if (p.bias)
+    store_wave_image<kRows, kCols, kPitch>(region, p.out, p.ldo, row0, col0, p.m, p.n, lane,
+                                           BiasOfLane(p.bias, col0 + image_column_of_lane<kCols>(lane), p.n));
+  else
+    store_wave_image<kRows, kCols, kPitch>(region, p.out, p.ldo, row0, col0, p.m, p.n, lane);
+}
 
 // acc[n] += (product[n] * row_scale) * (column_scales of lane n of this lane's row of 16).
 // The broadcast is the multiply-add's own operand modifier (the compiler keeps
@@ -301,8 +332,7 @@ __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) vo
             u32x2{pack_bf16x2(acc[i][j][4 * b], acc[i][j][4 * b + 1]),
                   pack_bf16x2(acc[i][j][4 * b + 2], acc[i][j][4 * b + 3])};
   wave_lds_sync();
-  store_wave_image<Cfg::kWaveM, Cfg::kWaveN, Cfg::kPitch>(region, p.out, p.ldo, m0 + wm * Cfg::kWaveM, n0 + wn * Cfg::kWaveN,
-                                                          p.m, p.n, lane);
+  store_fp8_product<Cfg::kWaveM, Cfg::kWaveN, Cfg::kPitch>(region, p, m0 + wm * Cfg::kWaveM, n0 + wn * Cfg::kWaveN, lane);
 }
 
 }  // namespace

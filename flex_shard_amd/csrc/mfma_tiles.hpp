@@ -452,25 +452,35 @@ __device__ __forceinline__ bool rows_are_16_byte(const uint16_t* p, int64_t ld) 
 
 // A wave's [kRows][kCols] image in LDS to `out` rows [row0, +) x columns
 // [col0, +), cut at rows x cols, whole row segments per store instruction.
-template <int kRows, int kCols, int kPitch>
+// `finish` has the last word on eight bf16 values of a lane's columns
+// [column_of_lane, +8).
+template <int kCols>
+__device__ __forceinline__ int image_column_of_lane(int lane) {
+  return lane % (kCols / 8) * 8;
+}
+template <int kRows, int kCols, int kPitch, typename Finish>
 __device__ __forceinline__ void store_wave_image(const uint8_t* region, uint16_t* out, int64_t ld, int64_t row0,
-                                                 int64_t col0, int64_t rows, int64_t cols, int lane) {
+                                                 int64_t col0, int64_t rows, int64_t cols, int lane, Finish finish) {
   constexpr int kLanesPerRow = kCols / 8, kRowsPerPass = 64 / kLanesPerRow;
   const bool vec = rows_are_16_byte(out, ld);
-  const int r0 = lane / kLanesPerRow, chunk = lane % kLanesPerRow;
-  const int64_t col = col0 + chunk * 8;
+  const int r0 = lane / kLanesPerRow;
+  const int64_t col = col0 + image_column_of_lane<kCols>(lane);
   if (col >= cols) return;
 #pragma unroll
   for (int pass = 0; pass < kRows / kRowsPerPass; ++pass) {
     const int r = pass * kRowsPerPass + r0;
     if (row0 + r >= rows) break;
-    const uint8_t* src = region + r * kPitch + chunk * 16;
+    const uint8_t* src = region + r * kPitch + image_column_of_lane<kCols>(lane) * 2;
     const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
     const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
-    store_row_piece(out + (row0 + r) * ld, col, cols, vec, u32x4{lo.x, lo.y, hi.x, hi.y});
+    store_row_piece(out + (row0 + r) * ld, col, cols, vec, finish(u32x4{lo.x, lo.y, hi.x, hi.y}));
   }
 }
-
+template <int kRows, int kCols, int kPitch>
+__device__ __forceinline__ void store_wave_image(const uint8_t* region, uint16_t* out, int64_t ld, int64_t row0,
+                                                 int64_t col0, int64_t rows, int64_t cols, int lane) {
+  store_wave_image<kRows, kCols, kPitch>(region, out, ld, row0, col0, rows, cols, lane, [](const u32x4& v) { return v; });
+}
 
 // What a launch of a tile kernel takes, from measurements: tiles of the chip's
 // one round at a time, per k-tile the less the emptier the round is (fewer

@@ -36,13 +36,21 @@ __all__ = [
     "REDUCE_PREMUL", "REDUCE_SUM", "SRC_BF16", "SRC_F16", "SRC_F32", "SRC_F32_AS_BF16", "SRC_F32_AS_F16",
     "MuonStepPlan", "QuantChunkSpec", "QuantPackPlan", "accumulate_grad", "act_quant_128x1_transposed", "act_quant_1x128", "act_quant_both",
     "copy_row_segments", "copy_segments", "fp8_gemm_1x128_128x1", "fp8_gemm_1x128_128x128", "fp8_gemm_1x128_128x128_dgrad",
-    "fp8_transpose", "gemm_nt", "gemm_nt_group", "muon_apply", "muon_prepare", "newton_schulz_multi",
+    "fp8_linear_backward", "fp8_transpose", "gemm_nt", "gemm_nt_group", "muon_apply", "muon_prepare", "newton_schulz_multi",
     "newton_schulz", "newton_schulz_noalloc", "newton_schulz_workspace_bytes", "pack_segments", "quantize_pack",
     "reduce_rows", "stream_ptr", "unpack_dequant", "zero_segments",
 ]
 
 
 def _require_gpu(*tensors: torch.Tensor) -> torch.device:
+    index = tensors[0].get_device()  # -1 for what is not on a GPU
+    for t in tensors:
+        if t.get_device() != index or index < 0:
+            _refuse_devices(tensors)
+    return tensors[0].device
+
+
+def _refuse_devices(tensors: Sequence[torch.Tensor]) -> None:
     device = tensors[0].device
     for t in tensors:
         if t.device.type != "cuda":
@@ -52,7 +60,6 @@ def _require_gpu(*tensors: torch.Tensor) -> torch.device:
             )
         if t.device != device:
             raise ValueError(f"tensors on different devices: {device} and {t.device}")
-    return device
 
 
 def stream_ptr(device: torch.device) -> int:
@@ -565,11 +572,14 @@ def act_quant_1x128(x: torch.Tensor, *, eps_fp32: bool = True) -> tuple[torch.Te
 
 
 def fp8_gemm_1x128_128x128(
-    xq: torch.Tensor, xs: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, out: torch.Tensor | None = None
+    xq: torch.Tensor, xs: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, out: torch.Tensor | None = None,
+    bias: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """``out[i, j] = bf16(sum_kb dot(xq[i, kb], wq[j, kb]) * xs[kb, i] * ws[j // 128, kb])``
     for float8_e4m3fn ``xq`` [m, k], ``wq`` [n, k] (rows contiguous, k a
-    multiple of 128), ``xs`` [k / 128, m] and ``ws`` [ceil(n / 128), >= k / 128]."""
+    multiple of 128), ``xs`` [k / 128, m] and ``ws`` [ceil(n / 128), >= k / 128].
+    ``bias``, bf16 of n contiguous elements, is added to the rounded product
+    (the bits of ``out + bias``)."""
     _require_gpu(xq, xs, wq, ws)
     for name, t in (("xq", xq), ("wq", wq)):
         if t.dtype not in (torch.float8_e4m3fn, torch.uint8) or t.ndim != 2 or t.stride(1) != 1:
@@ -588,8 +598,14 @@ def fp8_gemm_1x128_128x128(
     _require_gpu(xq, out)
     if out.dtype != torch.bfloat16 or tuple(out.shape) != (m, n) or out.stride(1) != 1:
         raise ValueError(f"out must be bf16 [{m}, {n}] with contiguous rows")
-    status = _native.lib().fsh_fp8_gemm_1x128_128x128(
-        xq.data_ptr(), xs.data_ptr(), wq.data_ptr(), ws.data_ptr(), out.data_ptr(), m, n, k, xq.stride(0),
+    bias_ptr = None
+    if bias is not None:
+        _require_gpu(xq, bias)
+        if bias.dtype != torch.bfloat16 or bias.numel() != n or not bias.is_contiguous():
+            raise ValueError(f"bias must be bf16 of {n} contiguous elements, got {bias.dtype} {tuple(bias.shape)}")
+        bias_ptr = bias.data_ptr()
+    status = _native.lib().fsh_fp8_gemm_1x128_128x128_bias(
+        xq.data_ptr(), xs.data_ptr(), wq.data_ptr(), ws.data_ptr(), bias_ptr, out.data_ptr(), m, n, k, xq.stride(0),
         wq.stride(0), out.stride(0), ws.stride(0), stream_ptr(xq.device),
     )
     _native.check(status, "fsh_fp8_gemm_1x128_128x128")
@@ -725,6 +741,65 @@ def fp8_gemm_1x128_128x1(
     )
     _native.check(status, "fsh_fp8_gemm_1x128_128x1")
     return out
+
+
+def fp8_linear_backward(
+    grad: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor, in_dim: int,
+    x_runs: tuple[torch.Tensor, torch.Tensor] | None, needs_x_grad: bool, needs_weight_grad: bool, needs_bias_grad: bool,
+) -> tuple[torch.Tensor | None, torch.Tensor | None, torch.Tensor | None]:
+    """Backward of ``x @ W.T + bias`` in one call: ``grad`` [tokens, out] bf16
+    (out padded with zero columns to a multiple of 8), ``wq`` [out, in padded
+    to a multiple of 16], ``ws`` its scales, ``x_runs`` the activation from
+    :func:`act_quant_128x1_transposed`.  Returns ``(grad_x [tokens, in_dim],
+    grad_w [grad's columns, x_runs' rows], grad_bias [grad's columns])``, None
+    where not wanted; the bias gradient only comes with the weight gradient."""
+    _require_gpu(grad, wq, ws)
+    if needs_x_grad:
+        _fp8_matrix("wq", wq)
+    if grad.dtype != torch.bfloat16 or grad.ndim != 2 or grad.stride(1) != 1:
+        raise ValueError("grad must be a bf16 matrix with contiguous rows")
+    tokens, out_cols = grad.shape
+    out_dim, in_cols = wq.shape
+    if out_cols != -(-out_dim // 8) * 8 or in_cols < in_dim:
+        raise ValueError(f"shapes do not match: grad {tuple(grad.shape)}, wq {tuple(wq.shape)}, in_dim {in_dim}")
+    if needs_x_grad and (
+        ws.dtype != torch.float32 or ws.ndim != 2 or not _unit_column_stride(ws) or ws.shape[0] < -(-out_dim // 128)
+        or ws.shape[1] < -(-in_dim // 128)
+    ):
+        raise ValueError(f"ws must be fp32 [>= {-(-out_dim // 128)}, >= {-(-in_dim // 128)}] with contiguous rows, got {tuple(ws.shape)}")
+    device = grad.device
+    runs_ptr = runs_scales_ptr = None
+    x_cols = 0
+    if needs_weight_grad:
+        if x_runs is None:
+            raise ValueError("the weight gradient needs the activation's token runs")
+        runs, runs_scales = x_runs
+        _require_gpu(grad, runs, runs_scales)
+        _fp8_matrix("x_runs", runs)
+        x_cols, padded = runs.shape
+        if padded != -(-tokens // 128) * 128 or not runs.is_contiguous():
+            raise ValueError(f"x_runs must be contiguous [in, tokens padded to {-(-tokens // 128) * 128}], got {tuple(runs.shape)}")
+        if runs_scales.dtype != torch.float32 or not runs_scales.is_contiguous() or tuple(runs_scales.shape) != (padded // 128, x_cols):
+            raise ValueError(f"the scales of x_runs must be contiguous fp32 of shape {(padded // 128, x_cols)}, got {tuple(runs_scales.shape)}")
+        runs_ptr, runs_scales_ptr = runs.data_ptr(), runs_scales.data_ptr()
+    grad_x = torch.empty((tokens, in_dim), dtype=torch.bfloat16, device=device) if needs_x_grad else None
+    grad_w = torch.empty((out_cols, x_cols), dtype=torch.bfloat16, device=device) if needs_weight_grad else None
+    grad_bias = None
+    if needs_bias_grad and needs_weight_grad:
+        grad_bias = torch.empty((out_cols,), dtype=torch.bfloat16, device=device)
+    lib = _native.lib()
+    nbytes = lib.fsh_fp8_linear_backward_scratch_bytes(
+        tokens, out_cols, in_cols, grad_x is not None, grad_w is not None, grad_bias is not None
+    )
+    scratch = torch.empty((max(nbytes, 1),), dtype=torch.uint8, device=device)
+    status = lib.fsh_fp8_linear_backward(
+        grad.data_ptr(), tokens, out_cols, grad.stride(0), wq.data_ptr(), out_dim, in_cols, in_dim, wq.stride(0),
+        ws.data_ptr(), ws.stride(0), runs_ptr, runs_scales_ptr, x_cols,
+        None if grad_x is None else grad_x.data_ptr(), None if grad_w is None else grad_w.data_ptr(),
+        None if grad_bias is None else grad_bias.data_ptr(), scratch.data_ptr(), nbytes, stream_ptr(device),
+    )
+    _native.check(status, "fsh_fp8_linear_backward")
+    return grad_x, grad_w, grad_bias
 
 
 def _muon_master_dtype(who: str, masters: Sequence[torch.Tensor], bf16: Sequence[torch.Tensor]) -> torch.dtype:

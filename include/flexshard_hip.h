@@ -341,12 +341,18 @@ int fsh_muon_apply_f32(float* param_dev, const void* direction_bf16_dev, int64_t
  * xq [m, k] and wq [n, k] E4M3FN bytes with row strides ldxq / ldwq, xs the
  * [k / 128, m] table above, ws the weight's [ceil(n / 128), ws_cols] scales,
  * out [m, n] bf16 with row stride ldo.  k must be a multiple of 128.
+ * The _bias form adds bias [n] (bf16, may be null) to the rounded product, as
+ * a bf16 addition after it would (blockwise_quant/linear.py:74-123).
  * ---------------------------------------------------------------------- */
 int fsh_act_quant_1x128(const void* x_dev, int64_t rows, int64_t cols, int64_t ldx, void* q_dev,
                         int64_t ldq, float* scales_dev, int32_t eps_mode, void* stream);
 int fsh_fp8_gemm_1x128_128x128(const void* xq_dev, const float* xs_dev, const void* wq_dev,
                                const float* ws_dev, void* out_dev, int64_t m, int64_t n, int64_t k,
                                int64_t ldxq, int64_t ldwq, int64_t ldo, int64_t ws_cols, void* stream);
+int fsh_fp8_gemm_1x128_128x128_bias(const void* xq_dev, const float* xs_dev, const void* wq_dev,
+                                    const float* ws_dev, const void* bias_dev, void* out_dev, int64_t m,
+                                    int64_t n, int64_t k, int64_t ldxq, int64_t ldwq, int64_t ldo,
+                                    int64_t ws_cols, void* stream);
 
 /* ------------------------------------------------------------------------
  * 9. Backward products of the same linear layer.  Replace the device work of
@@ -409,6 +415,25 @@ int fsh_fp8_gemm_1x128_128x128_dgrad(const void* gq_dev, const float* gs_dev, co
 int fsh_fp8_gemm_1x128_128x1(const void* aq_dev, const float* as_dev, const void* bq_dev,
                              const float* bs_dev, void* out_dev, int64_t m, int64_t n, int64_t k,
                              int64_t ldaq, int64_t ldbq, int64_t ldo, void* stream);
+
+/* The whole backward of the layer in one call: what the functions above give
+ * one after the other, bit for bit, with the weight's transpose in the launch
+ * that quantizes the gradient, and the bias gradient (sum over the tokens,
+ * blockwise_quant/linear.py:74-123) from the same pass over it.
+ * grad [tokens, out_cols] bf16 (out_cols = out_dim, or padded with zero
+ * columns to a multiple of 8); wq [out_dim, in_cols] with row stride ldwq
+ * (in_cols = in_dim rounded up to 16); x_runs / x_runs_scales the token-run
+ * form of the activation, [x_cols, tokens rounded up to 128].  Outputs, each
+ * null when not wanted: grad_x [tokens, in_dim], grad_w [out_cols, x_cols],
+ * grad_bias [out_cols] (only with grad_w), bf16, contiguous.  scratch_dev:
+ * 128-byte aligned, of at least the bytes the other function returns. */
+int64_t fsh_fp8_linear_backward_scratch_bytes(int64_t tokens, int64_t out_cols, int64_t in_cols, int32_t grad_x,
+                                              int32_t grad_w, int32_t grad_bias);
+int fsh_fp8_linear_backward(const void* grad_dev, int64_t tokens, int64_t out_cols, int64_t ldg, const void* wq_dev,
+                            int64_t out_dim, int64_t in_cols, int64_t in_dim, int64_t ldwq, const float* ws_dev,
+                            int64_t ws_cols, const void* x_runs_dev, const float* x_runs_scales_dev, int64_t x_cols,
+                            void* grad_x_dev, void* grad_w_dev, void* grad_bias_dev, void* scratch_dev,
+                            int64_t scratch_nbytes, void* stream);
 
 /* ------------------------------------------------------------------------
  * 10. One whole Muon step over matrices grouped by shape, for an owner's whole
