@@ -95,7 +95,13 @@ class BlockwiseFp8Weight(torch.Tensor):
             raise ValueError(f"BlockwiseFp8Weight expects 2D or stacked 2D data, got {data.shape}")
         if block_size <= 0:
             raise ValueError(f"block_size must be positive, got {block_size}")
-        _check_scale(_matrix_shape(data.shape), recip_scale, block_size)
+        # (written out for a 2-D weight: one is built per parameter and unshard)
+        shape = data.shape
+        if not (
+            len(shape) == 2 and type(block_size) is int and shape[0] > 0 and shape[1] > 0
+            and recip_scale.shape == (-(-shape[0] // block_size), -(-shape[1] // block_size))
+        ):
+            _check_scale(_matrix_shape(shape), recip_scale, block_size)
         if data.device != recip_scale.device:
             raise ValueError(
                 f"data and scale must be on the same device, got {data.device} and {recip_scale.device}"

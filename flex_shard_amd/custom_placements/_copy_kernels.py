@@ -252,13 +252,22 @@ def pack_segments_into_flat_buffer(
         )
     elif descriptor.input_ptrs.device != output.device or descriptor.input_ptrs.numel() != len(inputs):
         return None
+    return launch_pack_descriptor(descriptor, inputs, output)
+
+
+def launch_pack_descriptor(
+    descriptor: SegmentPackDescriptor, inputs: list[torch.Tensor], output: torch.Tensor
+) -> list[torch.Tensor]:
+    """The launch of :func:`pack_segments_into_flat_buffer` for a descriptor of
+    these inputs: contiguous tensors (of any shape) of one supported dtype on
+    the output's device."""
     staged = descriptor.update_input_ptrs(inputs)
     keep = [*descriptor.tensors, *staged, *inputs]
     if output.numel() == 0 or descriptor.nsegments == 0 or descriptor.max_segment_numel == 0:
         return keep
     hip_ops.pack_segments(
         descriptor.input_ptrs, descriptor.tensor_indices, descriptor.src_offsets, descriptor.numels,
-        descriptor.dst_offsets, descriptor.max_segment_numel, in_dtype, output,
+        descriptor.dst_offsets, descriptor.max_segment_numel, inputs[0].dtype, output,
     )
     return keep
 
@@ -269,6 +278,7 @@ __all__ = [
     "SegmentPackDescriptor",
     "copy_row_segments",
     "copy_segments",
+    "launch_pack_descriptor",
     "pack_segments_into_flat_buffer",
     "zero_segments",
 ]

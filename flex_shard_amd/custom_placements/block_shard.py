@@ -39,6 +39,7 @@ from ._copy_kernels import (
     SegmentPackDescriptor,
     copy_row_segments,
     copy_segments,
+    launch_pack_descriptor,
     pack_segments_into_flat_buffer,
 )
 from .utils import (
@@ -47,7 +48,6 @@ from .utils import (
     foreach_copy_,
     group_size,
     local_exchange_rows,
-    pack_segments_into_flat_buffer_if_supported,
     pack_tensors_into_flat_buffer_with_scratch,
     reduce_scatter_grads,
 )
@@ -680,7 +680,7 @@ class BucketedBlockShard(Placement):
         floats = (torch.float32, torch.bfloat16)
         first = tensors[0].dtype
         return dtype in floats and all(
-            t.device.type == "cuda" and t.dtype == first and t.dtype in floats and t.is_contiguous() for t in tensors
+            t.is_cuda and t.dtype == first and t.dtype in floats and t.is_contiguous() for t in tensors
         )
 
     def _pack_reduce_scatter_grad(
@@ -697,11 +697,17 @@ class BucketedBlockShard(Placement):
             )
         if send_rows.stride(1) != 1 or not self._packs_reduce_scatter_grad_in_one_pass(tensors, send_rows.dtype):
             raise AssertionError("BucketedBlockShard can't pack these grads in one pass.")
+        return self._pack_checked_grads(tensors, infos, send_rows)
+
+    def _pack_checked_grads(
+        self, tensors: list[torch.Tensor], infos: list["ParamInfo"], send_rows: torch.Tensor
+    ) -> list[torch.Tensor]:
+        """:meth:`_pack_reduce_scatter_grad` of grads that the single-launch
+        copy-in can write (``_packs_reduce_scatter_grad_in_one_pass``)."""
         row_stride = send_rows.stride(0)
         plan = self._reduce_copy_in_plan(infos, row_stride)
         out = send_rows.as_strided(((send_rows.size(0) - 1) * row_stride + send_rows.size(1),), (1,))
-        sources = [t.view(-1) for t in tensors]
-        key = (out.device, sources[0].dtype)
+        key = (out.device, tensors[0].dtype)
         descriptor = plan.descriptors.get(key)
         if descriptor is None:
             index, src, cnt, dst = [], [], [], []
@@ -717,14 +723,14 @@ class BucketedBlockShard(Placement):
                 cnt.append(n)
                 dst.append(d)
             descriptor = SegmentPackDescriptor.create(
-                ninputs=len(sources), tensor_indices=index, src_offsets=src, numels=cnt, dst_offsets=dst,
+                ninputs=len(tensors), tensor_indices=index, src_offsets=src, numels=cnt, dst_offsets=dst,
                 device=out.device,
             )
             plan.descriptors[key] = descriptor
-        keep = pack_segments_into_flat_buffer_if_supported(sources, [], [], [], [], out, descriptor=descriptor)
-        if keep is None:
+        device = out.get_device()
+        if device < 0 or any(t.get_device() != device for t in tensors) or descriptor.input_ptrs.numel() != len(tensors):
             raise AssertionError("BucketedBlockShard one-pass copy-in was declined by the HIP packer.")
-        return keep
+        return launch_pack_descriptor(descriptor, tensors, out)
 
     def prepare_reduce_grad(
         self, tensors: list[torch.Tensor], infos: list["ParamInfo"], mesh: Any, debug_fqn: str | None
@@ -746,7 +752,7 @@ class BucketedBlockShard(Placement):
         if self._packs_reduce_scatter_grad_in_one_pass(tensors, dtype):
             with record_range("FlexShard::reduce_scatter_copy_in", debug_fqn):
                 send = torch.empty(world_size * widest, dtype=dtype, device=device)
-                keep = self._pack_reduce_scatter_grad(tensors, infos, world_size, send.view(world_size, widest))
+                keep = self._pack_checked_grads(tensors, infos, send.view(world_size, widest))
             return PlacementPreparedReduceGrad(placement=self, buffers=[send, *keep], placement_state=state)
         # Compiling, off the GPU, or unusual dtypes: copy through a zeroed
         # gradient bucket with ATen.

@@ -160,6 +160,11 @@ class Fp8BucketedBlockShard(BlockwiseQuantBucketedBlockShard):
     def _param_scale_view(self, scale_index: int, scale: torch.Tensor, matrix_shape: torch.Size) -> torch.Tensor:
         return scale.view(_scale_shape(matrix_shape, self.block_size))
 
+    def _scale_view_shape(self, matrix_shape: torch.Size) -> tuple[int, int] | None:
+        if type(self)._param_scale_view is not Fp8BucketedBlockShard._param_scale_view:
+            return None  # a subclass lays its scales out otherwise
+        return _scale_shape(matrix_shape, self.block_size)
+
     def _make_quantized_weight(
         self, qdata: torch.Tensor, scales: tuple[torch.Tensor, ...], *, orig_dtype: torch.dtype, requires_grad: bool
     ) -> torch.Tensor:
@@ -264,10 +269,15 @@ class Fp8BucketedBlockShard(BlockwiseQuantBucketedBlockShard):
         compact_buf = self._compact_buffer(prepared, state.metadata, rank_rows.device) if compact else None
         with record_copy_out():
             hip_ops.unpack_dequant(rank_rows, table, starts, total_tiles, compact_buf, dequant_out.view(-1), self.block_size)
-        dequant = [
-            piece.view(info.global_shape)
-            for piece, info in zip(torch.split(dequant_out.view(-1), [i.global_numel for i in state.infos]), state.infos)
-        ]
+        plan = None if torch.compiler.is_compiling() else self._full_param_plan(state)
+        if plan is not None:
+            first = dequant_out.storage_offset()
+            dequant = [dequant_out.as_strided(shape, strides, first + start) for shape, strides, start, _, _ in plan.views]
+        else:
+            dequant = [
+                piece.view(info.global_shape)
+                for piece, info in zip(torch.split(dequant_out.view(-1), [i.global_numel for i in state.infos]), state.infos)
+            ]
         if compact_buf is None:
             return PlacementUnshardResult(full_params=[]), dequant
         result = PlacementUnshardResult(

@@ -246,11 +246,11 @@ def all_gather_rows(output: torch.Tensor, input: torch.Tensor, group: Any, *, as
         if group.local_row_only:
             rows[rank].copy_(input.reshape(-1))
             return None
+        if _gather_rows_in_one_launch(group, rows, input):
+            return None
         missing = sorted(set(range(world)) - {rank} - set(group.gather_rows))
         if missing:
             raise ValueError(f"LocalReduceGroup is missing the all-gather rows of ranks {missing}.")
-        if _gather_rows_in_one_launch(group, rows, input):
-            return None
         rows[rank].copy_(input.reshape(-1))
         for other, row in group.gather_rows.items():
             if other != rank:
@@ -271,11 +271,12 @@ def local_exchange_rows(group: Any, input: torch.Tensor) -> list[torch.Tensor] |
     world, rank = group.size(), group.rank()
     if world > MAX_COPY_ROWS or input.device.type != "cuda":
         return None
-    dtype, numel, device = input.dtype, input.numel(), input.device
+    dtype, numel, device = input.dtype, input.numel(), input.get_device()
+    gather_rows = group.gather_rows
     rows = []
     for r in range(world):
-        row = input if r == rank else group.gather_rows.get(r)
-        if row is None or row.dtype != dtype or row.numel() != numel or row.device != device or not row.is_contiguous():
+        row = input if r == rank else gather_rows.get(r)
+        if row is None or row.dtype != dtype or row.numel() != numel or row.get_device() != device or not row.is_contiguous():
             return None
         rows.append(row)
     return rows

@@ -27,7 +27,6 @@ Ordering uses events only; nothing here blocks the host:
 
 from __future__ import annotations
 
-import contextlib
 from typing import TYPE_CHECKING, Any
 
 import torch
@@ -143,7 +142,7 @@ def _get_bucket_placement(infos: list["ParamInfo"], operation: str) -> "Placemen
     lead = infos[0]
     wanted = lead.placement.bucket_compatibility_key()
     for info in infos[1:]:
-        if info.placement.bucket_compatibility_key() != wanted:
+        if info.placement is not lead.placement and info.placement.bucket_compatibility_key() != wanted:
             raise ValueError(
                 f"FlexShard bucket {operation} requires all parameters in a bucket to use compatible placements, "
                 f"but {lead.fqn!r} uses {lead.placement!r} and {info.fqn!r} uses {info.placement!r}."
@@ -168,10 +167,9 @@ def _prepare_and_run(
     prepared.persistent_buffers = persistent_buffers
     if persistent_buffers is None:
         return prepared, placement.run_prepared_unshard(prepared, async_op=async_op)
-    with contextlib.ExitStack() as guards:
-        guards.enter_context(torch.inference_mode(False))
-        guards.enter_context(torch.no_grad())
-        guards.enter_context(torch.autograd._unsafe_preserve_version_counter(tuple(persistent_buffers)))
+    with torch.inference_mode(False), torch.no_grad(), torch.autograd._unsafe_preserve_version_counter(
+        tuple(persistent_buffers)
+    ):
         work = placement.run_prepared_unshard(prepared, async_op=async_op)
     return prepared, work
 
