@@ -35,6 +35,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ u32x4 load_stream_u32x4(const void* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
 }
+__device__ __forceinline__ u32x2 load_stream_u32x2(const void* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p));
+}
 __device__ __forceinline__ f32x4 load_stream_f32x4(const void* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
 }
