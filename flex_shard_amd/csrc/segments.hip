@@ -60,7 +60,18 @@ __global__ __launch_bounds__(kThreads) void zero_segments_kernel(uint8_t* __rest
   zero_bytes(dst + dst_offsets[seg] * unit + begin, len, threadIdx.x, kThreads);
 }
 
-constexpr int64_t kPackSliceElems = 2048;  // one 8-element group per thread (larger slices measured slower)
+// A casting slice: four accesses per thread, all requested before the first is
+// stored, each contiguous across the wave with 16 bytes of fp32 per lane.
+// Bound by memory and, with small slices, by the chain of table loads at a
+// block's start: a layer's rank share (27 M elements) fp32 -> bf16 38 us with
+// one access per thread, 28 with two, 27 with four or eight, against 34 with
+// eight elements per thread in two 16-byte accesses 32 bytes apart; 12 M
+// elements bf16 -> fp32 20.5 / 15.5 / 15.8 / 19.1 against 17.7 us.
+constexpr int kCastUnroll = 4;
+// Elements of one block.  A launch whose thread count would pass 32 bits takes
+// larger slices.
+template <typename SRC, typename DST>
+constexpr int64_t kPackSliceElems = sizeof(SRC) == sizeof(DST) ? 2048 : kCastUnroll * 4 * kThreads;
 
 template <typename SRC, typename DST>
 __device__ __forceinline__ DST cast_elem(SRC v);
@@ -75,30 +86,26 @@ __device__ __forceinline__ uint16_t cast_elem<float, uint16_t>(float v) {
   return static_cast<uint16_t>(f32_to_bf16_bits(v));
 }
 
-// Eight consecutive elements, both pointers 16-byte aligned.
-__device__ __forceinline__ void cast_group_of_8(const uint16_t* src, float* dst) {
-  const u32x4 v = load_stream_u32x4(src);
-  const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-  f32x4 lo, hi;
-  lo.x = u32_as_f32(d[0] << 16); lo.y = u32_as_f32(d[0] & 0xFFFF0000u);
-  lo.z = u32_as_f32(d[1] << 16); lo.w = u32_as_f32(d[1] & 0xFFFF0000u);
-  hi.x = u32_as_f32(d[2] << 16); hi.y = u32_as_f32(d[2] & 0xFFFF0000u);
-  hi.z = u32_as_f32(d[3] << 16); hi.w = u32_as_f32(d[3] & 0xFFFF0000u);
-  reinterpret_cast<f32x4*>(dst)[0] = lo;
-  reinterpret_cast<f32x4*>(dst)[1] = hi;
-}
-__device__ __forceinline__ void cast_group_of_8(const float* src, uint16_t* dst) {
-  const f32x4 a = load_stream_f32x4(src), b = load_stream_f32x4(src + 4);
-  u32x4 o;
-  o.x = f32_to_bf16_bits(a.x) | (f32_to_bf16_bits(a.y) << 16);
-  o.y = f32_to_bf16_bits(a.z) | (f32_to_bf16_bits(a.w) << 16);
-  o.z = f32_to_bf16_bits(b.x) | (f32_to_bf16_bits(b.y) << 16);
-  o.w = f32_to_bf16_bits(b.z) | (f32_to_bf16_bits(b.w) << 16);
-  *reinterpret_cast<u32x4*>(dst) = o;
-}
-// Same-type pairs never reach the casting branch; these keep it compilable.
-__device__ __forceinline__ void cast_group_of_8(const float*, float*) {}
-__device__ __forceinline__ void cast_group_of_8(const uint16_t*, uint16_t*) {}
+// Four consecutive elements, 16 bytes of fp32 or 8 of bf16, as loaded and
+// cast to the other type.
+struct Bf16To32 {
+  typedef u32x2 Raw;
+  static __device__ __forceinline__ Raw load(const uint16_t* src) { return load_stream_u32x2(src); }
+  static __device__ __forceinline__ void store(float* dst, const Raw v) {
+    *reinterpret_cast<f32x4*>(dst) = f32x4{u32_as_f32(v.x << 16), u32_as_f32(v.x & 0xFFFF0000u), u32_as_f32(v.y << 16),
+                                           u32_as_f32(v.y & 0xFFFF0000u)};
+  }
+};
+struct F32ToBf16 {
+  typedef f32x4 Raw;
+  static __device__ __forceinline__ Raw load(const float* src) { return load_stream_f32x4(src); }
+  static __device__ __forceinline__ void store(uint16_t* dst, const Raw v) {
+    *reinterpret_cast<u32x2*>(dst) = u32x2{f32_to_bf16_bits(v.x) | (f32_to_bf16_bits(v.y) << 16),
+                                           f32_to_bf16_bits(v.z) | (f32_to_bf16_bits(v.w) << 16)};
+  }
+};
+__device__ __forceinline__ Bf16To32 caster(const uint16_t*, float*) { return {}; }
+__device__ __forceinline__ F32ToBf16 caster(const float*, uint16_t*) { return {}; }
 
 // Multi-input gather with cast.  A negative tensor index marks a zero-fill
 // segment.  Same-dtype segments move as bytes with the widest legal vector;
@@ -107,32 +114,40 @@ template <typename SRC, typename DST>
 __global__ __launch_bounds__(kThreads) void pack_segments_kernel(
     const int64_t* __restrict__ input_ptrs, const int64_t* __restrict__ tensor_indices,
     const int64_t* __restrict__ src_offsets, const int64_t* __restrict__ numels,
-    const int64_t* __restrict__ dst_offsets, DST* __restrict__ out, int64_t slices_per_segment) {
-  const int64_t seg = blockIdx.x / slices_per_segment;
-  const int64_t slice = blockIdx.x - seg * slices_per_segment;
-  const int64_t n = numels[seg];
-  const int64_t begin = slice * kPackSliceElems;
+    const int64_t* __restrict__ dst_offsets, DST* __restrict__ out, uint32_t slices_per_segment,
+    int64_t slice_elems) {
+  const uint32_t seg = blockIdx.x / slices_per_segment;
+  const int64_t begin = static_cast<int64_t>(blockIdx.x - seg * slices_per_segment) * slice_elems;
+  // (asked for together: what follows waits for them once)
+  const int64_t n = numels[seg], ti = tensor_indices[seg], src_offset = src_offsets[seg], dst_offset = dst_offsets[seg];
   if (begin >= n) return;
-  const int64_t len = (n - begin) < kPackSliceElems ? (n - begin) : kPackSliceElems;
-  DST* dst = out + dst_offsets[seg] + begin;
-  const int64_t ti = tensor_indices[seg];
+  const int64_t len = (n - begin) < slice_elems ? (n - begin) : slice_elems;
+  DST* dst = out + dst_offset + begin;
   if (ti < 0) {
     zero_bytes(reinterpret_cast<uint8_t*>(dst), len * static_cast<int64_t>(sizeof(DST)), threadIdx.x, kThreads);
     return;
   }
-  const SRC* src = reinterpret_cast<const SRC*>(static_cast<uintptr_t>(input_ptrs[ti])) + src_offsets[seg] + begin;
-  if (sizeof(SRC) == sizeof(DST)) {
+  const SRC* src = reinterpret_cast<const SRC*>(static_cast<uintptr_t>(input_ptrs[ti])) + src_offset + begin;
+  if constexpr (sizeof(SRC) == sizeof(DST)) {
     copy_bytes(reinterpret_cast<const uint8_t*>(src), reinterpret_cast<uint8_t*>(dst),
                len * static_cast<int64_t>(sizeof(DST)), threadIdx.x, kThreads);
   } else {
-    // Eight elements per thread and step when both sides start on a 16-byte
-    // boundary (16 bytes of bf16 against 32 of fp32); the rest, and slices
-    // that do not, go element by element.
+    // Four elements per thread and access when the fp32 side starts on a
+    // 16-byte boundary and the bf16 side on an 8-byte one; the rest, and
+    // slices that do not, go element by element.
+    typedef decltype(caster(src, dst)) Cast;
+    constexpr int64_t kStep = 4 * kThreads;
     int64_t done = 0;
-    if (((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0) {
-      const int64_t groups = len / 8;
-      for (int64_t g = threadIdx.x; g < groups; g += kThreads) cast_group_of_8(src + 8 * g, dst + 8 * g);
-      done = groups * 8;
+    if (reinterpret_cast<uintptr_t>(src) % (4 * sizeof(SRC)) == 0 && reinterpret_cast<uintptr_t>(dst) % (4 * sizeof(DST)) == 0) {
+      const int64_t i = 4 * static_cast<int64_t>(threadIdx.x);
+      for (; done + kCastUnroll * kStep <= len; done += kCastUnroll * kStep) {
+        typename Cast::Raw raw[kCastUnroll];
+#pragma unroll
+        for (int u = 0; u < kCastUnroll; ++u) raw[u] = Cast::load(src + done + u * kStep + i);
+#pragma unroll
+        for (int u = 0; u < kCastUnroll; ++u) Cast::store(dst + done + u * kStep + i, raw[u]);
+      }
+      for (; done + kStep <= len; done += kStep) Cast::store(dst + done + i, Cast::load(src + done + i));
     }
     for (int64_t i = done + threadIdx.x; i < len; i += kThreads) dst[i] = cast_elem<SRC, DST>(src[i]);
   }
@@ -219,25 +234,23 @@ FSH_API int fsh_pack_segments(const int64_t* input_ptrs_dev, const int64_t* tens
   if (nsegments == 0 || max_segment_numel == 0) return FSH_OK;
   if (!input_ptrs_dev || !tensor_indices_dev || !src_offsets_dev || !numels_dev || !dst_offsets_dev || !dst_dev)
     return fail(FSH_EINVAL, "fsh_pack_segments: null pointer");
-  const int64_t slices = ceil_div(max_segment_numel, kPackSliceElems);
-  const int64_t grid = nsegments * slices;
-  if (grid > 0x7FFFFFFFLL) return fail(FSH_ENOTSUP, "fsh_pack_segments: %lld workgroups exceed the grid limit", (long long)grid);
-  const dim3 g(static_cast<uint32_t>(grid)), b(kThreads);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define FSH_PACK_LAUNCH(SRC, DST)                                                                      \
-  hipLaunchKernelGGL((pack_segments_kernel<SRC, DST>), g, b, 0, s, input_ptrs_dev, tensor_indices_dev, \
-                     src_offsets_dev, numels_dev, dst_offsets_dev, static_cast<DST*>(dst_dev), slices)
-  if (src_dtype == FSH_DT_F32 && dst_dtype == FSH_DT_BF16) {
-    FSH_PACK_LAUNCH(float, uint16_t);
-  } else if (src_dtype == FSH_DT_BF16 && dst_dtype == FSH_DT_F32) {
-    FSH_PACK_LAUNCH(uint16_t, float);
-  } else if (src_dtype == FSH_DT_F32 && dst_dtype == FSH_DT_F32) {
-    FSH_PACK_LAUNCH(float, float);
-  } else if (src_dtype == FSH_DT_BF16 && dst_dtype == FSH_DT_BF16) {
-    FSH_PACK_LAUNCH(uint16_t, uint16_t);
-  } else {
-    return fail(FSH_EINVAL, "fsh_pack_segments: unsupported dtype pair (%d -> %d)", src_dtype, dst_dtype);
-  }
-#undef FSH_PACK_LAUNCH
-  return check_launch("fsh_pack_segments");
+  auto launch = [&](auto src_tag, auto dst_tag) -> int {
+    using SRC = decltype(src_tag);
+    using DST = decltype(dst_tag);
+    int64_t elems = kPackSliceElems<SRC, DST>;
+    while (nsegments * ceil_div(max_segment_numel, elems) >= (1 << 24) && elems < max_segment_numel) elems *= 2;
+    const int64_t slices = ceil_div(max_segment_numel, elems), grid = nsegments * slices;
+    if (grid > 0x7FFFFFFFLL)
+      return fail(FSH_ENOTSUP, "fsh_pack_segments: %lld workgroups exceed the grid limit", (long long)grid);
+    hipLaunchKernelGGL((pack_segments_kernel<SRC, DST>), dim3(static_cast<uint32_t>(grid)), dim3(kThreads), 0, s, input_ptrs_dev,
+                       tensor_indices_dev, src_offsets_dev, numels_dev, dst_offsets_dev, static_cast<DST*>(dst_dev),
+                       static_cast<uint32_t>(slices), elems);
+    return check_launch("fsh_pack_segments");
+  };
+  if (src_dtype == FSH_DT_F32 && dst_dtype == FSH_DT_BF16) return launch(float{}, uint16_t{});
+  if (src_dtype == FSH_DT_BF16 && dst_dtype == FSH_DT_F32) return launch(uint16_t{}, float{});
+  if (src_dtype == FSH_DT_F32 && dst_dtype == FSH_DT_F32) return launch(float{}, float{});
+  if (src_dtype == FSH_DT_BF16 && dst_dtype == FSH_DT_BF16) return launch(uint16_t{}, uint16_t{});
+  return fail(FSH_EINVAL, "fsh_pack_segments: unsupported dtype pair (%d -> %d)", src_dtype, dst_dtype);
 }
