@@ -20,14 +20,19 @@ namespace fsh {
 namespace {
 
 // ------------------------------------------------------------ 1x128 quantize
-// A workgroup owns 64 rows x 512 columns (4 scale blocks per row).  Sixteen
+// A workgroup owns 16 rows x 512 columns (4 scale blocks per row).  Sixteen
 // lanes own one run of 128 elements (16 bytes each); a wavefront load covers
-// four runs = 1 KB of one row.  All sixteen loads of a thread are issued
-// before the first is used.  The maximum of a run stays inside its row of 16
-// lanes (four DPP steps, no LDS, no barrier).  Scales go through LDS so that
-// they leave as 256-byte runs of the [k-block][row] table.
+// four runs = 1 KB of one row.  All four loads of a thread are issued before
+// the first is used.  The maximum of a run stays inside its row of 16 lanes
+// (four DPP steps, no LDS, no barrier).  Scales go through LDS so that they
+// leave as 64-byte runs of the [k-block][row] table.
+//
+// Bound by memory when large, by the chain of one thread's passes (each with
+// two divisions) when small.  With 64 rows per workgroup, sixteen passes (us,
+// 64 / 16 / 4 rows):  48 x 4096 5.5 / 4.2 / 4.0   1000 x 2048 7.5 / 4.1 / 4.0
+//   2048 x 4096 9.1 / 6.1 / 6.8   8192 x 4096 22.7 / 18.6 / 19.0   8192 x 14336 61.1 / 57.3 / 61.4
 constexpr int kActThreads = 256;
-constexpr int kActRows = 64;
+constexpr int kActRows = 16;
 constexpr int kActBlocks = 4;  // 128-element runs per row and workgroup
 constexpr int kActPasses = kActRows * kActBlocks * 16 / kActThreads;
 
@@ -50,7 +55,7 @@ __global__ __launch_bounds__(kActThreads) void act_quant_1x128_kernel(const ActQ
   u32x4 v[kActPasses];
 #pragma unroll
   for (int pass = 0; pass < kActPasses; ++pass) {
-    const int run = pass * 16 + run_lane;  // 0..255 within the tile
+    const int run = pass * 16 + run_lane;  // within the tile
     const int64_t row = row0 + run / kActBlocks;
     const int64_t col = (kb0 + run % kActBlocks) * 128 + sub * 8;
     v[pass] = u32x4{0, 0, 0, 0};
@@ -82,7 +87,7 @@ __global__ __launch_bounds__(kActThreads) void act_quant_1x128_kernel(const ActQ
     }
   }
   __syncthreads();
-  {
+  if (tid < kActBlocks * kActRows) {
     const int kbl = tid / kActRows, r = tid % kActRows;
     const int64_t kb = kb0 + kbl, row = row0 + r;
     if (row < p.rows && kb * 128 < p.ldq) p.scales[kb * p.rows + row] = lds_scales[tid];
