@@ -641,9 +641,25 @@ int launch_fp8_gemm(Fp8GemmParams& p, bool column_scales, const char* who, void*
   // half tiles, twice as many workgroups of half the length: e.g. the 896
   // tiles of a [14336, 4096] result take 3.5 rounds instead of 4.
   const Fp8TileKind kind = fp8_tile_kind(p.m, p.n, p.k);
-  if (kind == kFp8Tiles64) return launch_fp8_tiles<Fp8Tiles<2, 2, 1, 1, 3>, 3>(p, column_scales, static_cast<hipStream_t>(stream));
-  if (kind == kFp8Tiles128) return launch_fp8_tiles<Fp8Tiles<2, 2, 2, 2, 2>, 2>(p, column_scales, static_cast<hipStream_t>(stream));
   const int64_t units = compute_units();
+  const hipStream_t on = static_cast<hipStream_t>(stream);
+  // A compute unit with one workgroup to run has LDS to spare: more stages,
+  // i.e. more operand requests in flight.  Not where a unit runs several, whose
+  // requests cover one another's waits (us, fewer / more stages, weights from memory):
+  //   64 x 64, 3 / 4 stages:    48 x 14336, k 4096 18.6 / 16.2   48 x 4096, k 14336 48.2 / 36.1
+  //                             512 x 4096, k 4096 17.6 / 18.4 (column scales 20.6 / 19.2)   1024 x 4096, k 4096 32.5 / 32.6
+  //   128 x 128, 2 / 4 stages:  1024 x 4096, k 8192 55.9 / 46.9   1000 x 2048, k 5120 30.8 / 29.6   1000 x 5120, k 2048 20.3 / 28.3
+  // (eight stages of 64 x 64 tiles: 18.2 and 35.7 us on the first two, 0.4 us more where k is short)
+  if (kind == kFp8Tiles64) {
+    const int64_t few = ceil_div(p.m, (int64_t)64) * ceil_div(p.n, (int64_t)64);
+    if (few <= (column_scales ? 2 * units : units)) return launch_fp8_tiles<Fp8Tiles<2, 2, 1, 1, 4>, 2>(p, column_scales, on);
+    return launch_fp8_tiles<Fp8Tiles<2, 2, 1, 1, 3>, 3>(p, column_scales, on);
+  }
+  if (kind == kFp8Tiles128) {
+    if (ceil_div(p.m, (int64_t)128) * ceil_div(p.n, (int64_t)128) <= units)
+      return launch_fp8_tiles<Fp8Tiles<2, 2, 2, 2, 4>, 1>(p, column_scales, on);
+    return launch_fp8_tiles<Fp8Tiles<2, 2, 2, 2, 2>, 2>(p, column_scales, on);
+  }
   const int64_t tail = units > 0 ? tiles % units : 0;
   const int64_t cut = (tail > 0 && 2 * tail <= units) ? tail : 0;
   s.work_items = tiles - cut;
