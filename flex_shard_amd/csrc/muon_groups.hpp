@@ -269,38 +269,123 @@ __global__ __launch_bounds__(kNormThreads) void muon_apply_groups_kernel(const M
   }
 }
 
-// Reads matrix b of `in` ([rows, cols]), divides by max(||.||_F, eps) as bf16
-// tensor ops would (norm rounded to bf16, fp32 division, bf16 result), and
-// writes the result to `out_same` ([rows, cols]) and `out_t` ([cols, rows]);
-// either output may be null.
-// A workgroup owns a 64x64 tile: 16-byte loads and stores of 8 elements along
-// the rows, and for the transposed copy the tile goes through LDS and leaves
-// as 16-byte stores of 8 elements along the columns.  rows and cols are
-// multiples of 8, so an 8-element group is either whole or absent.
+// A matrix's norm from its partial sums: bf16(sqrt(sum)) floored at eps.
+__device__ __forceinline__ float norm_of_partials(const float* partial, int slices, float eps, float* lds) {
+  float total = 0.0f;
+  for (int j = threadIdx.x; j < slices; j += kNormThreads) total += partial[j];
+  total = block_sum(total, lds);
+  const float norm = bf16_bits_to_f32(f32_to_bf16_bits(sqrtf(total)));
+  return norm < eps ? eps : norm;
+}
+
+// The partials of a 7168 x 2048 matrix (7 KB) are as much to read as a block
+// of the normalization has data, ahead of its first store: from more than
+// kNormSlices slices on a launch of its own adds them up and leaves the norm in
+// place of the matrix's first partial (48 such and square matrices: 468 us in
+// one launch, 5 + 292 us in two with the cheaper division below).
+// Fewer are added up by every block, which costs less than the 5 us launch (20
+// matrices of at most 288 slices: 33.5 us in one launch, 4.8 + 30.5 in two).
+constexpr int kNormSlices = 512;
 constexpr int kNormTile = 64;
 constexpr int kNormPitch = kNormTile + 2;  // u16 per LDS row
 struct NormalizeGroup {
   const uint16_t* in;
   uint16_t* out_same;
   uint16_t* out_t;
-  const float* partial;  // [batch, slices]
-  int64_t rows, cols, tiles_c, tiles;
+  float* partial;        // [batch, slices]
+  int64_t rows, cols;
+  int32_t tiles, tiles_c;  // blocks per matrix; 64 x 64 tiles per row of tiles (transposing groups)
   int32_t slices;
   int32_t first_block;   // INT32_MAX past the last group
+  int32_t first_matrix;  // of all groups of the launch
 };
 struct NormalizeLaunch {
   NormalizeGroup group[kMaxMuonGroups];
   float eps_bf16;
+  int32_t norms_ready;  // norm_groups_kernel ran
 };
+__global__ __launch_bounds__(kNormThreads) void norm_groups_kernel(const NormalizeLaunch launch) {
+  __shared__ float lds[kNormThreads / 64];
+  int w = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxMuonGroups; ++i) w += static_cast<int>(blockIdx.x) >= launch.group[i].first_matrix ? 1 : 0;
+  const NormalizeGroup& p = launch.group[uniform_i32(w)];
+  float* partial = p.partial + (static_cast<int64_t>(blockIdx.x) - p.first_matrix) * p.slices;
+  const float norm = norm_of_partials(partial, p.slices, launch.eps_bf16, lds);  // all are read behind its barrier
+  if (threadIdx.x == 0) partial[0] = norm;
+}
+
+// bf16(x / norm), the bits of the correctly rounded fp32 quotient rounded to
+// bf16, for eight bf16 values: x times the reciprocal with one residual step.
+// Eight IEEE divisions and software roundings per vector (22 operations a
+// value) had the vector ALU as busy as the memory.  x and norm have eight
+// significant bits, so a quotient that is not a tie of the bf16 rounding is
+// 2^-17 away from one, and a tie is met exactly; 2^64 keeps the residuals of
+// small x out of the subnormals.  Norms outside [2^-60, 2^60], where the
+// scaled values could leave the range, and infinite or NaN ones divide.
+struct Normalizer {
+  float norm, recip;
+  bool divide;  // the same for the whole workgroup
+  __device__ __forceinline__ explicit Normalizer(float norm_of_matrix) {
+    norm = u32_as_f32(static_cast<uint32_t>(uniform_i32(static_cast<int>(f32_as_u32(norm_of_matrix)))));
+    divide = !(norm >= 0x1p-60f && norm <= 0x1p60f);
+    recip = 1.0f / norm;
+  }
+  __device__ __forceinline__ float quotient(float x) const {
+    const float scaled = x * 0x1p64f, q = scaled * recip;
+    return __builtin_fmaf(__builtin_fmaf(-q, norm, scaled), recip, q) * 0x1p-64f;
+  }
+  __device__ __forceinline__ u32x4 operator()(const u32x4& v) const {
+    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+    uint32_t out[4];
+    if (divide) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        out[j] = f32_to_bf16_bits(u32_as_f32(d[j] << 16) / norm) | (f32_to_bf16_bits(u32_as_f32(d[j] & 0xFFFF0000u) / norm) << 16);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) out[j] = pack_bf16x2(quotient(u32_as_f32(d[j] << 16)), quotient(u32_as_f32(d[j] & 0xFFFF0000u)));
+    }
+    return u32x4{out[0], out[1], out[2], out[3]};
+  }
+};
+
+// Divides matrix b of `in` ([rows, cols]) by its norm as bf16 tensor ops would
+// (fp32 division, bf16 result) and writes it to `out_same` ([rows, cols]) and
+// `out_t` ([cols, rows]); either may be null.  Bound by memory.
+// Without a transposed output a block takes 1024 consecutive 8-element vectors,
+// four per thread, requested together.  With one it owns a 64 x 64 tile:
+// 16-byte loads and stores of 8 elements along the rows, and the tile goes
+// through LDS and leaves as 16-byte stores of 8 elements along the columns.
+// rows and cols are multiples of 8, so an 8-element group is whole or absent.
 __global__ __launch_bounds__(kNormThreads) void normalize_groups_kernel(const NormalizeLaunch launch) {
   __shared__ uint16_t tile[kNormTile * kNormPitch];
   __shared__ float lds[kNormThreads / 64];
   const NormalizeGroup& p = launch.group[group_of_block(launch)];
   const int64_t rows = p.rows, cols = p.cols;
-  const int64_t block = static_cast<int64_t>(blockIdx.x) - p.first_block;
-  const int64_t b = block / p.tiles, t = block - b * p.tiles;
-  const int64_t r0 = t / p.tiles_c * kNormTile, c0 = t % p.tiles_c * kNormTile;
+  const uint32_t block = blockIdx.x - static_cast<uint32_t>(p.first_block);
+  const uint32_t b = block / static_cast<uint32_t>(p.tiles), t = block - b * static_cast<uint32_t>(p.tiles);
   const uint16_t* m = p.in + b * rows * cols;
+  const float* partial = p.partial + static_cast<int64_t>(b) * p.slices;
+  const auto norm_of_matrix = [&]() {
+    return launch.norms_ready ? *partial : norm_of_partials(partial, p.slices, launch.eps_bf16, lds);
+  };
+  uint16_t* o = p.out_same ? p.out_same + b * rows * cols : nullptr;
+  if (p.out_t == nullptr) {  // the same for the whole workgroup
+    const int64_t vectors = rows * cols / 8, g0 = t * kSliceVectors + threadIdx.x;
+    constexpr int kUnroll = static_cast<int>(kSliceVectors / kNormThreads);
+    u32x4 v[kUnroll];
+#pragma unroll
+    for (int k = 0; k < kUnroll; ++k)
+      if (g0 + k * kNormThreads < vectors) v[k] = load_stream_u32x4(m + (g0 + k * kNormThreads) * 8);
+    const Normalizer normalized(norm_of_matrix());
+#pragma unroll
+    for (int k = 0; k < kUnroll; ++k)
+      if (g0 + k * kNormThreads < vectors) store_stream_u32x4(o + (g0 + k * kNormThreads) * 8, normalized(v[k]));
+    return;
+  }
+  const uint32_t tile_r = t / static_cast<uint32_t>(p.tiles_c), tile_c = t - tile_r * static_cast<uint32_t>(p.tiles_c);
+  const int64_t r0 = static_cast<int64_t>(tile_r) * kNormTile, c0 = static_cast<int64_t>(tile_c) * kNormTile;
   const int q = threadIdx.x & 7, line = threadIdx.x >> 3;  // 8 groups of 8 elements per line, 32 lines per pass
   u32x4 v[2];
 #pragma unroll
@@ -308,32 +393,20 @@ __global__ __launch_bounds__(kNormThreads) void normalize_groups_kernel(const No
     const int64_t r = r0 + line + 32 * pass, c = c0 + 8 * q;
     if (r < rows && c < cols) v[pass] = load_stream_u32x4(m + r * cols + c);
   }
-  float total = 0.0f;
-  for (int j = threadIdx.x; j < p.slices; j += kNormThreads) total += p.partial[b * p.slices + j];
-  total = block_sum(total, lds);
-  float norm = bf16_bits_to_f32(f32_to_bf16_bits(sqrtf(total)));
-  norm = norm < launch.eps_bf16 ? launch.eps_bf16 : norm;
-  uint16_t* o = p.out_same ? p.out_same + b * rows * cols : nullptr;
-  uint16_t* ot = p.out_t ? p.out_t + b * rows * cols : nullptr;
+  const Normalizer normalized(norm_of_matrix());
+  uint16_t* ot = p.out_t + b * rows * cols;
 #pragma unroll
   for (int pass = 0; pass < 2; ++pass) {
     const int lr = line + 32 * pass;
     const int64_t r = r0 + lr, c = c0 + 8 * q;
     if (r < rows && c < cols) {
-      const uint32_t d[4] = {v[pass].x, v[pass].y, v[pass].z, v[pass].w};
-      uint32_t bits[8];
+      const u32x4 n = normalized(v[pass]);
+      if (o != nullptr) store_stream_u32x4(o + r * cols + c, n);
+      const uint32_t d[4] = {n.x, n.y, n.z, n.w};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        bits[2 * j] = f32_to_bf16_bits(u32_as_f32(d[j] << 16) / norm);
-        bits[2 * j + 1] = f32_to_bf16_bits(u32_as_f32(d[j] & 0xFFFF0000u) / norm);
-      }
-      if (o != nullptr) store_stream_u32x4(o + r * cols + c, pack8(bits));
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        *reinterpret_cast<uint32_t*>(&tile[lr * kNormPitch + 8 * q + 2 * j]) = bits[2 * j] | (bits[2 * j + 1] << 16);
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<uint32_t*>(&tile[lr * kNormPitch + 8 * q + 2 * j]) = d[j];
     }
   }
-  if (ot == nullptr) return;  // the same for the whole workgroup
   __syncthreads();
 #pragma unroll
   for (int pass = 0; pass < 2; ++pass) {

@@ -877,8 +877,11 @@ int ns_begin(const fsh_ns_problem& q, bool large, int32_t steps, NsState* st, No
   normalize->partial = partial;
   normalize->rows = rows;
   normalize->cols = cols;
-  normalize->tiles_c = ceil_div(cols, (int64_t)kNormTile);
-  normalize->tiles = normalize->tiles_c * ceil_div(rows, (int64_t)kNormTile);
+  const int64_t tiles_c = ceil_div(cols, (int64_t)kNormTile);
+  const int64_t tiles = transposed ? tiles_c * ceil_div(rows, (int64_t)kNormTile) : ceil_div(rows * cols / 8, kSliceVectors);
+  if (tiles >= INT32_MAX) return fail(FSH_ENOTSUP, "newton_schulz: more than %d blocks in one launch", INT32_MAX);
+  normalize->tiles_c = static_cast<int32_t>(tiles_c);
+  normalize->tiles = static_cast<int32_t>(tiles);
   normalize->slices = static_cast<int32_t>(slices_of(rows * cols / 8));
   return FSH_OK;
 }
@@ -893,11 +896,20 @@ int add_blocks(Group* group, int64_t blocks, int64_t batch, int64_t* total) {
 }
 
 int launch_normalize(NormalizeLaunch& launch, const NsState* st, int count, float eps, hipStream_t stream) {
-  int64_t blocks = 0;
-  for (int i = 0; i < count; ++i)
-    if (int rc = add_blocks(&launch.group[i], launch.group[i].tiles, st[i].batch, &blocks)) return rc;
-  for (int i = count; i < kMaxMuonGroups; ++i) launch.group[i].first_block = INT32_MAX;
+  int64_t blocks = 0, matrices = 0;
+  for (int i = 0; i < count; ++i) {
+    launch.group[i].first_matrix = static_cast<int32_t>(matrices);
+    matrices += st[i].batch;  // (fewer than blocks)
+    if (int rc = add_blocks(&launch.group[i], static_cast<int64_t>(launch.group[i].tiles), st[i].batch, &blocks)) return rc;
+  }
+  for (int i = count; i < kMaxMuonGroups; ++i) launch.group[i].first_block = launch.group[i].first_matrix = INT32_MAX;
   launch.eps_bf16 = bf16_round_host(eps);
+  launch.norms_ready = 0;
+  for (int i = 0; i < count; ++i) launch.norms_ready |= launch.group[i].slices > kNormSlices ? 1 : 0;
+  if (launch.norms_ready) {
+    hipLaunchKernelGGL(norm_groups_kernel, dim3(static_cast<uint32_t>(matrices)), dim3(kNormThreads), 0, stream, launch);
+    if (int rc = check_launch("norm_groups_kernel")) return rc;
+  }
   hipLaunchKernelGGL(normalize_groups_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kNormThreads), 0, stream, launch);
   return check_launch("normalize_groups_kernel");
 }
@@ -1012,7 +1024,7 @@ FSH_API int fsh_newton_schulz_multi(const fsh_ns_problem* problems, int32_t coun
     batch[i] = problems[i].batch;
     MuonGroupDev& g = sums.group[i];
     g.batch = static_cast<uint16_t*>(problems[i].x_dev);
-    g.partial = const_cast<float*>(normalize.group[i].partial);
+    g.partial = normalize.group[i].partial;
     g.vectors = problems[i].rows * problems[i].cols / 8;
     g.slices = normalize.group[i].slices;
   }
@@ -1096,7 +1108,7 @@ FSH_API int fsh_muon_step(const fsh_muon_group* groups, int32_t count, float ler
     q.momentum_ptrs = g.momentum_ptrs_dev;
     q.grad_ptrs = g.grad_ptrs_dev;
     q.batch = static_cast<uint16_t*>(g.batch_dev);
-    q.partial = const_cast<float*>(normalize.group[i].partial);
+    q.partial = normalize.group[i].partial;
     q.vectors = problems[i].rows * problems[i].cols / 8;
     q.rows = g.rows;
     q.cols = g.cols;
