@@ -223,6 +223,35 @@ __device__ __forceinline__ void muon_apply_slice(const MuonLaunch& launch, const
   const uint16_t* dir = q.batch + matrix * q.vectors * 8;
   const MasterVector<kF32, kPadded> master{q};
   constexpr int kUnroll = kF32 ? 2 : 4;
+  if (kF32 && !kPadded) {
+    // Every element is on its own, so fp32 masters go in chunks of four: one
+    // 16-byte access contiguous across the wave.  Eight per lane are two of
+    // them 32 bytes apart, each asking for half of every line (101 M
+    // parameters: 178 us that way, 158 us here, 6.4 TB/s).
+    constexpr int kChunks = 4;
+    float* out = static_cast<float*>(param);
+    for (int64_t c0 = 2 * begin + threadIdx.x; c0 < 2 * end; c0 += kChunks * kNormThreads) {
+      f32x4 p[kChunks];
+      u32x2 d[kChunks];
+#pragma unroll
+      for (int k = 0; k < kChunks; ++k)
+        if (c0 + k * kNormThreads < 2 * end) {
+          p[k] = load_stream_f32x4(out + (c0 + k * kNormThreads) * 4);
+          d[k] = load_stream_u32x2(dir + (c0 + k * kNormThreads) * 4);
+        }
+#pragma unroll
+      for (int k = 0; k < kChunks; ++k)
+        if (c0 + k * kNormThreads < 2 * end) {
+          const auto apply = [&](float value, uint32_t bits) {
+            return muon_apply_one_f32(value, u32_as_f32(bits), launch.decay, q.neg_lr, q.dir_scale);
+          };
+          *reinterpret_cast<f32x4*>(out + (c0 + k * kNormThreads) * 4) =
+              f32x4{apply(p[k].x, d[k].x << 16), apply(p[k].y, d[k].x & 0xFFFF0000u), apply(p[k].z, d[k].y << 16),
+                    apply(p[k].w, d[k].y & 0xFFFF0000u)};
+        }
+    }
+    return;
+  }
   for (int64_t g0 = begin + threadIdx.x; g0 < end; g0 += kUnroll * kNormThreads) {
     float pv[kUnroll][8];
     u32x4 draw[kUnroll];
