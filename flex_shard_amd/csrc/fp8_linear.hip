@@ -560,7 +560,8 @@ namespace fsh {
 namespace {
 
 // Which tiles a product takes: the ones with the lowest estimated time.
-// Measured (us with 64 x 64, 128 x 128, 256 x 256 tiles; block scales, the
+// Measured (us with 64 x 64 tiles of three stages, 128 x 128 of two, 256 x 256;
+// weights in the last-level cache; block scales, the
 // column-scale variant runs 5-10 % longer on all three):
 //   48 x 14336, k 4096     14.5   24.9   35.5      48 x 4096, k 14336  34.6  69.8  112
 //   256 x 4096, k 4096     13.0   23.4   27.6      1000 x 2048, k 5120 22.1  31.4  46.3
