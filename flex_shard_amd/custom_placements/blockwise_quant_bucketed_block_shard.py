@@ -131,12 +131,15 @@ GATHER_RING_SLOTS = 3
 class _QuantUnshardState:
     """The placement's private state of one prepared unshard."""
 
-    __slots__ = ("infos", "pg", "debug_fqn", "metadata", "copied_out")
+    __slots__ = ("infos", "pg", "debug_fqn", "metadata", "copied_out", "refilled")
 
     def __init__(self, infos: list, pg: Any, debug_fqn: str | None, metadata: quant_plan.QuantBucketMetadata) -> None:
         self.infos, self.pg, self.debug_fqn, self.metadata = infos, pg, debug_fqn, metadata
         #: the persistent buffers were refilled behind the exchange, in ``run_prepared_unshard``
         self.copied_out = False
+        #: the buffer that refill wrote, if it read the ranks' rows where they lie: the
+        #: gathered rows are unwritten then, and whatever needs them reads this instead
+        self.refilled: torch.Tensor | None = None
 
 
 # A forward pack that a backward re-gather may take once is remembered as a
@@ -899,10 +902,17 @@ class BlockwiseQuantBucketedBlockShard(BucketedBlockShard):
         with record_copy_out():
             copy_row_segments(rows, compact, descriptor)
         state.copied_out = True
+        state.refilled = compact
         return True
 
     def finish_prepared_unshard(self, prepared: PlacementPreparedUnshard) -> PlacementUnshardResult:
         state = self._unshard_state(prepared)
+        if state.refilled is not None:
+            compact = self._refilled_compact_buffer(prepared, state)
+            return PlacementUnshardResult(
+                full_params=self._full_params_from_compact(state, compact),
+                persistent_buffers=[compact] if prepared.persistent or prepared.persistent_buffers is not None else [],
+            )
         rows = prepared.buffers[1].view(len(state.metadata.rank_qdata_numels), prepared.buffers[0].numel())
         return self._finish_unshard_from_rank_rows(prepared, rows)
 
@@ -934,6 +944,16 @@ class BlockwiseQuantBucketedBlockShard(BucketedBlockShard):
             return prepared.persistent_buffers[0]
         _, scale_start, groups = self._compact_sizes(metadata)
         return torch.empty(scale_start + sum(groups), dtype=torch.uint8, device=device)
+
+    def _refilled_compact_buffer(self, prepared: PlacementPreparedUnshard, state: "_QuantUnshardState") -> torch.Tensor:
+        """:meth:`_compact_buffer` of an unshard whose refill left the gathered
+        rows unwritten, filled (it is another buffer than the refilled one only
+        if the caller has changed the persistent buffers since)."""
+        assert state.refilled is not None
+        compact = self._compact_buffer(prepared, state.metadata, state.refilled.device)
+        if compact is not state.refilled:
+            compact.copy_(state.refilled)
+        return compact
 
     def _full_params_from_compact(self, state: "_QuantUnshardState", compact: torch.Tensor) -> list[torch.Tensor]:
         """Per-parameter views of the compact buffer handed to the weight factory."""

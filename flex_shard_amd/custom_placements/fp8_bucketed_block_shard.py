@@ -190,12 +190,15 @@ class Fp8BucketedBlockShard(BlockwiseQuantBucketedBlockShard):
 
     # --------------------------------------------- fused compaction + dequant
     def _unpack_table(
-        self, state: "BlockwiseQuantBucketedBlockShard._QuantUnshardState", row_stride: int, device: torch.device
+        self, state: "BlockwiseQuantBucketedBlockShard._QuantUnshardState", row_stride: int | None, device: torch.device
     ):
         """Device table of ``fsh_unpack_chunk`` records, one per (rank, chunk),
-        built once per (bucket metadata, row stride, device)."""
+        built once per (bucket metadata, row stride, device).  ``row_stride``
+        None: the bytes are read from a compact buffer instead of the ranks'
+        rows."""
         metadata = state.metadata
-        key = (id(metadata), row_stride, device)
+        # (a compact buffer's table is one per stream: it is uploaded on the one it is first used on)
+        key = (id(metadata), hip_ops.stream_ptr(device) if row_stride is None else None, row_stride, device)
         cached = self._unpack_tables.get(key)
         if cached is not None and cached[0] is metadata:
             return cached[1:]
@@ -219,15 +222,12 @@ class Fp8BucketedBlockShard(BlockwiseQuantBucketedBlockShard):
                 assert chunk.rank == rank and chunk.fqn == pack_chunk.fqn
                 rows, in_dim = pack_chunk.local_shape
                 first_scale = scale_base[chunk.fqn] + (chunk.row_start // block) * tiles_c_of[chunk.fqn]
-                records += [
-                    rank * row_stride + chunk.qdata_offset,
-                    rank * row_stride + scale_cursor,
-                    rows,
-                    in_dim,
-                    chunk.global_dense_offset,
-                    scale_start + 4 * first_scale,
-                    chunk.global_dense_offset,
-                ]
+                compact_at = (chunk.global_dense_offset, scale_start + 4 * first_scale)
+                if row_stride is None:
+                    records += compact_at
+                else:
+                    records += [rank * row_stride + chunk.qdata_offset, rank * row_stride + scale_cursor]
+                records += [rows, in_dim, *compact_at, chunk.global_dense_offset]
                 tile_starts.append(tile_starts[-1] + _ceil_div(rows, block) * tiles_c_of[chunk.fqn])
                 scale_cursor += 4 * pack_chunk.scale_numels[0]
         table, table_host = _upload_i64(records, device)
@@ -251,24 +251,39 @@ class Fp8BucketedBlockShard(BlockwiseQuantBucketedBlockShard):
         ``dequant_dtype`` tensor per parameter, each a view of one flat buffer
         in parameter order.  Values equal ``BlockwiseFp8Weight.dequantize()`` on
         the gathered weight: fp32 product of the FP8 value and its tile's scale,
-        rounded once."""
+        rounded once.
+
+        A refill that read the ranks' rows where they lie has written no
+        gathered rows; its weights are dequantized from the refilled buffer,
+        which holds the same bytes and scales."""
         state = self._unshard_state(prepared)
-        if rank_rows is None:
-            rank_rows = prepared.buffers[1].view(len(state.metadata.rank_qdata_numels), prepared.buffers[0].numel())
-        self._check_rank_rows(state, rank_rows)
-        _require_gpu_rows(rank_rows, "The fused unpack")
-        if rank_rows.stride(1) != 1:
-            raise ValueError("gathered rank rows must have unit byte stride within a row")
-        row_stride = rank_rows.stride(0) if rank_rows.size(0) > 1 else rank_rows.size(1)
+        refilled = state.refilled if rank_rows is None else None
+        if refilled is not None:
+            rank_rows, row_stride = refilled, None
+        else:
+            if rank_rows is None:
+                rank_rows = prepared.buffers[1].view(len(state.metadata.rank_qdata_numels), prepared.buffers[0].numel())
+            self._check_rank_rows(state, rank_rows)
+            _require_gpu_rows(rank_rows, "The fused unpack")
+            if rank_rows.stride(1) != 1:
+                raise ValueError("gathered rank rows must have unit byte stride within a row")
+            row_stride = rank_rows.stride(0) if rank_rows.size(0) > 1 else rank_rows.size(1)
         table, starts, total_tiles, _hosts = self._unpack_table(state, row_stride, rank_rows.device)
         total = sum(info.global_numel for info in state.infos)
         if dequant_out is None:
             dequant_out = torch.empty(total, dtype=dequant_dtype, device=rank_rows.device)
         elif dequant_out.numel() != total or dequant_out.dtype != dequant_dtype or not dequant_out.is_contiguous():
             raise ValueError(f"dequant_out must be a contiguous {dequant_dtype} tensor of {total} elements")
-        compact_buf = self._compact_buffer(prepared, state.metadata, rank_rows.device) if compact else None
+        compact_buf = None
+        if compact and refilled is not None:
+            compact_buf = self._refilled_compact_buffer(prepared, state)
+        elif compact:
+            compact_buf = self._compact_buffer(prepared, state.metadata, rank_rows.device)
         with record_copy_out():
-            hip_ops.unpack_dequant(rank_rows, table, starts, total_tiles, compact_buf, dequant_out.view(-1), self.block_size)
+            hip_ops.unpack_dequant(
+                rank_rows, table, starts, total_tiles, compact_buf if refilled is None else None, dequant_out.view(-1),
+                self.block_size,
+            )
         plan = None if torch.compiler.is_compiling() else self._full_param_plan(state)
         if plan is not None:
             first = dequant_out.storage_offset()
