@@ -344,17 +344,18 @@ def reduce_scatter_grads(output: torch.Tensor, input: torch.Tensor, reduction: "
     and consumes the deposits; with a
     ``torch.distributed`` group it is one collective, as in the reference."""
     if isinstance(group, LocalReduceGroup):
+        # `deposited` names rows that were written: a reduction that is refused
+        # below leaves nothing behind that a second call would take for one.
+        missing = sorted(set(range(group.size())) - group.deposited - {group.rank()})
         own = None
         if group.rank() not in group.deposited:
             held = group.contributions
-            if input.is_contiguous() and input.device.type == "cuda" and input.dtype == output.dtype and (
+            if not missing and input.is_contiguous() and input.device.type == "cuda" and input.dtype == output.dtype and (
                 held is None or (held.dtype == input.dtype and held.device == input.device)
             ):
                 own = input.view(-1)
-                group.mark_deposited(group.rank())
             else:
                 group.deposit(group.rank(), input)
-        missing = sorted(set(range(group.size())) - group.deposited)
         if missing:
             raise ValueError(f"LocalReduceGroup is missing the contributions of ranks {missing}.")
         _local_reduce(output, group, reduction, own)
