@@ -29,6 +29,7 @@ from typing import Any
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 
 from .. import hip_ops
 from .blockwise_fp8_weight import BlockwiseFp8Weight
@@ -325,7 +326,8 @@ def _linear_forward(x: torch.Tensor, weight: BlockwiseFp8Weight, bias: torch.Ten
 
 
 def _apply_linear(x: torch.Tensor, weight: BlockwiseFp8Weight, bias: torch.Tensor | None, gemms) -> torch.Tensor:
-    if torch.is_grad_enabled() or torch._C._are_functorch_transforms_active():
+    # (inside a forward-mode level too: the function refuses a tangent, which the kernels would drop)
+    if torch.is_grad_enabled() or torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0:
         return _PrequantizedLinearFunction.apply(x, weight, bias, gemms)
     # Nothing to differentiate: no graph node, and the activation is quantized
     # in the one form that the product reads (host time of 48 tokens 34 -> 21 us).
