@@ -199,8 +199,10 @@ class Fp8BlockwiseGemms:
                 f"and weight input dim {in_dim}"
             )
         grad_bias = None
-        if needs_bias_grad and not (needs_weight_grad and grad_output_2d.dtype == torch.bfloat16):
-            # not from the quantizer's pass, which the weight gradient needs and which reads bf16
+        differentiable = torch.is_grad_enabled() and grad_output_2d.requires_grad
+        if needs_bias_grad and (differentiable or not (needs_weight_grad and grad_output_2d.dtype == torch.bfloat16)):
+            # not from the quantizer's pass, which the weight gradient needs, which reads bf16
+            # and whose sums a second backward could not go through
             grad_bias = grad_output_2d.sum(dim=0)
         if not (needs_x_grad or needs_weight_grad):
             return None, None, grad_bias
