@@ -252,12 +252,19 @@ class OwnedMuon:
             # views of a stacked parameter are taken per step: they follow a
             # parameter whose storage was replaced (``p.data = ...``) since
             self._matrices = self._as_matrices(self.params)
-        for keys, plan in self._plans:
-            members = [self._groups[key] for key in keys]
+        matrices = [
+            [
+                [[of[i] for i in self._groups[key]] for key in keys]
+                for of in (self._matrices, self._momentum_matrices, grad_matrices)
+            ]
+            for keys, _ in self._plans
+        ]
+        if len(self._plans) > 1:  # a step that one of the plans can't take updates nothing
+            for (_, plan), of_plan in zip(self._plans, matrices):
+                plan.check(*of_plan)
+        for (keys, plan), of_plan in zip(self._plans, matrices):
             plan.step(
-                [[self._matrices[i] for i in group] for group in members],
-                [[self._momentum_matrices[i] for i in group] for group in members],
-                [[grad_matrices[i] for i in group] for group in members],
+                *of_plan,
                 lerp_weight=1 - self.momentum, nesterov_weight=self.momentum, nesterov=self.nesterov,
                 decay_factor=1 - self.lr * self.weight_decay, coefficients=self.ns_coefficients, steps=self.ns_steps,
                 eps=self.eps,

@@ -897,9 +897,23 @@ class MuonStepPlan:
             slot.workspace_dev, slot.workspace_nbytes = workspace.data_ptr(), workspace.numel()
             slot.neg_adjusted_lr, slot.direction_scale = neg_lr, scale
 
-    def _refresh(self, table: torch.Tensor, current: list[int], tensors: Sequence[torch.Tensor], shape, dtype) -> None:
-        if len(tensors) != len(current):
-            raise ValueError(f"expected {len(current)} matrices of shape {shape}, got {len(tensors)}")
+    def check(
+        self, params: Sequence[Sequence[torch.Tensor]], momenta: Sequence[Sequence[torch.Tensor]],
+        grads: Sequence[Sequence[torch.Tensor]],
+    ) -> list[list[list[int]]]:
+        """The addresses of a step's matrices, per group and table; raises,
+        without having changed anything, if the step's kernels can't take them."""
+        for name, lists in (("parameter", params), ("momentum", momenta), ("gradient", grads)):
+            if len(lists) != len(self._shapes):
+                raise ValueError(f"expected {name} lists for {len(self._shapes)} groups, got {len(lists)}")
+        return [
+            [self._addresses(tensors, len(current), shape, dtype) for (_, current), tensors in zip(tables, (p, m, g))]
+            for tables, shape, dtype, p, m, g in zip(self._address_tables, self._shapes, self._dtypes, params, momenta, grads)
+        ]
+
+    def _addresses(self, tensors: Sequence[torch.Tensor], count: int, shape, dtype) -> list[int]:
+        if len(tensors) != count:
+            raise ValueError(f"expected {count} matrices of shape {shape}, got {len(tensors)}")
         addresses = []
         for t in tensors:
             if t.device != self._device:
@@ -909,12 +923,7 @@ class MuonStepPlan:
             if t.data_ptr() % 16 and not (shape[0] % 8 or shape[1] % 8):
                 raise ValueError("the Muon step kernels need 16-byte aligned matrices")
             addresses.append(t.data_ptr())
-        if addresses != current:
-            # A fresh pinned staging tensor per change: torch's host allocator
-            # keeps its block from reuse until the queued copy has read it, so
-            # nothing here waits for the GPU.
-            table.copy_(torch.tensor(addresses, dtype=torch.int64, pin_memory=True), non_blocking=True)
-            current[:] = addresses
+        return addresses
 
     def step(
         self, params: Sequence[Sequence[torch.Tensor]], momenta: Sequence[Sequence[torch.Tensor]],
@@ -938,12 +947,14 @@ class MuonStepPlan:
                 raise ValueError(f"expected one {name} per group ({len(self._shapes)}), got {len(values)}")
             for slot, value in zip(self._table, values):
                 setattr(slot, name, float(value))
-        for name, lists in (("parameter", params), ("momentum", momenta), ("gradient", grads)):
-            if len(lists) != len(self._shapes):
-                raise ValueError(f"expected {name} lists for {len(self._shapes)} groups, got {len(lists)}")
-        for tables, shape, dtype, p, m, g in zip(self._address_tables, self._shapes, self._dtypes, params, momenta, grads):
-            for (table, current), tensors in zip(tables, (p, m, g)):
-                self._refresh(table, current, tensors, shape, dtype)
+        for tables, wanted in zip(self._address_tables, self.check(params, momenta, grads)):
+            for (table, current), addresses in zip(tables, wanted):
+                if addresses != current:
+                    # A fresh pinned staging tensor per change: torch's host allocator
+                    # keeps its block from reuse until the queued copy has read it, so
+                    # nothing here waits for the GPU.
+                    table.copy_(torch.tensor(addresses, dtype=torch.int64, pin_memory=True), non_blocking=True)
+                    current[:] = addresses
         a, b, c = coefficients
         status = _native.lib().fsh_muon_step(
             self._table, len(self._shapes), lerp_weight, nesterov_weight, 1 if nesterov else 0, decay_factor, a, b, c,
