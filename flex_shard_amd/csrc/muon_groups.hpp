@@ -345,13 +345,15 @@ __global__ __launch_bounds__(kNormThreads) void norm_groups_kernel(const Normali
 }
 
 // bf16(x / norm), the bits of the correctly rounded fp32 quotient rounded to
-// bf16, for eight bf16 values: x times the reciprocal with one residual step.
-// Eight IEEE divisions and software roundings per vector (22 operations a
-// value) had the vector ALU as busy as the memory.  x and norm have eight
-// significant bits, so a quotient that is not a tie of the bf16 rounding is
-// 2^-17 away from one, and a tie is met exactly; 2^64 keeps the residuals of
-// small x out of the subnormals.  Norms outside [2^-60, 2^60], where the
-// scaled values could leave the range, and infinite or NaN ones divide.
+// bf16, for eight bf16 values: x times the reciprocal with one residual
+// correction (Markstein).  Eight IEEE divisions and software roundings per
+// vector (22 operations a value) had the vector ALU as busy as the memory.  x
+// and norm have eight significant bits, so a quotient that is not a tie of the
+// bf16 rounding is 2^-17 away from one, and a tie is met exactly; 2^64 keeps
+// the residuals of small x out of the subnormals.  The residual of a negative
+// zero is a positive one: the sign of x, which is the quotient's, is put back.
+// Norms outside [2^-60, 2^60], where the scaled values could leave the range,
+// and infinite or NaN ones divide.
 struct Normalizer {
   float norm, recip;
   bool divide;  // the same for the whole workgroup
@@ -373,7 +375,8 @@ struct Normalizer {
         out[j] = f32_to_bf16_bits(u32_as_f32(d[j] << 16) / norm) | (f32_to_bf16_bits(u32_as_f32(d[j] & 0xFFFF0000u) / norm) << 16);
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) out[j] = pack_bf16x2(quotient(u32_as_f32(d[j] << 16)), quotient(u32_as_f32(d[j] & 0xFFFF0000u)));
+      for (int j = 0; j < 4; ++j)
+        out[j] = pack_bf16x2(quotient(u32_as_f32(d[j] << 16)), quotient(u32_as_f32(d[j] & 0xFFFF0000u))) | (d[j] & 0x80008000u);
     }
     return u32x4{out[0], out[1], out[2], out[3]};
   }

@@ -41,6 +41,22 @@ def test_normalization_divides(device, shape, case):
     assert torch.equal(got[~got.isnan()], want[~got.isnan()])
 
 
+@pytest.mark.parametrize("case", ["usual", "tiny", "huge", "zero"])
+@pytest.mark.parametrize("shape", [(8, 8), (72, 200), (200, 72)])
+def test_normalization_keeps_the_sign_of_zero(device, shape, case):
+    """The int16 views are equal, zeros of either sign among the values."""
+    gen = torch.Generator().manual_seed(shape[1])
+    x = torch.randn(shape, generator=gen) * {"tiny": 2.0**-110, "huge": 2.0**52, "zero": 0.0}.get(case, 1.0)
+    x = x.bfloat16()
+    zero = torch.rand(shape, generator=gen) < 0.25
+    x[zero] = torch.where(torch.rand(shape, generator=gen) < 0.5, 0.0, -0.0).bfloat16()[zero]
+    x = x.to(device)
+    want = _normalized(x)
+    assert want[want == 0].signbit().any() and not want[want == 0].signbit().all()
+    got = hip_ops.newton_schulz(x.clone(), COEFFS, 0, 1e-7)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 # whole slices, slices that end inside a wave, less than one wave, odd rows and columns
 @pytest.mark.parametrize("shapes", [[(8, 8), (8, 520), (64, 1000)], [(1024, 1544), (1032, 72)], [(130, 77), (512, 512)]])
 def test_fp32_masters_equal_the_per_matrix_kernels(device, shapes):
