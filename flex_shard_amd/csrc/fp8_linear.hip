@@ -567,8 +567,23 @@ namespace {
 //   256 x 4096, k 4096     13.0   23.4   27.6      1000 x 2048, k 5120 22.1  31.4  46.3
 //   1024 x 4096, k 4096    30.7   26.9   38.3      2048 x 4096, k 4096 55.1  39.4  42.0
 //   1024 x 14336, k 4096   95.6   71.4   54.3      4096 x 4096, k 4096 112   73.0  58.8
-enum Fp8TileKind { kFp8Tiles64, kFp8Tiles128, kFp8Tiles256 };
-Fp8TileKind fp8_tile_kind(int64_t m, int64_t n, int64_t k) {
+//
+// A compute unit with one workgroup to run has LDS to spare: more stages,
+// i.e. more operand requests in flight ("deep").  Not where a unit runs several, whose
+// requests cover one another's waits (us, fewer / more stages, weights from memory):
+//   64 x 64, 3 / 4 stages:    48 x 14336, k 4096 18.6 / 16.2   48 x 4096, k 14336 48.2 / 36.1
+//                             512 x 4096, k 4096 17.6 / 18.4 (column scales 20.6 / 19.2)   1024 x 4096, k 4096 32.5 / 32.6
+//   128 x 128, 2 / 4 stages:  1024 x 4096, k 8192 55.9 / 46.9   1000 x 2048, k 5120 30.8 / 29.6   1000 x 5120, k 2048 20.3 / 28.3
+// (eight stages of 64 x 64 tiles: 18.2 and 35.7 us on the first two, 0.4 us more where k is short)
+enum Fp8TileKind {
+  kFp8Tiles64 = FSH_TILES_64,
+  kFp8Tiles64Deep = FSH_TILES_64_DEEP,
+  kFp8Tiles128 = FSH_TILES_128,
+  kFp8Tiles128Deep = FSH_TILES_128_DEEP,
+  kFp8Tiles256 = FSH_TILES_256,
+  kFp8Tiles256LongK = FSH_TILES_256_LONG_K,
+};
+Fp8TileKind fp8_tile_kind(int64_t m, int64_t n, int64_t k, bool column_scales, int64_t units) {
   static constexpr TileShape kShapes[] = {
       {64, 64, 768.0, 0.22, 0.34, 0.61, 2.0},    // three workgroups per compute unit
       {128, 128, 512.0, 0.56, 0.69, 1.07, 4.0},  // two
@@ -577,15 +592,21 @@ Fp8TileKind fp8_tile_kind(int64_t m, int64_t n, int64_t k) {
   const double ktiles = static_cast<double>(k / 128);
   int best = 0;
   double best_us = 0.0;
+  int64_t best_tiles = 0;
   for (int i = 0; i < 3; ++i) {
-    const double tiles = static_cast<double>(ceil_div(m, kShapes[i].m)) * static_cast<double>(ceil_div(n, kShapes[i].n));
-    const double us = rounds_us(kShapes[i], tiles, tiles * ktiles, ktiles);
+    const int64_t tiles = ceil_div(m, kShapes[i].m) * ceil_div(n, kShapes[i].n);
+    const double us = rounds_us(kShapes[i], static_cast<double>(tiles), static_cast<double>(tiles) * ktiles, ktiles);
     if (i == 0 || us < best_us) {
       best = i;
       best_us = us;
+      best_tiles = tiles;
     }
   }
-  return static_cast<Fp8TileKind>(best);
+  if (best == 0) return best_tiles <= (column_scales ? 2 * units : units) ? kFp8Tiles64Deep : kFp8Tiles64;
+  if (best == 1) return best_tiles <= units ? kFp8Tiles128Deep : kFp8Tiles128;
+  // The block-scale variant keeps one window of weight scales in LDS; a longer
+  // contraction takes the instantiation that refills it.
+  return !column_scales && k / 128 > Fp8Gemm::kMaxKTilesInLds ? kFp8Tiles256LongK : kFp8Tiles256;
 }
 
 template <typename Cfg, int kBlocksPerUnit>
@@ -637,30 +658,20 @@ int launch_fp8_gemm(Fp8GemmParams& p, bool column_scales, const char* who, void*
   const int64_t tiles = static_cast<int64_t>(s.tiles_m) * s.tiles_n;
   if (tiles > 0x3FFFFFFFLL) return fail(FSH_ENOTSUP, "%s: too many tiles", who);
   s.tiles_per_matrix = static_cast<int32_t>(tiles);
+  const int64_t units = compute_units();
+  const hipStream_t on = static_cast<hipStream_t>(stream);
+  const Fp8TileKind kind = fp8_tile_kind(p.m, p.n, p.k, column_scales, units);
+  switch (kind) {
+    case kFp8Tiles64: return launch_fp8_tiles<Fp8Tiles<2, 2, 1, 1, 3>, 3>(p, column_scales, on);
+    case kFp8Tiles64Deep: return launch_fp8_tiles<Fp8Tiles<2, 2, 1, 1, 4>, 2>(p, column_scales, on);
+    case kFp8Tiles128: return launch_fp8_tiles<Fp8Tiles<2, 2, 2, 2, 2>, 2>(p, column_scales, on);
+    case kFp8Tiles128Deep: return launch_fp8_tiles<Fp8Tiles<2, 2, 2, 2, 4>, 1>(p, column_scales, on);
+    default: break;
+  }
   // A workgroup holds a CU for a tile, so the tiles go through the chip in
   // rounds of one per CU.  A last round that is at most half full is cut into
   // half tiles, twice as many workgroups of half the length: e.g. the 896
   // tiles of a [14336, 4096] result take 3.5 rounds instead of 4.
-  const Fp8TileKind kind = fp8_tile_kind(p.m, p.n, p.k);
-  const int64_t units = compute_units();
-  const hipStream_t on = static_cast<hipStream_t>(stream);
-  // A compute unit with one workgroup to run has LDS to spare: more stages,
-  // i.e. more operand requests in flight.  Not where a unit runs several, whose
-  // requests cover one another's waits (us, fewer / more stages, weights from memory):
-  //   64 x 64, 3 / 4 stages:    48 x 14336, k 4096 18.6 / 16.2   48 x 4096, k 14336 48.2 / 36.1
-  //                             512 x 4096, k 4096 17.6 / 18.4 (column scales 20.6 / 19.2)   1024 x 4096, k 4096 32.5 / 32.6
-  //   128 x 128, 2 / 4 stages:  1024 x 4096, k 8192 55.9 / 46.9   1000 x 2048, k 5120 30.8 / 29.6   1000 x 5120, k 2048 20.3 / 28.3
-  // (eight stages of 64 x 64 tiles: 18.2 and 35.7 us on the first two, 0.4 us more where k is short)
-  if (kind == kFp8Tiles64) {
-    const int64_t few = ceil_div(p.m, (int64_t)64) * ceil_div(p.n, (int64_t)64);
-    if (few <= (column_scales ? 2 * units : units)) return launch_fp8_tiles<Fp8Tiles<2, 2, 1, 1, 4>, 2>(p, column_scales, on);
-    return launch_fp8_tiles<Fp8Tiles<2, 2, 1, 1, 3>, 3>(p, column_scales, on);
-  }
-  if (kind == kFp8Tiles128) {
-    if (ceil_div(p.m, (int64_t)128) * ceil_div(p.n, (int64_t)128) <= units)
-      return launch_fp8_tiles<Fp8Tiles<2, 2, 2, 2, 4>, 1>(p, column_scales, on);
-    return launch_fp8_tiles<Fp8Tiles<2, 2, 2, 2, 2>, 2>(p, column_scales, on);
-  }
   const int64_t tail = units > 0 ? tiles % units : 0;
   const int64_t cut = (tail > 0 && 2 * tail <= units) ? tail : 0;
   s.work_items = tiles - cut;
@@ -668,9 +679,7 @@ int launch_fp8_gemm(Fp8GemmParams& p, bool column_scales, const char* who, void*
   p.whole_grid = s.items_per_xcd * kXcds;
   p.half_items = 2 * cut;
   p.half_items_per_xcd = ceil_div(p.half_items, static_cast<int64_t>(kXcds));
-  // The block-scale variant keeps one window of weight scales in LDS; a longer
-  // contraction takes the instantiation that refills it.
-  const bool long_k = !column_scales && p.k / 128 > Fp8Gemm::kMaxKTilesInLds;
+  const bool long_k = kind == kFp8Tiles256LongK;
   static LdsReservation reserved_block_scales, reserved_block_scales_long, reserved_column_scales;
   if (int rc = column_scales
                    ? reserve_lds_once(reserved_column_scales, &fp8_gemm_blockwise_kernel<true>, Fp8Gemm::kLdsBytes)
@@ -680,17 +689,23 @@ int launch_fp8_gemm(Fp8GemmParams& p, bool column_scales, const char* who, void*
     return rc;
   const dim3 grid(static_cast<uint32_t>(p.whole_grid + p.half_items_per_xcd * kXcds)), block(Fp8Gemm::kThreads);
   if (column_scales)
-    hipLaunchKernelGGL(fp8_gemm_blockwise_kernel<true>, grid, block, Fp8Gemm::kLdsBytes, static_cast<hipStream_t>(stream), p);
+    hipLaunchKernelGGL(fp8_gemm_blockwise_kernel<true>, grid, block, Fp8Gemm::kLdsBytes, on, p);
   else if (long_k)
-    hipLaunchKernelGGL((fp8_gemm_blockwise_kernel<false, true>), grid, block, Fp8Gemm::kLdsBytes,
-                       static_cast<hipStream_t>(stream), p);
+    hipLaunchKernelGGL((fp8_gemm_blockwise_kernel<false, true>), grid, block, Fp8Gemm::kLdsBytes, on, p);
   else
-    hipLaunchKernelGGL(fp8_gemm_blockwise_kernel<false>, grid, block, Fp8Gemm::kLdsBytes, static_cast<hipStream_t>(stream), p);
+    hipLaunchKernelGGL(fp8_gemm_blockwise_kernel<false>, grid, block, Fp8Gemm::kLdsBytes, on, p);
   return check_launch("fp8_gemm_blockwise_kernel");
 }
 
 }  // namespace
 }  // namespace fsh
+
+FSH_API int fsh_fp8_gemm_tiles(int64_t m, int64_t n, int64_t k, int32_t column_scales) {
+  using namespace fsh;
+  if (m <= 0 || n <= 0 || k <= 0 || k % 128) return fail(FSH_EINVAL, "fsh_fp8_gemm_tiles: bad sizes");
+  const int64_t units = compute_units();
+  return fp8_tile_kind(m, n, k, column_scales != 0, units > 0 ? units : kXcds * 32);
+}
 
 FSH_API int fsh_fp8_gemm_1x128_128x128_bias(const void* xq_dev, const float* xs_dev, const void* wq_dev,
                                             const float* ws_dev, const void* bias_dev, void* out_dev, int64_t m,

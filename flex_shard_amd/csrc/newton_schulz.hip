@@ -465,7 +465,8 @@ struct PlannedGemm {
 //   2048 x 2048    11.5 / 30.6    9.7 / 22.7   11.6 / 28.0   16.8 / 42.8
 //   4096 x 2048    18.8 / 55.6   15.5 / 40.0   14.9 / 36.5   19.3 / 45.8
 //   4096 x 4096    35.9 / 108.5  27.3 / 80.5   28.0 / 74.6   22.9 / 61.7
-enum TileKind { kTiles64, kTiles128, kTiles128Deep, kTiles256x128, kTiles256 };
+enum TileKind { kTiles64, kTiles128, kTiles128Deep, kTiles256x128, kTiles256 };  // the order of kTileShapes
+constexpr int kTileNames[] = {FSH_TILES_64, FSH_TILES_128, FSH_TILES_128_DEEP, FSH_TILES_256X128, FSH_TILES_256};
 constexpr TileShape kTileShapes[] = {
     {64, 64, 768.0, 0.17, 0.40, 0.55, 1.7},       // three workgroups per compute unit
     {128, 128, 512.0, 0.37, 0.71, 1.02, 4.2},     // two
@@ -661,13 +662,17 @@ int launch_tiles_as(const TileLaunch& launch, hipStream_t stream) {
   return check_launch("gemm_nt_tiles_kernel");
 }
 
-int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stream) {
+LaunchWork work_of(const PlannedGemm* plans, const int* members, int n) {
   LaunchWork work;
   for (int k = 0; k < n; ++k) {
     const GemmParams& p = plans[members[k]].p;
     work.add(p.M, p.N, p.K, p.symmetric != 0, plans[members[k]].batch);
   }
-  const TileKind kind = small_tile_kind(work);
+  return work;
+}
+
+int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stream) {
+  const TileKind kind = small_tile_kind(work_of(plans, members, n));
   TileLaunch launch;
   if (int rc = fill_launch(plans, members, n, kTileShapes[kind].m, kTileShapes[kind].n, &launch)) return rc;
   switch (kind) {
@@ -763,6 +768,35 @@ FSH_API int fsh_gemm_bf16_nt_group(const fsh_gemm_desc* descs, int32_t count, vo
   for (int i = 0; i < count; ++i)
     if (int rc = fsh::check_k_major(descs[i])) return rc;
   return fsh::launch_gemms(descs, count, static_cast<hipStream_t>(stream));
+}
+
+FSH_API int fsh_gemm_bf16_tiles(const int64_t* sizes, int32_t count, int32_t* tiles) {
+  using namespace fsh;
+  constexpr int kMost = 16;  // products of one call that share launches
+  if (count < 0 || count > kMost || (count > 0 && (!sizes || !tiles))) return fail(FSH_EINVAL, "fsh_gemm_bf16_tiles: bad list");
+  static __attribute__((aligned(16))) uint8_t somewhere[16];  // (looked at for its alignment alone)
+  PlannedGemm plans[kMost];
+  for (int i = 0; i < count; ++i) {
+    fsh_gemm_desc d;
+    memset(&d, 0, sizeof(d));
+    d.a_dev = d.b_dev = d.c_dev = somewhere;
+    d.batch = sizes[5 * i]; d.m = sizes[5 * i + 1]; d.n = sizes[5 * i + 2]; d.k = sizes[5 * i + 3];
+    d.symmetric = sizes[5 * i + 4] != 0;
+    d.lda = d.ldb = d.k; d.ldc = d.n;
+    d.stride_a = d.m * d.k; d.stride_b = d.n * d.k; d.stride_c = d.m * d.n;
+    if (int rc = plan_gemm(d, &plans[i])) return rc;
+  }
+  if (int rc = choose_kernels(plans, count)) return rc;
+  for (int next = 0; next < count;) {  // the small-tile launches, as launch_planned fills them
+    int members[TileLaunch::kMaxProblems], n = 0;
+    for (; next < count && n < TileLaunch::kMaxProblems; ++next) {
+      if (plans[next].large) tiles[next] = FSH_TILES_256;
+      else members[n++] = next;
+    }
+    const TileKind kind = small_tile_kind(work_of(plans, members, n));
+    for (int k = 0; k < n; ++k) tiles[members[k]] = kTileNames[kind];
+  }
+  return FSH_OK;
 }
 
 // Workspace layout (bytes, each region 256-aligned):
@@ -1002,6 +1036,16 @@ int ns_iterate(NsState* st, int count, float a, float b, float c, int32_t steps,
 
 }  // namespace
 }  // namespace fsh
+
+FSH_API int fsh_newton_schulz_tiles(const fsh_ns_problem* problems, int32_t count, int32_t steps, int32_t* large) {
+  using namespace fsh;
+  if (count < 0 || count > FSH_MAX_NS_PROBLEMS || (count > 0 && (!problems || !large)))
+    return fail(FSH_EINVAL, "fsh_newton_schulz_tiles: bad list");
+  bool takes_large[FSH_MAX_NS_PROBLEMS];
+  ns_choose_large(problems, count, steps, takes_large);
+  for (int i = 0; i < count; ++i) large[i] = takes_large[i] ? 1 : 0;
+  return FSH_OK;
+}
 
 FSH_API int fsh_newton_schulz_multi(const fsh_ns_problem* problems, int32_t count, float a, float b, float c,
                                     int32_t steps, float eps, void* stream_) {

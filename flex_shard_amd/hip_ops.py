@@ -36,9 +36,9 @@ __all__ = [
     "REDUCE_PREMUL", "REDUCE_SUM", "SRC_BF16", "SRC_F16", "SRC_F32", "SRC_F32_AS_BF16", "SRC_F32_AS_F16",
     "MuonStepPlan", "QuantChunkSpec", "QuantPackPlan", "accumulate_grad", "act_quant_128x1_transposed", "act_quant_1x128", "act_quant_both",
     "copy_row_segments", "copy_segments", "fp8_gemm_1x128_128x1", "fp8_gemm_1x128_128x128", "fp8_gemm_1x128_128x128_dgrad",
-    "fp8_linear_backward", "fp8_transpose", "gemm_nt", "gemm_nt_group", "muon_apply", "muon_prepare", "newton_schulz_multi",
-    "newton_schulz", "newton_schulz_noalloc", "newton_schulz_workspace_bytes", "pack_segments", "quantize_pack",
-    "reduce_rows", "stream_ptr", "unpack_dequant", "zero_segments",
+    "fp8_gemm_tiles", "fp8_linear_backward", "fp8_transpose", "gemm_nt", "gemm_nt_group", "gemm_tiles", "muon_apply",
+    "muon_prepare", "newton_schulz_multi", "newton_schulz", "newton_schulz_large_tiles", "newton_schulz_noalloc",
+    "newton_schulz_workspace_bytes", "pack_segments", "quantize_pack", "reduce_rows", "stream_ptr", "unpack_dequant", "zero_segments",
 ]
 
 
@@ -524,6 +524,40 @@ def gemm_nt(
     status = _native.lib().fsh_gemm_bf16_nt(ctypes.byref(desc), stream_ptr(a.device))
     _native.check(status, "fsh_gemm_bf16_nt")
     return out
+
+
+#: the tiles a product can take, as ``gemm_tiles`` and ``fp8_gemm_tiles`` name them
+GEMM_TILES = ("64", "64 deep", "128", "128 deep", "256x128", "256", "256 long k")
+
+
+def gemm_tiles(*problems: tuple) -> tuple[str, ...]:
+    """The tiles that :func:`gemm_nt` (one problem) or :func:`gemm_nt_group` takes
+    for contiguous products of these sizes, ``(batch, m, n, k[, symmetric])``
+    each (no GPU needed)."""
+    sizes = [int(v) for problem in problems for v in (*problem, 0)[:5]]
+    tiles = (ctypes.c_int32 * len(problems))()
+    status = _native.lib().fsh_gemm_bf16_tiles((ctypes.c_int64 * len(sizes))(*sizes), len(problems), tiles)
+    _native.check(status, "fsh_gemm_bf16_tiles")
+    return tuple(GEMM_TILES[t] for t in tiles)
+
+
+def newton_schulz_large_tiles(*shapes: tuple[int, int, int], steps: int = 5) -> tuple[bool, ...]:
+    """Whether each (batch, rows, cols) of one :func:`newton_schulz_multi` call
+    iterates on the 256 x 256 tiles (no GPU needed)."""
+    problems = (_native.NsProblem * len(shapes))()
+    for q, (batch, rows, cols) in zip(problems, shapes):
+        q.batch, q.rows, q.cols = batch, rows, cols
+    large = (ctypes.c_int32 * len(shapes))()
+    _native.check(_native.lib().fsh_newton_schulz_tiles(problems, len(shapes), steps, large), "fsh_newton_schulz_tiles")
+    return tuple(map(bool, large))
+
+
+def fp8_gemm_tiles(m: int, n: int, k: int, *, column_scales: bool = False) -> str:
+    """The tiles of an [m, n] scaled FP8 product over ``k`` (no GPU needed);
+    ``column_scales``: :func:`fp8_gemm_1x128_128x1`."""
+    kind = _native.lib().fsh_fp8_gemm_tiles(m, n, k, 1 if column_scales else 0)
+    _native.check(min(kind, 0), "fsh_fp8_gemm_tiles")
+    return GEMM_TILES[kind]
 
 
 def gemm_nt_group(problems: Sequence[dict]) -> list[torch.Tensor]:

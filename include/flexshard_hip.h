@@ -298,6 +298,26 @@ int fsh_gemm_bf16_nt(const fsh_gemm_desc* desc, void* stream);
  * share launches.  Same results as `count` calls of fsh_gemm_bf16_nt. */
 int fsh_gemm_bf16_nt_group(const fsh_gemm_desc* descs, int32_t count, void* stream);
 
+/* Which tiles products take, for tests that mean to reach a kernel: the
+ * launch rules' choice for contiguous, aligned matrices of these sizes, without
+ * a GPU.  "Deep": more operand requests in flight.
+ * fsh_gemm_bf16_tiles: sizes [count, 5] (batch, m, n, k, symmetric) of the
+ * products of one call (at most 16), their FSH_TILES_* to tiles [count].
+ * fsh_newton_schulz_tiles: for the problems of one call of (6) (rows, cols and
+ * batch are read) whether each iterates on the 256 x 256 tiles.
+ * fsh_fp8_gemm_tiles: the FSH_TILES_* of a product of (8) and (9), negative on
+ * bad sizes; column_scales: of fsh_fp8_gemm_1x128_128x1. */
+#define FSH_TILES_64 0
+#define FSH_TILES_64_DEEP 1
+#define FSH_TILES_128 2
+#define FSH_TILES_128_DEEP 3
+#define FSH_TILES_256X128 4
+#define FSH_TILES_256 5
+#define FSH_TILES_256_LONG_K 6
+int fsh_gemm_bf16_tiles(const int64_t* sizes, int32_t count, int32_t* tiles);
+int fsh_newton_schulz_tiles(const fsh_ns_problem* problems, int32_t count, int32_t steps, int32_t* large);
+int fsh_fp8_gemm_tiles(int64_t m, int64_t n, int64_t k, int32_t column_scales);
+
 /* ------------------------------------------------------------------------
  * 7. Muon elementwise steps in bf16 (fp32 math, one rounding per reference
  * tensor op).  Replace dist_muon/optimizer.py:2049-2068 (_prepare_muon_input:

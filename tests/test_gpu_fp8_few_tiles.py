@@ -11,15 +11,21 @@ pytestmark = pytest.mark.gpu
 E4M3 = torch.float8_e4m3fn
 
 
-# 64 x 64 tiles of four and of three stages, 128 x 128 tiles of four and of two
-@pytest.mark.parametrize("m,n", [(1, 8), (65, 200), (64, 16 * 1024 + 8), (1030, 2050), (1090, 3080), (1000, 5120)])
+# 64 x 64 tiles of four stages ("deep") and of three, 128 x 128 tiles of four ("deep") and of two
+@pytest.mark.parametrize(
+    "m,n,tiles,with_column_scales",
+    [(1, 8, "64 deep", "64 deep"), (65, 200, "64 deep", "64 deep"), (64, 16 * 1024 + 8, "64", "64 deep"),
+     (1030, 2050, "64", "64"), (1090, 3080, "128 deep", "128 deep"), (1000, 5120, "128", "128")],
+)
 @pytest.mark.parametrize("ktiles", [1, 2, 3, 4, 5, 6, 9])
-def test_every_number_of_k_tiles(device, m, n, ktiles):
+def test_every_number_of_k_tiles(device, m, n, ktiles, tiles, with_column_scales):
     """Small integers and power-of-two scales: every partial sum is exact in
     fp32 whatever the order, so the output is the one bf16 rounding of the
     exact result."""
     gen = torch.Generator().manual_seed(m + n + ktiles)
     k = 128 * ktiles
+    assert hip_ops.fp8_gemm_tiles(m, n, k) == tiles
+    assert hip_ops.fp8_gemm_tiles(m, n, k, column_scales=True) == with_column_scales
 
     def integers(rows):
         return torch.randint(-2, 3, (rows, k), generator=gen).float().to(E4M3).to(device)

@@ -144,10 +144,11 @@ def test_gemm_rejects_what_the_kernel_cannot_take(device):
 
 
 def test_contraction_longer_than_one_window_of_weight_scales(device):
-    """The block-scale variant keeps 256 k-tiles of weight scales in LDS and
-    refills the window when the loop crosses it: k = 2 windows + 3 k-tiles,
-    every weight scale different, against the oracle's product; forward and
-    input-gradient (scale table read across) forms."""
+    """k = two windows of the 256 x 256 kernel (256 k-tiles of weight scales each)
+    + 3 k-tiles, every weight scale different, against the oracle's product;
+    forward and input-gradient (scale table read across) forms.  So few rows
+    and columns take 64 x 64 tiles, which request the scales of every k-tile
+    with its operands; the next test refills the window."""
     gen = torch.Generator().manual_seed(5)
     m, n, k = 96, 384, 2 * 32768 + 384
     x = torch.randn(m, k, generator=gen).bfloat16()
@@ -163,6 +164,37 @@ def test_contraction_longer_than_one_window_of_weight_scales(device):
         xq.to(device), xs.to(device), wq.to(device), ws.t().contiguous().to(device), in_dim=n
     )
     assert torch.equal(got_t, got)
+
+
+@pytest.mark.parametrize("m,n", [(4096, 4096), (4000, 4100)])
+def test_window_of_weight_scales_refilled_in_the_loop(device, m, n):
+    """The 256 x 256 kernel keeps 256 k-tiles of weight scales in LDS and refills
+    the window when the loop crosses it (here once, three k-tiles before the
+    end).  Operands in -1..1 and power-of-two scales: every sum is a multiple
+    of 2^-2 below 2^18 and so exact in fp32, and the outputs are the one bf16
+    rounding of it; forward and input-gradient (scale table read across) forms."""
+    ktiles = 256 + 3
+    k = 128 * ktiles
+    assert hip_ops.fp8_gemm_tiles(m, n, k) == "256 long k"
+    gen = torch.Generator(device=device)
+    gen.manual_seed(m + n)
+
+    def integers(rows):
+        return torch.randint(-1, 2, (rows, k), generator=gen, device=device, dtype=torch.int8).to(torch.float32).to(E4M3)
+
+    def powers(*shape):
+        return torch.exp2(torch.randint(-1, 2, shape, generator=gen, device=device).float())
+
+    xq, wq, xs, ws = integers(m), integers(n), powers(ktiles, m), powers(-(-n // 128), ktiles)
+    got = hip_ops.fp8_gemm_1x128_128x128(xq, xs, wq, ws)
+    for rows in (slice(0, 200), slice(m - 130, m)):  # whole rows of the result, both ends
+        want = torch.zeros(rows.stop - rows.start, n, device=device)
+        for kb in range(ktiles):
+            run = slice(128 * kb, 128 * kb + 128)
+            product = xq[rows, run].float() @ wq[:, run].float().t()
+            want += product * xs[kb, rows, None] * ws[:, kb].repeat_interleave(128)[None, :n]
+        assert torch.equal(got[rows], want.bfloat16())
+    assert torch.equal(hip_ops.fp8_gemm_1x128_128x128_dgrad(xq, xs, wq, ws.t().contiguous(), in_dim=n), got)
 
 
 def test_projections_that_share_an_activation_quantize_it_once(device):

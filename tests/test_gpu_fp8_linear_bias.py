@@ -21,11 +21,15 @@ def _weight(gen, out_dim, in_dim, device):
 
 
 @pytest.mark.parametrize(
-    "tokens,out_dim,in_dim",
-    [(1, 200, 128), (65, 1003, 256), (1000, 2052, 512), (4096, 4100, 256), (4100, 8199, 128)],  # 64, 64, 128, 256, 256 + half tiles
+    "tokens,out_dim,in_dim,tiles",
+    [
+        (1, 200, 128, "64 deep"), (65, 1003, 256, "64 deep"), (1000, 2052, 512, "64"), (1091, 3081, 512, "128 deep"),
+        (1001, 5123, 256, "128"), (4096, 4100, 256, "256"), (4100, 8199, 128, "256"),  # the last with half tiles
+    ],
 )
-def test_bias_in_the_epilogue(device, tokens, out_dim, in_dim):
+def test_bias_in_the_epilogue(device, tokens, out_dim, in_dim, tiles):
     """Bit for bit the separate bf16 addition, ragged rows and columns included."""
+    assert hip_ops.fp8_gemm_tiles(tokens, out_dim, in_dim) == tiles
     gen = torch.Generator().manual_seed(tokens + out_dim)
     wq, ws = _weight(gen, out_dim, in_dim, device)
     xq, xs = hip_ops.act_quant_1x128(torch.randn(tokens, in_dim, generator=gen).bfloat16().to(device))

@@ -1,7 +1,8 @@
 """The tile kernels of the bf16 NT product at the sizes where they can go
 wrong: ragged rows and columns, contractions that end inside a k-tile or hold
 fewer k-tiles than the pipeline is deep, every tile size the launch rule
-chooses between, and several problems in one launch."""
+chooses between (the rule is asked which one a case takes), and several
+problems in one launch."""
 
 import pytest
 import torch
@@ -15,8 +16,10 @@ CASES = [
     (1, 1, 1, 8), (1, 64, 64, 64), (1, 65, 63, 72), (2, 130, 257, 136), (1, 129, 127, 520), (3, 33, 300, 248),
     # 128 x 128 tiles, operands requested three k-tiles ahead (240 tiles)
     (1, 1920, 1928, 264), (1, 1923, 1837, 392), (1, 1920, 1920, 576),
-    # 128 x 128 tiles, two workgroups per compute unit (640 tiles)
-    (32, 520, 500, 456), (32, 512, 512, 512), (32, 513, 511, 520),
+    # 64 x 64 tiles, more than the chip holds at once (2304 and 2304 tiles)
+    (32, 520, 500, 456), (32, 513, 511, 520),
+    # 128 x 128 tiles, two workgroups per compute unit
+    (32, 512, 512, 512), (9, 1544, 1288, 72),
     # 256 x 256 tiles, resident workgroups
     (20, 1024, 1280, 1024),
 ]
@@ -59,6 +62,47 @@ def test_ragged_symmetric_products_with_a_diagonal_term(device, batch, n, k):
     ref = torch.bmm(a.double(), a.double().transpose(1, 2).contiguous()) + 1.5 * torch.eye(n, device=device, dtype=torch.float64)
     assert _close(got, ref)
     assert torch.equal(got, hip_ops.gemm_nt(a, a, diag_add=1.5))  # the same sums, every tile computed
+
+
+@pytest.mark.parametrize(
+    "tiles,batch,m,n,k",
+    [
+        ("64", 2, 130, 257, 136), ("64", 32, 513, 511, 520), ("128", 32, 512, 512, 512), ("128", 8, 337, 1500, 200),
+        ("128 deep", 1, 1923, 1837, 392), ("256x128", 3, 1433, 1433, 1000), ("256x128", 3, 1159, 2000, 1000),
+        ("256x128", 20, 200, 1500, 1000), ("256", 7, 1536, 1280, 64), ("256", 20, 1024, 1280, 1024),
+    ],
+)
+def test_small_integers_on_every_kind_of_tile(device, tiles, batch, m, n, k):
+    """Sums of products of small integers are exact in fp32 whatever the order,
+    so the outputs are the one bf16 rounding of the exact result."""
+    assert hip_ops.gemm_tiles((batch, m, n, k)) == (tiles,)
+    a, b, d = (t.round().clamp(-3, 3) for t in _operands(batch, m, n, k, device, m + n + k))
+    pad = 512
+    bufs = [torch.full((batch * m * n + 2 * pad,), 7.0, dtype=torch.bfloat16, device=device) for _ in range(2)]
+    c, ct = bufs[0][pad:-pad].view(batch, m, n), bufs[1][pad:-pad].view(batch, n, m)
+    hip_ops.gemm_nt(a, b, d=d, alpha=0.5, beta=2.0, out=c, out_t=ct)
+    want = (0.5 * torch.bmm(a.float(), b.float().transpose(1, 2).contiguous()) + 2.0 * d.float()).bfloat16()
+    assert torch.equal(c, want)
+    assert torch.equal(ct, want.transpose(1, 2).contiguous())
+    for buf in bufs:
+        assert (buf[:pad] == 7).all() and (buf[-pad:] == 7).all()
+
+
+@pytest.mark.parametrize(
+    "tiles,batch,n,k",
+    [("64", 4, 300, 200), ("128", 6, 1536, 192), ("256x128", 7, 1283, 1544), ("256x128", 1, 3000, 3000), ("256", 10, 1536, 128)],
+)
+def test_small_integers_in_symmetric_products(device, tiles, batch, n, k):
+    assert hip_ops.gemm_tiles((batch, n, n, k, True)) == (tiles,)
+    a, _, d = (t.round().clamp(-3, 3) for t in _operands(batch, n, n, k, device, n + k))
+    d = torch.triu(d) + torch.triu(d, 1).transpose(1, 2)
+    pad = 512
+    buf = torch.full((batch * n * n + 2 * pad,), 7.0, dtype=torch.bfloat16, device=device)
+    c = buf[pad:-pad].view(batch, n, n)
+    hip_ops.gemm_nt(a, a, d=d, alpha=0.5, beta=2.0, symmetric=True, diag_add=1.5, out=c)
+    want = 0.5 * torch.bmm(a.float(), a.float().transpose(1, 2).contiguous()) + 2.0 * d.float()
+    assert torch.equal(c, (want + 1.5 * torch.eye(n, device=device)).bfloat16())
+    assert (buf[:pad] == 7).all() and (buf[-pad:] == 7).all()
 
 
 def test_more_problems_than_one_launch_holds(device):

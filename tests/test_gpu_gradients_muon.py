@@ -493,12 +493,13 @@ def test_newton_schulz_matches_torch_muon_routine(device, shape, golden):
 
 @pytest.mark.parametrize("shape,steps", [((20, 1024, 1280), 5), ((20, 1280, 1024), 5), ((24, 1024, 1024), 4), ((20, 1280, 1024), 1)])
 def test_newton_schulz_with_one_orientation_carried(device, shape, steps, golden):
-    """Batches with whole 256 x 256 x 64 tiles and at least 192 of them carry
+    """Batches of whole 256 x 256 x 64 tiles that the rule gives the large-tile kernel carry
     only X^T between steps (G from its k-major rows; a wide input's last step
     written as X' = P X): wide, tall and square inputs, odd, even and single
     step counts, first and last matrix against torch's routine."""
     from torch.optim._muon import _zeropower_via_newtonschulz as torch_ns
 
+    assert hip_ops.newton_schulz_large_tiles(shape, steps=steps) == (True,)
     tol = golden["muon_tolerance"]["atol"]
     gen = torch.Generator().manual_seed(8)
     g = torch.randn(shape, generator=gen).bfloat16()
@@ -583,8 +584,8 @@ def _gemm_reference(a, b, d=None, alpha=1.0, beta=0.0):
     [
         (6, 1536, 1536, 192),  # 256x256x64 whole-tile kernel, 3 k-tiles
         (7, 1536, 1280, 64),  # same kernel, single k-tile, padding workgroups in the grid
-        (1, 512, 384, 96),  # 128x128x32 whole-tile kernel
-        (9, 1544, 1288, 72),  # 256x256 predicated kernel
+        (1, 512, 384, 96),  # 64x64 tiles
+        (9, 1544, 1288, 72),  # 128x128 tiles, ragged rows, columns and contraction
     ],
 )
 def test_gemm_tile_paths(device, batch, m, n, k):
@@ -652,21 +653,25 @@ def test_gemm_diagonal_addend(device, batch, n, k, symmetric):
     assert ((shifted[eye].cpu().double() - want).abs() <= 0.51 * ulp + 1e-3).all()
 
 
-def test_gemm_group_equals_separate_calls(device):
-    """Problems of different shapes and kernels in one call: the ones on the
-    large-tile kernel share a launch (longest k first), every result is bit
+@pytest.mark.parametrize(
+    "times,tiles", [(1, ("128",) * 6), (3, ("256", "256", "64", "256", "64", "256"))]
+)
+def test_gemm_group_equals_separate_calls(device, times, tiles):
+    """Problems of different shapes and kernels in one call: the ones on one
+    kernel share launches (longest k first), every result is bit
     for bit what a call of its own gives, and nothing outside the outputs is
     written."""
     gen = torch.Generator().manual_seed(21)
     specs = [
         # (batch, m, n, k, symmetric, with d, with out_t)
-        (10, 1536, 1536, 128, True, False, False),  # large tile, short k
-        (7, 1536, 1280, 320, False, True, True),  # large tile, long k, all outputs
-        (1, 512, 384, 96, False, True, False),  # 128x128 whole-tile kernel
-        (10, 1536, 1536, 192, True, True, False),  # large tile, symmetric with addend
-        (2, 264, 136, 72, False, False, True),  # predicated kernel
-        (8, 1280, 1280, 64, False, False, False),  # large tile, one k-tile
+        (10 * times, 1536, 1536, 128, True, False, False),  # whole 256x256 tiles, short k
+        (7 * times, 1536, 1280, 320, False, True, True),  # whole 256x256 tiles, long k, all outputs
+        (1, 512, 384, 96, False, True, False),  # whole 128x128 tiles
+        (10 * times, 1536, 1536, 192, True, True, False),  # whole 256x256 tiles, symmetric with addend
+        (2, 264, 136, 72, False, False, True),  # ragged
+        (8 * times, 1280, 1280, 64, False, False, False),  # whole 256x256 tiles, one k-tile
     ]
+    assert hip_ops.gemm_tiles(*(spec[:5] for spec in specs)) == tiles
     pad = 1024
     problems, buffers = [], []
     for batch, m, n, k, symmetric, with_d, with_t in specs:
@@ -697,13 +702,16 @@ def test_gemm_group_equals_separate_calls(device):
     assert hip_ops.gemm_nt_group([]) == []
 
 
-def test_gemm_static_schedule_when_tiles_are_equally_long(device):
+@pytest.mark.parametrize("batch,tiles", [(11, "128"), (14, "256")])  # 6 x 7 x batch = 462 and 588 tiles of 256 x 256
+def test_gemm_static_schedule_when_tiles_are_equally_long(device, batch, tiles):
     """More large tiles than compute units, all with the same k: one resident
     workgroup per compute unit walks the tiles of both problems (next tile's
-    operands requested during the epilogue).  Against fp64 and against the
-    symmetric / transposed identities, with guard bands."""
+    operands requested during the epilogue); somewhat fewer, on the 128 x 128
+    tiles.  Against fp64 and against the symmetric / transposed identities,
+    with guard bands."""
     gen = torch.Generator().manual_seed(33)
-    batch, m, n, k = 11, 1536, 1792, 192  # 6 x 7 x 11 = 462 tiles
+    m, n, k = 1536, 1792, 192
+    assert hip_ops.gemm_tiles((batch, m, n, k), (9, 1280, 1280, k, True)) == (tiles, tiles)
     a = torch.randn(batch, m, k, generator=gen).bfloat16().to(device)
     b = torch.randn(batch, n, k, generator=gen).bfloat16().to(device)
     d = torch.randn(batch, m, n, generator=gen).bfloat16().to(device)
@@ -730,11 +738,19 @@ def test_gemm_static_schedule_when_tiles_are_equally_long(device):
     assert torch.equal(x, c)
 
 
-def test_newton_schulz_multi_equals_one_call_per_shape(device):
+@pytest.mark.parametrize(
+    "shapes,large",
+    [
+        ([(40, 1024, 768), (48, 768, 768), (5, 256, 1024), (1, 64, 96)], 0),  # the first alone would take large tiles
+        ([(48, 1024, 1024), (5, 256, 1024), (2, 304, 200), (1, 64, 96)], 2),
+    ],
+)
+def test_newton_schulz_multi_equals_one_call_per_shape(device, shapes, large):
     """Shape groups iterated together (each product issued for all groups at
     once) against one call per group: identical bits, tall, wide and square,
     large-tile and small-tile kernels mixed."""
-    shapes = [(40, 1024, 768), (48, 768, 768), (5, 256, 1024), (1, 64, 96)]  # the first two fill the large tile
+    assert hip_ops.newton_schulz_large_tiles(*shapes) == tuple(i < large for i in range(len(shapes)))
+    assert hip_ops.newton_schulz_large_tiles(shapes[0]) == (True,)
     inputs = [seeded_normal(shape, 1.0, 30 + i, device) for i, shape in enumerate(shapes)]
     together = [x.clone() for x in inputs]
     hip_ops.newton_schulz_multi([(x, None) for x in together], COEFFS, 5, 1e-7)
@@ -1089,6 +1105,7 @@ def test_fused_muon_step_equals_the_per_matrix_kernels(device, nesterov):
     one-orientation flow, two steps (the second with momentum in place and
     gradients at new addresses)."""
     shapes = [(1024, 1280)] * 20 + [(768, 256)] * 3 + [(64, 96)] + [(256, 256)] * 2
+    assert hip_ops.newton_schulz_large_tiles((20, 1024, 1280), (3, 768, 256), (1, 64, 96), (2, 256, 256)) == (True, True, False, True)
     start = [seeded_normal(s, 0.02, 700 + i, device) for i, s in enumerate(shapes)]
     mine = [p.clone() for p in start]
     theirs = [p.clone() for p in start]
@@ -1134,8 +1151,8 @@ def test_newton_schulz_takes_any_shape(device, shape, golden):
 
 
 def test_owned_muon_with_odd_shapes_and_a_learning_rate_schedule(device, golden):
-    """Matrices the batched step cannot take (rows or columns not multiples of
-    8) go through the per-matrix kernels beside the batched groups, and a
+    """Matrices whose rows or columns are not multiples of 8 (padded in the
+    batched step) beside ones whose are, and a
     learning rate changed between steps moves the step size and the weight
     decay together: three steps against torch.optim.Muon under the same
     schedule."""
@@ -1169,6 +1186,7 @@ def test_muon_step_plan_with_scaled_directions_equals_the_per_matrix_kernels(dev
     epilogue (large-tile group) and the batched update kernel (small group)
     must give the bits of prepare -> Newton-Schulz -> apply(direction_scale)."""
     groups = [((1024, 1280), 20, -3e-3, 0.75), ((64, 96), 2, -1.5e-3, 1.5)]
+    assert hip_ops.newton_schulz_large_tiles((20, 1024, 1280), (2, 64, 96)) == (True, False)
     plan = hip_ops.MuonStepPlan(groups, device)
     params, momenta, grads, ref_params, ref_momenta = [], [], [], [], []
     for gi, (shape, n, _, _) in enumerate(groups):

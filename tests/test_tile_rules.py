@@ -1,0 +1,43 @@
+"""The launch rules of the products as their host-only queries report them."""
+
+import pytest
+
+from flex_shard_amd import hip_ops
+
+
+def test_every_kind_of_tile_is_chosen_somewhere():
+    bf16 = {
+        hip_ops.gemm_tiles((batch, m, m, k, symmetric))[0]
+        for batch in (1, 7, 24) for m in (40, 520, 1283, 2048, 3000) for k in (64, 520, 1544) for symmetric in (False, True)
+    }
+    assert bf16 == {"64", "128", "128 deep", "256x128", "256"}
+    fp8 = {
+        hip_ops.fp8_gemm_tiles(m, n, k, column_scales=scales)
+        for m in (1, 1000, 1090, 8192) for n in (200, 2052, 3080, 5120, 14336) for k in (128, 4096, 33152) for scales in (False, True)
+    }
+    assert fp8 == set(hip_ops.GEMM_TILES) - {"256x128"}
+
+
+def test_problems_of_one_call_share_the_choice():
+    """Whole 256 x 256 tiles go together or not at all, ragged problems beside
+    them; more problems than a launch holds are looked at launch by launch."""
+    ragged, few, many = (2, 264, 136, 72), (8, 1280, 1280, 64), (40, 1536, 1536, 192)
+    assert hip_ops.gemm_tiles(ragged, many, few) == ("64", "256", "256")
+    assert len(set(hip_ops.gemm_tiles(few, ragged))) == 1 and hip_ops.gemm_tiles() == ()
+    assert hip_ops.gemm_tiles(*[(1, 64, 64, 64)] * 8, (1, 1920, 1928, 264)) == ("64",) * 8 + ("128 deep",)
+    assert hip_ops.newton_schulz_large_tiles((24, 7168, 2048), (24, 2048, 2048), (1, 64, 96)) == (True, True, False)
+    assert hip_ops.newton_schulz_large_tiles((1, 2048, 2048)) == (False,)
+    assert hip_ops.newton_schulz_large_tiles((24, 7168, 2048), steps=0) == (False,)
+
+
+def test_bad_sizes_are_refused():
+    for sizes in ((0, 8, 8, 8), (1, 8, 8, 12)):
+        with pytest.raises(RuntimeError, match="gemm"):
+            hip_ops.gemm_tiles(sizes)
+    with pytest.raises(RuntimeError, match="symmetric"):
+        hip_ops.gemm_tiles((1, 8, 16, 8, True))
+    with pytest.raises(RuntimeError, match="bad list"):
+        hip_ops.gemm_tiles(*[(1, 8, 8, 8)] * 17)
+    for sizes in ((0, 8, 128), (8, 8, 100)):
+        with pytest.raises(RuntimeError, match="bad sizes"):
+            hip_ops.fp8_gemm_tiles(*sizes)

@@ -20,9 +20,13 @@ def _with_workspace(x):
 
 def test_noalloc_newton_schulz_equals_the_workspace_entry_point(device):
     torch.cuda.synchronize()
-    # large-tile, one-orientation flow: 192 matrices of 256 x 256 (96.2 MB of scratch) ...
+    # 192 matrices of 256 x 256 (96.2 MB of scratch) and, on the large tiles with one orientation
+    # carried, 26 of 768 x 768 (117 MB) ...
     first = seeded_normal((192, 256, 256), 1.0, 51, device)
-    # ... then a smaller, tall batch on the small-tile kernels, over what the first call left behind
+    large = seeded_normal((26, 768, 768), 1.0, 55, device)
+    assert hip_ops.newton_schulz_large_tiles(large.shape) == (True,)
+    assert torch.equal(hip_ops.newton_schulz_noalloc(large.clone(), COEFFS, 5, 1e-7), _with_workspace(large))
+    # ... then a smaller, tall batch, over what the first calls left behind
     second = seeded_normal((3, 200, 136), 1.0, 52, device)
     third = seeded_normal((2, 512, 768), 1.0, 53, device)
     want = [_with_workspace(x) for x in (first, second, third)]
