@@ -400,7 +400,7 @@ __device__ __forceinline__ void store_tile_in_halves(const GemmParams& p, int64_
 }
 
 // Scheduling-group masks of __builtin_amdgcn_sched_group_barrier.
-constexpr int kSchedValu = 0x002, kSchedMfma = 0x008, kSchedVmemRead = 0x020, kSchedDsRead = 0x100, kSchedDsWrite = 0x200;
+constexpr int kSchedMfma = 0x008, kSchedDsRead = 0x100;
 
 // gfx950 loads 16 bytes per lane from global memory straight into LDS: lane l
 // of a wave writes LDS bytes [M0 + 16 l, M0 + 16 l + 16).  The address is a
@@ -413,14 +413,14 @@ __device__ inline void dma_load_16(uint32_t voffset, const uint8_t* base, uint32
 __device__ inline void dma_load_16_at(const uint8_t* src, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory");
 }
-// The 4-byte form: lane l writes LDS bytes [M0 + 4 l, M0 + 4 l + 4).
+// 4 bytes per lane: lane l writes LDS bytes [M0 + 4 l, M0 + 4 l + 4).
 __device__ inline void dma_load_4_at(const uint8_t* src, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds_addr) : "memory");
 }
 template <int kInFlight>
 __device__ inline void wait_for_dma_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kInFlight) : "memory"); }
 __device__ inline void wait_for_dma_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// The 4-byte form: lane l writes LDS bytes [M0 + 4 l, M0 + 4 l + 4).
+// 4 bytes per lane from a uniform base plus a 32-bit per-lane offset.
 __device__ inline void dma_touch_4(uint32_t voffset, const uint8_t* base, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(voffset), "s"(base), "s"(lds_addr) : "memory");
 }

@@ -19,7 +19,7 @@ namespace {
 constexpr int kNormThreads = 256;
 constexpr int kMaxMuonGroups = FSH_MAX_NS_PROBLEMS;
 constexpr int64_t kSliceVectors = 1024;  // 8-element vectors per block and slice
-constexpr int64_t kMaxSlices = 2048;     // per matrix: a block of the normalization adds up all partial sums
+constexpr int64_t kMaxSlices = 2048;     // per matrix: one block adds up all partial sums (see kNormSlices)
 
 // Slices (and partial sums of squares) of a matrix of `vectors` 8-element
 // vectors; a matter of the matrix alone, so that the order of the additions is

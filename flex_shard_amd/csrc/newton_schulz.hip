@@ -831,7 +831,7 @@ struct NsState {
   bool single;  // only X^T is carried from step to step (G = X X^T is then computed from its k-major rows)
 };
 
-// Workspace offset of the [batch, 64] norm partials.
+// Workspace offset of the norm partials.
 int64_t ns_partial_offset(int64_t batch, int64_t rows, int64_t cols) {
   const int64_t s = rows < cols ? rows : cols, l = rows < cols ? cols : rows;
   return 2 * align256(batch * s * l * 2) + 2 * align256(batch * s * s * 2);
@@ -1199,8 +1199,9 @@ FSH_API int fsh_muon_step(const fsh_muon_group* groups, int32_t count, float ler
 namespace fsh {
 namespace {
 
-// The norm partials of a batch that otherwise fills the scratch: 4 bytes per
-// 8192 elements or per matrix, and at most a quarter of the bytes are elements.
+// The norm partials of a batch that otherwise fills the scratch: 4 bytes for
+// each slices_of() slice of a matrix, i.e. per 8192 elements or per matrix if it has
+// fewer, and at most a quarter of the bytes are elements.
 constexpr int64_t kScratchPartials = 1 << 20;
 static __device__ __align__(256) uint8_t scratch[FSH_NS_STATIC_SCRATCH_BYTES + kScratchPartials];
 
@@ -1242,7 +1243,8 @@ FSH_API int fsh_newton_schulz_noalloc(void* x_dev, int64_t batch, int64_t rows, 
                 "fsh_newton_schulz_noalloc: batch %lld of %lld x %lld exceeds the %lld-byte static scratch; call "
                 "fsh_newton_schulz with a workspace of fsh_newton_schulz_workspace_bytes()",
                 (long long)batch, (long long)rows, (long long)cols, (long long)FSH_NS_STATIC_SCRATCH_BYTES);
-  // (everything but the norm partials, which have room of their own behind the advertised size)
+  // The norm partials have room of their own behind the advertised size, against
+  // which a matrix counts 64 of them, however many it has.
   const int64_t need = ns_partial_offset(batch, rows, cols) + align256(batch * 64 * 4);
   if (need > FSH_NS_STATIC_SCRATCH_BYTES || fsh_newton_schulz_workspace_bytes(batch, rows, cols) > FSH_NS_STATIC_SCRATCH_BYTES + kScratchPartials)
     return fail(FSH_ENOTSUP,

@@ -109,7 +109,7 @@ __device__ __forceinline__ F32ToBf16 caster(const float*, uint16_t*) { return {}
 
 // Multi-input gather with cast.  A negative tensor index marks a zero-fill
 // segment.  Same-dtype segments move as bytes with the widest legal vector;
-// casting segments convert element by element (coalesced across the wave).
+// casting segments convert four elements per access where both sides allow it.
 template <typename SRC, typename DST>
 __global__ __launch_bounds__(kThreads) void pack_segments_kernel(
     const int64_t* __restrict__ input_ptrs, const int64_t* __restrict__ tensor_indices,

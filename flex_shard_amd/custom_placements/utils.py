@@ -384,18 +384,6 @@ def make_segment_pack_descriptor_if_supported(
     )
 
 
-def pack_segments_into_flat_buffer_if_supported(
-    inputs, tensor_indices, src_offsets, numels, dst_offsets, out, descriptor=None
-) -> list[torch.Tensor] | None:
-    """HIP descriptor packing when the inputs qualify, else None (caller falls
-    back to ``foreach_copy_``)."""
-    if torch.compiler.is_compiling():
-        return None
-    return pack_segments_into_flat_buffer(
-        inputs, tensor_indices, src_offsets, numels, dst_offsets, out, descriptor=descriptor
-    )
-
-
 __all__ = [
     "LocalReduceGroup",
     "all_gather_rows",
@@ -406,7 +394,6 @@ __all__ = [
     "group_size",
     "local_exchange_rows",
     "make_segment_pack_descriptor_if_supported",
-    "pack_segments_into_flat_buffer_if_supported",
     "pack_tensors_into_flat_buffer",
     "pack_tensors_into_flat_buffer_with_scratch",
     "reduce_grads_on_one_rank",

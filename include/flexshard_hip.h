@@ -254,10 +254,11 @@ int fsh_newton_schulz_multi(const fsh_ns_problem* problems, int32_t count, float
  * library runs on until the process ends; its address on the current device
  * is resolved on the first call on that device (so make that first call
  * outside any graph capture).  The call allocates and frees nothing.  A batch
- * whose fsh_newton_schulz_workspace_bytes() exceeds the static scratch is
- * rejected with FSH_ENOTSUP.  All calls on one GPU share the one array: calls
- * that overlap on a GPU (different streams, or threads) race and must be
- * serialized by the caller; calls on one stream are ordered by the stream.
+ * whose fsh_newton_schulz_workspace_bytes() (counting 64 norm partials per
+ * matrix) exceeds the static scratch is rejected with FSH_ENOTSUP.  All calls
+ * on one GPU share the one array: calls that overlap on a GPU (different
+ * streams, or threads) race and must be serialized by the caller; calls on one
+ * stream are ordered by the stream.
  * Results are those of fsh_newton_schulz, bit for bit. */
 #define FSH_NS_STATIC_SCRATCH_BYTES (128LL << 20)
 int fsh_newton_schulz_noalloc(void* x_dev, int64_t batch, int64_t rows, int64_t cols, float a, float b,
