@@ -181,10 +181,10 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
     const uint8_t* b_src = Bb + kt * Cfg::kRowBytes;
 #pragma unroll
     for (int q = 0; q < Cfg::kLoadsA; ++q)
-      dma_load_16(a_voff[q], a_src, stage_off + fill_lds + q * Cfg::kFillRows * Cfg::kRowBytes);
+      dma_load_16(a_voff[q], a_src, stage_off + fill_lds, q * Cfg::kFillRows * Cfg::kRowBytes);
 #pragma unroll
     for (int q = 0; q < Cfg::kLoadsB; ++q)
-      dma_load_16(b_voff[q], b_src, stage_off + Cfg::kABytes + fill_lds + q * Cfg::kFillRows * Cfg::kRowBytes);
+      dma_load_16(b_voff[q], b_src, stage_off + fill_lds, Cfg::kABytes + q * Cfg::kFillRows * Cfg::kRowBytes);
   };
 
   // Fragment side: row = lane & 31 of a 32-row block; chunks 4 kh + 2 h and
@@ -251,9 +251,9 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
     if (part >= Cfg::kLoadsA) {
       const int q = part - Cfg::kLoadsA;
       dma_load_16(b_voff[q], Bb + kt * Cfg::kRowBytes,
-                  stage_off + Cfg::kABytes + fill_lds + q * Cfg::kFillRows * Cfg::kRowBytes);
+                  stage_off + fill_lds, Cfg::kABytes + q * Cfg::kFillRows * Cfg::kRowBytes);
     } else {
-      dma_load_16(a_voff[part], Ab + kt * Cfg::kRowBytes, stage_off + fill_lds + part * Cfg::kFillRows * Cfg::kRowBytes);
+      dma_load_16(a_voff[part], Ab + kt * Cfg::kRowBytes, stage_off + fill_lds, part * Cfg::kFillRows * Cfg::kRowBytes);
     }
     if (part == 0) issue_scale_loads(kt, stage);
   };

@@ -405,9 +405,17 @@ constexpr int kSchedMfma = 0x008, kSchedDsRead = 0x100;
 // gfx950 loads 16 bytes per lane from global memory straight into LDS: lane l
 // of a wave writes LDS bytes [M0 + 16 l, M0 + 16 l + 16).  The address is a
 // uniform 64-bit base plus a 32-bit per-lane offset.  Inline asm: the compiler
-// neither reorders these against other memory operations nor counts them.
-__device__ inline void dma_load_16(uint32_t voffset, const uint8_t* base, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voffset), "s"(base), "s"(lds_addr) : "memory");
+// neither reorders these against other memory operations nor counts them.  The
+// instruction set asks for one wait state between a scalar write of M0 and a
+// load to LDS, which the compiler inserts for its own instructions only.  It
+// costs the large-tile products 0.5 % (48 Newton-Schulz matrices 16.28 -> 16.36 ms),
+// as an idle state or as an addition to the lane's address that would be a
+// scalar one otherwise.
+// `lds_step`, a constant after unrolling, is added on the way into M0: the
+// addresses of a k-tile's requests then need no scalar registers of their own.
+__device__ __forceinline__ void dma_load_16(uint32_t voffset, const uint8_t* base, uint32_t lds_addr, uint32_t lds_step) {
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voffset), "s"(base), "s"(lds_addr),
+               "i"(lds_step) : "memory", "scc");
 }
 // The same with a per-lane 64-bit address.
 __device__ inline void dma_load_16_at(const uint8_t* src, uint32_t lds_addr) {
@@ -422,7 +430,7 @@ __device__ inline void wait_for_dma_loads_but() { asm volatile("s_waitcnt vmcnt(
 __device__ inline void wait_for_dma_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // 4 bytes per lane from a uniform base plus a 32-bit per-lane offset.
 __device__ inline void dma_touch_4(uint32_t voffset, const uint8_t* base, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(voffset), "s"(base), "s"(lds_addr) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voffset), "s"(base), "s"(lds_addr) : "memory");
 }
 
 constexpr int max_int(int a, int b) { return a > b ? a : b; }

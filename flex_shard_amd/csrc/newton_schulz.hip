@@ -145,9 +145,9 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
     const uint32_t a_voff = fill_row0 * a_row_bytes + fill_chunk * 16, b_voff = fill_row0 * b_row_bytes + fill_chunk * 16;
 #pragma unroll
     for (int q = q_first; q < q_last; ++q) {
-      dma_load_16(a_voff, a_src + static_cast<uint64_t>(kRowsPerLoadStep * q) * a_row_bytes, stage_off + fill_lds + q * 4096);
+      dma_load_16(a_voff, a_src + static_cast<uint64_t>(kRowsPerLoadStep * q) * a_row_bytes, stage_off + fill_lds, q * 4096);
       dma_load_16(b_voff, b_src + static_cast<uint64_t>(kRowsPerLoadStep * q) * b_row_bytes,
-                  stage_off + Cfg::kOperandBytes + fill_lds + q * 4096);
+                  stage_off + fill_lds, Cfg::kOperandBytes + q * 4096);
     }
   };
 
@@ -279,10 +279,10 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
     const int q = idx >> 1;
     if (idx & 1)
       dma_load_16(fill_row0 * b_row_bytes + fill_chunk * 16, b_src + static_cast<uint64_t>(kRowsPerLoadStep * q) * b_row_bytes,
-                  stage + Cfg::kOperandBytes + fill_lds + q * 4096);
+                  stage + fill_lds, Cfg::kOperandBytes + q * 4096);
     else
       dma_load_16(fill_row0 * a_row_bytes + fill_chunk * 16, a_src + static_cast<uint64_t>(kRowsPerLoadStep * q) * a_row_bytes,
-                  stage + fill_lds + q * 4096);
+                  stage + fill_lds, q * 4096);
   };
   auto k_tile = [&](int64_t kt, int64_t ktiles, auto more_tag, auto first_tag) {
     constexpr bool more = decltype(more_tag)::value;
