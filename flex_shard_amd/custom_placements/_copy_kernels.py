@@ -15,6 +15,7 @@ from dataclasses import dataclass
 import torch
 
 from .. import hip_ops
+from .._native import MAX_COPY_ROWS
 
 # Split segments are capped at this many so descriptor tables stay small.
 _MAX_SEGMENTS = 65535
@@ -101,11 +102,12 @@ def copy_segments(source: torch.Tensor, output: torch.Tensor, descriptor: Segmen
 class RowCopyDescriptor:
     """Byte segments ``(row, source offset, nbytes, destination offset)`` of
     separately allocated source rows, on the device: the layout alone, since
-    the rows' addresses come with every launch."""
+    the rows' addresses come with every launch.  A launch carries the addresses
+    of ``MAX_COPY_ROWS`` rows; more rows are several parts."""
 
-    table: torch.Tensor
-    max_nbytes: int
-    _staged_host: torch.Tensor
+    #: per launch: first row, segment table (rows counted from the first), longest segment
+    parts: list[tuple[int, torch.Tensor, int]]
+    _staged_hosts: tuple[torch.Tensor, ...]
 
     @classmethod
     def create(
@@ -115,20 +117,27 @@ class RowCopyDescriptor:
         piece = max_piece_nbytes
         while sum(-(-n // piece) for _, _, n, _ in segments) > _MAX_SEGMENTS:
             piece *= 2
-        columns: list[list[int]] = [[], [], [], []]
+        by_part: dict[int, list[list[int]]] = {}
         for row, src, nbytes, dst in segments:
+            columns = by_part.setdefault(row // MAX_COPY_ROWS, [[], [], [], []])
             for done in range(0, nbytes, piece):
                 step = min(piece, nbytes - done)
-                for column, value in zip(columns, (row, src + done, step, dst + done)):
+                for column, value in zip(columns, (row % MAX_COPY_ROWS, src + done, step, dst + done)):
                     column.append(value)
-        table, host = _upload_i64([v for column in columns for v in column], device)
-        return cls(table.view(4, -1), max(columns[2], default=0), host)
+        parts, hosts = [], []
+        for part, columns in sorted(by_part.items()):
+            if columns[0]:
+                table, host = _upload_i64([v for column in columns for v in column], device)
+                parts.append((part * MAX_COPY_ROWS, table.view(4, -1), max(columns[2])))
+                hosts.append(host)
+        return cls(parts, tuple(hosts))
 
 
 def copy_row_segments(rows: Sequence[torch.Tensor], output: torch.Tensor, descriptor: RowCopyDescriptor) -> None:
-    """Copy every segment of ``descriptor`` from ``rows`` to ``output`` in one launch."""
-    if descriptor.max_nbytes:
-        hip_ops.copy_row_segments(rows, output, descriptor.table, descriptor.max_nbytes)
+    """Copy every segment of ``descriptor`` from ``rows`` to ``output``, one
+    launch for every ``MAX_COPY_ROWS`` rows."""
+    for first, table, max_nbytes in descriptor.parts:
+        hip_ops.copy_row_segments(rows[first : first + MAX_COPY_ROWS], output, table, max_nbytes)
 
 
 def zero_segments(output: torch.Tensor, descriptor: SegmentCopyDescriptor) -> None:

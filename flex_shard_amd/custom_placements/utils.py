@@ -17,7 +17,6 @@ import torch
 import torch.distributed as dist
 
 from .. import hip_ops
-from .._native import MAX_COPY_ROWS
 from ._copy_kernels import (
     RowCopyDescriptor,
     SegmentPackDescriptor,
@@ -263,13 +262,13 @@ def all_gather_rows(output: torch.Tensor, input: torch.Tensor, group: Any, *, as
 
 def local_exchange_rows(group: Any, input: torch.Tensor) -> list[torch.Tensor] | None:
     """The rows a local all-gather of ``input`` consists of, in rank order,
-    when one launch can read them all where they lie (a
+    when a launch can read them where they lie (a
     :class:`LocalReduceGroup` whose rows are contiguous GPU tensors of
     ``input``'s dtype and length); None otherwise."""
     if not isinstance(group, LocalReduceGroup) or group.local_row_only or torch.compiler.is_compiling():
         return None
     world, rank = group.size(), group.rank()
-    if world > MAX_COPY_ROWS or input.device.type != "cuda":
+    if input.device.type != "cuda":
         return None
     dtype, numel, device = input.dtype, input.numel(), input.get_device()
     gather_rows = group.gather_rows

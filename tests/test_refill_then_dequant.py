@@ -27,8 +27,9 @@ class _ViewShard(Fp8BucketedBlockShard):
 
 def _copy_rows(rows, output, descriptor):
     flat = output.view(-1)
-    for row, src, nbytes, dst in descriptor.table.t().tolist():
-        flat[dst : dst + nbytes] = rows[row].view(-1)[src : src + nbytes]
+    for first, table, _ in descriptor.parts:
+        for row, src, nbytes, dst in table.t().tolist():
+            flat[dst : dst + nbytes] = rows[first + row].view(-1)[src : src + nbytes]
 
 
 def _unpack(rows, table, starts, total_tiles, compact, dequant, block):
