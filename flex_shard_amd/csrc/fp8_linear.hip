@@ -41,6 +41,7 @@ struct ActQuantParams {
   uint8_t* q;
   float* scales;
   int64_t rows, cols, ldx, ldq;  // elements; ldq = cols rounded up to 128
+  int64_t first_row;             // of this launch
   int32_t col_groups;            // ceil(ceil(cols / 128) / 4)
   float eps;
 };
@@ -50,7 +51,7 @@ __global__ __launch_bounds__(kActThreads) void act_quant_1x128_kernel(const ActQ
   const int tid = threadIdx.x;
   const int sub = tid & 15, run_lane = tid >> 4;
   const int64_t tile_r = blockIdx.x / p.col_groups, tile_c = blockIdx.x % p.col_groups;
-  const int64_t row0 = tile_r * kActRows, kb0 = tile_c * kActBlocks;
+  const int64_t row0 = p.first_row + tile_r * kActRows, kb0 = tile_c * kActBlocks;
 
   u32x4 v[kActPasses];
 #pragma unroll
@@ -549,11 +550,18 @@ FSH_API int fsh_act_quant_1x128(const void* x_dev, int64_t rows, int64_t cols, i
   float eps_bf16;
   memcpy(&eps_bf16, &bits, 4);
   p.eps = eps_mode == FSH_EPS_FP32 ? eps32 : eps_bf16;
-  const int64_t grid = ceil_div(rows, (int64_t)kActRows) * col_groups;
-  if (grid > 0x7FFFFFFFLL || col_groups > 0x7FFFFFFFLL) return fail(FSH_ENOTSUP, "fsh_act_quant_1x128: too many tiles");
-  hipLaunchKernelGGL(act_quant_1x128_kernel, dim3(static_cast<uint32_t>(grid)), dim3(kActThreads), 0,
-                     static_cast<hipStream_t>(stream), p);
-  return check_launch("act_quant_1x128_kernel");
+  // A launch's threads are counted in 32 bits: 2^24 - 1 workgroups.  A narrow
+  // matrix of more rows than that (268 M of up to 512 columns) takes several.
+  constexpr int64_t kMaxGrid = (1LL << 32) / kActThreads - 1;
+  if (col_groups > kMaxGrid) return fail(FSH_ENOTSUP, "fsh_act_quant_1x128: too many tiles");
+  const int64_t rows_per_launch = kMaxGrid / col_groups * kActRows;
+  for (p.first_row = 0; p.first_row < rows; p.first_row += rows_per_launch) {
+    const int64_t left = rows - p.first_row, now = left < rows_per_launch ? left : rows_per_launch;
+    hipLaunchKernelGGL(act_quant_1x128_kernel, dim3(static_cast<uint32_t>(ceil_div(now, (int64_t)kActRows) * col_groups)),
+                       dim3(kActThreads), 0, static_cast<hipStream_t>(stream), p);
+    if (int rc = check_launch("act_quant_1x128_kernel")) return rc;
+  }
+  return FSH_OK;
 }
 
 namespace fsh {

@@ -379,3 +379,18 @@ def test_quantizers_and_transpose_on_a_matrix_beyond_two_to_the_32_bytes(device)
     for r, c in ((slice(0, 300), slice(0, 300)), (slice(rows - 300, rows), slice(cols - 300, cols))):
         assert torch.equal(t[c, r].view(torch.uint8), q[r, c].view(torch.uint8).t())
 
+
+
+def test_row_quantizer_on_more_rows_than_one_launch_takes(device):
+    """2^28 + 40 rows of 8 columns: 16 rows a workgroup are more workgroups than
+    the 2^24 - 1 of a launch.  Both ends and the rows around the second
+    launch's first against calls of their own."""
+    rows, boundary = 2**28 + 40, (2**24 - 1) * 16
+    x = torch.zeros((rows, 8), device=device, dtype=torch.bfloat16)
+    for part in (slice(0, 100), slice(boundary - 100, rows)):
+        x[part].normal_()
+    q, s = hip_ops.act_quant_1x128(x)
+    for part in (slice(0, 128), slice(boundary - 128, boundary), slice(boundary, rows)):
+        want_q, want_s = hip_ops.act_quant_1x128(x[part].clone())
+        assert torch.equal(q[part].view(torch.uint8), want_q.view(torch.uint8)) and torch.equal(s[:, part], want_s)
+    assert not q[128 : boundary - 128].view(torch.int64).any()
