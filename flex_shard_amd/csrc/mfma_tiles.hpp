@@ -211,9 +211,9 @@ __device__ __forceinline__ void wave_lds_sync() {
 //
 // The upper and then the lower 64 rows of the wave's 128x128 sub-tile are
 // taken in turn, in a staging region of 17 KB per wave that only the wave
-// itself touches.  The region then fits beside one k-loop stage, which leaves
-// the other stage free to receive the next tile's first operands while this
-// runs, and no step needs a workgroup barrier (whose memory fence would wait
+// itself touches.  The region then fits beside two of the k loop's operand
+// slots, which receive the next tile's first operands while this runs, and no
+// step needs a workgroup barrier (whose memory fence would wait
 // for those loads).
 template <typename Cfg>
 struct HalfTileEpilogue {
@@ -398,9 +398,6 @@ __device__ __forceinline__ void store_tile_in_halves(const GemmParams& p, int64_
   else
     store_tile_in_halves_as<Cfg, kEpiGeneric>(p, batch, m0, n0, wm, wn, lane, mirror, acc, staging);
 }
-
-// Scheduling-group masks of __builtin_amdgcn_sched_group_barrier.
-constexpr int kSchedMfma = 0x008, kSchedDsRead = 0x100;
 
 // gfx950 loads 16 bytes per lane from global memory straight into LDS: lane l
 // of a wave writes LDS bytes [M0 + 16 l, M0 + 16 l + 16).  The address is a

@@ -28,8 +28,7 @@ namespace {
 // gfx950 can load 16 bytes per lane from global memory straight into LDS
 // (global_load_lds_dwordx4: lane l of a wave writes LDS bytes
 // [M0 + 16 l, M0 + 16 l + 16)), so a k-tile needs no staging registers and
-// no ds_write, and the loads of tile t+1 are waited for only at the end of
-// tile t.  A wave-level load fills 1 KB of LDS = 8 tile rows of 128 bytes
+// no ds_write.  A wave-level load fills 1 KB of LDS = 8 tile rows of 128 bytes
 // with no padding, so bank conflicts are avoided by an XOR swizzle instead:
 // the 16-byte chunk c of row r is stored in slot c ^ ((r >> 1) & 7) of its
 // row, done on the global side by letting the lane that fills slot s of row r
@@ -44,31 +43,28 @@ namespace {
 // reorders nor counts; everything else in the loop is compiler-visible and is
 // pinned around them with sched_barrier.
 //
-// The part does not hold its peak clock under this kernel (1.5-1.6 GHz on
-// random operands, 2.3 GHz on zeros, by the shader-clock counter against the
-// 100 MHz one).  Cycle counters in the loop put under 5 % of a k-tile into the
-// wait for operands and the barrier together; asking for every operand line
-// once more, a few k-tiles ahead, to pull it into L2 (4-byte requests into a
-// scrap area) made all three products 2-5 % slower and is gone.
+// The part does not hold its peak clock under this kernel: 1.65 GHz on random
+// operands with the matrix cores 82 % busy (8192^3, by the counters).
 struct DmaGemm {
   static constexpr int BM = 256, BN = 256, BK = 64, WM = 2, WN = 2, TM = 4, TN = 4;
   static constexpr int kThreads = 256, kWaveM = 128, kWaveN = 128, KS = BK / 16;
   static constexpr int kRowBytes = BK * 2;                   // 128
-  static constexpr int kOperandBytes = BM * kRowBytes;       // 32 KB per operand and stage
-  static constexpr int kStageBytes = 2 * kOperandBytes;      // 64 KB
-  static constexpr int kLoopLdsBytes = 2 * kStageBytes;
-  static constexpr int kLoadsPerOperand = BM / 8 / 4;        // wave-level 1 KB loads per wave: 8
+  static constexpr int kOperandBytes = BM * kRowBytes;       // 32 KB per operand and k-tile
+  static constexpr int kSlots = 5;                           // ring of operand slots
+  static constexpr int kRingBytes = kSlots * kOperandBytes;  // 160 KB, all of a compute unit's LDS
+  static constexpr int kLoads = BM / 8 / 4;                  // wave-level 1 KB requests per wave and operand: 8
 };
 
-// LDS of the kernel: two operand stages, the epilogue's staging region from
-// stage 1 upward.
-constexpr int kDmaGemmLdsBytes = DmaGemm::kStageBytes + max_int(DmaGemm::kStageBytes, HalfTileEpilogue<DmaGemm>::kLdsBytes);
+// LDS of the kernel: the ring; the epilogue's staging region lies from slot 2 upward.
+constexpr int kDmaGemmLdsBytes = DmaGemm::kRingBytes;
+constexpr int kDmaGemmStaging = 2 * DmaGemm::kOperandBytes;
+static_assert(kDmaGemmStaging + HalfTileEpilogue<DmaGemm>::kLdsBytes <= kDmaGemmLdsBytes, "the epilogue works beside slots 0 and 1");
 
 // kPersistent: the grid is one workgroup per compute unit and workgroup g
 // takes the ids g, g + gridDim.x, ... of the launch (the same XCD every time,
 // and the 32 workgroups of an XCD stay on 32 neighbouring tiles).  While the
 // epilogue of a tile runs, the first operands of the next one are already on
-// their way into stage 0.  The schedule is static, so the host uses it only
+// their way.  The schedule is static, so the host uses it only
 // when all tiles of the launch are equally long; otherwise each id is its own
 // workgroup and the hardware hands them out as compute units come free.
 //
@@ -138,17 +134,16 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
     return uniform_ptr(reinterpret_cast<const uint8_t*>(
         q.B + batch * q.sB + static_cast<int64_t>(tn) * Cfg::BN * (kKMajor ? 1 : q.ldb)));
   };
-  auto issue_tile_load = [&](const uint8_t* a_src, const uint8_t* b_src, uint32_t a_row_bytes, uint32_t b_row_bytes,
-                             int stage_off, int q_first, int q_last) {
-    // The part of the address that depends on q goes into the scalar base, so
-    // that one lane offset per operand serves all eight loads.
-    const uint32_t a_voff = fill_row0 * a_row_bytes + fill_chunk * 16, b_voff = fill_row0 * b_row_bytes + fill_chunk * 16;
+  // Request q of an operand's k-tile at `src` into the ring slot at `slot`.
+  // The part of the address that depends on q goes into the scalar base, so
+  // that one lane offset per operand serves all eight.
+  auto issue_one = [&](const uint8_t* src, uint32_t row_bytes, int slot, int q) {
+    dma_load_16(fill_row0 * row_bytes + fill_chunk * 16, src + static_cast<uint64_t>(kRowsPerLoadStep * q) * row_bytes,
+                slot + fill_lds, q * 4096);
+  };
+  auto issue_operand = [&](const uint8_t* src, uint32_t row_bytes, int slot, int count) {
 #pragma unroll
-    for (int q = q_first; q < q_last; ++q) {
-      dma_load_16(a_voff, a_src + static_cast<uint64_t>(kRowsPerLoadStep * q) * a_row_bytes, stage_off + fill_lds, q * 4096);
-      dma_load_16(b_voff, b_src + static_cast<uint64_t>(kRowsPerLoadStep * q) * b_row_bytes,
-                  stage_off + fill_lds, Cfg::kOperandBytes + q * 4096);
-    }
+    for (int q = 0; q < count; ++q) issue_one(src, row_bytes, slot, q);
   };
 
   // Operand pointer of k-tile kt: 128 bytes along the rows, or 64 rows down.
@@ -182,14 +177,14 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       a_frag[ks] = (frag_base ^ (ks * 32)) + wm * Cfg::kWaveM * Cfg::kRowBytes;
-      b_frag[ks] = (frag_base ^ (ks * 32)) + Cfg::kOperandBytes + wn * Cfg::kWaveN * Cfg::kRowBytes;
+      b_frag[ks] = (frag_base ^ (ks * 32)) + wn * Cfg::kWaveN * Cfg::kRowBytes;
     }
     const int t = l & 15, g = l >> 4;
     const uint32_t common = static_cast<uint32_t>(((g >> 1) * 8 + (t >> 2)) * 512 + (g & 1) * 32 + (t & 3) * 8);
 #pragma unroll
     for (int i = 0; i < TM; ++i) a_frag_km[i] = common + wm * 256 + ((i ^ (t >> 2)) * 64);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) b_frag_km[j] = Cfg::kOperandBytes + common + wn * 256 + ((j ^ (t >> 2)) * 64);
+    for (int j = 0; j < TN; ++j) b_frag_km[j] = common + wn * 256 + ((j ^ (t >> 2)) * 64);
   };
   derive_lane_values(lane);
 
@@ -202,23 +197,22 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
     const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)(lds_bytes + offset + 2048));
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  auto read_a = [&](int set, int stage_off, int ks, int i) {
+  auto read_a = [&](int set, int slot, int ks, int i) {
     if (kKMajor)
-      af[set][i] = read_transposed(stage_off + a_frag_km[i] + ks * 8192);
+      af[set][i] = read_transposed(slot + a_frag_km[i] + ks * 8192);
     else
-      af[set][i] = *reinterpret_cast<const bf16x8*>(lds_bytes + stage_off + a_frag[ks] + i * 32 * Cfg::kRowBytes);
+      af[set][i] = *reinterpret_cast<const bf16x8*>(lds_bytes + slot + a_frag[ks] + i * 32 * Cfg::kRowBytes);
   };
-  auto read_b = [&](int set, int stage_off, int ks, int j) {
+  auto read_b = [&](int set, int slot, int ks, int j) {
     if (kKMajor)
-      bf[set][j] = read_transposed(stage_off + b_frag_km[j] + ks * 8192);
+      bf[set][j] = read_transposed(slot + b_frag_km[j] + ks * 8192);
     else
-      bf[set][j] = *reinterpret_cast<const bf16x8*>(lds_bytes + stage_off + b_frag[ks] + j * 32 * Cfg::kRowBytes);
+      bf[set][j] = *reinterpret_cast<const bf16x8*>(lds_bytes + slot + b_frag[ks] + j * 32 * Cfg::kRowBytes);
   };
-  auto read_frags = [&](int set, int stage_off, int ks) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) read_a(set, stage_off, ks, i);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) read_b(set, stage_off, ks, j);
+  // Fragment g of k step ks: the TM of operand A, then the TN of B.
+  auto read_frag = [&](int set, int a_slot, int b_slot, int ks, int g) {
+    if (g < TM) read_a(set, a_slot, ks, g);
+    else read_b(set, b_slot, ks, g - TM);
   };
   auto mfma = [&](int set, int i, int j) {
     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[set][j], af[set][i], acc[i][j], 0, 0, 0);
@@ -246,109 +240,88 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   uint32_t a_row_bytes = static_cast<uint32_t>(launch.problem[which].lda * 2);
   uint32_t b_row_bytes = static_cast<uint32_t>(launch.problem[which].ldb * 2);
   FSH_STAMP(1);
-  issue_tile_load(Ab, Bb, a_row_bytes, b_row_bytes, 0, 0, Cfg::kLoadsPerOperand);
+  issue_operand(Ab, a_row_bytes, 0, Cfg::kLoads);
+  issue_operand(Bb, b_row_bytes, Cfg::kOperandBytes, Cfg::kLoads);
 
-  // One k-tile, rotated by a quarter: the barrier that hands over the next
-  // tile's operands sits before the last k step, so that step's MFMAs cover
-  // the first fragment reads of the next tile (otherwise exposed after every
-  // barrier) and the requests for the tile after it (the stage they fill was
-  // released by the same barrier: every wave holds its last fragments of it
-  // in registers).
-  //   entering:  set 0 holds the fragments of (kt, k step 0); the operands of
-  //              kt + 1 are on their way
-  //   k steps 0 .. KS-2: MFMAs while the next step's fragments are read
-  //   wait for kt + 1, barrier
-  //   k step KS-1: one MFMA, one fragment read of (kt + 1, 0), one pair of
-  //              requests for kt + 2 at a time
 #ifdef FSH_TRACE
   uint64_t trace_wait = 0, trace_barrier = 0, trace_ktiles = 0, trace_tile_wait = 0, trace_tile_barrier = 0, trace_tiles = 0, trace_kloop = 0, trace_epi = 0, trace_steps = 0, trace_last = 0, trace_mark = 0;
   const uint64_t trace_begin = __builtin_amdgcn_s_memtime();
 #endif
-  // Requests for a k-tile's operands.  A wave cannot issue anything else
-  // while a request waits to be accepted, and with all four waves asking at
-  // once each request takes about 80 cycles: cycle counters put the last k
-  // step, when it carried all sixteen requests of a wave, at 1250 cycles
-  // against 512 of matrix work.  The requests are therefore spread over two k
-  // steps, one per two MFMAs: eight behind the barrier that released their
-  // stage and eight in the first k step of the next k-tile, which still
-  // leaves them two k steps to land.  (Spread over all four k steps, the late
-  // ones were waited for.)
-  constexpr int kFirstRequests = 8, kSecondRequests = 16 - kFirstRequests;  // 6 / 10, 10 / 6 and 12 / 4 measured the same or slower
-  // request idx (0 .. 15) of a k-tile: operand A for even idx, B for odd, wave-level load idx / 2
-  auto issue_one = [&](int idx, const uint8_t* a_src, const uint8_t* b_src, int stage) {
-    const int q = idx >> 1;
-    if (idx & 1)
-      dma_load_16(fill_row0 * b_row_bytes + fill_chunk * 16, b_src + static_cast<uint64_t>(kRowsPerLoadStep * q) * b_row_bytes,
-                  stage + fill_lds, Cfg::kOperandBytes + q * 4096);
-    else
-      dma_load_16(fill_row0 * a_row_bytes + fill_chunk * 16, a_src + static_cast<uint64_t>(kRowsPerLoadStep * q) * a_row_bytes,
-                  stage + fill_lds, q * 4096);
-  };
-  auto k_tile = [&](int64_t kt, int64_t ktiles, auto more_tag, auto first_tag) {
-    constexpr bool more = decltype(more_tag)::value;
-    constexpr bool first = decltype(first_tag)::value;  // k-tile 0 of an output tile
-    const int stage_off = static_cast<int>(kt & 1) * Cfg::kStageBytes;
-    const int next_off = stage_off ^ Cfg::kStageBytes;
-#pragma unroll
-    for (int ks = 0; ks + 1 < KS; ++ks) {
-      if (ks == 0 && more && !first) {
-        // the second eight requests for k-tile kt + 1 (the first eight went out in the last k step of kt - 1)
-        const uint8_t* a_cur = k_tile_ptr(Ab, a_row_bytes, kt + 1);
-        const uint8_t* b_cur = k_tile_ptr(Bb, b_row_bytes, kt + 1);
-#pragma unroll
-        for (int g = 0; g < TM * TN; ++g) {
-          mfma(0, g / TN, g % TN);
-          if (g < TM) read_a(1, stage_off, 1, g);
-          else if (g < TM + TN) read_b(1, stage_off, 1, g - TM);
-          if ((g + 1) * kSecondRequests / 16 != g * kSecondRequests / 16)
-            issue_one(kFirstRequests + g * kSecondRequests / 16, a_cur, b_cur, next_off);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        continue;
+  // The k loop.  What bounds it: the request path of a compute unit takes one
+  // of the 64 requests of a k-tile (16 per wave) per 16 cycles, so they need
+  // half of the 2048 cycles of the MFMAs, and a wave that issues a request
+  // into a busy path cannot issue MFMAs.  Packed into two of the four k steps,
+  // as two 64 KB stages ask for (a stage is free only once the k-tile in it
+  // has been read), they cost 500 of the 3000 cycles a k-tile took, and the
+  // wait for the last ones up to 460.  The ring holds two and a half k-tiles
+  // instead: operand n of the sequence A(0), B(0), A(1), B(1), ... lives in
+  // slot n % 5, so A is requested two k-tiles ahead while both operands of the
+  // next one are still on their way, and every k step carries four requests of
+  // a wave, one per four MFMAs.
+  //
+  // The barrier that hands over k-tile kt + 1 sits before the last k step of
+  // kt: that step's MFMAs cover the first fragment reads of kt + 1, and the
+  // slots of kt are free (every wave holds its last fragments in registers).
+  //   k step 0:     requests 4-7 of B(kt + 1)
+  //   k steps 1, 2: A(kt + 2) into the fifth slot
+  //   wait for all but A(kt + 2), barrier
+  //   k step 3:     requests 0-3 of B(kt + 2) into the slot of A(kt)
+  // Each step reads the next one's fragments.
+  // Us before / after (two stages / ring): 24 x 7168 x 2048, k 2048 1327 / 1185;
+  // the same, k-major and symmetric, k 7168 786 / 728; 8192^3 901 / 821; 4096^3
+  // 108 / 102.  Eight requests behind the barrier and the rest in any split
+  // over the other steps, or all four of a step at once: the same or 2 % slower.
+  constexpr int kPerStep = 2 * Cfg::kLoads / KS;
+  static_assert(KS == 4 && Cfg::kLoads == 2 * kPerStep, "the sequence above");
+  const auto next_slot = [](int slot) { return slot + Cfg::kOperandBytes == Cfg::kRingBytes ? 0 : slot + Cfg::kOperandBytes; };
+  int a_slot = 0;  // of the current k-tile's operand A
+  // more: k-tile kt + 1 exists; more2: kt + 2 exists; zero: k-tile 0 of an output tile
+  auto k_tile = [&](int64_t kt, auto more_tag, auto more2_tag, auto zero_tag) {
+    constexpr bool more = decltype(more_tag)::value, more2 = decltype(more2_tag)::value, zero = decltype(zero_tag)::value;
+    const int b_slot = next_slot(a_slot), a_next = next_slot(b_slot), b_next = next_slot(a_next), a_after = next_slot(b_next);
+    const uint8_t* b_src1 = k_tile_ptr(Bb, b_row_bytes, kt + 1);
+    const uint8_t* a_src2 = k_tile_ptr(Ab, a_row_bytes, kt + 2);
+    const uint8_t* b_src2 = k_tile_ptr(Bb, b_row_bytes, kt + 2);
+    // MFMA g of k step ks with what goes out behind it.
+    auto slice = [&](int ks, int g) {
+      if (zero && ks == 0) mfma_from_zero(0, g / TN, g % TN);
+      else mfma(ks & 1, g / TN, g % TN);
+      if (g < TM + TN) {
+        if (ks + 1 < KS) read_frag((ks + 1) & 1, a_slot, b_slot, ks + 1, g);
+        else if (more) read_frag(0, a_next, b_next, 0, g);
       }
-      read_frags((ks + 1) & 1, stage_off, ks + 1);
-#pragma unroll
-      for (int g = 0; g < TM * TN; ++g) {
-        if (first && ks == 0) mfma_from_zero(0, g / TN, g % TN);
-        else mfma(ks & 1, g / TN, g % TN);
+      if ((g + 1) % (TM * TN / kPerStep) == 0) {
+        const int r = g / (TM * TN / kPerStep);
+        if (ks == 0 && more) issue_one(b_src1, b_row_bytes, b_next, kPerStep + r);
+        if ((ks == 1 || ks == 2) && more2) issue_one(a_src2, a_row_bytes, a_after, (ks - 1) * kPerStep + r);
+        if (ks == 3 && more2) issue_one(b_src2, b_row_bytes, a_slot, r);
       }
+      __builtin_amdgcn_sched_barrier(0);
+    };
 #pragma unroll
-      for (int g = 0; g < TM + TN; ++g) {
-        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, kKMajor ? 2 : 1, 0);
-        __builtin_amdgcn_sched_group_barrier(kSchedMfma, TM * TN / (TM + TN), 0);
-      }
-    }
+    for (int ks = 0; ks + 1 < KS; ++ks)
+#pragma unroll
+      for (int g = 0; g < TM * TN; ++g) slice(ks, g);
 #ifdef FSH_TRACE
     const uint64_t tr0 = __builtin_amdgcn_s_memtime();
     trace_steps += tr0 - trace_mark;
 #endif
-    if (more) {  // this wave's part of the next tile has landed
-      wait_for_dma_loads();
-    }
+    // This wave's part of k-tile kt + 1 has landed; A(kt + 2) stays in flight.
+    if (more2) wait_for_dma_loads_but<Cfg::kLoads>();
+    else if (more) wait_for_dma_loads();
 #ifdef FSH_TRACE
     const uint64_t tr1 = __builtin_amdgcn_s_memtime();
 #endif
-    __syncthreads();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #ifdef FSH_TRACE
     const uint64_t tr2 = __builtin_amdgcn_s_memtime();
     trace_wait += tr1 - tr0;
     trace_barrier += tr2 - tr1;
     trace_ktiles += 1;
 #endif
-    const bool more2 = more && kt + 2 < ktiles;
-    const uint8_t* a_next = k_tile_ptr(Ab, a_row_bytes, kt + 2);
-    const uint8_t* b_next = k_tile_ptr(Bb, b_row_bytes, kt + 2);
 #pragma unroll
-    for (int g = 0; g < TM * TN; ++g) {
-      mfma((KS - 1) & 1, g / TN, g % TN);
-      if (more) {
-        if (g < TM) read_a(0, next_off, 0, g);
-        else if (g < TM + TN) read_b(0, next_off, 0, g - TM);
-      }
-      if (more2 && (g + 1) * kFirstRequests / 16 != g * kFirstRequests / 16)
-        issue_one(g * kFirstRequests / 16, a_next, b_next, stage_off);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    for (int g = 0; g < TM * TN; ++g) slice(KS - 1, g);
+    a_slot = a_next;
 #ifdef FSH_TRACE
     trace_mark = __builtin_amdgcn_s_memtime();
     trace_last += trace_mark - tr2;
@@ -380,26 +353,35 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
     const uint64_t tk0 = __builtin_amdgcn_s_memtime();
     trace_mark = tk0;
 #endif
-    read_frags(0, 0, 0);
-    if (ktiles > 1)
-      issue_tile_load(k_tile_ptr(Ab, a_row_bytes, 1), k_tile_ptr(Bb, b_row_bytes, 1), a_row_bytes, b_row_bytes,
-                      Cfg::kStageBytes, 0, Cfg::kLoadsPerOperand);
+    a_slot = 0;
+#pragma unroll
+    for (int g = 0; g < TM + TN; ++g) read_frag(0, 0, Cfg::kOperandBytes, 0, g);
+    if (ktiles > 1) {
+      issue_operand(k_tile_ptr(Ab, a_row_bytes, 1), a_row_bytes, 2 * Cfg::kOperandBytes, Cfg::kLoads);
+      issue_operand(k_tile_ptr(Bb, b_row_bytes, 1), b_row_bytes, 3 * Cfg::kOperandBytes, kPerStep);
+    }
     FSH_STAMP(2);
 
-    if (ktiles > 1) {
-      k_tile(0, ktiles, std::true_type{}, std::true_type{});
-      for (int64_t kt = 1; kt + 1 < ktiles; ++kt) k_tile(kt, ktiles, std::true_type{}, std::false_type{});
-      k_tile(ktiles - 1, ktiles, std::false_type{}, std::false_type{});
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    if (ktiles > 2) {
+      k_tile(0, yes, yes, yes);
+      for (int64_t kt = 1; kt + 2 < ktiles; ++kt) k_tile(kt, yes, yes, no);
     } else {
-      k_tile(0, ktiles, std::false_type{}, std::true_type{});
+#pragma unroll
+      for (int g = 0; g < TM * TN; ++g)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[g / TN][g % TN][r] = 0.0f;
     }
+    if (ktiles > 1) k_tile(ktiles - 2, yes, no, no);
+    k_tile(ktiles - 1, no, no, no);
     FSH_STAMP(3);
 #ifdef FSH_TRACE
     trace_kloop += __builtin_amdgcn_s_memtime() - tk0;
 #endif
 
-    // Both stages are free now.  The next tile's first operands go to stage 0
-    // while the epilogue stages its output beside it, from stage 1 upward.
+    // All slots are free now.  The next tile's first operands go to slots 0 and
+    // 1 while the epilogue stages its output beside them.
     int next_which = 0, next_tm = 0, next_tn = 0;
     int64_t next_batch = 0;
     bool have_next = false;
@@ -412,14 +394,15 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
         Bb = b_base(next_which, next_batch, next_tn);
         a_row_bytes = static_cast<uint32_t>(launch.problem[next_which].lda * 2);
         b_row_bytes = static_cast<uint32_t>(launch.problem[next_which].ldb * 2);
-        issue_tile_load(Ab, Bb, a_row_bytes, b_row_bytes, 0, 0, Cfg::kLoadsPerOperand);
+        issue_operand(Ab, a_row_bytes, 0, Cfg::kLoads);
+        issue_operand(Bb, b_row_bytes, Cfg::kOperandBytes, Cfg::kLoads);
       }
     }
 #ifdef FSH_TRACE
     const uint64_t te0 = __builtin_amdgcn_s_memtime();
 #endif
     store_tile_in_halves<Cfg>(p, batch, static_cast<int64_t>(tm) * Cfg::BM, static_cast<int64_t>(tn) * Cfg::BN, wm,
-                              wn, lane, p.symmetric && tm != tn, acc, lds_bytes + Cfg::kStageBytes);
+                              wn, lane, p.symmetric && tm != tn, acc, lds_bytes + kDmaGemmStaging);
 #ifdef FSH_TRACE
     trace_epi += __builtin_amdgcn_s_memtime() - te0;
 #endif
