@@ -140,9 +140,15 @@ __device__ inline void store_staged_rows(const uint8_t* region, uint16_t* dst, i
   for (int pass = 0; pass < kRows / kRowsPerPass; ++pass) {
     const int r = pass * kRowsPerPass + r0;
     const uint8_t* src = region + r * kPitch + chunk * 16;
-    const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
-    const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
-    *reinterpret_cast<u32x4*>(base + pass * pass_bytes + lane_off) = u32x4{lo.x, lo.y, hi.x, hi.y};
+    u32x4 v;
+    if (kPitch % 16 == 0) {
+      v = *reinterpret_cast<const u32x4*>(src);
+    } else {
+      const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
+      const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
+      v = u32x4{lo.x, lo.y, hi.x, hi.y};
+    }
+    *reinterpret_cast<u32x4*>(base + pass * pass_bytes + lane_off) = v;
   }
 }
 
@@ -195,9 +201,9 @@ __device__ __forceinline__ void wave_lds_sync() {
 // Epilogue of the large-tile kernel, staged through LDS.
 //
 // The accumulate is issued as mfma(B, A), so accumulator r of block (i, j)
-// belongs to output row m = lane%32 and column n = 8*(r/4) + 4*(lane/32) + r%4
-// of the block.  In that layout a store instruction would touch 32 rows with
-// 16 bytes each, and the transposed output would leave as 2-byte stores.
+// belongs to output row m = lane%16 and column n = 4*(lane/16) + r of the
+// 16x16 block.  In that layout a store instruction would touch 16 rows with
+// 32 bytes each, and the transposed output would leave as 2-byte stores.
 // Instead:
 //   1. D is loaded row-wise (16 bytes per lane) into the staging region; the
 //      finals = bf16(fma(beta, D, alpha*acc)) are computed in registers and
@@ -206,8 +212,9 @@ __device__ __forceinline__ void wave_lds_sync() {
 //      lane, 256 contiguous bytes per row;
 //   3. for a transposed (or mirrored) output the finals are read back in
 //      accumulator layout, written again as [col][row] and leave the same way.
-// The LDS row pitch is the row plus 8 bytes: 8-byte writes of 16 lanes then
-// cover all banks, and so do the row-wise 8-byte reads of a half-wave.
+// The LDS row pitch is the row plus 16 bytes: 8-byte writes of 32 lanes (16
+// rows, two groups of columns) then cover all banks, and rows are read 16 bytes
+// at a time.
 //
 // The upper and then the lower 64 rows of the wave's 128x128 sub-tile are
 // taken in turn, in a staging region of 17 KB per wave that only the wave
@@ -218,7 +225,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 template <typename Cfg>
 struct HalfTileEpilogue {
   static constexpr int kRows = Cfg::kWaveM / 2;                 // 64
-  static constexpr int kPitch = Cfg::kWaveN * 2 + 8;            // [row][col] image
+  static constexpr int kPitch = Cfg::kWaveN * 2 + 16;           // [row][col] image
   static constexpr int kPitchT = kRows * 2 + 8;                 // [col][row] image
   static constexpr int kRegion =
       (kRows * kPitch > Cfg::kWaveN * kPitchT) ? kRows * kPitch : Cfg::kWaveN * kPitchT;
@@ -239,12 +246,12 @@ constexpr int kEpiGeneric = 0, kEpiPlain = 1, kEpiPoly = 2, kEpiUpdate = 3;
 // table would have to live in scratch memory.)
 template <typename Cfg, int kMode>
 __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int64_t batch, int64_t m0, int64_t n0, int wm,
-                                               int wn, int lane, bool mirror, const f32x16 (&acc)[Cfg::TM][Cfg::TN],
+                                               int wn, int lane, bool mirror, const f32x4 (&acc)[Cfg::TM][Cfg::TN],
                                                uint8_t* staging) {
   using Epi = HalfTileEpilogue<Cfg>;
   using R = DRows<Cfg>;
   constexpr int TM = Cfg::TM, TN = Cfg::TN, HM = TM / 2;
-  static_assert(TM % 2 == 0 && Epi::kRows == HM * 32, "two halves of whole 32-row blocks");
+  static_assert(TM % 2 == 0 && Epi::kRows == HM * 16, "two halves of whole 16-row blocks");
   const bool has_d = kMode == kEpiPlain ? false : (kMode == kEpiPoly || kMode == kEpiUpdate) ? true : p.D != nullptr;
   // (a pointer loaded from a table is a per-lane value to the compiler: said to be uniform here)
   uint16_t* C = kMode == kEpiUpdate ? reinterpret_cast<uint16_t*>(uniform_i64(p.update_ptrs[batch])) : p.C + batch * p.sC;
@@ -255,7 +262,7 @@ __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int
   const int64_t ldct = mirror ? p.ldc : p.ldct;
   const int64_t wave_row = m0 + wm * Cfg::kWaveM, wave_col = n0 + wn * Cfg::kWaveN;
   uint8_t* region = staging + (wm * Cfg::WN + wn) * Epi::kRegion;
-  const int r_lane = lane & 31, h = lane >> 5;
+  const int r_lane = lane & 15, c_lane = 4 * (lane >> 4);
   const bool unit_alpha = (kMode == kEpiPlain || kMode == kEpiUpdate) ? true : kMode == kEpiPoly ? false : p.alpha == 1.0f;
   // Block tiles and wave sub-tiles are square, so C's diagonal runs through
   // the (i, i) blocks of the diagonal sub-tiles of the diagonal tiles.
@@ -273,74 +280,65 @@ __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int
 #pragma unroll
       for (int q = 0; q < R::kPasses; ++q) {
         uint8_t* d = region + (r0 + q * R::kRowsPerPass) * Epi::kPitch + chunk * 16;
-        *reinterpret_cast<u32x2*>(d) = u32x2{drows[hf].t[q].x, drows[hf].t[q].y};
-        *reinterpret_cast<u32x2*>(d + 8) = u32x2{drows[hf].t[q].z, drows[hf].t[q].w};
+        *reinterpret_cast<u32x4*>(d) = drows[hf].t[q];
       }
       if (hf == 0) load_d_rows_from<Cfg>(D, ldd, m0, n0, wm, wn, lane, 1, drows[1]);
       wave_lds_sync();
     }
 #pragma unroll
     for (int ih = 0; ih < HM; ++ih) {
-      u32x2 fin[TN][4];  // packed bf16 finals of this 32-row block, accumulator layout
+      u32x2 fin[TN];  // packed bf16 finals of this 16-row block, accumulator layout
       const int i = hf * HM + ih;
-      u32x2 dv[TN][4];
+      u32x2 dv[TN];
       if (has_d) {
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int b = 0; b < 4; ++b)
-            dv[j][b] = *reinterpret_cast<const u32x2*>(region + (ih * 32 + r_lane) * Epi::kPitch +
-                                                       (j * 32 + 8 * b + 4 * h) * 2);
+          dv[j] = *reinterpret_cast<const u32x2*>(region + (ih * 16 + r_lane) * Epi::kPitch + (j * 16 + c_lane) * 2);
       }
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+      for (int j = 0; j < TN; ++j) {
+        float v[4];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          float v[4];
-#pragma unroll
-          for (int t = 0; t < 4; ++t) v[t] = unit_alpha ? acc[i][j][4 * b + t] : p.alpha * acc[i][j][4 * b + t];
-          if (kMode == kEpiUpdate) {
-            // The rounding sequence of the separate update kernel: direction
-            // to bf16 (scaled and rounded again when the scale is not 1),
-            // decayed parameter to bf16, then one multiply and one add.
-            const uint32_t d01 = pack_bf16x2(v[0], v[1]), d23 = pack_bf16x2(v[2], v[3]);
-            float d[4] = {u32_as_f32(d01 << 16), u32_as_f32(d01 & 0xFFFF0000u), u32_as_f32(d23 << 16),
-                          u32_as_f32(d23 & 0xFFFF0000u)};
-            if (p.update_dir_scale != 1.0f) {
-              const uint32_t s01 = pack_bf16x2(d[0] * p.update_dir_scale, d[1] * p.update_dir_scale);
-              const uint32_t s23 = pack_bf16x2(d[2] * p.update_dir_scale, d[3] * p.update_dir_scale);
-              d[0] = u32_as_f32(s01 << 16); d[1] = u32_as_f32(s01 & 0xFFFF0000u);
-              d[2] = u32_as_f32(s23 << 16); d[3] = u32_as_f32(s23 & 0xFFFF0000u);
-            }
-            const uint32_t p01 = pack_bf16x2(u32_as_f32(dv[j][b].x << 16) * p.update_decay,
-                                             u32_as_f32(dv[j][b].x & 0xFFFF0000u) * p.update_decay);
-            const uint32_t p23 = pack_bf16x2(u32_as_f32(dv[j][b].y << 16) * p.update_decay,
-                                             u32_as_f32(dv[j][b].y & 0xFFFF0000u) * p.update_decay);
-            v[0] = u32_as_f32(p01 << 16) + p.update_neg_lr * d[0];
-            v[1] = u32_as_f32(p01 & 0xFFFF0000u) + p.update_neg_lr * d[1];
-            v[2] = u32_as_f32(p23 << 16) + p.update_neg_lr * d[2];
-            v[3] = u32_as_f32(p23 & 0xFFFF0000u) + p.update_neg_lr * d[3];
-          } else if (has_d) {
-            v[0] = __builtin_fmaf(p.beta, u32_as_f32(dv[j][b].x << 16), v[0]);
-            v[1] = __builtin_fmaf(p.beta, u32_as_f32(dv[j][b].x & 0xFFFF0000u), v[1]);
-            v[2] = __builtin_fmaf(p.beta, u32_as_f32(dv[j][b].y << 16), v[2]);
-            v[3] = __builtin_fmaf(p.beta, u32_as_f32(dv[j][b].y & 0xFFFF0000u), v[3]);
+        for (int t = 0; t < 4; ++t) v[t] = unit_alpha ? acc[i][j][t] : p.alpha * acc[i][j][t];
+        if (kMode == kEpiUpdate) {
+          // The rounding sequence of the separate update kernel: direction
+          // to bf16 (scaled and rounded again when the scale is not 1),
+          // decayed parameter to bf16, then one multiply and one add.
+          const uint32_t d01 = pack_bf16x2(v[0], v[1]), d23 = pack_bf16x2(v[2], v[3]);
+          float d[4] = {u32_as_f32(d01 << 16), u32_as_f32(d01 & 0xFFFF0000u), u32_as_f32(d23 << 16),
+                        u32_as_f32(d23 & 0xFFFF0000u)};
+          if (p.update_dir_scale != 1.0f) {
+            const uint32_t s01 = pack_bf16x2(d[0] * p.update_dir_scale, d[1] * p.update_dir_scale);
+            const uint32_t s23 = pack_bf16x2(d[2] * p.update_dir_scale, d[3] * p.update_dir_scale);
+            d[0] = u32_as_f32(s01 << 16); d[1] = u32_as_f32(s01 & 0xFFFF0000u);
+            d[2] = u32_as_f32(s23 << 16); d[3] = u32_as_f32(s23 & 0xFFFF0000u);
           }
-          if (kMode != kEpiPlain && kMode != kEpiUpdate && i == j) {
-            // a select per final rather than a branch per block (adding zero
-            // elsewhere would turn a -0 into +0)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) v[t] = (on_diagonal && r_lane == 8 * b + 4 * h + t) ? v[t] + p.diag_add : v[t];
-          }
-          fin[j][b] = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+          const uint32_t p01 = pack_bf16x2(u32_as_f32(dv[j].x << 16) * p.update_decay,
+                                           u32_as_f32(dv[j].x & 0xFFFF0000u) * p.update_decay);
+          const uint32_t p23 = pack_bf16x2(u32_as_f32(dv[j].y << 16) * p.update_decay,
+                                           u32_as_f32(dv[j].y & 0xFFFF0000u) * p.update_decay);
+          v[0] = u32_as_f32(p01 << 16) + p.update_neg_lr * d[0];
+          v[1] = u32_as_f32(p01 & 0xFFFF0000u) + p.update_neg_lr * d[1];
+          v[2] = u32_as_f32(p23 << 16) + p.update_neg_lr * d[2];
+          v[3] = u32_as_f32(p23 & 0xFFFF0000u) + p.update_neg_lr * d[3];
+        } else if (has_d) {
+          v[0] = __builtin_fmaf(p.beta, u32_as_f32(dv[j].x << 16), v[0]);
+          v[1] = __builtin_fmaf(p.beta, u32_as_f32(dv[j].x & 0xFFFF0000u), v[1]);
+          v[2] = __builtin_fmaf(p.beta, u32_as_f32(dv[j].y << 16), v[2]);
+          v[3] = __builtin_fmaf(p.beta, u32_as_f32(dv[j].y & 0xFFFF0000u), v[3]);
         }
+        if (kMode != kEpiPlain && kMode != kEpiUpdate && i == j) {
+          // a select per final rather than a branch per block (adding zero
+          // elsewhere would turn a -0 into +0)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) v[t] = (on_diagonal && r_lane == c_lane + t) ? v[t] + p.diag_add : v[t];
+        }
+        fin[j] = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      }
       // A lane's finals replace exactly the D values it read itself.
 #pragma unroll
       for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-          *reinterpret_cast<u32x2*>(region + (ih * 32 + r_lane) * Epi::kPitch + (j * 32 + 8 * b + 4 * h) * 2) =
-              fin[j][b];
+        *reinterpret_cast<u32x2*>(region + (ih * 16 + r_lane) * Epi::kPitch + (j * 16 + c_lane) * 2) = fin[j];
     }
     if (hf == 1) FSH_STAMP(9);
     wave_lds_sync();
@@ -350,29 +348,23 @@ __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int
     if (Ct != nullptr) {  // uniform over the workgroup
       // The finals come back in accumulator layout (every read before the
       // first write: the transposed image reuses the region).
-      u32x2 fin[HM][TN][4];
+      u32x2 fin[HM][TN];
 #pragma unroll
       for (int ih = 0; ih < HM; ++ih)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int b = 0; b < 4; ++b)
-            fin[ih][j][b] = *reinterpret_cast<const u32x2*>(region + (ih * 32 + r_lane) * Epi::kPitch +
-                                                            (j * 32 + 8 * b + 4 * h) * 2);
+          fin[ih][j] = *reinterpret_cast<const u32x2*>(region + (ih * 16 + r_lane) * Epi::kPitch + (j * 16 + c_lane) * 2);
       wave_lds_sync();  // these reads and the row reads are done before the region is reused
 #pragma unroll
       for (int ih = 0; ih < HM; ++ih)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-          for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              const uint32_t pair = (t >> 1) ? fin[ih][j][b].y : fin[ih][j][b].x;
-              *reinterpret_cast<uint16_t*>(region + (j * 32 + 8 * b + 4 * h + t) * Epi::kPitchT +
-                                           (ih * 32 + r_lane) * 2) =
-                  static_cast<uint16_t>((t & 1) ? (pair >> 16) : pair);
-            }
+          for (int t = 0; t < 4; ++t) {
+            const uint32_t pair = (t >> 1) ? fin[ih][j].y : fin[ih][j].x;
+            *reinterpret_cast<uint16_t*>(region + (j * 16 + c_lane + t) * Epi::kPitchT + (ih * 16 + r_lane) * 2) =
+                static_cast<uint16_t>((t & 1) ? (pair >> 16) : pair);
+          }
       if (hf == 1) FSH_STAMP(12);
       wave_lds_sync();
       store_staged_rows<Cfg::kWaveN, Epi::kRows * 2, Epi::kPitchT>(
@@ -385,7 +377,7 @@ __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int
 
 template <typename Cfg>
 __device__ __forceinline__ void store_tile_in_halves(const GemmParams& p, int64_t batch, int64_t m0, int64_t n0, int wm, int wn,
-                                            int lane, bool mirror, const f32x16 (&acc)[Cfg::TM][Cfg::TN],
+                                            int lane, bool mirror, const f32x4 (&acc)[Cfg::TM][Cfg::TN],
                                             uint8_t* staging) {
   // uniform over the launch's problem, so one branch per tile
   const bool has_d = p.D != nullptr, diag = p.diag_add != 0.0f, unit_alpha = p.alpha == 1.0f;

@@ -12,7 +12,8 @@
 // A tall input is its own X^T, so no transpose kernel is needed in either
 // case, and the result lands in the caller's buffer without a copy.
 //
-// GEMM kernels: 256 threads (2x2 wavefronts) on v_mfma_f32_32x32x16_bf16,
+// GEMM kernels: 256 threads (2x2 wavefronts) on v_mfma_f32_16x16x32_bf16 (the
+// smaller tiles: 32x32x16),
 // operands global -> LDS directly: 256x256x64 tiles for large problems of
 // whole tiles (below), smaller tiles for everything else (gemm_tiles.hpp).
 #include "gemm_tiles.hpp"
@@ -43,11 +44,12 @@ namespace {
 // reorders nor counts; everything else in the loop is compiler-visible and is
 // pinned around them with sched_barrier.
 //
-// The part does not hold its peak clock under this kernel: 1.65 GHz on random
-// operands with the matrix cores 82 % busy (8192^3, by the counters).
+// The part does not hold its peak clock under this kernel: 1.84 GHz on random
+// operands with the matrix cores 83 % busy (8192^3, by the counters).
 struct DmaGemm {
-  static constexpr int BM = 256, BN = 256, BK = 64, WM = 2, WN = 2, TM = 4, TN = 4;
-  static constexpr int kThreads = 256, kWaveM = 128, kWaveN = 128, KS = BK / 16;
+  static constexpr int BM = 256, BN = 256, BK = 64, WM = 2, WN = 2;
+  static constexpr int kThreads = 256, kWaveM = 128, kWaveN = 128;
+  static constexpr int TM = kWaveM / 16, TN = kWaveN / 16, KS = BK / 32;  // 16x16x32 products
   static constexpr int kRowBytes = BK * 2;                   // 128
   static constexpr int kOperandBytes = BM * kRowBytes;       // 32 KB per operand and k-tile
   static constexpr int kSlots = 5;                           // ring of operand slots
@@ -60,6 +62,12 @@ constexpr int kDmaGemmLdsBytes = DmaGemm::kRingBytes;
 constexpr int kDmaGemmStaging = 2 * DmaGemm::kOperandBytes;
 static_assert(kDmaGemmStaging + HalfTileEpilogue<DmaGemm>::kLdsBytes <= kDmaGemmLdsBytes, "the epilogue works beside slots 0 and 1");
 
+// (The empty statement keeps the cleared registers in place.)
+__device__ __forceinline__ void clear_accumulators(f32x4& acc) {
+  acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  asm volatile("" : "+a"(acc));
+}
+
 // kPersistent: the grid is one workgroup per compute unit and workgroup g
 // takes the ids g, g + gridDim.x, ... of the launch (the same XCD every time,
 // and the 32 workgroups of an XCD stay on 32 neighbouring tiles).  While the
@@ -70,14 +78,14 @@ static_assert(kDmaGemmStaging + HalfTileEpilogue<DmaGemm>::kLdsBytes <= kDmaGemm
 //
 // kKMajor: both operands are given k-major, A as [K, M] and B as [K, N] (row
 // strides lda / ldb), i.e. the product is A^T B.  A k-tile of an operand is
-// then 64 rows of 512 bytes.  It lands in LDS as it is (chunk c of k-row r in
-// slot c ^ 4 (r & 3)), and the fragments come out of it through the
-// transposing LDS read of gfx950 (ds_read_b64_tr_b16): within 16 lanes, lane
-// 4 j + q passes the address of four consecutive columns 4 q .. 4 q + 3 of
-// k-row j, and lane t receives column t of k-rows 0 .. 3 -- four consecutive
-// k of one output row, half of an MFMA operand.  The products and their order
-// are those of the k-contiguous form on the transposed operands, so the
-// results are bit-identical.
+// then 64 rows of 512 bytes.  They land in LDS whole (the row order and the
+// swizzle are at the load side below), and the fragments come out of it
+// through the transposing LDS read of gfx950 (ds_read_b64_tr_b16): within 16
+// lanes, lane 4 j + q passes the address of four consecutive columns 4 q ..
+// 4 q + 3 of k-row j, and lane t receives column t of k-rows 0 .. 3 -- four
+// consecutive k of one output row, half of an MFMA operand.  The products and
+// their order are those of the k-contiguous form on the transposed operands,
+// so the results are bit-identical.
 template <bool kPersistent, bool kKMajor>
 __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const GemmLaunch launch) {
   using Cfg = DmaGemm;
@@ -112,13 +120,14 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
 
   // Load side.  Wave-level load q (0..7) of this wave fills tile rows
   // [32 q + 8 wave, +8); lane l fills slot l & 7 of row l >> 3 there.
-  // (k-major: load q fills k-rows [8 q + 2 wave, +2); lane l fills slot
-  // l & 31 of row l >> 5 there.)
+  // (k-major: load q fills k-rows r and r + 8, r = 16 (q / 2) + 4 (q % 2) + wave;
+  // lane l fills slot l & 31 of row r + 8 (l >> 5).  K-row 16 a + 8 b + c thus
+  // lies at byte 1024 (8 a + c) + 512 b of its slot.)
   // (The per-lane values of both sides are derived from the lane number again
   // at the start of every tile, see derive_lane_values below.)
-  uint32_t fill_row0 = 0;
-  int fill_chunk = 0;
-  constexpr uint32_t kRowsPerLoadStep = kKMajor ? 8 : 32;
+  uint32_t a_row_bytes = 0, b_row_bytes = 0;
+  uint32_t a_voff[Cfg::kLoads], b_voff[Cfg::kLoads];
+  const auto request_row = [](int q) -> uint32_t { return kKMajor ? 16 * (q / 2) + 4 * (q % 2) : 32 * q; };
   // M0 takes the LDS byte address relative to the workgroup's allocation.
   typedef __attribute__((address_space(3))) uint8_t* lds_address;
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_address)lds_bytes));
@@ -135,15 +144,12 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
         q.B + batch * q.sB + static_cast<int64_t>(tn) * Cfg::BN * (kKMajor ? 1 : q.ldb)));
   };
   // Request q of an operand's k-tile at `src` into the ring slot at `slot`.
-  // The part of the address that depends on q goes into the scalar base, so
-  // that one lane offset per operand serves all eight.
-  auto issue_one = [&](const uint8_t* src, uint32_t row_bytes, int slot, int q) {
-    dma_load_16(fill_row0 * row_bytes + fill_chunk * 16, src + static_cast<uint64_t>(kRowsPerLoadStep * q) * row_bytes,
-                slot + fill_lds, q * 4096);
+  auto issue_one = [&](const uint8_t* src, const uint32_t (&voff)[Cfg::kLoads], int slot, int q) {
+    dma_load_16(voff[q], src, slot + fill_lds, q * 4096);
   };
-  auto issue_operand = [&](const uint8_t* src, uint32_t row_bytes, int slot, int count) {
+  auto issue_operand = [&](const uint8_t* src, const uint32_t (&voff)[Cfg::kLoads], int slot) {
 #pragma unroll
-    for (int q = 0; q < count; ++q) issue_one(src, row_bytes, slot, q);
+    for (int q = 0; q < Cfg::kLoads; ++q) issue_one(src, voff, slot, q);
   };
 
   // Operand pointer of k-tile kt: 128 bytes along the rows, or 64 rows down.
@@ -151,16 +157,17 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
     return kKMajor ? base + kt * (static_cast<int64_t>(Cfg::BK) * row_bytes) : base + kt * Cfg::kRowBytes;
   };
 
-  // Fragment side.  Lane l reads row l & 31 of a 32-row block, k chunk
-  // 2 ks + (l >> 5); its slot is that chunk XOR ((row >> 1) & 7), i.e. the
-  // ks = 0 address with bits 5..6 flipped by ks.
+  // Fragment side.  Lane l reads row l & 15 of a 16-row block, k chunk
+  // 4 ks + (l >> 4); its slot is that chunk XOR ((row >> 1) & 7), i.e. the
+  // ks = 0 address with bit 6 flipped by ks.
   uint32_t a_frag[KS], b_frag[KS];
-  // k-major fragments: lane l = 16 g + t of a wave serves output row
-  // 16 (g & 1) + t of a 32-row block and the k octet g >> 1 of a k step; it
-  // passes the address of columns 4 (t & 3) .. + 3 of k-row (t >> 2) of its
-  // octet's first half, then of its second half (4 rows = 2048 bytes down).
-  // The block index enters the slot through the swizzle: i ^ (k-row & 3).
-  uint32_t a_frag_km[TM], b_frag_km[TN];
+  // k-major fragments: lane l = 16 g + t of a wave serves output row t of a
+  // 16-row block and the k octet g of a k step; it passes the address of
+  // columns 4 (t & 3) .. + 3 of k-row (t >> 2) of its octet's first half, then
+  // of its second half (4 rows = 4096 bytes on).  The block index enters the
+  // slot through the swizzle: chunk ^ 4 (k-row & 3) ^ 2 (octet & 1), one address
+  // per block in the upper bits (i ^ (k-row & 3)) and two in the lower one.
+  uint32_t a_frag_km[TM / 2][2], b_frag_km[TN / 2][2];
   // All per-lane addresses of the k loop, from the lane number.  Called with
   // a lane number the compiler cannot see through at the start of every tile:
   // the values then live from there to the end of the k loop only.  Kept
@@ -168,46 +175,56 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   // spilled some of them and reloaded them inside the k loop, and a reload is
   // a vector memory load: the wait for it also waited for every operand
   // request in flight.
+  const auto opaque = [](int l) {
+    asm volatile("" : "+v"(l));
+    return l;
+  };
   auto derive_lane_values = [&](int l) {
-    const int fill_row = kKMajor ? l >> 5 : l >> 3;
-    fill_row0 = static_cast<uint32_t>((kKMajor ? 2 : 8) * wave + fill_row);
-    fill_chunk = kKMajor ? (l & 31) ^ (4 * static_cast<int>(fill_row0 & 3)) : (l & 7) ^ static_cast<int>((fill_row0 >> 1) & 7);
-    const int frag_row = l & 31;
-    const uint32_t frag_base = static_cast<uint32_t>(frag_row * Cfg::kRowBytes + (((l >> 5) ^ ((frag_row >> 1) & 7)) * 16));
+    const uint32_t fill_row = kKMajor ? wave + 8 * (l >> 5) : 8 * wave + (l >> 3);
+    // (k-row & 3 of a k-major request is the wave's number)
+    const uint32_t fill_chunk = kKMajor ? (l & 31) ^ (4 * wave) ^ (2 * (l >> 5)) : (l & 7) ^ ((fill_row >> 1) & 7);
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      a_frag[ks] = (frag_base ^ (ks * 32)) + wm * Cfg::kWaveM * Cfg::kRowBytes;
-      b_frag[ks] = (frag_base ^ (ks * 32)) + wn * Cfg::kWaveN * Cfg::kRowBytes;
+    for (int q = 0; q < Cfg::kLoads; ++q) {
+      a_voff[q] = (fill_row + request_row(q)) * a_row_bytes + fill_chunk * 16;
+      b_voff[q] = (fill_row + request_row(q)) * b_row_bytes + fill_chunk * 16;
     }
     const int t = l & 15, g = l >> 4;
-    const uint32_t common = static_cast<uint32_t>(((g >> 1) * 8 + (t >> 2)) * 512 + (g & 1) * 32 + (t & 3) * 8);
+    const uint32_t frag_base = static_cast<uint32_t>(t * Cfg::kRowBytes + ((g ^ ((t >> 1) & 7)) * 16));
 #pragma unroll
-    for (int i = 0; i < TM; ++i) a_frag_km[i] = common + wm * 256 + ((i ^ (t >> 2)) * 64);
+    for (int ks = 0; ks < KS; ++ks) {
+      a_frag[ks] = (frag_base ^ (ks * 64)) + wm * Cfg::kWaveM * Cfg::kRowBytes;
+      b_frag[ks] = (frag_base ^ (ks * 64)) + wn * Cfg::kWaveN * Cfg::kRowBytes;
+    }
+    const uint32_t common = static_cast<uint32_t>((g >> 1) * 8192 + (t >> 2) * 1024 + (g & 1) * 512 + (t & 3) * 8);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) b_frag_km[j] = common + wn * 256 + ((j ^ (t >> 2)) * 64);
+    for (int i = 0; i < TM / 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) a_frag_km[i][e] = common + wm * 256 + ((i ^ (t >> 2)) * 64) + ((e ^ (g & 1)) * 32);
+#pragma unroll
+    for (int j = 0; j < TN / 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) b_frag_km[j][e] = common + wn * 256 + ((j ^ (t >> 2)) * 64) + ((e ^ (g & 1)) * 32);
   };
-  derive_lane_values(lane);
-
-  f32x16 acc[TM][TN];
+  f32x4 acc[TM][TN];
   bf16x8 af[2][TM], bf[2][TN];
   auto read_transposed = [&](uint32_t offset) -> bf16x8 {
     typedef short i16x4 __attribute__((__vector_size__(4 * sizeof(short))));
     typedef __attribute__((address_space(3))) i16x4* lds_i16x4;
     const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)(lds_bytes + offset));
-    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)(lds_bytes + offset + 2048));
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)(lds_bytes + offset + 4096));
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
   auto read_a = [&](int set, int slot, int ks, int i) {
     if (kKMajor)
-      af[set][i] = read_transposed(slot + a_frag_km[i] + ks * 8192);
+      af[set][i] = read_transposed(slot + a_frag_km[i / 2][i % 2] + ks * 16384);
     else
-      af[set][i] = *reinterpret_cast<const bf16x8*>(lds_bytes + slot + a_frag[ks] + i * 32 * Cfg::kRowBytes);
+      af[set][i] = *reinterpret_cast<const bf16x8*>(lds_bytes + slot + a_frag[ks] + i * 16 * Cfg::kRowBytes);
   };
   auto read_b = [&](int set, int slot, int ks, int j) {
     if (kKMajor)
-      bf[set][j] = read_transposed(slot + b_frag_km[j] + ks * 8192);
+      bf[set][j] = read_transposed(slot + b_frag_km[j / 2][j % 2] + ks * 16384);
     else
-      bf[set][j] = *reinterpret_cast<const bf16x8*>(lds_bytes + slot + b_frag[ks] + j * 32 * Cfg::kRowBytes);
+      bf[set][j] = *reinterpret_cast<const bf16x8*>(lds_bytes + slot + b_frag[ks] + j * 16 * Cfg::kRowBytes);
   };
   // Fragment g of k step ks: the TM of operand A, then the TN of B.
   auto read_frag = [&](int set, int a_slot, int b_slot, int ks, int g) {
@@ -215,15 +232,8 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
     else read_b(set, b_slot, ks, g - TM);
   };
   auto mfma = [&](int set, int i, int j) {
-    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[set][j], af[set][i], acc[i][j], 0, 0, 0);
+    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[set][j], af[set][i], acc[i][j], 0, 0, 0);
   };
-  // The first k step of a tile starts its accumulators from a zero operand
-  // instead of from 256 cleared registers.
-  auto mfma_from_zero = [&](int set, int i, int j) {
-    const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[set][j], af[set][i], zero, 0, 0, 0);
-  };
-
   // Current tile: plain scalars, reassigned per tile.
   int which = 0, tm = 0, tn = 0;
   int64_t batch = 0;
@@ -237,71 +247,71 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   }
   const uint8_t* Ab = a_base(which, batch, tm);
   const uint8_t* Bb = b_base(which, batch, tn);
-  uint32_t a_row_bytes = static_cast<uint32_t>(launch.problem[which].lda * 2);
-  uint32_t b_row_bytes = static_cast<uint32_t>(launch.problem[which].ldb * 2);
+  a_row_bytes = static_cast<uint32_t>(launch.problem[which].lda * 2);
+  b_row_bytes = static_cast<uint32_t>(launch.problem[which].ldb * 2);
   FSH_STAMP(1);
-  issue_operand(Ab, a_row_bytes, 0, Cfg::kLoads);
-  issue_operand(Bb, b_row_bytes, Cfg::kOperandBytes, Cfg::kLoads);
+  derive_lane_values(lane);
+  issue_operand(Ab, a_voff, 0);
+  issue_operand(Bb, b_voff, Cfg::kOperandBytes);
 
 #ifdef FSH_TRACE
   uint64_t trace_wait = 0, trace_barrier = 0, trace_ktiles = 0, trace_tile_wait = 0, trace_tile_barrier = 0, trace_tiles = 0, trace_kloop = 0, trace_epi = 0, trace_steps = 0, trace_last = 0, trace_mark = 0;
   const uint64_t trace_begin = __builtin_amdgcn_s_memtime();
 #endif
-  // The k loop.  What bounds it: the request path of a compute unit takes one
-  // of the 64 requests of a k-tile (16 per wave) per 16 cycles, so they need
-  // half of the 2048 cycles of the MFMAs, and a wave that issues a request
-  // into a busy path cannot issue MFMAs.  Packed into two of the four k steps,
-  // as two 64 KB stages ask for (a stage is free only once the k-tile in it
-  // has been read), they cost 500 of the 3000 cycles a k-tile took, and the
-  // wait for the last ones up to 460.  The ring holds two and a half k-tiles
-  // instead: operand n of the sequence A(0), B(0), A(1), B(1), ... lives in
-  // slot n % 5, so A is requested two k-tiles ahead while both operands of the
-  // next one are still on their way, and every k step carries four requests of
-  // a wave, one per four MFMAs.
+  // The k loop.  What bounds it: power, then the issue slots of the one wave
+  // per SIMD.  The request path of a compute unit takes one of the 64 requests
+  // of a k-tile (16 per wave) per 16 cycles, so they need half of the 2048
+  // cycles of the MFMAs, and a wave that issues a request into a busy path
+  // cannot issue MFMAs.  Packed into half of the k-tile, as two 64 KB stages
+  // ask for (a stage is free only once the k-tile in it has been read), they
+  // cost 500 of the 3000 cycles a k-tile took, and the wait for the last ones
+  // up to 460.  The ring holds two and a half k-tiles instead: operand n of the
+  // sequence A(0), B(0), A(1), B(1), ... lives in slot n % 5, so A is requested
+  // two k-tiles ahead while both operands of the next one are still on their
+  // way, and a request goes out every eighth MFMA.
   //
   // The barrier that hands over k-tile kt + 1 sits before the last k step of
   // kt: that step's MFMAs cover the first fragment reads of kt + 1, and the
   // slots of kt are free (every wave holds its last fragments in registers).
-  //   k step 0:     requests 4-7 of B(kt + 1)
-  //   k steps 1, 2: A(kt + 2) into the fifth slot
+  //   k step 0:     A(kt + 2) into the fifth slot
   //   wait for all but A(kt + 2), barrier
-  //   k step 3:     requests 0-3 of B(kt + 2) into the slot of A(kt)
+  //   k step 1:     B(kt + 2) into the slot of A(kt)
   // Each step reads the next one's fragments.
-  // Us before / after (two stages / ring): 24 x 7168 x 2048, k 2048 1327 / 1185;
-  // the same, k-major and symmetric, k 7168 786 / 728; 8192^3 901 / 821; 4096^3
-  // 108 / 102.  Eight requests behind the barrier and the rest in any split
-  // over the other steps, or all four of a step at once: the same or 2 % slower.
-  constexpr int kPerStep = 2 * Cfg::kLoads / KS;
-  static_assert(KS == 4 && Cfg::kLoads == 2 * kPerStep, "the sequence above");
+  //
+  // 16x16x32 MFMAs read and write half as many accumulators per product as
+  // 32x32x16 ones and draw less power for it: the part then runs this loop at
+  // 1.84 instead of 1.67 GHz.
+  // Us with two stages and 32x32x16 / ring / ring and 16x16x32:
+  //   24 x 7168 x 2048, k 2048 1327 / 1190 / 1115    8192^3 901 / 821 / 755   4096^3 108 / 104 / 93
+  //   24 x 2048 x 2048, k 7168, k-major and symmetric 786 / 728 / 712
+  // Where in its step a request or a read goes out, and the order of the
+  // MFMAs, matter by 1 %: two rows of blocks at a time is the best by that.
+  constexpr int kMfmas = TM * TN, kReadEvery = 2;  // a fragment read behind every second MFMA
+  static_assert(KS == 2, "the sequence above");
   const auto next_slot = [](int slot) { return slot + Cfg::kOperandBytes == Cfg::kRingBytes ? 0 : slot + Cfg::kOperandBytes; };
   int a_slot = 0;  // of the current k-tile's operand A
-  // more: k-tile kt + 1 exists; more2: kt + 2 exists; zero: k-tile 0 of an output tile
-  auto k_tile = [&](int64_t kt, auto more_tag, auto more2_tag, auto zero_tag) {
-    constexpr bool more = decltype(more_tag)::value, more2 = decltype(more2_tag)::value, zero = decltype(zero_tag)::value;
+  // more: k-tile kt + 1 exists; more2: kt + 2 exists
+  auto k_tile = [&](int64_t kt, auto more_tag, auto more2_tag) {
+    constexpr bool more = decltype(more_tag)::value, more2 = decltype(more2_tag)::value;
     const int b_slot = next_slot(a_slot), a_next = next_slot(b_slot), b_next = next_slot(a_next), a_after = next_slot(b_next);
-    const uint8_t* b_src1 = k_tile_ptr(Bb, b_row_bytes, kt + 1);
     const uint8_t* a_src2 = k_tile_ptr(Ab, a_row_bytes, kt + 2);
     const uint8_t* b_src2 = k_tile_ptr(Bb, b_row_bytes, kt + 2);
     // MFMA g of k step ks with what goes out behind it.
     auto slice = [&](int ks, int g) {
-      if (zero && ks == 0) mfma_from_zero(0, g / TN, g % TN);
-      else mfma(ks & 1, g / TN, g % TN);
-      if (g < TM + TN) {
-        if (ks + 1 < KS) read_frag((ks + 1) & 1, a_slot, b_slot, ks + 1, g);
-        else if (more) read_frag(0, a_next, b_next, 0, g);
+      mfma(ks, g / (2 * TN) * 2 + g % 2, g % (2 * TN) / 2);
+      if (g % kReadEvery == kReadEvery - 1 && g / kReadEvery < TM + TN) {
+        if (ks == 0) read_frag(1, a_slot, b_slot, 1, g / kReadEvery);
+        else if (more) read_frag(0, a_next, b_next, 0, g / kReadEvery);
       }
-      if ((g + 1) % (TM * TN / kPerStep) == 0) {
-        const int r = g / (TM * TN / kPerStep);
-        if (ks == 0 && more) issue_one(b_src1, b_row_bytes, b_next, kPerStep + r);
-        if ((ks == 1 || ks == 2) && more2) issue_one(a_src2, a_row_bytes, a_after, (ks - 1) * kPerStep + r);
-        if (ks == 3 && more2) issue_one(b_src2, b_row_bytes, a_slot, r);
+      if ((g + 1) % (kMfmas / Cfg::kLoads) == 0 && more2) {
+        const int r = g / (kMfmas / Cfg::kLoads);
+        if (ks == 0) issue_one(a_src2, a_voff, a_after, r);
+        else issue_one(b_src2, b_voff, a_slot, r);
       }
       __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll
-    for (int ks = 0; ks + 1 < KS; ++ks)
-#pragma unroll
-      for (int g = 0; g < TM * TN; ++g) slice(ks, g);
+    for (int g = 0; g < kMfmas; ++g) slice(0, g);
 #ifdef FSH_TRACE
     const uint64_t tr0 = __builtin_amdgcn_s_memtime();
     trace_steps += tr0 - trace_mark;
@@ -320,7 +330,7 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
     trace_ktiles += 1;
 #endif
 #pragma unroll
-    for (int g = 0; g < TM * TN; ++g) slice(KS - 1, g);
+    for (int g = 0; g < kMfmas; ++g) slice(1, g);
     a_slot = a_next;
 #ifdef FSH_TRACE
     trace_mark = __builtin_amdgcn_s_memtime();
@@ -331,12 +341,11 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   while (true) {
     const GemmParams& p = launch.problem[which];
     const int64_t ktiles = p.K / Cfg::BK;
-    {
-      int lane_again = lane;
-      asm volatile("" : "+v"(lane_again));
-      derive_lane_values(lane_again);
-    }
+    derive_lane_values(opaque(lane));
     FSH_STAMP(6);
+    // Under the wait for the first operands and for the previous tile's stores.
+#pragma unroll
+    for (int g = 0; g < kMfmas; ++g) clear_accumulators(acc[g / TN][g % TN]);
 #ifdef FSH_TRACE
     const uint64_t ts0 = __builtin_amdgcn_s_memtime();
 #endif
@@ -357,24 +366,16 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
 #pragma unroll
     for (int g = 0; g < TM + TN; ++g) read_frag(0, 0, Cfg::kOperandBytes, 0, g);
     if (ktiles > 1) {
-      issue_operand(k_tile_ptr(Ab, a_row_bytes, 1), a_row_bytes, 2 * Cfg::kOperandBytes, Cfg::kLoads);
-      issue_operand(k_tile_ptr(Bb, b_row_bytes, 1), b_row_bytes, 3 * Cfg::kOperandBytes, kPerStep);
+      issue_operand(k_tile_ptr(Ab, a_row_bytes, 1), a_voff, 2 * Cfg::kOperandBytes);
+      issue_operand(k_tile_ptr(Bb, b_row_bytes, 1), b_voff, 3 * Cfg::kOperandBytes);
     }
     FSH_STAMP(2);
 
     constexpr std::true_type yes{};
     constexpr std::false_type no{};
-    if (ktiles > 2) {
-      k_tile(0, yes, yes, yes);
-      for (int64_t kt = 1; kt + 2 < ktiles; ++kt) k_tile(kt, yes, yes, no);
-    } else {
-#pragma unroll
-      for (int g = 0; g < TM * TN; ++g)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[g / TN][g % TN][r] = 0.0f;
-    }
-    if (ktiles > 1) k_tile(ktiles - 2, yes, no, no);
-    k_tile(ktiles - 1, no, no, no);
+    for (int64_t kt = 0; kt + 2 < ktiles; ++kt) k_tile(kt, yes, yes);
+    if (ktiles > 1) k_tile(ktiles - 2, yes, no);
+    k_tile(ktiles - 1, no, no);
     FSH_STAMP(3);
 #ifdef FSH_TRACE
     trace_kloop += __builtin_amdgcn_s_memtime() - tk0;
@@ -394,15 +395,16 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
         Bb = b_base(next_which, next_batch, next_tn);
         a_row_bytes = static_cast<uint32_t>(launch.problem[next_which].lda * 2);
         b_row_bytes = static_cast<uint32_t>(launch.problem[next_which].ldb * 2);
-        issue_operand(Ab, a_row_bytes, 0, Cfg::kLoads);
-        issue_operand(Bb, b_row_bytes, Cfg::kOperandBytes, Cfg::kLoads);
+        derive_lane_values(opaque(lane));
+        issue_operand(Ab, a_voff, 0);
+        issue_operand(Bb, b_voff, Cfg::kOperandBytes);
       }
     }
 #ifdef FSH_TRACE
     const uint64_t te0 = __builtin_amdgcn_s_memtime();
 #endif
     store_tile_in_halves<Cfg>(p, batch, static_cast<int64_t>(tm) * Cfg::BM, static_cast<int64_t>(tn) * Cfg::BN, wm,
-                              wn, lane, p.symmetric && tm != tn, acc, lds_bytes + kDmaGemmStaging);
+                              wn, opaque(lane), p.symmetric && tm != tn, acc, lds_bytes + kDmaGemmStaging);
 #ifdef FSH_TRACE
     trace_epi += __builtin_amdgcn_s_memtime() - te0;
 #endif
@@ -444,10 +446,10 @@ struct PlannedGemm {
 // ---- Which tiles a launch takes.
 // Measured over 13 shapes from 512^2 to 8192 x 6144 at k = 512 and 2048 (us for
 // k = 512 / 2048, tiles of 64 x 64, 128 x 128, 256 x 128, 256 x 256; k-tiles of 64):
-//   1024 x 1024     5.5 / 10.4    8.1 / 17.4   10.2 / 25.4   15.5 / 38.7
-//   2048 x 2048    11.5 / 30.6    9.7 / 22.7   11.6 / 28.0   16.8 / 42.8
-//   4096 x 2048    18.8 / 55.6   15.5 / 40.0   14.9 / 36.5   19.3 / 45.8
-//   4096 x 4096    35.9 / 108.5  27.3 / 80.5   28.0 / 74.6   22.9 / 61.7
+//   1024 x 1024     5.5 / 10.4    8.1 / 17.4   10.2 / 25.4   16.3 / 38.9
+//   2048 x 2048    11.5 / 30.6    9.7 / 22.7   11.6 / 28.0   17.2 / 40.6
+//   4096 x 2048    18.8 / 55.6   15.5 / 40.0   14.9 / 36.5   18.8 / 43.4
+//   4096 x 4096    35.9 / 108.5  27.3 / 80.5   28.0 / 74.6   22.4 / 53.3
 enum TileKind { kTiles64, kTiles128, kTiles128Deep, kTiles256x128, kTiles256 };  // the order of kTileShapes
 constexpr int kTileNames[] = {FSH_TILES_64, FSH_TILES_128, FSH_TILES_128_DEEP, FSH_TILES_256X128, FSH_TILES_256};
 constexpr TileShape kTileShapes[] = {
