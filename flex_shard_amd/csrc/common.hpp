@@ -63,6 +63,32 @@ __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
   return (f != f) ? 0x7FC0u : r;
 }
 
+// The bits of f32_to_bf16_bits for eight floats, packed in pairs: one
+// v_cvt_pk_bf16_f32 per pair, which rounds alike and differs in NaNs alone (it
+// keeps their sign and payload); they are looked for once per eight.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+// Each bf16 half that is a NaN becomes 0x7FC0.
+__device__ __forceinline__ uint32_t canonical_nan_pair(uint32_t w) {
+  if ((w & 0x7FFFu) > 0x7F80u) w = (w & 0xFFFF0000u) | 0x7FC0u;
+  if ((w & 0x7FFF0000u) > 0x7F800000u) w = (w & 0xFFFFu) | 0x7FC00000u;
+  return w;
+}
+__device__ __forceinline__ u32x4 pack8_bf16(const float (&f)[8]) {
+  u32x4 w;
+  bool nan = false;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    w[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{f[2 * j], f[2 * j + 1]}), bf16x2));
+    nan |= __builtin_isunordered(f[2 * j], f[2 * j + 1]) != 0;
+  }
+  if (nan) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = canonical_nan_pair(w[j]);
+  }
+  return w;
+}
+
 // float -> fp16 bits, round to nearest even over the whole range, subnormal
 // results included, in integer arithmetic plus one fp32 add: the hardware
 // conversion rounded exact ties of subnormal results away from zero (e.g.

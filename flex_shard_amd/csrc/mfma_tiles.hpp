@@ -154,11 +154,9 @@ __device__ inline void store_staged_rows(const uint8_t* region, uint16_t* dst, i
 
 // Two floats -> packed bf16 pair (low half = first), round to nearest even:
 // one v_cvt_pk_bf16_f32 on gfx950.
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  const f32x2_t v = {lo, hi};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+  const f32x2 v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
 // Half of a wave's D tile (its upper or lower kWaveM/2 rows), loaded the way

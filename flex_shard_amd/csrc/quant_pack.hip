@@ -321,22 +321,64 @@ struct QuantFastParams {
   uint8_t* payload;
   int64_t zero_begin[2];
   int64_t zero_len[2];
+  uint32_t ragged;  // bit i: chunk i (quantize_pack_ragged_kernel)
 };
 
 // Two floats -> two bf16 in one word (low half first), round to nearest even:
 // one v_cvt_pk_bf16_f32.  Finite values and infinities get the bits of
-// f32_to_bf16_bits; a NaN keeps its sign and payload (see canonical_nan_pair).
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
+// f32_to_bf16_bits; a NaN keeps its sign and payload (see canonical_nan_pair, which gives it the canonical one).
 __device__ __forceinline__ uint32_t round_pair_to_bf16(float lo, float hi) {
-  const f32x2_t pair = {lo, hi};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2_t));
+  const f32x2 pair = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2));
 }
-// Each bf16 half that is a NaN becomes 0x7FC0, what f32_to_bf16_bits gives.
-__device__ __forceinline__ uint32_t canonical_nan_pair(uint32_t w) {
-  if ((w & 0x7FFFu) > 0x7F80u) w = (w & 0xFFFF0000u) | 0x7FC0u;
-  if ((w & 0x7FFF0000u) > 0x7F800000u) w = (w & 0xFFFFu) | 0x7FC00000u;
-  return w;
+// Eight elements of a row and their eight bytes.  `n` of them exist (eight but
+// for the last group of a width that is no multiple of eight); RAGGED ones are
+// aligned to the element only, which global memory instructions may be.
+template <bool RAGGED>
+__device__ __forceinline__ u32x4 load_bf16_group(const uint8_t* p, uint32_t n) {
+  if (!RAGGED) return load_stream_u32x4(p);
+  u32x4 v = {0, 0, 0, 0};
+  if (n >= 8) {
+    __builtin_memcpy(&v, p, sizeof(v));
+    return v;
+  }
+  const uint16_t* e = reinterpret_cast<const uint16_t*>(p);
+#pragma unroll
+  for (uint32_t j = 0; j < 7; ++j)
+    if (j < n) v[j >> 1] |= static_cast<uint32_t>(e[j]) << (16 * (j & 1));
+  return v;
+}
+template <bool RAGGED>
+__device__ __forceinline__ void load_f32_group(const uint8_t* p, uint32_t n, f32x4* a, f32x4* b) {
+  if (!RAGGED) {
+    *a = load_stream_f32x4(p);
+    *b = load_stream_f32x4(p + 16);
+    return;
+  }
+  if (n >= 8) {
+    __builtin_memcpy(a, p, sizeof(*a));
+    __builtin_memcpy(b, p + 16, sizeof(*b));
+    return;
+  }
+  const float* e = reinterpret_cast<const float*>(p);
+#pragma unroll
+  for (uint32_t j = 0; j < 7; ++j)
+    if (j < n) (j < 4 ? *a : *b)[j & 3] = e[j];
+}
+template <bool RAGGED>
+__device__ __forceinline__ void store_fp8_group(uint8_t* p, uint32_t n, uint32_t lo, uint32_t hi) {
+  if (!RAGGED) {
+    store_stream_u32x2(p, lo, hi);
+    return;
+  }
+  if (n >= 8) {
+    const u32x2 v = {lo, hi};
+    __builtin_memcpy(p, &v, sizeof(v));  // (a plain store: the caches put the pieces of a line together)
+    return;
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < 7; ++j)
+    if (j < n) p[j] = static_cast<uint8_t>((j < 4 ? lo : hi) >> (8 * (j & 3)));
 }
 
 // F32: the shard is an fp32 master; every element is rounded to bf16 as it is
@@ -344,7 +386,8 @@ __device__ __forceinline__ uint32_t canonical_nan_pair(uint32_t w) {
 // rows at a time: 79 registers and six workgroups per compute unit instead of
 // 91 and five with all sixteen loads in flight (forced to 72 or 64 registers
 // the compiler spills and the launch is 4 % slower).
-template <bool FULL, bool F32>
+// RAGGED: rows start anywhere and end inside a group of eight.
+template <bool FULL, bool F32, bool RAGGED = false>
 __device__ __forceinline__ void quant_tile128_fast(const FastChunk& ch, uint32_t tr, uint32_t tc, float eps,
                                                    uint32_t* lds) {
   const uint32_t tid = threadIdx.x;
@@ -353,6 +396,7 @@ __device__ __forceinline__ void quant_tile128_fast(const FastChunk& ch, uint32_t
   const uint32_t col = tc * 128u + g * 8u;
   const bool col_ok = FULL || col < static_cast<uint32_t>(ch.in_dim);
   const uint32_t rows = static_cast<uint32_t>(ch.rows);
+  const uint32_t n = FULL || !RAGGED ? 8 : static_cast<uint32_t>(ch.in_dim) - col;  // elements left in the row (if col_ok)
   const int64_t src_row_bytes = ch.src_row_bytes;
   const int64_t dst_row_bytes = ch.in_dim;
   const uint8_t* sp = ch.src + static_cast<int64_t>(row0) * src_row_bytes + static_cast<int64_t>(col) * (F32 ? 4 : 2);
@@ -364,10 +408,10 @@ __device__ __forceinline__ void quant_tile128_fast(const FastChunk& ch, uint32_t
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       if (FULL) {
-        v[k] = load_stream_u32x4(sp + 16 * k * src_row_bytes);
+        v[k] = load_bf16_group<RAGGED>(sp + 16 * k * src_row_bytes, 8);
       } else {
         v[k] = u32x4{0, 0, 0, 0};
-        if (col_ok && row0 + 16u * k < rows) v[k] = load_stream_u32x4(sp + 16 * k * src_row_bytes);
+        if (col_ok && row0 + 16u * k < rows) v[k] = load_bf16_group<RAGGED>(sp + 16 * k * src_row_bytes, n);
       }
     }
   } else {
@@ -380,8 +424,7 @@ __device__ __forceinline__ void quant_tile128_fast(const FastChunk& ch, uint32_t
         a[j] = f32x4{0.f, 0.f, 0.f, 0.f};
         b[j] = a[j];
         if (FULL || (col_ok && row0 + 16u * k < rows)) {
-          a[j] = load_stream_f32x4(sp + 16 * k * src_row_bytes);
-          b[j] = load_stream_f32x4(sp + 16 * k * src_row_bytes + 16);
+          load_f32_group<RAGGED>(sp + 16 * k * src_row_bytes, n, &a[j], &b[j]);
         }
       }
 #pragma unroll
@@ -439,7 +482,7 @@ __device__ __forceinline__ void quant_tile128_fast(const FastChunk& ch, uint32_t
         const float e1 = u32_as_f32(d[j] & 0xFFFF0000u) * scale;
         w[j >> 1] = cvt2_fp8(e0, e1, w[j >> 1], (j & 1) != 0);
       }
-      store_stream_u32x2(dp + 16 * k * dst_row_bytes, w[0], w[1]);
+      store_fp8_group<RAGGED>(dp + 16 * k * dst_row_bytes, n, w[0], w[1]);
     }
   }
 }
@@ -492,6 +535,42 @@ __global__ __launch_bounds__(kThreads) void quantize_pack_f32_master_kernel(cons
     quant_tile128_fast<false, true>(ch, tr, tc, prm.eps, lds);
 }
 
+// The launch when some chunk's rows are not 16-byte friendly: an odd width, a
+// shard or a payload position off the vector grid.  Such a tile's accesses go
+// out unaligned and its rows begin and end inside memory lines that the tiles
+// beside it share, so each XCD takes a contiguous run of tiles: neighbours
+// then meet in its L2.  The element-wise path, which used to take every chunk of
+// such a launch: 8.2 M elements in five chunks, one of width 343, 47.7 us, here
+// 10.8; 31 M in two of 2605 and 2816 columns among five 82 -> 22 us.
+template <int N, bool F32>
+__global__ __launch_bounds__(kThreads) void quantize_pack_ragged_kernel(const QuantFastParams<N> prm, int32_t tiles_per_xcd) {
+  __shared__ uint32_t lds[4];
+  const int32_t first_pad = 8 * tiles_per_xcd;  // workgroup ids go round-robin to the 8 XCDs
+  int32_t tile = static_cast<int32_t>(blockIdx.x);
+  if (tile >= first_pad) {
+    zero_pad_slice(prm.payload, prm.zero_begin, prm.zero_len, tile - first_pad);
+    return;
+  }
+  tile = (tile & 7) * tiles_per_xcd + (tile >> 3);
+  int c = 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) c += tile >= prm.next_begin[i] ? 1 : 0;
+  if (c >= prm.nchunks) return;
+  const FastChunk ch = prm.chunks[c];
+  const uint32_t t = static_cast<uint32_t>(tile - ch.tile_begin);
+  const uint32_t tr = t / static_cast<uint32_t>(ch.tiles_c);
+  const uint32_t tc = t - tr * static_cast<uint32_t>(ch.tiles_c);
+  const bool full = (tr + 1) * 128u <= static_cast<uint32_t>(ch.rows) &&
+                    (tc + 1) * 128u <= static_cast<uint32_t>(ch.in_dim);
+  if ((prm.ragged >> c & 1) == 0) {
+    if (full) quant_tile128_fast<true, F32>(ch, tr, tc, prm.eps, lds);
+    else quant_tile128_fast<false, F32>(ch, tr, tc, prm.eps, lds);
+  } else {
+    if (full) quant_tile128_fast<true, F32, true>(ch, tr, tc, prm.eps, lds);
+    else quant_tile128_fast<false, F32, true>(ch, tr, tc, prm.eps, lds);
+  }
+}
+
 template <int N, bool F32>
 void launch_bf16_kernel(const QuantParams& prm, int64_t tiles, int64_t grid, hipStream_t stream) {
   QuantFastParams<N> fast;
@@ -521,7 +600,12 @@ void launch_bf16_kernel(const QuantParams& prm, int64_t tiles, int64_t grid, hip
   }
   fast.eps = prm.eps[F32 ? FSH_SRC_F32_AS_BF16 : FSH_SRC_BF16];
   fast.nchunks = nchunks;
-  if (F32)
+  for (int i = 0; i < nchunks; ++i) fast.ragged |= (prm.chunks[i].fast ? 0u : 1u) << i;
+  if (fast.ragged) {
+    const int64_t per_xcd = ceil_div(tiles, (int64_t)8);
+    hipLaunchKernelGGL((quantize_pack_ragged_kernel<N, F32>), dim3(static_cast<uint32_t>(8 * per_xcd + (grid - tiles))), dim3(kThreads),
+                       0, stream, fast, static_cast<int32_t>(per_xcd));
+  } else if (F32)
     hipLaunchKernelGGL(quantize_pack_f32_master_kernel<N>, dim3(static_cast<uint32_t>(grid)), dim3(kThreads), 0,
                        stream, fast);
   else
@@ -655,7 +739,8 @@ static int quantize_pack_impl(const fsh_quant_chunk* chunks, int32_t nchunks, vo
   prm.eps[FSH_SRC_F16] = prm.eps[FSH_SRC_F32_AS_F16] = eps_mode == FSH_EPS_FP32 ? eps32 : 0.0f;
 
   int64_t tiles = 0;
-  bool all_bf16_fast = true, all_f32_master_fast = true;
+  // one source kind, 128 x 128 tiles: the 32-bit kernels
+  bool all_bf16 = block == 128, all_f32_master = block == 128;
   for (int i = 0; i < nchunks; ++i) {
     const fsh_quant_chunk& in = chunks[i];
     if (in.src_dev == nullptr || in.rows <= 0 || in.in_dim <= 0 || in.src_row_stride < in.in_dim)
@@ -686,8 +771,8 @@ static int quantize_pack_impl(const fsh_quant_chunk* chunks, int32_t nchunks, vo
     out.fast = block == 128 && aligned(in.src_dev, 16) && (in.src_row_stride * elem) % 16 == 0 &&
                in.in_dim % 8 == 0 && in.qdata_offset % 8 == 0;
     const bool small = in.rows < (1LL << 30) && in.in_dim < (1LL << 30);
-    all_bf16_fast = all_bf16_fast && out.fast && in.src_kind == FSH_SRC_BF16 && small;
-    all_f32_master_fast = all_f32_master_fast && out.fast && in.src_kind == FSH_SRC_F32_AS_BF16 && small;
+    all_bf16 = all_bf16 && in.src_kind == FSH_SRC_BF16 && small;
+    all_f32_master = all_f32_master && in.src_kind == FSH_SRC_F32_AS_BF16 && small;
     tiles += tiles_r * tiles_c;
   }
   prm.total_tiles = tiles;
@@ -701,12 +786,12 @@ static int quantize_pack_impl(const fsh_quant_chunk* chunks, int32_t nchunks, vo
   if (grid == 0) return FSH_OK;
   if (grid > 0x7FFFFFFFLL) return fail(FSH_ENOTSUP, "fsh_quantize_pack: %lld workgroups exceed the grid limit", (long long)grid);
   if (!launch) return FSH_OK;
-  if (all_bf16_fast) {
+  if (all_bf16) {
     if (nchunks < 8)
       launch_bf16_kernel<8, false>(prm, tiles, grid, static_cast<hipStream_t>(stream));
     else
       launch_bf16_kernel<FSH_MAX_QUANT_CHUNKS, false>(prm, tiles, grid, static_cast<hipStream_t>(stream));
-  } else if (all_f32_master_fast && nchunks > 0) {
+  } else if (all_f32_master && nchunks > 0) {
     if (nchunks < 8)
       launch_bf16_kernel<8, true>(prm, tiles, grid, static_cast<hipStream_t>(stream));
     else
