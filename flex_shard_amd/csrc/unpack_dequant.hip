@@ -2,23 +2,22 @@
 // buffer fused with blockwise dequantization to bf16 (or fp32), one pass over
 // the FP8 bytes.
 //
-// A workgroup owns one block x block tile of one (rank, parameter) chunk.  For
-// block = 128 each thread moves 8 FP8 bytes per row pass: one 8-byte load, one
-// 8-byte store into the compact buffer, four v_cvt_pk_f32_fp8 + multiplies by
-// the tile's reciprocal scale, and one 16-byte bf16 store.  Where the width or
-// the addresses are not multiples of eight (an odd width; rank rows at odd
-// byte offsets inside a mixed bucket) the same accesses go out unaligned,
-// which global memory instructions may be, and only a row's last, partial
-// group of eight moves byte by byte.  Other block sizes take an element-wise
-// path.
+// A chunk is one contiguous run of bytes, and so are its compact bytes and its
+// dequantized values.  For block = 128 its T tiles' worth of workgroups split
+// that run into T consecutive pieces: eight FP8 bytes per thread and pass (one
+// 8-byte load, one 8-byte store into the compact buffer, four v_cvt_pk_f32_fp8
+// + multiplies by the tile's reciprocal scale, one 16-byte bf16 store), each
+// access contiguous across the wave whatever the width, the dequantized stores
+// whole memory lines.  Only the wider output's alignment is arranged; FP8
+// bytes at odd offsets (an odd width; rank rows inside a mixed bucket) go out
+// unaligned, which global memory instructions may be.  Bound by memory.  Other
+// block sizes and widths below eight take an element-wise path.
 #include "common.hpp"
 
 namespace fsh {
 namespace {
 
 constexpr int kThreads = 256;
-
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float load_f32_any(const uint8_t* p) {
   if ((reinterpret_cast<uintptr_t>(p) & 3) == 0) return *reinterpret_cast<const float*>(p);
@@ -49,8 +48,9 @@ __device__ __forceinline__ void dequant4(uint32_t w, float s, float* out) {
   out[3] = hi.y * s;
 }
 
-// `kAligned`: FP8 bytes and compact bytes of every group of eight on 8-byte,
-// dequantized values on 16-byte boundaries.
+// `kAligned`: FP8 bytes of every group of eight on 8-byte boundaries, and the
+// compact bytes of a piece from a memory line's start: they stream.  Pieces of
+// lines stay in the caches until the rest of the line is there.
 template <typename V, bool kAligned>
 __device__ __forceinline__ V load_group(const uint8_t* p) {
   // A plain load: with the nontemporal hint this kernel, three quarters of
@@ -69,14 +69,6 @@ __device__ __forceinline__ void store_group(uint8_t* p, const u32x2& v) {
   else
     __builtin_memcpy(p, &v, sizeof(v));
 }
-template <bool kAligned>
-__device__ __forceinline__ void store_group(uint8_t* p, const u32x4& v) {
-  if (kAligned)
-    store_stream_u32x4(p, v);
-  else
-    __builtin_memcpy(p, &v, sizeof(v));
-}
-
 template <int DQ>
 __device__ __forceinline__ void store_value(uint8_t* dq, int64_t idx, float f) {
   if (DQ == FSH_DT_BF16)
@@ -87,69 +79,115 @@ __device__ __forceinline__ void store_value(uint8_t* dq, int64_t idx, float f) {
     reinterpret_cast<float*>(dq)[idx] = f;
 }
 
-// One 128 x 128 tile.  16 threads per tile row, 8 FP8 bytes each: every load
-// and store instruction of a wave then covers whole contiguous row segments
-// (128 B of FP8, 256 B of bf16), which the memory pipeline needs for
-// full-width requests.  16 rows per pass, 8 passes, all loads issued up
-// front; rows past the chunk's end are clamped for the load and skipped for
-// the stores.
-template <int DQ, bool kAligned>
-__device__ __forceinline__ void unpack_tile(const uint8_t* src, uint8_t* cq, uint8_t* dq, int64_t rows, int64_t in_dim,
-                                            int64_t tr, int64_t tc, float scale, int tid) {
-  const int g = tid & 15, r0 = tid >> 4;
-  const int64_t col = tc * 128 + g * 8;
-  if (col >= in_dim) return;
-  if (!kAligned && col + 8 > in_dim) {  // the row's last bytes
-    for (int k = 0; k < 8; ++k) {
-      const int64_t row = tr * 128 + r0 + 16 * k;
-      if (row >= rows) break;
-      for (int64_t idx = row * in_dim + col; idx < (row + 1) * in_dim; ++idx) {
-        const uint8_t b = src[idx];
-        if (cq) cq[idx] = b;
-        if (dq) store_value<DQ>(dq, idx, __builtin_amdgcn_cvt_f32_fp8(static_cast<int>(b), 0) * scale);
-      }
-    }
+// a / b of a >= 0 and b > 0 that are the same in every lane (a 64-bit division
+// is a few hundred cycles ahead of a workgroup's first load).
+__device__ __forceinline__ int64_t divide(int64_t a, int64_t b) {
+  if (((a | b) >> 32) == 0) return static_cast<uint32_t>(a) / static_cast<uint32_t>(b);
+  return a / b;
+}
+
+// Eight dequantized values to dq[idx ..], 16-byte aligned.
+template <int DQ>
+__device__ __forceinline__ void store_values8(uint8_t* dq, uint32_t idx, const float (&f)[8]) {
+  if (DQ == FSH_DT_F32) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      store_stream_u32x4(dq + idx * 4 + 16 * j, u32x4{f32_as_u32(f[4 * j]), f32_as_u32(f[4 * j + 1]),
+                                                      f32_as_u32(f[4 * j + 2]), f32_as_u32(f[4 * j + 3])});
     return;
   }
-  u32x2 vin[8];
-  int64_t idxs[8];
+  u32x4 o;
+  if (DQ == FSH_DT_BF16) {
+    o = pack8_bf16(f);
+  } else {
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int64_t row = tr * 128 + r0 + 16 * k;
-    idxs[k] = (row < rows ? row : rows - 1) * in_dim + col;
-    vin[k] = load_group<u32x2, kAligned>(src + idxs[k]);
+    for (int j = 0; j < 4; ++j) o[j] = f32_to_f16_bits(f[2 * j]) | (f32_to_f16_bits(f[2 * j + 1]) << 16);
+  }
+  store_stream_u32x4(dq + idx * 2, o);
+}
+
+// Piece t of `tiles` of a chunk.  `scales`: the chunk's table [rows / 128][in_dim / 128].
+// With a tile's own 128 rows per workgroup, memory lines were written in pieces
+// wherever the width is no multiple of 128, and completed by workgroups on
+// other XCDs.  Us there / here: 25.5 M values of widths 3344 and 384 54 / 33,
+// 87 M of 2605 to 10112 83 / 59 (6.1 TB/s), 14 M of 1000 to 3000 28 / 17, the
+// eight rank rows of a 218 M layer 146 / 131 (6.7 TB/s), 67 M of 4096 on one
+// rank 44 / 46.
+template <int DQ, bool kAligned>
+__device__ __forceinline__ void unpack_piece(const uint8_t* src, uint8_t* cq, uint8_t* dq, const uint8_t* scales, int64_t rows,
+                                             int64_t in_dim, int64_t tiles_c, int64_t t, int64_t tiles, int64_t lead, int tid) {
+  constexpr int kElem = DQ == FSH_DT_F32 ? 4 : 2, kPasses = 8;
+  const int64_t n = rows * in_dim;
+  const bool scales_aligned = (reinterpret_cast<uintptr_t>(scales) & 3) == 0;  // (the same for the whole launch)
+  const auto scale_at = [&](int64_t row, uint32_t col) {
+    const uint8_t* p = scales + 4 * ((row >> 7) * tiles_c + (col >> 7));
+    return scales_aligned ? *reinterpret_cast<const float*>(p) : load_f32_any(p);
+  };
+  lead = lead < n ? lead : n;
+  const int64_t groups = (n - lead) / 8, per = (divide(groups + tiles - 1, tiles) + 15) / 16 * 16;
+  const int64_t edge = t == 0 && tid < lead ? tid : t == tiles - 1 && lead + 8 * groups + tid < n ? lead + 8 * groups + tid : -1;
+  if (edge >= 0) {  // (fewer than 128 elements in front, than eight behind; a chunk of one piece has both ends)
+    for (int64_t idx = edge; idx >= 0;) {
+      const uint8_t b = src[idx];
+      if (cq) cq[idx] = b;
+      const int64_t row = idx / in_dim;
+      if (dq) store_value<DQ>(dq, idx, __builtin_amdgcn_cvt_f32_fp8(static_cast<int>(b), 0) * scale_at(row, static_cast<uint32_t>(idx - row * in_dim)));
+      const int64_t last = lead + 8 * groups + tid;
+      idx = idx < lead && t == tiles - 1 && last < n ? last : -1;
+    }
+  }
+  const int64_t first = t * per, end = first + per < groups ? first + per : groups;  // per <= 2048: a tile has 16384 elements at most
+  const int64_t idx0 = lead + 8 * first, row0 = divide(idx0, in_dim);
+  const uint32_t width = static_cast<uint32_t>(in_dim), col0 = static_cast<uint32_t>(idx0 - row0 * in_dim);
+  const bool splits = (width & 7) != 0 || (col0 & 7) != 0;  // groups that reach into the next tile or row
+  const uint32_t count = first < end ? static_cast<uint32_t>(end - first) : 0;
+  src += idx0;
+  if (cq) cq += idx0;
+  if (dq) dq += idx0 * kElem;
+  u32x2 vin[kPasses];
+  uint32_t cols[kPasses], belows[kPasses];
+  float scale[kPasses];
+#pragma unroll
+  for (int k = 0; k < kPasses; ++k) {
+    const uint32_t g = k * kThreads + tid;
+    if (g >= count) break;
+    vin[k] = load_group<u32x2, kAligned>(src + 8 * g);
+    const uint32_t c = col0 + 8 * g;
+    belows[k] = c / width;
+    cols[k] = c - belows[k] * width;
+    if (dq) scale[k] = scale_at(row0 + belows[k], cols[k]);
   }
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    if (tr * 128 + r0 + 16 * k >= rows) break;
-    const int64_t idx = idxs[k];
-    const u32x2 v = vin[k];
-    if (cq) store_group<kAligned>(cq + idx, v);
-    if (dq) {
-      float f[8];
-      dequant4(v.x, scale, f);
-      dequant4(v.y, scale, f + 4);
-      if (DQ == FSH_DT_BF16) {
-        u32x4 o;
-        o.x = f32_to_bf16_bits(f[0]) | (f32_to_bf16_bits(f[1]) << 16);
-        o.y = f32_to_bf16_bits(f[2]) | (f32_to_bf16_bits(f[3]) << 16);
-        o.z = f32_to_bf16_bits(f[4]) | (f32_to_bf16_bits(f[5]) << 16);
-        o.w = f32_to_bf16_bits(f[6]) | (f32_to_bf16_bits(f[7]) << 16);
-        store_group<kAligned>(dq + idx * 2, o);
-      } else if (DQ == FSH_DT_F16) {
-        u32x4 o;
-        o.x = f32_to_f16_bits(f[0]) | (f32_to_f16_bits(f[1]) << 16);
-        o.y = f32_to_f16_bits(f[2]) | (f32_to_f16_bits(f[3]) << 16);
-        o.z = f32_to_f16_bits(f[4]) | (f32_to_f16_bits(f[5]) << 16);
-        o.w = f32_to_f16_bits(f[6]) | (f32_to_f16_bits(f[7]) << 16);
-        store_group<kAligned>(dq + idx * 2, o);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          store_group<kAligned>(dq + idx * 4 + 16 * j, u32x4{f32_as_u32(f[4 * j]), f32_as_u32(f[4 * j + 1]),
-                                                             f32_as_u32(f[4 * j + 2]), f32_as_u32(f[4 * j + 3])});
+  for (int k = 0; k < kPasses; ++k) {
+    const uint32_t g = k * kThreads + tid;
+    if (g >= count) break;
+    if (cq) store_group<kAligned>(cq + 8 * g, vin[k]);
+    if (!dq) continue;
+    float f[8];
+    if (!splits) {
+      dequant4(vin[k].x, scale[k], f);
+      dequant4(vin[k].y, scale[k], f + 4);
+    } else {
+      dequant4(vin[k].x, 1.0f, f);
+      dequant4(vin[k].y, 1.0f, f + 4);
+      // Of the group, `cut` elements belong to the first tile; what follows may
+      // cross one more edge (a column block's, then the row's).
+      const uint32_t in_row = width - cols[k], in_tile = 128 - (cols[k] & 127);
+      const uint32_t cut = in_row < in_tile ? in_row : in_tile;
+      float s1 = scale[k], s2 = scale[k];
+      uint32_t cut2 = 8;
+      if (cut < 8) {
+        const int64_t row = row0 + belows[k];
+        s1 = cut == in_row ? scale_at(row + 1, 0) : scale_at(row, cols[k] + cut);
+        if (cut < in_row && in_row < 8) {
+          cut2 = in_row;
+          s2 = scale_at(row + 1, 0);
+        }
       }
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) f[j] *= j < cut ? scale[k] : j < cut2 ? s1 : s2;
     }
+    store_values8<DQ>(dq, 8 * g, f);
   }
 }
 
@@ -181,29 +219,31 @@ __global__ __launch_bounds__(kThreads) void unpack_dequant_kernel(
   const fsh_unpack_chunk ch = chunks[lo];
   const int64_t tiles_c = (ch.in_dim + block - 1) / block;
   const int64_t t = bid - tile_starts[lo];
-  const int64_t tr = t / tiles_c, tc = t - tr * tiles_c;
   const int tid = threadIdx.x;
   constexpr int kElem = DQ == FSH_DT_F32 ? 4 : 2;
 
-  const float scale = load_f32_any(rows + ch.src_scale_offset + 4 * (tr * tiles_c + tc));
-  if (compact != nullptr && tid == 0)
-    store_f32_any(compact + ch.dst_scale_offset + 4 * (tr * tiles_c + tc), scale);
+  const uint8_t* scales = rows + ch.src_scale_offset;
+  const float scale = load_f32_any(scales + 4 * t);
+  if (compact != nullptr && tid == 0) store_f32_any(compact + ch.dst_scale_offset + 4 * t, scale);
 
   const uint8_t* src = rows + ch.src_qdata_offset;
   uint8_t* cq = compact ? compact + ch.dst_qdata_offset : nullptr;
   uint8_t* dq = dequant ? dequant + ch.dst_dequant_offset * kElem : nullptr;
-  if (block == 128) {
-    // Four parameters of 1000 to 3000 rows and columns (14 MB, none a multiple of
-    // 16 wide), which the element-wise path used to take: 53.8 us there, 21.9 here.
-    const uintptr_t bytes_at = reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(cq) | static_cast<uintptr_t>(ch.in_dim);
-    if ((bytes_at & 7) == 0 && (reinterpret_cast<uintptr_t>(dq) & 15) == 0)
-      unpack_tile<DQ, true>(src, cq, dq, ch.rows, ch.in_dim, tr, tc, scale, tid);
+  if (block == 128 && ch.in_dim >= 8 && ch.in_dim < (1LL << 31)) {
+    // The pieces start `lead` elements in, where the wider output's memory lines do.
+    const int64_t lead = dq ? (-reinterpret_cast<uintptr_t>(dq) & 255) / kElem : (-reinterpret_cast<uintptr_t>(cq) & 127);
+    const bool on_lines = (cq == nullptr || ((reinterpret_cast<uintptr_t>(cq) + lead) & 127) == 0) &&
+                          ((reinterpret_cast<uintptr_t>(src) + lead) & 7) == 0;
+    const int64_t tiles = ((ch.rows + 127) / 128) * tiles_c;
+    if (on_lines)
+      unpack_piece<DQ, true>(src, cq, dq, scales, ch.rows, ch.in_dim, tiles_c, t, tiles, lead, tid);
     else
-      unpack_tile<DQ, false>(src, cq, dq, ch.rows, ch.in_dim, tr, tc, scale, tid);
+      unpack_piece<DQ, false>(src, cq, dq, scales, ch.rows, ch.in_dim, tiles_c, t, tiles, lead, tid);
     return;
   }
 
   // Element-wise path.
+  const int64_t tr = t / tiles_c, tc = t - tr * tiles_c;
   const int64_t row0 = tr * block, col0 = tc * block;
   const int64_t nrows = (ch.rows - row0) < block ? (ch.rows - row0) : block;
   const int64_t ncols = (ch.in_dim - col0) < block ? (ch.in_dim - col0) : block;
