@@ -124,11 +124,12 @@ __device__ __forceinline__ T* uniform_ptr(T* ptr) {
 }
 
 // Stores a [rows][row_bytes] bf16 image held in LDS (pitch bytes apart) to
-// global rows `ld` elements apart, 16 bytes per lane.  `dst` is the same in
-// every lane: each store is a scalar base (advanced per pass) plus one 32-bit
-// lane offset, so the passes share a single address register.
+// global rows `ld` elements apart, 16 bytes per lane, cut at rows_left x
+// cols_left (a multiple of 8).  `dst` is the same in every lane: each store is
+// a scalar base (advanced per pass) plus one 32-bit lane offset, so the passes
+// share a single address register.
 template <int kRows, int kRowBytes, int kPitch>
-__device__ inline void store_staged_rows(const uint8_t* region, uint16_t* dst, int64_t ld, int lane) {
+__device__ inline void store_staged_rows(const uint8_t* region, uint16_t* dst, int64_t ld, int rows_left, int cols_left, int lane) {
   constexpr int kLanesPerRow = kRowBytes / 16;
   constexpr int kRowsPerPass = 64 / kLanesPerRow;
   static_assert(kRowBytes % 16 == 0 && 64 % kLanesPerRow == 0 && kRows % kRowsPerPass == 0, "staged store shape");
@@ -136,6 +137,7 @@ __device__ inline void store_staged_rows(const uint8_t* region, uint16_t* dst, i
   const uint32_t lane_off = static_cast<uint32_t>(r0) * static_cast<uint32_t>(ld * 2) + chunk * 16;
   uint8_t* base = uniform_ptr(reinterpret_cast<uint8_t*>(dst));
   const int64_t pass_bytes = uniform_i64(static_cast<int64_t>(kRowsPerPass) * ld * 2);
+  const int rows = chunk * 8 < cols_left ? rows_left : 0;  // of this lane's columns
 #pragma unroll
   for (int pass = 0; pass < kRows / kRowsPerPass; ++pass) {
     const int r = pass * kRowsPerPass + r0;
@@ -148,7 +150,7 @@ __device__ inline void store_staged_rows(const uint8_t* region, uint16_t* dst, i
       const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
       v = u32x4{lo.x, lo.y, hi.x, hi.y};
     }
-    *reinterpret_cast<u32x4*>(base + pass * pass_bytes + lane_off) = v;
+    if (r < rows) *reinterpret_cast<u32x4*>(base + pass * pass_bytes + lane_off) = v;
   }
 }
 
@@ -175,15 +177,19 @@ struct DRows {
 // `d` is matrix `batch` of D (row stride ldd elements).
 template <typename Cfg>
 __device__ __forceinline__ void load_d_rows_from(const uint16_t* d, int64_t ldd, int64_t m0, int64_t n0, int wm, int wn,
-                                                 int lane, int half, DRows<Cfg>& rows) {
+                                                 int lane, int half, int rows_left, int cols_left, DRows<Cfg>& rows) {
   using R = DRows<Cfg>;
   const int r0 = lane / R::kLanesPerRow, chunk = lane % R::kLanesPerRow;
   const uint32_t lane_off = static_cast<uint32_t>(r0) * static_cast<uint32_t>(ldd * 2) + chunk * 16;
   const uint8_t* base = uniform_ptr(reinterpret_cast<const uint8_t*>(
       d + (m0 + wm * Cfg::kWaveM + half * (Cfg::kWaveM / 2)) * ldd + n0 + wn * Cfg::kWaveN));
   const int64_t pass_bytes = uniform_i64(static_cast<int64_t>(R::kRowsPerPass) * ldd * 2);
+  const int live = chunk * 8 < cols_left ? rows_left : 0;  // rows of this lane's columns
 #pragma unroll
-  for (int q = 0; q < R::kPasses; ++q) rows.t[q] = *reinterpret_cast<const u32x4*>(base + q * pass_bytes + lane_off);
+  for (int q = 0; q < R::kPasses; ++q) {
+    rows.t[q] = u32x4{0, 0, 0, 0};
+    if (q * R::kRowsPerPass + r0 < live) rows.t[q] = *reinterpret_cast<const u32x4*>(base + q * pass_bytes + lane_off);
+  }
 }
 
 // Orders the LDS traffic of one wave: lanes exchange data through the wave's
@@ -242,7 +248,7 @@ constexpr int kEpiGeneric = 0, kEpiPlain = 1, kEpiPoly = 2, kEpiUpdate = 3;
 
 // (Always inlined: as a real call the accumulators and the launch's problem
 // table would have to live in scratch memory.)
-template <typename Cfg, int kMode>
+template <typename Cfg, int kMode, bool kRagged>
 __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int64_t batch, int64_t m0, int64_t n0, int wm,
                                                int wn, int lane, bool mirror, const f32x4 (&acc)[Cfg::TM][Cfg::TN],
                                                uint8_t* staging) {
@@ -259,6 +265,9 @@ __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int
   uint16_t* Ct = mirror ? C : (p.Ct ? p.Ct + batch * p.sCt : nullptr);
   const int64_t ldct = mirror ? p.ldc : p.ldct;
   const int64_t wave_row = m0 + wm * Cfg::kWaveM, wave_col = n0 + wn * Cfg::kWaveN;
+  // Rows and columns of the wave's sub-tile that exist (0 or less: none).
+  const auto left = [](int64_t size, int64_t at) { return kRagged && size - at < 256 ? static_cast<int>(size - at) : 256; };
+  const int rows_left = left(p.M, wave_row), cols_left = left(p.N, wave_col);
   uint8_t* region = staging + (wm * Cfg::WN + wn) * Epi::kRegion;
   const int r_lane = lane & 15, c_lane = 4 * (lane >> 4);
   const bool unit_alpha = (kMode == kEpiPlain || kMode == kEpiUpdate) ? true : kMode == kEpiPoly ? false : p.alpha == 1.0f;
@@ -269,7 +278,7 @@ __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int
   // The lower half of D is requested once the upper half has left its
   // registers for LDS, and lands while the upper half is worked on.
   DRows<Cfg> drows[2];
-  if (has_d) load_d_rows_from<Cfg>(D, ldd, m0, n0, wm, wn, lane, 0, drows[0]);
+  if (has_d) load_d_rows_from<Cfg>(D, ldd, m0, n0, wm, wn, lane, 0, rows_left, cols_left, drows[0]);
 #pragma unroll
   for (int hf = 0; hf < 2; ++hf) {
     if (has_d) {
@@ -280,7 +289,7 @@ __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int
         uint8_t* d = region + (r0 + q * R::kRowsPerPass) * Epi::kPitch + chunk * 16;
         *reinterpret_cast<u32x4*>(d) = drows[hf].t[q];
       }
-      if (hf == 0) load_d_rows_from<Cfg>(D, ldd, m0, n0, wm, wn, lane, 1, drows[1]);
+      if (hf == 0) load_d_rows_from<Cfg>(D, ldd, m0, n0, wm, wn, lane, 1, rows_left - Epi::kRows, cols_left, drows[1]);
       wave_lds_sync();
     }
 #pragma unroll
@@ -341,7 +350,7 @@ __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int
     if (hf == 1) FSH_STAMP(9);
     wave_lds_sync();
     store_staged_rows<Epi::kRows, Cfg::kWaveN * 2, Epi::kPitch>(
-        region, C + (wave_row + hf * Epi::kRows) * p.ldc + wave_col, p.ldc, lane);
+        region, C + (wave_row + hf * Epi::kRows) * p.ldc + wave_col, p.ldc, rows_left - hf * Epi::kRows, cols_left, lane);
     if (hf == 1) FSH_STAMP(10);
     if (Ct != nullptr) {  // uniform over the workgroup
       // The finals come back in accumulator layout (every read before the
@@ -366,27 +375,27 @@ __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int
       if (hf == 1) FSH_STAMP(12);
       wave_lds_sync();
       store_staged_rows<Cfg::kWaveN, Epi::kRows * 2, Epi::kPitchT>(
-          region, Ct + wave_col * ldct + wave_row + hf * Epi::kRows, ldct, lane);
+          region, Ct + wave_col * ldct + wave_row + hf * Epi::kRows, ldct, cols_left, rows_left - hf * Epi::kRows, lane);
     }
     if (hf == 0) FSH_STAMP(8);
     if (hf == 0) wave_lds_sync();  // before the lower half overwrites the region
   }
 }
 
-template <typename Cfg>
+template <typename Cfg, bool kRagged>
 __device__ __forceinline__ void store_tile_in_halves(const GemmParams& p, int64_t batch, int64_t m0, int64_t n0, int wm, int wn,
                                             int lane, bool mirror, const f32x4 (&acc)[Cfg::TM][Cfg::TN],
                                             uint8_t* staging) {
   // uniform over the launch's problem, so one branch per tile
   const bool has_d = p.D != nullptr, diag = p.diag_add != 0.0f, unit_alpha = p.alpha == 1.0f;
   if (p.update_ptrs != nullptr)
-    store_tile_in_halves_as<Cfg, kEpiUpdate>(p, batch, m0, n0, wm, wn, lane, mirror, acc, staging);
+    store_tile_in_halves_as<Cfg, kEpiUpdate, kRagged>(p, batch, m0, n0, wm, wn, lane, mirror, acc, staging);
   else if (!has_d && !diag && unit_alpha)
-    store_tile_in_halves_as<Cfg, kEpiPlain>(p, batch, m0, n0, wm, wn, lane, mirror, acc, staging);
+    store_tile_in_halves_as<Cfg, kEpiPlain, kRagged>(p, batch, m0, n0, wm, wn, lane, mirror, acc, staging);
   else if (has_d && !unit_alpha)
-    store_tile_in_halves_as<Cfg, kEpiPoly>(p, batch, m0, n0, wm, wn, lane, mirror, acc, staging);
+    store_tile_in_halves_as<Cfg, kEpiPoly, kRagged>(p, batch, m0, n0, wm, wn, lane, mirror, acc, staging);
   else
-    store_tile_in_halves_as<Cfg, kEpiGeneric>(p, batch, m0, n0, wm, wn, lane, mirror, acc, staging);
+    store_tile_in_halves_as<Cfg, kEpiGeneric, kRagged>(p, batch, m0, n0, wm, wn, lane, mirror, acc, staging);
 }
 
 // gfx950 loads 16 bytes per lane from global memory straight into LDS: lane l

@@ -24,7 +24,7 @@ namespace fsh {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Large whole-tile problems: 256x256x64 tiles with global->LDS loads.
+// Large problems: 256x256x64 tiles with global->LDS loads.
 //
 // gfx950 can load 16 bytes per lane from global memory straight into LDS
 // (global_load_lds_dwordx4: lane l of a wave writes LDS bytes
@@ -86,7 +86,11 @@ __device__ __forceinline__ void clear_accumulators(f32x4& acc) {
 // consecutive k of one output row, half of an MFMA operand.  The products and
 // their order are those of the k-contiguous form on the transposed operands,
 // so the results are bit-identical.
-template <bool kPersistent, bool kKMajor>
+//
+// kRagged: some problem of the launch does not consist of whole tiles.  A
+// separate instantiation: the limits in the epilogue and at a tile's start cost
+// launches of whole tiles 1-2 %.
+template <bool kPersistent, bool kKMajor, bool kRagged>
 __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const GemmLaunch launch) {
   using Cfg = DmaGemm;
 #ifdef FSH_TRACE
@@ -97,7 +101,6 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   constexpr int TM = Cfg::TM, TN = Cfg::TN, KS = Cfg::KS;
 
   const int tid = threadIdx.x;
-  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
 
@@ -124,10 +127,11 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   // lane l fills slot l & 31 of row r + 8 (l >> 5).  K-row 16 a + 8 b + c thus
   // lies at byte 1024 (8 a + c) + 512 b of its slot.)
   // (The per-lane values of both sides are derived from the lane number again
-  // at the start of every tile, see derive_lane_values below.)
+  // at the start of every tile, see below.)
   uint32_t a_row_bytes = 0, b_row_bytes = 0;
+  int a_left = 0, b_left = 0;  // rows of the operands from the tile's first on, 256 at most
   uint32_t a_voff[Cfg::kLoads], b_voff[Cfg::kLoads];
-  const auto request_row = [](int q) -> uint32_t { return kKMajor ? 16 * (q / 2) + 4 * (q % 2) : 32 * q; };
+  const auto request_row = [](int q) -> int { return kKMajor ? 16 * (q / 2) + 4 * (q % 2) : 32 * q; };
   // M0 takes the LDS byte address relative to the workgroup's allocation.
   typedef __attribute__((address_space(3))) uint8_t* lds_address;
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_address)lds_bytes));
@@ -168,26 +172,38 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   // slot through the swizzle: chunk ^ 4 (k-row & 3) ^ 2 (octet & 1), one address
   // per block in the upper bits (i ^ (k-row & 3)) and two in the lower one.
   uint32_t a_frag_km[TM / 2][2], b_frag_km[TN / 2][2];
-  // All per-lane addresses of the k loop, from the lane number.  Called with
-  // a lane number the compiler cannot see through at the start of every tile:
-  // the values then live from there to the end of the k loop only.  Kept
-  // across the epilogue (which needs every register it can get), the compiler
-  // spilled some of them and reloaded them inside the k loop, and a reload is
-  // a vector memory load: the wait for it also waited for every operand
-  // request in flight.
-  const auto opaque = [](int l) {
-    asm volatile("" : "+v"(l));
+  // All per-lane addresses of the k loop are derived from the lane's number at
+  // the start of every tile: the values then live from there to the end of the
+  // k loop only.  Kept across the epilogue (which needs every register it can
+  // get), the compiler spilled some of them and reloaded them inside the k
+  // loop, and a reload is a vector memory load: the wait for it also waited
+  // for every operand request in flight.
+  // (So is that number itself, in two instructions.)
+  const auto lane_now = []() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
     return l;
   };
-  auto derive_lane_values = [&](int l) {
-    const uint32_t fill_row = kKMajor ? wave + 8 * (l >> 5) : 8 * wave + (l >> 3);
+  // `octets` of a k-tile's eight exist.  What lies past the matrix is read from
+  // its last row (k-major: column octet), what lies past K from the last octet:
+  // the one is never stored, the other is zeroed in the fragments.
+  auto derive_requests = [&](int l, int octets) {
+    const int fill_row = kKMajor ? wave + 8 * (l >> 5) : 8 * wave + (l >> 3);
     // (k-row & 3 of a k-major request is the wave's number)
-    const uint32_t fill_chunk = kKMajor ? (l & 31) ^ (4 * wave) ^ (2 * (l >> 5)) : (l & 7) ^ ((fill_row >> 1) & 7);
+    const int fill_chunk = kKMajor ? (l & 31) ^ (4 * wave) ^ (2 * (l >> 5)) : (l & 7) ^ ((fill_row >> 1) & 7);
+    const auto offset = [&](int q, int left, uint32_t row_bytes) {
+      const int row = fill_row + request_row(q);
+      const int row_there = !kRagged ? row : kKMajor ? min(row, 8 * octets - 1) : min(row, left - 1);
+      const int chunk_there = !kRagged ? fill_chunk : kKMajor ? min(fill_chunk, left / 8 - 1) : min(fill_chunk, octets - 1);
+      return static_cast<uint32_t>(row_there) * row_bytes + static_cast<uint32_t>(chunk_there * 16);
+    };
 #pragma unroll
     for (int q = 0; q < Cfg::kLoads; ++q) {
-      a_voff[q] = (fill_row + request_row(q)) * a_row_bytes + fill_chunk * 16;
-      b_voff[q] = (fill_row + request_row(q)) * b_row_bytes + fill_chunk * 16;
+      a_voff[q] = offset(q, a_left, a_row_bytes);
+      b_voff[q] = offset(q, b_left, b_row_bytes);
     }
+  };
+  auto derive_fragments = [&](int l) {
     const int t = l & 15, g = l >> 4;
     const uint32_t frag_base = static_cast<uint32_t>(t * Cfg::kRowBytes + ((g ^ ((t >> 1) & 7)) * 16));
 #pragma unroll
@@ -245,14 +261,26 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   } else if (!locate(id, which, batch, tm, tn)) {
     return;  // whole workgroup, before any barrier
   }
-  const uint8_t* Ab = a_base(which, batch, tm);
-  const uint8_t* Bb = b_base(which, batch, tn);
-  a_row_bytes = static_cast<uint32_t>(launch.problem[which].lda * 2);
-  b_row_bytes = static_cast<uint32_t>(launch.problem[which].ldb * 2);
+  const uint8_t* Ab = nullptr;
+  const uint8_t* Bb = nullptr;
+  // The first operands of a tile, into slots 0 and 1.
+  auto begin_tile = [&](int problem, int64_t matrix, int r, int c) {
+    const GemmParams& q = launch.problem[problem];
+    Ab = a_base(problem, matrix, r);
+    Bb = b_base(problem, matrix, c);
+    a_row_bytes = static_cast<uint32_t>(q.lda * 2);
+    b_row_bytes = static_cast<uint32_t>(q.ldb * 2);
+    if (kRagged) {
+      const int64_t m_left = q.M - static_cast<int64_t>(r) * Cfg::BM, n_left = q.N - static_cast<int64_t>(c) * Cfg::BN;
+      a_left = static_cast<int>(m_left < Cfg::BM ? m_left : Cfg::BM);
+      b_left = static_cast<int>(n_left < Cfg::BN ? n_left : Cfg::BN);
+    }
+    derive_requests(lane_now(), kRagged && q.K < Cfg::BK ? static_cast<int>(q.K / 8) : 8);
+    issue_operand(Ab, a_voff, 0);
+    issue_operand(Bb, b_voff, Cfg::kOperandBytes);
+  };
   FSH_STAMP(1);
-  derive_lane_values(lane);
-  issue_operand(Ab, a_voff, 0);
-  issue_operand(Bb, b_voff, Cfg::kOperandBytes);
+  begin_tile(which, batch, tm, tn);
 
 #ifdef FSH_TRACE
   uint64_t trace_wait = 0, trace_barrier = 0, trace_ktiles = 0, trace_tile_wait = 0, trace_tile_barrier = 0, trace_tiles = 0, trace_kloop = 0, trace_epi = 0, trace_steps = 0, trace_last = 0, trace_mark = 0;
@@ -291,7 +319,8 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   const auto next_slot = [](int slot) { return slot + Cfg::kOperandBytes == Cfg::kRingBytes ? 0 : slot + Cfg::kOperandBytes; };
   int a_slot = 0;  // of the current k-tile's operand A
   // more: k-tile kt + 1 exists; more2: kt + 2 exists
-  auto k_tile = [&](int64_t kt, auto more_tag, auto more2_tag) {
+  int tail = 0;  // octets of the last k-tile, 0 if it is whole
+  auto k_tile = [&](int kt, auto more_tag, auto more2_tag) {
     constexpr bool more = decltype(more_tag)::value, more2 = decltype(more2_tag)::value;
     const int b_slot = next_slot(a_slot), a_next = next_slot(b_slot), b_next = next_slot(a_next), a_after = next_slot(b_next);
     const uint8_t* a_src2 = k_tile_ptr(Ab, a_row_bytes, kt + 2);
@@ -310,8 +339,22 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
       }
       __builtin_amdgcn_sched_barrier(0);
     };
+    // Past K both operands are zero (the other's last values could be infinite).
+    auto zero_past_k = [&](int ks) {
+      const bool live = 4 * ks + (lane_now() >> 4) < tail;
+      const auto masked = [&](bf16x8& f) {
+        const u32x4 w = __builtin_bit_cast(u32x4, f);
+        f = __builtin_bit_cast(bf16x8, live ? w : u32x4{0, 0, 0, 0});
+      };
+#pragma unroll
+      for (int i = 0; i < TM; ++i) masked(af[ks][i]);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) masked(bf[ks][j]);
+    };
+    if (kRagged && !more && tail) zero_past_k(0);
 #pragma unroll
     for (int g = 0; g < kMfmas; ++g) slice(0, g);
+    if (kRagged && !more && tail) zero_past_k(1);
 #ifdef FSH_TRACE
     const uint64_t tr0 = __builtin_amdgcn_s_memtime();
     trace_steps += tr0 - trace_mark;
@@ -340,8 +383,10 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
 
   while (true) {
     const GemmParams& p = launch.problem[which];
-    const int64_t ktiles = p.K / Cfg::BK;
-    derive_lane_values(opaque(lane));
+    const int ktiles = static_cast<int>((p.K + Cfg::BK - 1) / Cfg::BK);
+    if (kRagged) tail = static_cast<int>(p.K / 8) & 7;
+    derive_requests(lane_now(), 8);
+    derive_fragments(lane_now());
     FSH_STAMP(6);
     // Under the wait for the first operands and for the previous tile's stores.
 #pragma unroll
@@ -366,6 +411,7 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
 #pragma unroll
     for (int g = 0; g < TM + TN; ++g) read_frag(0, 0, Cfg::kOperandBytes, 0, g);
     if (ktiles > 1) {
+      if (kRagged && ktiles == 2 && tail) derive_requests(lane_now(), tail);
       issue_operand(k_tile_ptr(Ab, a_row_bytes, 1), a_voff, 2 * Cfg::kOperandBytes);
       issue_operand(k_tile_ptr(Bb, b_row_bytes, 1), b_voff, 3 * Cfg::kOperandBytes);
     }
@@ -373,7 +419,10 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
 
     constexpr std::true_type yes{};
     constexpr std::false_type no{};
-    for (int64_t kt = 0; kt + 2 < ktiles; ++kt) k_tile(kt, yes, yes);
+    for (int kt = 0; kt + 2 < ktiles; ++kt) {
+      if (kRagged && kt + 3 == ktiles && tail) derive_requests(lane_now(), tail);  // the last k-tile's go out in this one
+      k_tile(kt, yes, yes);
+    }
     if (ktiles > 1) k_tile(ktiles - 2, yes, no);
     k_tile(ktiles - 1, no, no);
     FSH_STAMP(3);
@@ -390,21 +439,13 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
       id = uniform_i64(id + stride);
       while (id < launch.total_workgroups && !(have_next = locate(id, next_which, next_batch, next_tm, next_tn)))
         id = uniform_i64(id + stride);
-      if (have_next) {
-        Ab = a_base(next_which, next_batch, next_tm);
-        Bb = b_base(next_which, next_batch, next_tn);
-        a_row_bytes = static_cast<uint32_t>(launch.problem[next_which].lda * 2);
-        b_row_bytes = static_cast<uint32_t>(launch.problem[next_which].ldb * 2);
-        derive_lane_values(opaque(lane));
-        issue_operand(Ab, a_voff, 0);
-        issue_operand(Bb, b_voff, Cfg::kOperandBytes);
-      }
+      if (have_next) begin_tile(next_which, next_batch, next_tm, next_tn);
     }
 #ifdef FSH_TRACE
     const uint64_t te0 = __builtin_amdgcn_s_memtime();
 #endif
-    store_tile_in_halves<Cfg>(p, batch, static_cast<int64_t>(tm) * Cfg::BM, static_cast<int64_t>(tn) * Cfg::BN, wm,
-                              wn, opaque(lane), p.symmetric && tm != tn, acc, lds_bytes + kDmaGemmStaging);
+    store_tile_in_halves<Cfg, kRagged>(p, batch, static_cast<int64_t>(tm) * Cfg::BM, static_cast<int64_t>(tn) * Cfg::BN, wm,
+                              wn, lane_now(), p.symmetric && tm != tn, acc, lds_bytes + kDmaGemmStaging);
 #ifdef FSH_TRACE
     trace_epi += __builtin_amdgcn_s_memtime() - te0;
 #endif
@@ -436,11 +477,11 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   }
 }
 
-// A validated problem and whether it takes the large-tile kernel.
+// A validated problem, whether the large-tile kernel can take it and whether it does.
 struct PlannedGemm {
   GemmParams p;
   int64_t batch;
-  bool large;
+  bool fits, large;
 };
 
 // ---- Which tiles a launch takes.
@@ -457,7 +498,7 @@ constexpr TileShape kTileShapes[] = {
     {128, 128, 512.0, 0.37, 0.71, 1.02, 4.2},     // two
     {128, 128, 256.0, 0.35, 0.43, 0.52, 3.2},     // one, its operands requested three k-tiles ahead
     {256, 128, 256.0, 0.54, 0.68, 0.91, 5.5},     // one of eight waves
-    {256, 256, 256.0, 0.96, 1.10, 1.58, 8.0},     // one
+    {256, 256, 256.0, 0.94, 1.02, 1.38, 8.5},     // one
 };
 // The products of one launch, as the tiles of every kind see them.
 struct LaunchWork {
@@ -493,13 +534,16 @@ TileKind small_tile_kind(const LaunchWork& w) {
 }
 double small_tiles_us(const LaunchWork& w) { return launch_us(small_tile_kind(w), w); }
 
-// The 256 x 256 kernel takes whole tiles with 16-byte accesses in the epilogue and 32-bit tile spans.
+// The 256 x 256 kernel has 16-byte accesses in the epilogue and 32-bit tile spans.
 bool fits_large_tiles(const GemmParams& p) {
-  return p.M % DmaGemm::BM == 0 && p.N % DmaGemm::BN == 0 && p.K % DmaGemm::BK == 0 && p.ldc % 8 == 0 &&
+  return p.M % 8 == 0 && p.N % 8 == 0 && p.K % 8 == 0 && p.ldc % 8 == 0 &&
          (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && p.sC % 8 == 0 &&
          (p.Ct == nullptr || (p.ldct % 8 == 0 && (reinterpret_cast<uintptr_t>(p.Ct) & 15) == 0 && p.sCt % 8 == 0)) &&
          (p.D == nullptr || (p.ldd % 8 == 0 && (reinterpret_cast<uintptr_t>(p.D) & 15) == 0 && p.sD % 8 == 0)) &&
          static_cast<int64_t>(DmaGemm::BM) * p.lda * 2 < (1LL << 31) && static_cast<int64_t>(DmaGemm::BN) * p.ldb * 2 < (1LL << 31);
+}
+bool whole_large_tiles(const GemmParams& p) {
+  return p.M % DmaGemm::BM == 0 && p.N % DmaGemm::BN == 0 && p.K % DmaGemm::BK == 0;
 }
 
 // The Muon update an epilogue applies instead of storing its product (see
@@ -549,7 +593,8 @@ int plan_gemm(const fsh_gemm_desc& d, PlannedGemm* plan, const GemmUpdate* updat
   if (const char* e = getenv("FSH_GEMM_TRACE")) p.trace = reinterpret_cast<uint64_t*>(strtoull(e, nullptr, 0));
 #endif
   plan->batch = d.batch;
-  plan->large = fits_large_tiles(p);  // may take the large-tile kernel; choose_kernels decides whether it does
+  plan->fits = fits_large_tiles(p);
+  plan->large = plan->fits && whole_large_tiles(p);  // may take the large-tile kernel; choose_kernels decides whether it does
   return FSH_OK;
 }
 
@@ -611,31 +656,37 @@ int fill_launch(PlannedGemm* plans, const int* members, int n, int64_t tile_m, i
   return FSH_OK;
 }
 
+template <bool kPersistent, bool kKMajor, bool kRagged>
+int launch_large_as(const GemmLaunch& launch, int64_t workgroups, hipStream_t stream) {
+  static LdsReservation reserved;
+  constexpr auto* kernel = &gemm_nt_dma_kernel<kPersistent, kKMajor, kRagged>;
+  if (int rc = reserve_lds_once(reserved, kernel, kDmaGemmLdsBytes)) return rc;
+  hipLaunchKernelGGL((gemm_nt_dma_kernel<kPersistent, kKMajor, kRagged>), dim3(static_cast<uint32_t>(workgroups)),
+                     dim3(DmaGemm::kThreads), kDmaGemmLdsBytes, stream, launch);
+  return check_launch("gemm_nt_dma_kernel");
+}
 int launch_large_tiles(const GemmLaunch& launch, bool k_major, hipStream_t stream) {
-  static LdsReservation reserved_dma, reserved_persistent, reserved_dma_km, reserved_persistent_km;
-  constexpr int kLds = kDmaGemmLdsBytes;
   // Equally long tiles and more of them than compute units: one resident
   // workgroup per compute unit walks a static schedule.
-  bool equal_k = true;
-  for (int k = 1; k < GemmLaunch::kMaxProblems; ++k)
-    equal_k = equal_k && (launch.first_workgroup[k] == INT32_MAX || launch.problem[k].K == launch.problem[0].K);
+  bool equal_k = true, ragged = false;
+  for (int k = 0; k < GemmLaunch::kMaxProblems; ++k) {
+    if (launch.first_workgroup[k] == INT32_MAX) continue;
+    equal_k = equal_k && launch.problem[k].K == launch.problem[0].K;
+    ragged = ragged || !whole_large_tiles(launch.problem[k]);
+  }
   const int64_t units = compute_units(), total = launch.total_workgroups;
   const bool resident = equal_k && units >= kXcds && units % kXcds == 0 && total > units;
-  const dim3 grid(static_cast<uint32_t>(resident ? units : total)), block(DmaGemm::kThreads);
-  if (resident && k_major) {
-    if (int rc = reserve_lds_once(reserved_persistent_km, &gemm_nt_dma_kernel<true, true>, kLds)) return rc;
-    hipLaunchKernelGGL((gemm_nt_dma_kernel<true, true>), grid, block, kLds, stream, launch);
-  } else if (resident) {
-    if (int rc = reserve_lds_once(reserved_persistent, &gemm_nt_dma_kernel<true, false>, kLds)) return rc;
-    hipLaunchKernelGGL((gemm_nt_dma_kernel<true, false>), grid, block, kLds, stream, launch);
-  } else if (k_major) {
-    if (int rc = reserve_lds_once(reserved_dma_km, &gemm_nt_dma_kernel<false, true>, kLds)) return rc;
-    hipLaunchKernelGGL((gemm_nt_dma_kernel<false, true>), grid, block, kLds, stream, launch);
-  } else {
-    if (int rc = reserve_lds_once(reserved_dma, &gemm_nt_dma_kernel<false, false>, kLds)) return rc;
-    hipLaunchKernelGGL((gemm_nt_dma_kernel<false, false>), grid, block, kLds, stream, launch);
+  const int64_t workgroups = resident ? units : total;
+  switch ((resident ? 4 : 0) + (k_major ? 2 : 0) + (ragged ? 1 : 0)) {
+    case 0: return launch_large_as<false, false, false>(launch, workgroups, stream);
+    case 1: return launch_large_as<false, false, true>(launch, workgroups, stream);
+    case 2: return launch_large_as<false, true, false>(launch, workgroups, stream);
+    case 3: return launch_large_as<false, true, true>(launch, workgroups, stream);
+    case 4: return launch_large_as<true, false, false>(launch, workgroups, stream);
+    case 5: return launch_large_as<true, false, true>(launch, workgroups, stream);
+    case 6: return launch_large_as<true, true, false>(launch, workgroups, stream);
+    default: return launch_large_as<true, true, true>(launch, workgroups, stream);
   }
-  return check_launch("gemm_nt_dma_kernel");
 }
 
 template <typename Cfg, int kBlocksPerUnit>
@@ -708,7 +759,10 @@ int launch_gemms(const fsh_gemm_desc* descs, int count, hipStream_t stream, cons
     const int n = count - begin < kChunk ? count - begin : kChunk;
     for (int i = 0; i < n; ++i) {
       if (int rc = plan_gemm(descs[begin + i], &plans[i], updates ? &updates[begin + i] : nullptr)) return rc;
-      if (large != nullptr && !large[begin + i]) plans[i].large = false;
+      if (large != nullptr) {
+        plans[i].large = large[begin + i];
+        if (large[begin + i] && !plans[i].fits) return fail(FSH_ENOTSUP, "gemm: a product does not fit the large tiles");
+      }
     }
     if (large == nullptr)
       if (int rc = choose_kernels(plans, n)) return rc;
@@ -824,23 +878,45 @@ int64_t ns_partial_offset(int64_t batch, int64_t rows, int64_t cols) {
 
 // Which problems run on the large-tile kernel: all that consist of its whole
 // tiles or none, whichever is estimated to take less time over an iteration's
-// three products together with the other problems of the call.
-void ns_choose_large(const fsh_ns_problem* problems, int count, int32_t steps, bool* large) {
-  double with_large_us = 0.0, without_us = 0.0;
+// three products together with the other problems of the call (by a margin of
+// 5 %, which is what the estimates are off by); then those with ragged edges
+// as well, all whose short side fills a tile or none.  Whole Muon steps, us
+// without / with ragged ones: one 5573 x 5573 and four small 4762 / 3434;
+// 16 of 444 x 384, 1224 x 2176 and 1024 x 5248 4003 / 3176; 1 of 5494 x 4608
+// and 16 of 256 x 5888 3232 / 2328; 16 of 832 x 2944, 334 x 960 and 2 of 2605 x
+// 6784 3411 / 2712; 16 of 1100 x 1300 1182 / 941.
+constexpr int64_t kRaggedLarge = 256;
+double ns_iteration_us(const fsh_ns_problem* problems, int count, const bool* large) {
+  double us = 0.0;
   for (int which = 0; which < 3; ++which) {
-    LaunchWork in_large, small, all;
+    LaunchWork in_large, small;
     for (int i = 0; i < count; ++i) {
       const fsh_ns_problem& q = problems[i];
       const int64_t s = q.rows < q.cols ? q.rows : q.cols, l = q.rows < q.cols ? q.cols : q.rows;
-      large[i] = steps > 0 && s > 0 && s % 256 == 0 && l % 256 == 0 && l < (1LL << 22);
       const int64_t m = which == 2 ? l : s, k = which == 0 ? l : s;
-      all.add(m, s, k, which != 2, q.batch);
       (large[i] ? in_large : small).add(m, s, k, which != 2, q.batch);
     }
-    with_large_us += launch_us(kTiles256, in_large) + small_tiles_us(small);
-    without_us += small_tiles_us(all);
+    us += launch_us(kTiles256, in_large) + small_tiles_us(small);
   }
-  for (int i = 0; i < count; ++i) large[i] = large[i] && with_large_us < without_us;
+  return us;
+}
+void ns_choose_large(const fsh_ns_problem* problems, int count, int32_t steps, bool* large) {
+  constexpr double kMargin = 0.95;
+  bool whole[FSH_MAX_NS_PROBLEMS], ragged[FSH_MAX_NS_PROBLEMS];
+  for (int i = 0; i < count; ++i) {
+    const fsh_ns_problem& q = problems[i];
+    const int64_t s = q.rows < q.cols ? q.rows : q.cols, l = q.rows < q.cols ? q.cols : q.rows;
+    large[i] = false;
+    whole[i] = steps > 0 && s > 0 && s % 256 == 0 && l % 256 == 0 && l < (1LL << 22);
+    ragged[i] = whole[i] || (steps > 0 && s >= kRaggedLarge && l < (1LL << 22));
+  }
+  double us = ns_iteration_us(problems, count, large);
+  for (const bool* choice : {whole, ragged}) {
+    const double with = ns_iteration_us(problems, count, choice);
+    if (with >= kMargin * us) continue;
+    us = with;
+    for (int i = 0; i < count; ++i) large[i] = choice[i];
+  }
 }
 
 // Checks a problem and lays out its buffers; `normalize` receives its part of
@@ -1159,8 +1235,8 @@ FSH_API int fsh_muon_step(const fsh_muon_group* groups, int32_t count, float ler
   // separate launch applies them.
   GemmUpdate updates[FSH_MAX_NS_PROBLEMS];
   for (int i = 0; i < count; ++i) {
-    // (the epilogue writes bf16 parameters; fp32 masters take the separate launch)
-    const bool fused = st[i].single && groups[i].master_dtype == FSH_DT_BF16;
+    // (the epilogue writes bf16 parameters in rows of 16-byte pieces; fp32 masters and odd widths take the separate launch)
+    const bool fused = st[i].single && groups[i].master_dtype == FSH_DT_BF16 && !launch.group[i].padded;
     updates[i].ptrs = fused ? groups[i].param_ptrs_dev : nullptr;
     updates[i].decay = decay_factor;
     updates[i].neg_lr = groups[i].neg_adjusted_lr;
