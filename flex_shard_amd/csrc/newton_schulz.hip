@@ -504,6 +504,7 @@ constexpr TileShape kTileShapes[] = {
 struct LaunchWork {
   double tiles[5] = {0, 0, 0, 0, 0}, tile_ktiles[5] = {0, 0, 0, 0, 0};
   double max_ktiles = 0.0;
+  bool transposed = false;  // some product is written transposed as well
   void add(int64_t m, int64_t n, int64_t k, bool symmetric, int64_t batch);
 };
 int64_t count_tiles(int64_t m, int64_t n, bool symmetric, int64_t tile_m, int64_t tile_n) {
@@ -522,7 +523,10 @@ void LaunchWork::add(int64_t m, int64_t n, int64_t k, bool symmetric, int64_t ba
 // Tiles of a shorter contraction count by their share of the longest one.
 double launch_us(TileKind kind, const LaunchWork& w) {
   if (w.max_ktiles == 0.0) return 0.0;
-  return rounds_us(kTileShapes[kind], w.tiles[kind], w.tile_ktiles[kind], w.max_ktiles);
+  // A second output lengthens the end of every round: 128 KB more of each 256 x 256 tile leave at a time.
+  TileShape shape = kTileShapes[kind];
+  if (w.transposed) shape.ends += kind == kTiles256 ? 12.0 : 3.0;
+  return rounds_us(shape, w.tiles[kind], w.tile_ktiles[kind], w.max_ktiles);
 }
 TileKind small_tile_kind(const LaunchWork& w) {
   TileKind best = kTiles64;
@@ -532,6 +536,7 @@ TileKind small_tile_kind(const LaunchWork& w) {
   }
   return best;
 }
+constexpr double kEstimateMargin = 0.95;  // the estimates are off by about 5 %
 double small_tiles_us(const LaunchWork& w) { return launch_us(small_tile_kind(w), w); }
 
 // The 256 x 256 kernel has 16-byte accesses in the epilogue and 32-bit tile spans.
@@ -750,7 +755,34 @@ int launch_planned(PlannedGemm* plans, int count, hipStream_t stream) {
   return FSH_OK;
 }
 
-// `large` (null: decided here): the problems that take the large-tile kernel.
+// Products of a Newton-Schulz iteration whose flow either kernel can serve:
+// `plans[i].large` is set already where the flow asks for the large tiles; the
+// others join them, all that fill a tile or none, if that is estimated to be
+// faster by 10 %: two estimates are compared, each off by half of that.  One or
+// two matrices of 2000 to 3300 a side come out so in their third product, whose
+// tiles are a round and a bit on the small kernels and less than one here.
+// Whole Muon steps, us: one 3072 x 3072 890 -> 798; 2248 x 2248 and 2176 x 2176
+// 860 -> 782.
+void choose_free_products(PlannedGemm* plans, int count) {
+  LaunchWork in_large, rest, all;
+  bool any = false;
+  const auto candidate = [](const PlannedGemm& q) { return !q.large && q.fits && q.p.M >= 256 && q.p.N >= 256; };
+  for (int i = 0; i < count; ++i) {
+    const GemmParams& p = plans[i].p;
+    if (plans[i].large) continue;
+    const bool joins = candidate(plans[i]);
+    any = any || joins;
+    all.add(p.M, p.N, p.K, p.symmetric != 0, plans[i].batch);
+    all.transposed = all.transposed || p.Ct != nullptr;
+    LaunchWork& its = joins ? in_large : rest;
+    its.add(p.M, p.N, p.K, p.symmetric != 0, plans[i].batch);
+    its.transposed = its.transposed || p.Ct != nullptr;
+  }
+  if (!any || launch_us(kTiles256, in_large) + small_tiles_us(rest) >= 0.9 * small_tiles_us(all)) return;
+  for (int i = 0; i < count; ++i) plans[i].large = plans[i].large || candidate(plans[i]);
+}
+
+// `large` (null: decided here): the problems that take the large-tile kernel at least.
 int launch_gemms(const fsh_gemm_desc* descs, int count, hipStream_t stream, const GemmUpdate* updates = nullptr,
                  const bool* large = nullptr) {
   constexpr int kChunk = 16;
@@ -764,8 +796,10 @@ int launch_gemms(const fsh_gemm_desc* descs, int count, hipStream_t stream, cons
         if (large[begin + i] && !plans[i].fits) return fail(FSH_ENOTSUP, "gemm: a product does not fit the large tiles");
       }
     }
-    if (large == nullptr)
-      if (int rc = choose_kernels(plans, n)) return rc;
+    if (large != nullptr)
+      choose_free_products(plans, n);
+    else if (int rc = choose_kernels(plans, n))
+      return rc;
     if (int rc = launch_planned(plans, n, stream)) return rc;
   }
   return FSH_OK;
@@ -878,8 +912,7 @@ int64_t ns_partial_offset(int64_t batch, int64_t rows, int64_t cols) {
 
 // Which problems run on the large-tile kernel: all that consist of its whole
 // tiles or none, whichever is estimated to take less time over an iteration's
-// three products together with the other problems of the call (by a margin of
-// 5 %, which is what the estimates are off by); then those with ragged edges
+// three products together with the other problems of the call (by a margin); then those with ragged edges
 // as well, all whose short side fills a tile or none.  Whole Muon steps, us
 // without / with ragged ones: one 5573 x 5573 and four small 4762 / 3434;
 // 16 of 444 x 384, 1224 x 2176 and 1024 x 5248 4003 / 3176; 1 of 5494 x 4608
@@ -901,7 +934,6 @@ double ns_iteration_us(const fsh_ns_problem* problems, int count, const bool* la
   return us;
 }
 void ns_choose_large(const fsh_ns_problem* problems, int count, int32_t steps, bool* large) {
-  constexpr double kMargin = 0.95;
   bool whole[FSH_MAX_NS_PROBLEMS], ragged[FSH_MAX_NS_PROBLEMS];
   for (int i = 0; i < count; ++i) {
     const fsh_ns_problem& q = problems[i];
@@ -913,7 +945,7 @@ void ns_choose_large(const fsh_ns_problem* problems, int count, int32_t steps, b
   double us = ns_iteration_us(problems, count, large);
   for (const bool* choice : {whole, ragged}) {
     const double with = ns_iteration_us(problems, count, choice);
-    if (with >= kMargin * us) continue;
+    if (with >= kEstimateMargin * us) continue;
     us = with;
     for (int i = 0; i < count; ++i) large[i] = choice[i];
   }

@@ -28,7 +28,23 @@ def test_ragged_sizes_against_64_bits(device, shape, steps):
     workspace = torch.full((nbytes + 4096,), 0x55, dtype=torch.uint8, device=device)
     hip_ops.newton_schulz_multi([(mine, workspace[:nbytes])], COEFFS, steps, 1e-7)
     assert (x[:guard] == 7).all() and (x[-guard:] == 7).all() and (workspace[nbytes:] == 0x55).all()
-    for b in (0, batch - 1):
+    _check(mine, start, steps, (0, batch - 1))
+
+
+@pytest.mark.parametrize("shape", [(1, 2248, 2248), (1, 3072, 3072), (1, 2600, 2200)])
+def test_third_product_alone_on_large_tiles(device, shape):
+    """Few matrices iterate on the small tiles; their third product, with its
+    transposed output, may still take the large ones."""
+    assert hip_ops.newton_schulz_large_tiles(shape) == (False,)
+    mine = seeded_normal(shape, 1.0, sum(shape), device)
+    start = mine.double()
+    hip_ops.newton_schulz_multi([(mine, None)], COEFFS, 3, 1e-7)
+    _check(mine, start, 3, (0,))
+
+
+def _check(mine, start, steps, which):
+    rows, cols = mine.shape[1:]
+    for b in which:
         ref = start[b] if rows <= cols else start[b].T.contiguous()
         ref = ref / ref.norm()
         for _ in range(steps):
