@@ -8,12 +8,12 @@
 //   out[m][n] = bf16( sum over k-blocks kb of
 //                     dot(xq[m][kb], wq[n][kb]) * (xs[kb][m] * ws[n / 128][kb]) )
 //
-// Matrix cores: v_mfma_f32_32x32x64_f8f6f4 (64 FP8 products per lane pair and
-// instruction, twice the rate of the 32x32x16 FP8 form on gfx950).  A k-tile
-// is one scale block (128 bytes of each row), so its partial products are
-// accumulated from zero in a scratch accumulator and folded into the result
-// with one fused multiply-add per element; the folds of one 32x32 block run
-// on the vector ALU while the matrix core works on the next.
+// Matrix cores: v_mfma_f32_16x16x128_f8f6f4 here, 32x32x64 in the smaller tiles
+// (twice the rate of the 32x32x16 FP8 form on gfx950).  A k-tile is one scale
+// block (128 bytes of each row), so its partial products are accumulated from
+// zero in a scratch accumulator and folded into the result with one fused
+// multiply-add per element; the folds of one block run on the vector ALU while
+// the matrix core works on the next ones.
 #include "fp8_tiles.hpp"
 
 namespace fsh {
@@ -98,27 +98,37 @@ __global__ __launch_bounds__(kActThreads) void act_quant_1x128_kernel(const ActQ
 // ----------------------------------------------------------------- FP8 GEMM
 // 256 x 256 output tile per workgroup (262 flop per operand byte, which is
 // what keeps the request rate to L2 within reach at FP8 speed), eight waves of
-// 64 x 128 (two by four 32x32 blocks).  A wave's 128 accumulators stay in
+// 64 x 128 (four by eight 16x16 blocks).  A wave's 128 accumulators stay in
 // architectural VGPRs, where the vector ALU folds into them, and two waves
 // share a SIMD, so one wave's folds run under the other's MFMAs.  Operand
 // tiles are 128 bytes per row and k-tile and travel global -> LDS directly,
 // 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7), into one of two 64 KB
-// stages.  A lane feeds the matrix core bytes [32 h, 32 h + 32) of each half
-// of its row (h = lane / 32), i.e. chunks 2h and 2h+1 of a 64-byte half.
+// stages.
+//
+// Bound by the vector ALU and, in the block-scale form, by power (matrix cores
+// 64 % busy at 1.73 GHz; column scales 51 % at 1.93: two vector operations per
+// element and k-block).  A 16x16x128 MFMA is a block's whole product of a
+// k-tile: four registers that a fold can follow four blocks later, where the
+// two 32x32x64 ones before it held sixteen and had to be folded behind the next
+// pair; and the k-tile is a tag's two instantiations instead of a branch per
+// request.  8192 tokens, us before / after: 4096 x 4096 141 / 127, 14336 x 4096
+// 441 / 411, 4096 x 14336 383 / 355; weight gradients 133 / 126, 470 / 443, 467 /
+// 439.  Same bits.
 //
 // TM_ = 1 is the half tile (128 x 256, waves of 32 x 128) that the tiles of a
 // last, at most half-full round are cut into; it keeps the LDS layout of the
 // whole tile and fills the first half of the A area.
 template <int TM_>
 struct Fp8GemmCfg {
-  static constexpr int BM = 128 * TM_, BN = 256, BK = 128, WM = 4, WN = 2, TM = TM_, TN = 4;
+  static constexpr int BM = 128 * TM_, BN = 256, BK = 128, WM = 4, WN = 2;
   static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves, kWaveM = BM / WM, kWaveN = BN / WN;
+  static constexpr int TM = kWaveM / 16, TN = kWaveN / 16;  // blocks of 16 x 16 per wave
   static constexpr int kRowBytes = 128;
   static constexpr int kABytes = 256 * kRowBytes;              // 32 KB (half of it used by the half tile)
   static constexpr int kStageBytes = (256 + BN) * kRowBytes;   // 64 KB
   static constexpr int kFillRows = 8 * kWaves;                 // tile rows per wave-level load of all waves
   static constexpr int kLoadsA = BM / kFillRows, kLoadsB = BN / kFillRows;  // per wave: 4 (2) and 4
-  static constexpr int kPitch = kWaveN * 2 + 8;                // epilogue staging, bytes
+  static constexpr int kPitch = kWaveN * 2 + 16;               // epilogue staging, bytes
   static constexpr int kRegion = kWaveM * kPitch;              // per wave
   static constexpr int kStages = 2;
   static constexpr int kScaleSlots = 64;                        // row scales per wave and stage (one 4-byte request per lane)
@@ -188,36 +198,35 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
       dma_load_16(b_voff[q], b_src, stage_off + fill_lds, Cfg::kABytes + q * Cfg::kFillRows * Cfg::kRowBytes);
   };
 
-  // Fragment side: row = lane & 31 of a 32-row block; chunks 4 kh + 2 h and
-  // 4 kh + 2 h + 1 of the row (kh = 64-byte half), each in slot chunk ^ ((row >> 1) & 7).
-  const int frag_row = lane & 31, h = lane >> 5;
-  uint32_t frag_off[2][2];
+  // Fragment side: row = lane & 15 of a 16-row block, chunks g and g + 4 of its
+  // eight (g = lane / 16), each in slot chunk ^ ((row >> 1) & 7).  Any split of
+  // the 128 bytes over the four g will do that both operands share; with chunks
+  // 2 g and 2 g + 1 the reads met in the banks (25 % of the kernel's cycles by
+  // the counter: the LDS serves a 16-byte read to lanes of two neighbouring g at
+  // a time, whose slots stay apart if their chunks differ in bit 0).
+  const int frag_row = lane & 15, group = lane >> 4;
+  uint32_t frag_off[2];
 #pragma unroll
-  for (int kh = 0; kh < 2; ++kh)
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-      frag_off[kh][c] = static_cast<uint32_t>(frag_row * Cfg::kRowBytes + (((4 * kh + 2 * h + c) ^ ((frag_row >> 1) & 7)) * 16));
-  auto read_frag = [&](int stage_off, int operand_off, int block, int kh) -> v8i32 {
-    const uint8_t* base = lds_bytes + stage_off + operand_off + block * 32 * Cfg::kRowBytes;
-    const u32x4 lo = *reinterpret_cast<const u32x4*>(base + frag_off[kh][0]);
-    const u32x4 hi = *reinterpret_cast<const u32x4*>(base + frag_off[kh][1]);
+  for (int c = 0; c < 2; ++c)
+    frag_off[c] = static_cast<uint32_t>(frag_row * Cfg::kRowBytes + (((group + 4 * c) ^ ((frag_row >> 1) & 7)) * 16));
+  auto read_frag = [&](int stage_off, int operand_off, int block) -> v8i32 {
+    const uint8_t* base = lds_bytes + stage_off + operand_off + block * 16 * Cfg::kRowBytes;
+    const u32x4 lo = *reinterpret_cast<const u32x4*>(base + frag_off[0]);
+    const u32x4 hi = *reinterpret_cast<const u32x4*>(base + frag_off[1]);
     return v8i32{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z), static_cast<int>(lo.w),
                  static_cast<int>(hi.x), static_cast<int>(hi.y), static_cast<int>(hi.z), static_cast<int>(hi.w)};
   };
 
-  // Scales: a lane owns output row lane & 31 of each of its two 32-row blocks,
-  // so it needs xs[kb][row] for two rows and the one weight scale of the
-  // wave's 128 columns.
+  // Scales: a lane owns output row lane & 15 of each of its 16-row blocks, so it
+  // needs xs[kb][row] of those and the one weight scale of the wave's 128 columns.
   const int64_t wcol = n0 + wn * Cfg::kWaveN;
   const int64_t wblock = (wcol < p.n ? wcol : p.n - 1) / 128;
 
-  f32x16 acc[TM][TN];
+  f32x4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // Two stages: the operands of k-tile kt + 1 are in flight while kt is
   // multiplied.  The row scales ride the same global->LDS path (two 4-byte-
@@ -302,56 +311,53 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
     t_mark = now;
   };
 #endif
-  // The k loop is rotated by one block: the barrier that hands over k-tile
-  // kt + 1 sits before the last 32x32 block of k-tile kt, and behind that
-  // block's MFMAs the wave already reads what the first block of kt + 1 needs
-  // (its first A and B fragments).  The first MFMAs after a
-  // barrier thus never wait for an LDS read, which every wave of the
-  // workgroup would otherwise do at the same moment.
-  //   carried into a k-tile: afrag[0], bfrag[0]
-  constexpr int kBSets = kColumnScales ? 1 : 2;  // the per-column variant has registers for one set of B fragments only
+  // The k loop is rotated by a column of blocks: the barrier that hands over
+  // k-tile kt + 1 sits before the last column of k-tile kt, and behind each of
+  // its MFMAs the wave reads the fragment of kt + 1 that takes the place of the
+  // one just used.
+  //   carried into a k-tile: afrag, bfrag[0]
   constexpr int kBlocks = TM * TN;
-  v8i32 afrag[TM][2], bfrag[kBSets][2];
-  float s[TM], cs_rows[TN];
+  v8i32 afrag[TM], bfrag[2];
+  constexpr int kScaleRegs = TN / 4;
+  float s[TM], cs_rows[kScaleRegs];
   // Row scales of the wave's rows for the k-tile in `stage`, times the weight
   // block's scale in the block-scale variant.
   auto read_row_scales = [&](float (&dst)[TM], int stage, int64_t kt) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
       dst[i] = *reinterpret_cast<const float*>(lds_bytes + Cfg::kScaleOffset + stage * Cfg::kScaleStageBytes +
-                                               (wave * Cfg::kScaleSlots + i * 32 + frag_row) * 4);
+                                               (wave * Cfg::kScaleSlots + i * 16 + frag_row) * 4);
     if (!kColumnScales) {
       const float ws_now = ws_lds[kLongK ? (kt & (Cfg::kMaxKTilesInLds - 1)) : kt];
 #pragma unroll
       for (int i = 0; i < TM; ++i) dst[i] *= ws_now;
     }
   };
-  // Per-column scales: register j holds, in every row of 16 lanes, the 16
-  // scales of column block j that the lanes of that row fold with (lane n of
-  // the row the scale of accumulator element n), so a fold takes element n's
-  // scale from lane n of its own row through the data-parallel-primitive
-  // broadcast of the multiply-add itself: no scale is read from LDS between a
-  // product and its fold.
-  auto read_column_scales = [&](float (&dst)[TN], int stage) {
+  // Per-column scales: register q holds, in every row of 16 lanes, the 16
+  // scales that the lanes of that row fold column blocks 4 q .. 4 q + 3 with:
+  // lane 4 b + r of the row the scale of accumulator r of block 4 q + b.  A fold
+  // takes it through the data-parallel-primitive broadcast of the multiply-add
+  // itself: no scale is read from LDS between a product and its fold.
+  auto read_column_scales = [&](float (&dst)[kScaleRegs], int stage) {
     if (kColumnScales) {
       const uint8_t* cscale_lds = lds_bytes + Cfg::kWeightScaleOffset + stage * 1024 +
-                                  (wn * Cfg::kWaveN + 8 * ((lane & 15) >> 2) + 4 * h + (lane & 3)) * 4;
+                                  (wn * Cfg::kWaveN + 16 * ((lane & 15) >> 2) + 4 * group + (lane & 3)) * 4;
 #pragma unroll
-      for (int j = 0; j < TN; ++j) dst[j] = *reinterpret_cast<const float*>(cscale_lds + j * 32 * 4);
+      for (int q = 0; q < kScaleRegs; ++q) dst[q] = *reinterpret_cast<const float*>(cscale_lds + q * 64 * 4);
     }
   };
-  auto read_first_frags = [&](int stage_off) {
+  auto read_a = [&](int stage_off, int i) { afrag[i] = read_frag(stage_off, 0, wm * TM + i); };
+  auto read_b = [&](int stage_off, int j) { bfrag[j & 1] = read_frag(stage_off, Cfg::kABytes, wn * TN + j); };
+  read_b(0, 0);
 #pragma unroll
-    for (int kh = 0; kh < 2; ++kh) bfrag[0][kh] = read_frag(stage_off, Cfg::kABytes, wn * (Cfg::kWaveN / 32), kh);
-#pragma unroll
-    for (int kh = 0; kh < 2; ++kh) afrag[0][kh] = read_frag(stage_off, 0, wm * (Cfg::kWaveM / 32), kh);
-  };
-  read_first_frags(0);
+  for (int i = 0; i < TM; ++i) read_a(0, i);
 
   int stage = 0;
-  for (int64_t kt = 0; kt < ktiles; ++kt) {
+  // more: k-tile kt + 1 exists (its stage was released by the barrier inside kt - 1).
+  // A tag, so that no request sits behind a branch of its own.
+  auto k_tile = [&](int64_t kt, auto more_tag) {
+    constexpr bool more = decltype(more_tag)::value;
     const int stage_off = stage * Cfg::kStageBytes;
-    const bool more = kt + 1 < ktiles;  // the next k-tile's stage was released by the barrier inside kt - 1
     // The scales are first needed by the fold behind the second block's MFMAs.
     read_row_scales(s, stage, kt);
     read_column_scales(cs_rows, stage);
@@ -362,29 +368,21 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       issue_weight_scale_window(kt + 1);
     }
-    // Fragments are read in the order the blocks need them: the other A row
-    // blocks under the MFMAs of the first column block (they stay for the
-    // whole k-tile), each further B column block while the previous one is
-    // multiplied.
-    // The wave's eight 32x32 blocks, column block by column block: two MFMAs, back
-    // to back, give a block's partial product for this scale block.  It is
-    // folded into the result (16 fused multiply-adds, or multiply + fused
-    // multiply-add with per-column scales) one block later, behind that
-    // block's MFMAs: a fold that reads the product of the MFMA issued just
-    // before it waits for the matrix core to drain (measured: 122 against 100
-    // time units per block for the arrangement used here).
-    // Blocks between a product and its fold.  One: the other wave of the SIMD
-    // keeps the matrix core busy while this one waits for its own product,
-    // and the registers of a third product are needed elsewhere.
-    constexpr int kLag = 1;
-    f32x16 part[kLag + 1];
-    auto fold = [&](int blk, const f32x16& product) {
+    // The wave's 16x16 blocks, column by column.  One 16x16x128 MFMA gives a
+    // block's partial product for this scale block; it is folded into the result
+    // (4 fused multiply-adds, or multiply + fused multiply-add with per-column
+    // scales) kLag blocks later: a fold that reads the product of an MFMA issued
+    // just before it waits for the matrix core to drain.
+    constexpr int kLag = 4;
+    f32x4 part[kLag + 1];
+    auto fold = [&](int blk) {
       const int pi = blk % TM, pj = blk / TM;
+      const f32x4& product = part[blk % (kLag + 1)];
       if (kColumnScales) {
-        fold_with_row_broadcast(acc[pi][pj], product, s[pi], cs_rows[pj]);
+        fold_with_row_broadcast(acc[pi][pj], product, s[pi], cs_rows[pj / 4], pj % 4);
       } else {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[pi][pj][r] = __builtin_fmaf(product[r], s[pi], acc[pi][pj][r]);
+        for (int r = 0; r < 4; ++r) acc[pi][pj][r] = __builtin_fmaf(product[r], s[pi], acc[pi][pj][r]);
       }
       // An empty statement that "uses" the folded block keeps its arithmetic
       // on this side of the next scheduling barrier.
@@ -393,8 +391,8 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
 #pragma unroll
     for (int blk = 0; blk < kBlocks; ++blk) {
       const int i = blk % TM, j = blk / TM;
-      const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (blk == kBlocks - 1) {
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+      if (blk == kBlocks - TM) {
         // Every fragment of this k-tile is in registers: hand the stage over.
 #ifdef FSH_TRACE
         lap(t_compute);
@@ -403,20 +401,13 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
 #ifdef FSH_TRACE
         lap(t_wait);
 #endif
-        __syncthreads();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #ifdef FSH_TRACE
         lap(t_barrier);
 #endif
       }
-      if (j == 0 && i + 1 < TM) {  // next row block's A fragments
-#pragma unroll
-        for (int kh = 0; kh < 2; ++kh) afrag[i + 1][kh] = read_frag(stage_off, 0, wm * (Cfg::kWaveM / 32) + i + 1, kh);
-      }
-      if (kBSets == 2 && i == TM - 1 && j + 1 < TN) {  // next column block's B fragments, one block ahead
-#pragma unroll
-        for (int kh = 0; kh < 2; ++kh)
-          bfrag[(j + 1) % kBSets][kh] = read_frag(stage_off, Cfg::kABytes, wn * (Cfg::kWaveN / 32) + j + 1, kh);
-      }
+      // The next column's B fragment, a column ahead.
+      if (i == 0 && j + 1 < TN) read_b(stage_off, j + 1);
       // Wave priority falls as the k-tile proceeds: of the two waves of a SIMD
       // the one that is behind wins the issue slot, so both reach the barrier
       // together (with equal priorities the older wave runs ahead and then
@@ -426,39 +417,29 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
       if (blk * 4 == 1 * kBlocks) __builtin_amdgcn_s_setprio(2);
       if (blk * 4 == 2 * kBlocks) __builtin_amdgcn_s_setprio(1);
       if (blk * 4 == 3 * kBlocks) __builtin_amdgcn_s_setprio(0);
-      f32x16 product =
-          __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bfrag[j % kBSets][0], afrag[i][0], zero, 0, 0, 0, 0, 0, 0);
-      product =
-          __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bfrag[j % kBSets][1], afrag[i][1], product, 0, 0, 0, 0, 0, 0);
-      part[blk % (kLag + 1)] = product;
+      part[blk % (kLag + 1)] =
+          __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bfrag[j & 1], afrag[i], zero, 0, 0, 0, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
-      if (kBSets == 1 && i == TM - 1 && j + 1 < TN) {  // behind the last MFMAs that read the current set
-#pragma unroll
-        for (int kh = 0; kh < 2; ++kh)
-          bfrag[0][kh] = read_frag(stage_off, Cfg::kABytes, wn * (Cfg::kWaveN / 32) + j + 1, kh);
-      }
-      if (blk == kBlocks - 1 && more) {  // behind the last MFMAs of this k-tile: what the next one starts with
-        read_first_frags(stage_off ^ Cfg::kStageBytes);
+      if (blk >= kBlocks - TM && more) {  // what the next k-tile starts with
+        const int next_off = stage_off ^ Cfg::kStageBytes;
+        if (i == 0) read_b(next_off, 0);
+        read_a(next_off, i);
       }
       // The next k-tile's requests leave during the first half of this one, so
       // the data has the second half to arrive (spread over all blocks, the last
       // requests were still in flight at the hand-over: 0.15-0.35 us of every
-      // 2 us k-tile went to waiting for them; moved one block earlier still,
-      // behind the hand-over barrier of the previous k-tile, the per-column
-      // variant ran out of registers).
-      constexpr int kIssueBlocks = kBlocks / 2;
-      constexpr int kPartsPerBlock = (Cfg::kLoadsA + Cfg::kLoadsB + kIssueBlocks - 1) / kIssueBlocks;
-      if (more && blk < kIssueBlocks) {
-#pragma unroll
-        for (int part = 0; part < kPartsPerBlock; ++part) issue_k_tile_part(kt + 1, stage ^ 1, blk * kPartsPerBlock + part);
-      }
-      if (blk >= kLag) fold(blk - kLag, part[(blk - kLag) % (kLag + 1)]);
+      // 2 us k-tile went to waiting for them).
+      constexpr int kParts = Cfg::kLoadsA + Cfg::kLoadsB, kIssueEvery = kBlocks / 2 / kParts;
+      if (more && blk % kIssueEvery == kIssueEvery - 1 && blk < kBlocks / 2) issue_k_tile_part(kt + 1, stage ^ 1, blk / kIssueEvery);
+      if (blk >= kLag) fold(blk - kLag);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int blk = kBlocks - kLag; blk < kBlocks; ++blk) fold(blk, part[blk % (kLag + 1)]);
+    for (int blk = kBlocks - kLag; blk < kBlocks; ++blk) fold(blk);
     stage ^= 1;
-  }
+  };
+  for (int64_t kt = 0; kt + 1 < ktiles; ++kt) k_tile(kt, std::true_type{});
+  k_tile(ktiles - 1, std::false_type{});
 #ifdef FSH_TRACE
   if (p.schedule.trace && lane == 0) {
     uint64_t* out = p.schedule.trace + (static_cast<int64_t>(blockIdx.x) * Cfg::kWaves + wave) * 8;
@@ -473,11 +454,8 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        *reinterpret_cast<u32x2*>(region + (i * 32 + frag_row) * Cfg::kPitch + (j * 32 + 8 * b + 4 * h) * 2) =
-            u32x2{pack_bf16x2(acc[i][j][4 * b], acc[i][j][4 * b + 1]),
-                  pack_bf16x2(acc[i][j][4 * b + 2], acc[i][j][4 * b + 3])};
+      *reinterpret_cast<u32x2*>(region + (i * 16 + frag_row) * Cfg::kPitch + (j * 16 + 4 * group) * 2) =
+          u32x2{pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3])};
   wave_lds_sync();
   store_fp8_product<Cfg::kWaveM, Cfg::kWaveN, Cfg::kPitch>(region, p, m0 + wm * Cfg::kWaveM, n0 + wn * Cfg::kWaveN, lane);
 #ifdef FSH_TRACE
@@ -595,7 +573,7 @@ Fp8TileKind fp8_tile_kind(int64_t m, int64_t n, int64_t k, bool column_scales, i
   static constexpr TileShape kShapes[] = {
       {64, 64, 768.0, 0.22, 0.34, 0.61, 2.0},    // three workgroups per compute unit
       {128, 128, 512.0, 0.56, 0.69, 1.07, 4.0},  // two
-      {256, 256, 256.0, 0.75, 1.06, 1.59, 5.0},  // one; a round of at most half as many is cut into half tiles
+      {256, 256, 256.0, 0.72, 0.99, 1.48, 5.0},  // one; a round of at most half as many is cut into half tiles
   };
   const double ktiles = static_cast<double>(k / 128);
   int best = 0;

@@ -72,6 +72,28 @@ __device__ __forceinline__ void fold_with_row_broadcast(f32x16& acc, const f32x1
   }
 }
 
+// The same for a block of 16 x 16: element r takes the scale of lane 4 block + r
+// of its row of 16 lanes (block is a constant after unrolling).
+template <int N>
+__device__ __forceinline__ float fold_one_with_row_broadcast(float sum, float scaled, float column_scales) {
+  asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(sum) : "v"(column_scales), "v"(scaled), "n"(N));
+  return sum;
+}
+template <int kBlock>
+__device__ __forceinline__ void fold_block_with_row_broadcast(f32x4& acc, const f32x4& product, float row_scale, float column_scales) {
+  acc[0] = fold_one_with_row_broadcast<4 * kBlock + 0>(acc[0], product[0] * row_scale, column_scales);
+  acc[1] = fold_one_with_row_broadcast<4 * kBlock + 1>(acc[1], product[1] * row_scale, column_scales);
+  acc[2] = fold_one_with_row_broadcast<4 * kBlock + 2>(acc[2], product[2] * row_scale, column_scales);
+  acc[3] = fold_one_with_row_broadcast<4 * kBlock + 3>(acc[3], product[3] * row_scale, column_scales);
+}
+__device__ __forceinline__ void fold_with_row_broadcast(f32x4& acc, const f32x4& product, float row_scale, float column_scales,
+                                                        int block) {
+  if (block == 0) fold_block_with_row_broadcast<0>(acc, product, row_scale, column_scales);
+  else if (block == 1) fold_block_with_row_broadcast<1>(acc, product, row_scale, column_scales);
+  else if (block == 2) fold_block_with_row_broadcast<2>(acc, product, row_scale, column_scales);
+  else fold_block_with_row_broadcast<3>(acc, product, row_scale, column_scales);
+}
+
 // Four waves, WM x WN, each TM x TN blocks of 32 x 32; a k-tile is one scale
 // block (128 bytes of every row) with its row scales and column scales.
 template <int WM_, int WN_, int TM_, int TN_, int kStages_>
