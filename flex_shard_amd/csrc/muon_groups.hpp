@@ -163,6 +163,63 @@ __device__ __forceinline__ float muon_prepare_slice(const MuonLaunch& launch, co
   const MasterVector<kF32, kPadded> master{q};
   constexpr int kUnroll = kF32 ? 2 : 4;
   float s = 0.0f;
+  if constexpr (kF32 && !kPadded) {
+    // fp32 accesses contiguous across the wave: lane l takes the four-element
+    // chunks l and 64 + l of its 64 vectors.  (Vector by vector, a lane's two
+    // 16-byte accesses lie 32 bytes apart and each asks for half of every line:
+    // 101 M elements 281 us that way, 269 here, 253 with streaming stores.)  The rounded results then
+    // change lanes, so that lane l has vector l: the sums of squares keep their
+    // order.
+    const int lane = threadIdx.x & 63;
+    const int64_t chunks = 2 * end;
+    float* moms = static_cast<float*>(mom);
+    const float* grads = static_cast<const float*>(grad);
+    for (int64_t w0 = begin + threadIdx.x - lane; w0 < end; w0 += kUnroll * kNormThreads) {  // (the same in the whole wave)
+      f32x4 mv[kUnroll][2], gv[kUnroll][2];
+#pragma unroll
+      for (int k = 0; k < kUnroll; ++k)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int64_t c = 2 * (w0 + k * kNormThreads) + 64 * h + lane;
+          mv[k][h] = gv[k][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (c < chunks) {
+            mv[k][h] = load_stream_f32x4(moms + c * 4);
+            gv[k][h] = load_stream_f32x4(grads + c * 4);
+          }
+        }
+#pragma unroll
+      for (int k = 0; k < kUnroll; ++k) {
+        u32x2 words[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int64_t c = 2 * (w0 + k * kNormThreads) + 64 * h + lane;
+          uint32_t ob[4];
+          float mo[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            muon_prepare_one_f32(mv[k][h][j], gv[k][h][j], launch.one_minus_mu, launch.mu, launch.nesterov, &mo[j], &ob[j]);
+          words[h] = u32x2{ob[0] | (ob[1] << 16), ob[2] | (ob[3] << 16)};
+          if (c < chunks) __builtin_nontemporal_store(f32x4{mo[0], mo[1], mo[2], mo[3]}, reinterpret_cast<f32x4*>(moms + c * 4));
+        }
+        u32x4 u;
+#pragma unroll
+        for (int part = 0; part < 2; ++part)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int from = ((2 * lane + part) & 63) * 4;
+            const int first = __builtin_amdgcn_ds_bpermute(from, static_cast<int>(words[0][j]));
+            const int second = __builtin_amdgcn_ds_bpermute(from, static_cast<int>(words[1][j]));
+            u[2 * part + j] = static_cast<uint32_t>(lane < 32 ? first : second);
+          }
+        const int64_t g = w0 + k * kNormThreads + lane;
+        if (g < end) {
+          store_stream_u32x4(out + g * 8, u);
+          s = add_squares8(s, u);
+        }
+      }
+    }
+    return s;
+  }
   for (int64_t g0 = begin + threadIdx.x; g0 < end; g0 += kUnroll * kNormThreads) {
     float mv[kUnroll][8], gv[kUnroll][8];
 #pragma unroll
