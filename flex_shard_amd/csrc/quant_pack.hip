@@ -399,7 +399,14 @@ __device__ __forceinline__ void quant_tile128_fast(const FastChunk& ch, uint32_t
   const uint32_t n = FULL || !RAGGED ? 8 : static_cast<uint32_t>(ch.in_dim) - col;  // elements left in the row (if col_ok)
   const int64_t src_row_bytes = ch.src_row_bytes;
   const int64_t dst_row_bytes = ch.in_dim;
-  const uint8_t* sp = ch.src + static_cast<int64_t>(row0) * src_row_bytes + static_cast<int64_t>(col) * (F32 ? 4 : 2);
+  // Whole tiles of aligned fp32 rows are read 16 bytes a lane, contiguous across
+  // the row's sixteen lanes: columns 4 g .. and 64 + 4 g ...  (Eight consecutive
+  // elements a lane are two accesses 32 bytes apart, each asking for half of
+  // every line: 80 M elements 77 us that way, 66 here; 23 M 23.0 and 20.5.)  The
+  // FP8 bytes change lanes before they are stored.
+  constexpr bool kQuarters = F32 && FULL && !RAGGED;
+  const uint8_t* sp = ch.src + static_cast<int64_t>(row0) * src_row_bytes +
+                      static_cast<int64_t>(kQuarters ? tc * 128u + g * 4u : col) * (F32 ? 4 : 2);
   uint8_t* dp = ch.qdst + static_cast<int64_t>(row0) * dst_row_bytes + col;
   float* scale_slot = ch.scales + static_cast<int64_t>(tr) * ch.tiles_c + tc;
 
@@ -423,7 +430,10 @@ __device__ __forceinline__ void quant_tile128_fast(const FastChunk& ch, uint32_t
         const int k = 4 * half + j;
         a[j] = f32x4{0.f, 0.f, 0.f, 0.f};
         b[j] = a[j];
-        if (FULL || (col_ok && row0 + 16u * k < rows)) {
+        if (kQuarters) {
+          a[j] = load_stream_f32x4(sp + 16 * k * src_row_bytes);
+          b[j] = load_stream_f32x4(sp + 16 * k * src_row_bytes + 256);
+        } else if (FULL || (col_ok && row0 + 16u * k < rows)) {
           load_f32_group<RAGGED>(sp + 16 * k * src_row_bytes, n, &a[j], &b[j]);
         }
       }
@@ -473,17 +483,27 @@ __device__ __forceinline__ void quant_tile128_fast(const FastChunk& ch, uint32_t
 
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    if (FULL || (col_ok && row0 + 16u * k < rows)) {
-      const uint32_t d[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-      uint32_t w[2] = {0, 0};
+    const uint32_t d[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+    uint32_t w[2] = {0, 0};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float e0 = u32_as_f32(d[j] << 16) * scale;
-        const float e1 = u32_as_f32(d[j] & 0xFFFF0000u) * scale;
-        w[j >> 1] = cvt2_fp8(e0, e1, w[j >> 1], (j & 1) != 0);
-      }
-      store_fp8_group<RAGGED>(dp + 16 * k * dst_row_bytes, n, w[0], w[1]);
+    for (int j = 0; j < 4; ++j) {
+      const float e0 = u32_as_f32(d[j] << 16) * scale;
+      const float e1 = u32_as_f32(d[j] & 0xFFFF0000u) * scale;
+      w[j >> 1] = cvt2_fp8(e0, e1, w[j >> 1], (j & 1) != 0);
     }
+    if (kQuarters) {  // columns 8 g .. of the lane are the row's quarters 2 g and 2 g + 1
+      uint32_t own[2];
+#pragma unroll
+      for (int part = 0; part < 2; ++part) {
+        const int from = static_cast<int>(((tid & 48u) + ((2u * g + part) & 15u)) * 4u);
+        const int low = __builtin_amdgcn_ds_bpermute(from, static_cast<int>(w[0]));
+        const int high = __builtin_amdgcn_ds_bpermute(from, static_cast<int>(w[1]));
+        own[part] = static_cast<uint32_t>(g < 8u ? low : high);
+      }
+      w[0] = own[0];
+      w[1] = own[1];
+    }
+    if (FULL || (col_ok && row0 + 16u * k < rows)) store_fp8_group<RAGGED>(dp + 16 * k * dst_row_bytes, n, w[0], w[1]);
   }
 }
 
