@@ -161,7 +161,7 @@ __device__ __forceinline__ float muon_prepare_slice(const MuonLaunch& launch, co
   const void* grad = reinterpret_cast<const void*>(uniform_i64(q.grad_ptrs[matrix]));
   uint16_t* out = q.batch + matrix * q.vectors * 8;
   const MasterVector<kF32, kPadded> master{q};
-  constexpr int kUnroll = kF32 ? 2 : 4;
+  constexpr int kUnroll = kF32 || kPadded ? 2 : 4;  // (four odd vectors would cost the whole launch occupancy)
   float s = 0.0f;
   if constexpr (kF32 && !kPadded) {
     // fp32 accesses contiguous across the wave: lane l takes the four-element
@@ -303,7 +303,7 @@ __device__ __forceinline__ void muon_apply_slice(const MuonLaunch& launch, const
   void* param = reinterpret_cast<void*>(uniform_i64(q.param_ptrs[matrix]));
   const uint16_t* dir = q.batch + matrix * q.vectors * 8;
   const MasterVector<kF32, kPadded> master{q};
-  constexpr int kUnroll = kF32 ? 2 : 4;
+  constexpr int kUnroll = kF32 || kPadded ? 2 : 4;  // (four odd vectors would cost the whole launch occupancy)
   if (kF32 && !kPadded) {
     // Every element is on its own, so fp32 masters go in chunks of four: one
     // 16-byte access contiguous across the wave.  Eight per lane are two of
