@@ -111,8 +111,9 @@ __device__ __forceinline__ void store_values8(uint8_t* dq, uint32_t idx, const f
 // wherever the width is no multiple of 128, and completed by workgroups on
 // other XCDs.  Us there / here: 25.5 M values of widths 3344 and 384 54 / 33,
 // 87 M of 2605 to 10112 83 / 59 (6.1 TB/s), 14 M of 1000 to 3000 28 / 17, the
-// eight rank rows of a 218 M layer 146 / 131 (6.7 TB/s), 67 M of 4096 on one
-// rank 44 / 46.
+// eight rank rows of a 218 M layer still in the last-level cache, as after a
+// gather, 146 / 131 (6.7 TB/s).  Slower here: the same rows from HBM 158 / 164,
+// 67 M of 4096 on one rank 44 / 46.
 template <int DQ, bool kAligned>
 __device__ __forceinline__ void unpack_piece(const uint8_t* src, uint8_t* cq, uint8_t* dq, const uint8_t* scales, int64_t rows,
                                              int64_t in_dim, int64_t tiles_c, int64_t t, int64_t tiles, int64_t lead, int tid) {
