@@ -86,14 +86,16 @@ __device__ __forceinline__ int64_t divide(int64_t a, int64_t b) {
   return a / b;
 }
 
-// Eight dequantized values to dq[idx ..], 16-byte aligned.
+// Eight dequantized values to dq[idx ..], 16-byte aligned.  fp32 ones are two
+// stores of every other 16 bytes: plain, so that the caches put them together
+// (59 M values to fp32, just gathered: 130 us with the streaming hint, 57 without).
 template <int DQ>
 __device__ __forceinline__ void store_values8(uint8_t* dq, uint32_t idx, const float (&f)[8]) {
   if (DQ == FSH_DT_F32) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      store_stream_u32x4(dq + idx * 4 + 16 * j, u32x4{f32_as_u32(f[4 * j]), f32_as_u32(f[4 * j + 1]),
-                                                      f32_as_u32(f[4 * j + 2]), f32_as_u32(f[4 * j + 3])});
+      *reinterpret_cast<u32x4*>(dq + idx * 4 + 16 * j) = u32x4{f32_as_u32(f[4 * j]), f32_as_u32(f[4 * j + 1]),
+                                                               f32_as_u32(f[4 * j + 2]), f32_as_u32(f[4 * j + 3])};
     return;
   }
   u32x4 o;
@@ -109,11 +111,19 @@ __device__ __forceinline__ void store_values8(uint8_t* dq, uint32_t idx, const f
 // Piece t of `tiles` of a chunk.  `scales`: the chunk's table [rows / 128][in_dim / 128].
 // With a tile's own 128 rows per workgroup, memory lines were written in pieces
 // wherever the width is no multiple of 128, and completed by workgroups on
-// other XCDs.  Us there / here: 25.5 M values of widths 3344 and 384 54 / 33,
-// 87 M of 2605 to 10112 83 / 59 (6.1 TB/s), 14 M of 1000 to 3000 28 / 17, the
-// eight rank rows of a 218 M layer still in the last-level cache, as after a
-// gather, 146 / 131 (6.7 TB/s).  Slower here: the same rows from HBM 158 / 164,
-// 67 M of 4096 on one rank 44 / 46.
+// other XCDs.  All loads of a piece go out ahead of its first store and without
+// a branch between them, and nothing that waits for memory (the ends of a run
+// that are no whole group, the scale's own copy) comes before them.  Us with a
+// tile per workgroup / a branch per load / here, rows from HBM and (just
+// gathered, in the last-level cache):
+//   218 M layer on eight ranks      169 / 165 / 153     (162 / 150 / 146)
+//   67 M of 4096 on one             58 / 56 / 52        (44 / 47 / 45)
+//   33 M of 4104 on three           57 / 36 / 31        (55 / 32 / 26)
+//   16.8 M of 4096 on one           17.6 / 17.6 / 17.9  (15.4 / 16.9 / 16.4)
+//   2.1 M of 4096 on one            7.9 / 9.9 / 8.2     (9.2 / 10.4 / 9.2)
+//   59 M of 4096 to fp32            90 / 121 / 83       (102 / 130 / 57)
+// A tile per workgroup stays up to 1 us ahead on whole tiles of 8 to 17 M
+// elements from HBM (one scale instead of one per group): no second form for that.
 template <int DQ, bool kAligned>
 __device__ __forceinline__ void unpack_piece(const uint8_t* src, uint8_t* cq, uint8_t* dq, const uint8_t* scales, int64_t rows,
                                              int64_t in_dim, int64_t tiles_c, int64_t t, int64_t tiles, int64_t lead, int tid) {
@@ -126,43 +136,34 @@ __device__ __forceinline__ void unpack_piece(const uint8_t* src, uint8_t* cq, ui
   };
   lead = lead < n ? lead : n;
   const int64_t groups = (n - lead) / 8, per = (divide(groups + tiles - 1, tiles) + 15) / 16 * 16;
-  const int64_t edge = t == 0 && tid < lead ? tid : t == tiles - 1 && lead + 8 * groups + tid < n ? lead + 8 * groups + tid : -1;
-  if (edge >= 0) {  // (fewer than 128 elements in front, than eight behind; a chunk of one piece has both ends)
-    for (int64_t idx = edge; idx >= 0;) {
-      const uint8_t b = src[idx];
-      if (cq) cq[idx] = b;
-      const int64_t row = idx / in_dim;
-      if (dq) store_value<DQ>(dq, idx, __builtin_amdgcn_cvt_f32_fp8(static_cast<int>(b), 0) * scale_at(row, static_cast<uint32_t>(idx - row * in_dim)));
-      const int64_t last = lead + 8 * groups + tid;
-      idx = idx < lead && t == tiles - 1 && last < n ? last : -1;
-    }
-  }
   const int64_t first = t * per, end = first + per < groups ? first + per : groups;  // per <= 2048: a tile has 16384 elements at most
   const int64_t idx0 = lead + 8 * first, row0 = divide(idx0, in_dim);
   const uint32_t width = static_cast<uint32_t>(in_dim), col0 = static_cast<uint32_t>(idx0 - row0 * in_dim);
   const bool splits = (width & 7) != 0 || (col0 & 7) != 0;  // groups that reach into the next tile or row
   const uint32_t count = first < end ? static_cast<uint32_t>(end - first) : 0;
-  src += idx0;
-  if (cq) cq += idx0;
-  if (dq) dq += idx0 * kElem;
+  const uint8_t* run = src + idx0;
+  uint8_t* run_cq = cq ? cq + idx0 : nullptr;
+  uint8_t* run_dq = dq ? dq + idx0 * kElem : nullptr;
   u32x2 vin[kPasses];
   uint32_t cols[kPasses], belows[kPasses];
   float scale[kPasses];
+  if (count > 0) {
 #pragma unroll
-  for (int k = 0; k < kPasses; ++k) {
-    const uint32_t g = k * kThreads + tid;
-    if (g >= count) break;
-    vin[k] = load_group<u32x2, kAligned>(src + 8 * g);
-    const uint32_t c = col0 + 8 * g;
-    belows[k] = c / width;
-    cols[k] = c - belows[k] * width;
-    if (dq) scale[k] = scale_at(row0 + belows[k], cols[k]);
+    for (int k = 0; k < kPasses; ++k) {
+      // (groups past the piece's end: its last one again)
+      const uint32_t g = min(static_cast<uint32_t>(k * kThreads + tid), count - 1);
+      vin[k] = load_group<u32x2, kAligned>(run + 8 * g);
+      const uint32_t c = col0 + 8 * g;
+      belows[k] = c / width;
+      cols[k] = c - belows[k] * width;
+      if (dq) scale[k] = scale_at(row0 + belows[k], cols[k]);
+    }
   }
 #pragma unroll
   for (int k = 0; k < kPasses; ++k) {
     const uint32_t g = k * kThreads + tid;
     if (g >= count) break;
-    if (cq) store_group<kAligned>(cq + 8 * g, vin[k]);
+    if (cq) store_group<kAligned>(run_cq + 8 * g, vin[k]);
     if (!dq) continue;
     float f[8];
     if (!splits) {
@@ -188,7 +189,18 @@ __device__ __forceinline__ void unpack_piece(const uint8_t* src, uint8_t* cq, ui
 #pragma unroll
       for (uint32_t j = 0; j < 8; ++j) f[j] *= j < cut ? scale[k] : j < cut2 ? s1 : s2;
     }
-    store_values8<DQ>(dq, 8 * g, f);
+    store_values8<DQ>(run_dq, 8 * g, f);
+  }
+  const int64_t edge = t == 0 && tid < lead ? tid : t == tiles - 1 && lead + 8 * groups + tid < n ? lead + 8 * groups + tid : -1;
+  if (edge >= 0) {  // (fewer than 128 elements in front, than eight behind; a chunk of one piece has both ends)
+    for (int64_t idx = edge; idx >= 0;) {
+      const uint8_t b = src[idx];
+      if (cq) cq[idx] = b;
+      const int64_t row = idx / in_dim;
+      if (dq) store_value<DQ>(dq, idx, __builtin_amdgcn_cvt_f32_fp8(static_cast<int>(b), 0) * scale_at(row, static_cast<uint32_t>(idx - row * in_dim)));
+      const int64_t last = lead + 8 * groups + tid;
+      idx = idx < lead && t == tiles - 1 && last < n ? last : -1;
+    }
   }
 }
 
@@ -225,7 +237,6 @@ __global__ __launch_bounds__(kThreads) void unpack_dequant_kernel(
 
   const uint8_t* scales = rows + ch.src_scale_offset;
   const float scale = load_f32_any(scales + 4 * t);
-  if (compact != nullptr && tid == 0) store_f32_any(compact + ch.dst_scale_offset + 4 * t, scale);
 
   const uint8_t* src = rows + ch.src_qdata_offset;
   uint8_t* cq = compact ? compact + ch.dst_qdata_offset : nullptr;
@@ -240,10 +251,12 @@ __global__ __launch_bounds__(kThreads) void unpack_dequant_kernel(
       unpack_piece<DQ, true>(src, cq, dq, scales, ch.rows, ch.in_dim, tiles_c, t, tiles, lead, tid);
     else
       unpack_piece<DQ, false>(src, cq, dq, scales, ch.rows, ch.in_dim, tiles_c, t, tiles, lead, tid);
+    if (compact != nullptr && tid == 0) store_f32_any(compact + ch.dst_scale_offset + 4 * t, scale);
     return;
   }
 
   // Element-wise path.
+  if (compact != nullptr && tid == 0) store_f32_any(compact + ch.dst_scale_offset + 4 * t, scale);
   const int64_t tr = t / tiles_c, tc = t - tr * tiles_c;
   const int64_t row0 = tr * block, col0 = tc * block;
   const int64_t nrows = (ch.rows - row0) < block ? (ch.rows - row0) : block;
