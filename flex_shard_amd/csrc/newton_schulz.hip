@@ -275,7 +275,7 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
       a_left = static_cast<int>(m_left < Cfg::BM ? m_left : Cfg::BM);
       b_left = static_cast<int>(n_left < Cfg::BN ? n_left : Cfg::BN);
     }
-    derive_requests(lane_now(), kRagged && q.K < Cfg::BK ? static_cast<int>(q.K / 8) : 8);
+    derive_requests(lane_now(), 8);  // (a contraction that ends inside a k-tile has at least three)
     issue_operand(Ab, a_voff, 0);
     issue_operand(Bb, b_voff, Cfg::kOperandBytes);
   };
@@ -411,7 +411,6 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
 #pragma unroll
     for (int g = 0; g < TM + TN; ++g) read_frag(0, 0, Cfg::kOperandBytes, 0, g);
     if (ktiles > 1) {
-      if (kRagged && ktiles == 2 && tail) derive_requests(lane_now(), tail);
       issue_operand(k_tile_ptr(Ab, a_row_bytes, 1), a_voff, 2 * Cfg::kOperandBytes);
       issue_operand(k_tile_ptr(Bb, b_row_bytes, 1), b_voff, 3 * Cfg::kOperandBytes);
     }
@@ -540,8 +539,10 @@ constexpr double kEstimateMargin = 0.95;  // the estimates are off by about 5 %
 double small_tiles_us(const LaunchWork& w) { return launch_us(small_tile_kind(w), w); }
 
 // The 256 x 256 kernel has 16-byte accesses in the epilogue and 32-bit tile spans.
+// It aims its requests at a k-tile that the contraction ends in only inside the
+// k loop, two k-tiles ahead: with the tile's third at the earliest.
 bool fits_large_tiles(const GemmParams& p) {
-  return p.M % 8 == 0 && p.N % 8 == 0 && p.K % 8 == 0 && p.ldc % 8 == 0 &&
+  return p.M % 8 == 0 && p.N % 8 == 0 && p.K % 8 == 0 && (p.K % DmaGemm::BK == 0 || p.K > 2 * DmaGemm::BK) && p.ldc % 8 == 0 &&
          (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && p.sC % 8 == 0 &&
          (p.Ct == nullptr || (p.ldct % 8 == 0 && (reinterpret_cast<uintptr_t>(p.Ct) & 15) == 0 && p.sCt % 8 == 0)) &&
          (p.D == nullptr || (p.ldd % 8 == 0 && (reinterpret_cast<uintptr_t>(p.D) & 15) == 0 && p.sD % 8 == 0)) &&
