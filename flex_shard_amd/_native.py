@@ -172,6 +172,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "fsh_gemm_bf16_nt": (c_int, [POINTER(GemmDesc), c_void_p]),
     "fsh_gemm_bf16_tiles": (c_int, [POINTER(c_int64), c_int32, POINTER(c_int32)]),
     "fsh_newton_schulz_tiles": (c_int, [POINTER(NsProblem), c_int32, c_int32, POINTER(c_int32)]),
+    "fsh_newton_schulz_product_tiles": (c_int, [POINTER(NsProblem), c_int32, c_int32, c_int32, c_int32, POINTER(c_int32)]),
     "fsh_fp8_gemm_tiles": (c_int, [c_int64, c_int64, c_int64, c_int32]),
     "fsh_gemm_bf16_nt_group": (c_int, [POINTER(GemmDesc), c_int32, c_void_p]),
     "fsh_act_quant_1x128": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p, c_int32, c_void_p]),

@@ -786,27 +786,43 @@ void choose_free_products(PlannedGemm* plans, int count) {
   for (int i = 0; i < count; ++i) plans[i].large = plans[i].large || candidate(plans[i]);
 }
 
-// `large` (null: decided here): the problems that take the large-tile kernel at least.
+// Plans `count` products that may share launches.  `large` (null: decided here):
+// the problems that take the large-tile kernel at least.
+constexpr int kPlannedTogether = 16;
+int plan_gemms(const fsh_gemm_desc* descs, int count, const GemmUpdate* updates, const bool* large, PlannedGemm* plans) {
+  for (int i = 0; i < count; ++i) {
+    if (int rc = plan_gemm(descs[i], &plans[i], updates ? &updates[i] : nullptr)) return rc;
+    if (large != nullptr) {
+      plans[i].large = large[i];
+      if (large[i] && !plans[i].fits) return fail(FSH_ENOTSUP, "gemm: a product does not fit the large tiles");
+    }
+  }
+  if (large == nullptr) return choose_kernels(plans, count);
+  choose_free_products(plans, count);
+  return FSH_OK;
+}
 int launch_gemms(const fsh_gemm_desc* descs, int count, hipStream_t stream, const GemmUpdate* updates = nullptr,
                  const bool* large = nullptr) {
-  constexpr int kChunk = 16;
-  PlannedGemm plans[kChunk];
-  for (int begin = 0; begin < count; begin += kChunk) {
-    const int n = count - begin < kChunk ? count - begin : kChunk;
-    for (int i = 0; i < n; ++i) {
-      if (int rc = plan_gemm(descs[begin + i], &plans[i], updates ? &updates[begin + i] : nullptr)) return rc;
-      if (large != nullptr) {
-        plans[i].large = large[begin + i];
-        if (large[begin + i] && !plans[i].fits) return fail(FSH_ENOTSUP, "gemm: a product does not fit the large tiles");
-      }
-    }
-    if (large != nullptr)
-      choose_free_products(plans, n);
-    else if (int rc = choose_kernels(plans, n))
-      return rc;
+  PlannedGemm plans[kPlannedTogether];
+  for (int begin = 0; begin < count; begin += kPlannedTogether) {
+    const int n = count - begin < kPlannedTogether ? count - begin : kPlannedTogether;
+    if (int rc = plan_gemms(descs + begin, n, updates ? updates + begin : nullptr, large ? large + begin : nullptr, plans)) return rc;
     if (int rc = launch_planned(plans, n, stream)) return rc;
   }
   return FSH_OK;
+}
+
+// The FSH_TILES_* that launch_planned takes for planned products.
+void report_tiles(const PlannedGemm* plans, int count, int32_t* tiles) {
+  for (int next = 0; next < count;) {  // the small-tile launches, as launch_planned fills them
+    int members[TileLaunch::kMaxProblems], n = 0;
+    for (; next < count && n < TileLaunch::kMaxProblems; ++next) {
+      if (plans[next].large) tiles[next] = FSH_TILES_256;
+      else members[n++] = next;
+    }
+    const TileKind kind = small_tile_kind(work_of(plans, members, n));
+    for (int k = 0; k < n; ++k) tiles[members[k]] = kTileNames[kind];
+  }
 }
 
 // A caller's k-major product: refused below 192 large tiles, where a
@@ -849,10 +865,9 @@ FSH_API int fsh_gemm_bf16_nt_group(const fsh_gemm_desc* descs, int32_t count, vo
 
 FSH_API int fsh_gemm_bf16_tiles(const int64_t* sizes, int32_t count, int32_t* tiles) {
   using namespace fsh;
-  constexpr int kMost = 16;  // products of one call that share launches
-  if (count < 0 || count > kMost || (count > 0 && (!sizes || !tiles))) return fail(FSH_EINVAL, "fsh_gemm_bf16_tiles: bad list");
+  if (count < 0 || count > kPlannedTogether || (count > 0 && (!sizes || !tiles))) return fail(FSH_EINVAL, "fsh_gemm_bf16_tiles: bad list");
   static __attribute__((aligned(16))) uint8_t somewhere[16];  // (looked at for its alignment alone)
-  PlannedGemm plans[kMost];
+  PlannedGemm plans[kPlannedTogether];
   for (int i = 0; i < count; ++i) {
     fsh_gemm_desc d;
     memset(&d, 0, sizeof(d));
@@ -864,15 +879,7 @@ FSH_API int fsh_gemm_bf16_tiles(const int64_t* sizes, int32_t count, int32_t* ti
     if (int rc = plan_gemm(d, &plans[i])) return rc;
   }
   if (int rc = choose_kernels(plans, count)) return rc;
-  for (int next = 0; next < count;) {  // the small-tile launches, as launch_planned fills them
-    int members[TileLaunch::kMaxProblems], n = 0;
-    for (; next < count && n < TileLaunch::kMaxProblems; ++next) {
-      if (plans[next].large) tiles[next] = FSH_TILES_256;
-      else members[n++] = next;
-    }
-    const TileKind kind = small_tile_kind(work_of(plans, members, n));
-    for (int k = 0; k < n; ++k) tiles[members[k]] = kTileNames[kind];
-  }
+  report_tiles(plans, count, tiles);
   return FSH_OK;
 }
 
@@ -1141,6 +1148,31 @@ FSH_API int fsh_newton_schulz_tiles(const fsh_ns_problem* problems, int32_t coun
   bool takes_large[FSH_MAX_NS_PROBLEMS];
   ns_choose_large(problems, count, steps, takes_large);
   for (int i = 0; i < count; ++i) large[i] = takes_large[i] ? 1 : 0;
+  return FSH_OK;
+}
+
+FSH_API int fsh_newton_schulz_product_tiles(const fsh_ns_problem* problems, int32_t count, int32_t steps, int32_t product,
+                                            int32_t last_step, int32_t* tiles) {
+  using namespace fsh;
+  if (count < 0 || count > FSH_MAX_NS_PROBLEMS || (count > 0 && (!problems || !tiles)) || steps <= 0 || product < 0 || product > 2)
+    return fail(FSH_EINVAL, "fsh_newton_schulz_product_tiles: bad list, step count or product");
+  void* const somewhere = reinterpret_cast<void*>(static_cast<uintptr_t>(4096));  // (looked at for its alignment alone)
+  bool large[FSH_MAX_NS_PROBLEMS];
+  ns_choose_large(problems, count, steps, large);
+  fsh_gemm_desc descs[FSH_MAX_NS_PROBLEMS];
+  for (int i = 0; i < count; ++i) {
+    fsh_ns_problem q = problems[i];
+    q.x_dev = q.workspace_dev = somewhere;
+    q.workspace_nbytes = fsh_newton_schulz_workspace_bytes(q.batch, q.rows, q.cols);
+    NsState st;
+    NormalizeGroup unused;
+    if (int rc = ns_begin(q, large[i], steps, &st, &unused)) return rc;
+    descs[i] = ns_product(st, product, 1.0f, 1.0f, 1.0f, last_step != 0);
+  }
+  PlannedGemm plans[kPlannedTogether];
+  static_assert(FSH_MAX_NS_PROBLEMS <= kPlannedTogether, "one group of launches");
+  if (int rc = plan_gemms(descs, count, nullptr, large, plans)) return rc;
+  report_tiles(plans, count, tiles);
   return FSH_OK;
 }
 

@@ -38,6 +38,7 @@ __all__ = [
     "copy_row_segments", "copy_segments", "fp8_gemm_1x128_128x1", "fp8_gemm_1x128_128x128", "fp8_gemm_1x128_128x128_dgrad",
     "fp8_gemm_tiles", "fp8_linear_backward", "fp8_transpose", "gemm_nt", "gemm_nt_group", "gemm_tiles", "muon_apply",
     "muon_prepare", "newton_schulz_multi", "newton_schulz", "newton_schulz_large_tiles", "newton_schulz_noalloc",
+    "newton_schulz_product_tiles",
     "newton_schulz_workspace_bytes", "pack_segments", "quantize_pack", "reduce_rows", "stream_ptr", "unpack_dequant", "zero_segments",
 ]
 
@@ -541,15 +542,31 @@ def gemm_tiles(*problems: tuple) -> tuple[str, ...]:
     return tuple(GEMM_TILES[t] for t in tiles)
 
 
-def newton_schulz_large_tiles(*shapes: tuple[int, int, int], steps: int = 5) -> tuple[bool, ...]:
-    """Whether each (batch, rows, cols) of one :func:`newton_schulz_multi` call
-    iterates on the 256 x 256 tiles (no GPU needed)."""
+def _ns_problem_sizes(shapes: Sequence[tuple[int, int, int]]):
     problems = (_native.NsProblem * len(shapes))()
     for q, (batch, rows, cols) in zip(problems, shapes):
         q.batch, q.rows, q.cols = batch, rows, cols
+    return problems
+
+
+def newton_schulz_large_tiles(*shapes: tuple[int, int, int], steps: int = 5) -> tuple[bool, ...]:
+    """Whether each (batch, rows, cols) of one :func:`newton_schulz_multi` call
+    iterates on the 256 x 256 tiles (no GPU needed)."""
     large = (ctypes.c_int32 * len(shapes))()
-    _native.check(_native.lib().fsh_newton_schulz_tiles(problems, len(shapes), steps, large), "fsh_newton_schulz_tiles")
+    status = _native.lib().fsh_newton_schulz_tiles(_ns_problem_sizes(shapes), len(shapes), steps, large)
+    _native.check(status, "fsh_newton_schulz_tiles")
     return tuple(map(bool, large))
+
+
+def newton_schulz_product_tiles(*shapes: tuple[int, int, int], product: int, steps: int = 5, last: bool = False) -> tuple[str, ...]:
+    """The tiles that product 0 (G), 1 (P) or 2 (X') of an iteration (``last``:
+    the last one) takes for each (batch, rows, cols) of one
+    :func:`newton_schulz_multi` call (no GPU needed)."""
+    tiles = (ctypes.c_int32 * len(shapes))()
+    status = _native.lib().fsh_newton_schulz_product_tiles(
+        _ns_problem_sizes(shapes), len(shapes), steps, product, 1 if last else 0, tiles)
+    _native.check(status, "fsh_newton_schulz_product_tiles")
+    return tuple(GEMM_TILES[t] for t in tiles)
 
 
 def fp8_gemm_tiles(m: int, n: int, k: int, *, column_scales: bool = False) -> str:

@@ -306,6 +306,10 @@ int fsh_gemm_bf16_nt_group(const fsh_gemm_desc* descs, int32_t count, void* stre
  * products of one call (at most 16), their FSH_TILES_* to tiles [count].
  * fsh_newton_schulz_tiles: for the problems of one call of (6) (rows, cols and
  * batch are read) whether each iterates on the 256 x 256 tiles.
+ * fsh_newton_schulz_product_tiles: the FSH_TILES_* of each of those problems'
+ * product 0 (G = X X^T), 1 (P) or 2 (X' = P X) of one iteration, the last one if
+ * last_step; a problem that iterates on smaller tiles may take the large ones
+ * for a product on its own.
  * fsh_fp8_gemm_tiles: the FSH_TILES_* of a product of (8) and (9), negative on
  * bad sizes; column_scales: of fsh_fp8_gemm_1x128_128x1. */
 #define FSH_TILES_64 0
@@ -317,6 +321,8 @@ int fsh_gemm_bf16_nt_group(const fsh_gemm_desc* descs, int32_t count, void* stre
 #define FSH_TILES_256_LONG_K 6
 int fsh_gemm_bf16_tiles(const int64_t* sizes, int32_t count, int32_t* tiles);
 int fsh_newton_schulz_tiles(const fsh_ns_problem* problems, int32_t count, int32_t steps, int32_t* large);
+int fsh_newton_schulz_product_tiles(const fsh_ns_problem* problems, int32_t count, int32_t steps, int32_t product,
+                                    int32_t last_step, int32_t* tiles);
 int fsh_fp8_gemm_tiles(int64_t m, int64_t n, int64_t k, int32_t column_scales);
 
 /* ------------------------------------------------------------------------

@@ -1,6 +1,7 @@
 """Newton-Schulz on the 256 x 256 tiles where sizes are not whole tiles: edge
-tiles of a few rows and columns, contractions that end in any octet of a
-k-tile, tall, wide and square, and the update behind them."""
+tiles of a few rows and columns, contractions that end in every octet of a
+k-tile (bit for bit against the small tiles), tall, wide and square, products
+that take the large tiles on their own, and the update behind them."""
 
 import pytest
 import torch
@@ -31,15 +32,47 @@ def test_ragged_sizes_against_64_bits(device, shape, steps):
     _check(mine, start, steps, (0, batch - 1))
 
 
-@pytest.mark.parametrize("shape", [(1, 2248, 2248), (1, 3072, 3072), (1, 2600, 2200)])
+# Short sides that end in octet 0 .. 7 of a k-tile; long ones in 1, 4, 7, 2, 5, 0, 3, 6.
+OCTETS = [(26, 704, 712), (26, 672, 648), (26, 656, 696), (26, 720, 664), (26, 672, 680), (26, 704, 680), (26, 688, 728), (26, 752, 696)]
+PRODUCTS = [(product, last) for product in (0, 1, 2) for last in (False, True)]
+
+
+def _tiles(shape):
+    return {hip_ops.newton_schulz_product_tiles(shape, product=product, last=last)[0] for product, last in PRODUCTS}
+
+
+@pytest.mark.parametrize("shape", OCTETS)
+def test_every_octet_equals_the_small_tiles_bit_for_bit(device, shape):
+    """The batch fills the large tiles; one of its matrices alone takes small ones."""
+    assert _tiles(shape) == {"256"} and "256" not in _tiles((1, *shape[1:]))
+    together = seeded_normal(shape, 1.0, sum(shape), device)
+    alone = {b: together[b : b + 1].clone() for b in (0, 11, 25)}
+    hip_ops.newton_schulz_multi([(together, None)], COEFFS, 3, 1e-7)
+    for b, x in alone.items():
+        hip_ops.newton_schulz_multi([(x, None)], COEFFS, 3, 1e-7)
+        assert torch.equal(together[b], x[0]), b
+
+
+# Short sides that end in octet 2, 4, 6, 7 (wide) and 1, 3, 5, 2 (tall).
+FREE = [(2, 1936, 2200), (2, 2016, 2200), (2, 2096, 2200), (2, 1976, 2200), (2, 2216, 2056), (2, 2216, 2008), (2, 2216, 1960), (2, 2216, 1936)]
+
+
+@pytest.mark.parametrize("shape", FREE)
 def test_third_product_alone_on_large_tiles(device, shape):
     """Few matrices iterate on the small tiles; their third product, with its
-    transposed output, may still take the large ones."""
+    transposed output, may still take the large ones.  One matrix of the two
+    declines that, with the same bits."""
     assert hip_ops.newton_schulz_large_tiles(shape) == (False,)
-    mine = seeded_normal(shape, 1.0, sum(shape), device)
-    start = mine.double()
-    hip_ops.newton_schulz_multi([(mine, None)], COEFFS, 3, 1e-7)
-    _check(mine, start, 3, (0,))
+    tiles = {q: hip_ops.newton_schulz_product_tiles(shape, product=q[0], last=q[1])[0] for q in PRODUCTS}
+    assert {q for q, kind in tiles.items() if kind == "256"} == {(2, False), (2, True)}
+    assert "256" not in _tiles((1, *shape[1:]))
+    together = seeded_normal(shape, 1.0, sum(shape), device)
+    alone = together[1:].clone()
+    start = together.double()
+    hip_ops.newton_schulz_multi([(together, None)], COEFFS, 3, 1e-7)
+    hip_ops.newton_schulz_multi([(alone, None)], COEFFS, 3, 1e-7)
+    assert torch.equal(together[1], alone[0])
+    _check(together, start, 3, (0,))
 
 
 def _check(mine, start, steps, which):

@@ -30,7 +30,23 @@ def test_problems_of_one_call_share_the_choice():
     assert hip_ops.newton_schulz_large_tiles((24, 7168, 2048), steps=0) == (False,)
 
 
+def test_third_product_takes_large_tiles_within_one_round_only():
+    """Problems that iterate on the small tiles: their third product joins the
+    256 x 256 ones up to a round of 256 of them, and only where that is faster."""
+    third = lambda *shapes, **kw: hip_ops.newton_schulz_product_tiles(*shapes, product=2, **kw)  # noqa: E731
+    assert hip_ops.newton_schulz_large_tiles((2, 2048, 3072)) == hip_ops.newton_schulz_large_tiles((3, 2048, 3072)) == (False,)
+    assert third((2, 2048, 3072)) == third((2, 3072, 2048)) == third((1, 3072, 3072), last=True) == ("256",)  # 192 and 144 tiles
+    assert third((3, 2048, 3072)) == third((3, 3072, 2048)) == ("256x128",)  # 288 tiles
+    assert third((1, 2248, 2248)) == third((1, 2600, 2200)) == ("256x128",)  # 81 and 99: too few to gain by it
+    assert third((24, 2048, 2048), (1, 64, 96)) == ("256", "64") and third() == ()
+    for product in (0, 1):
+        assert hip_ops.newton_schulz_product_tiles((2, 2048, 3072), product=product) != ("256",)
+
+
 def test_bad_sizes_are_refused():
+    for shape, kw in (((1, 64, 64), {"product": 3}), ((1, 64, 64), {"product": 0, "steps": 0}), ((1, 64, 60), {"product": 0}), ((0, 64, 64), {"product": 0})):
+        with pytest.raises(RuntimeError, match="newton_schulz"):
+            hip_ops.newton_schulz_product_tiles(shape, **kw)
     for sizes in ((0, 8, 8, 8), (1, 8, 8, 12)):
         with pytest.raises(RuntimeError, match="gemm"):
             hip_ops.gemm_tiles(sizes)
