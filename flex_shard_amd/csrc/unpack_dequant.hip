@@ -112,18 +112,20 @@ __device__ __forceinline__ void store_values8(uint8_t* dq, uint32_t idx, const f
 // With a tile's own 128 rows per workgroup, memory lines were written in pieces
 // wherever the width is no multiple of 128, and completed by workgroups on
 // other XCDs.  All loads of a piece go out ahead of its first store and without
-// a branch between them, and nothing that waits for memory (the ends of a run
-// that are no whole group, the scale's own copy) comes before them.  Us with a
-// tile per workgroup / a branch per load / here, rows from HBM and (just
-// gathered, in the last-level cache):
-//   218 M layer on eight ranks      169 / 165 / 153     (162 / 150 / 146)
-//   67 M of 4096 on one             58 / 56 / 52        (44 / 47 / 45)
-//   33 M of 4104 on three           57 / 36 / 31        (55 / 32 / 26)
-//   16.8 M of 4096 on one           17.6 / 17.6 / 17.9  (15.4 / 16.9 / 16.4)
-//   2.1 M of 4096 on one            7.9 / 9.9 / 8.2     (9.2 / 10.4 / 9.2)
-//   59 M of 4096 to fp32            90 / 121 / 83       (102 / 130 / 57)
-// A tile per workgroup stays up to 1 us ahead on whole tiles of 8 to 17 M
-// elements from HBM (one scale instead of one per group): no second form for that.
+// a branch between them, the FP8 bytes ahead of the scales, whose addresses take
+// a division, and nothing that waits for memory (the ends of a run that are no
+// whole group, the scale's own copy) comes before them.  Us with a tile per
+// workgroup / a branch per load / here, rows from HBM and (just gathered, in the
+// last-level cache):
+//   218 M layer on eight ranks      169 / 163 / 152     (168 / 159 / 150)
+//   67 M of 4096 on one             57 / 56 / 50        (44 / 46 / 44)
+//   33 M of 4104 on three           61 / 36 / 30        (57 / 30 / 25)
+//   16.8 M of 4096 on one           18.1 / 16.7 / 16.1  (15.1 / 16.0 / 15.4)
+//   8.4 M of 4096 on one            10.4 / 11.0 / 10.3  (10.2 / 11.1 / 10.4)
+//   2.1 M of 4096 on one            8.1 / 10.3 / 8.3    (8.9 / 10.1 / 8.9)
+//   59 M of 4096 to fp32            96 / 118 / 86       (110 / 125 / 61)
+// With byte and scale loads in turn the layer took 149 and the others up to 12 %
+// longer.  A tile per workgroup is nowhere ahead by more than 3 %: no second form.
 template <int DQ, bool kAligned>
 __device__ __forceinline__ void unpack_piece(const uint8_t* src, uint8_t* cq, uint8_t* dq, const uint8_t* scales, int64_t rows,
                                              int64_t in_dim, int64_t tiles_c, int64_t t, int64_t tiles, int64_t lead, int tid) {
@@ -148,15 +150,18 @@ __device__ __forceinline__ void unpack_piece(const uint8_t* src, uint8_t* cq, ui
   uint32_t cols[kPasses], belows[kPasses];
   float scale[kPasses];
   if (count > 0) {
+    // (groups past the piece's end: its last one again)
+    const auto group_of = [&](int k) { return min(static_cast<uint32_t>(k * kThreads + tid), count - 1); };
 #pragma unroll
-    for (int k = 0; k < kPasses; ++k) {
-      // (groups past the piece's end: its last one again)
-      const uint32_t g = min(static_cast<uint32_t>(k * kThreads + tid), count - 1);
-      vin[k] = load_group<u32x2, kAligned>(run + 8 * g);
-      const uint32_t c = col0 + 8 * g;
-      belows[k] = c / width;
-      cols[k] = c - belows[k] * width;
-      if (dq) scale[k] = scale_at(row0 + belows[k], cols[k]);
+    for (int k = 0; k < kPasses; ++k) vin[k] = load_group<u32x2, kAligned>(run + 8 * group_of(k));
+    if (dq) {
+#pragma unroll
+      for (int k = 0; k < kPasses; ++k) {
+        const uint32_t c = col0 + 8 * group_of(k);
+        belows[k] = c / width;
+        cols[k] = c - belows[k] * width;
+        scale[k] = scale_at(row0 + belows[k], cols[k]);
+      }
     }
   }
 #pragma unroll
