@@ -111,9 +111,10 @@ __global__ __launch_bounds__(kActThreads) void act_quant_1x128_kernel(const ActQ
 // k-tile: four registers that a fold can follow four blocks later, where the
 // two 32x32x64 ones before it held sixteen and had to be folded behind the next
 // pair; and the k-tile is a tag's two instantiations instead of a branch per
-// request.  8192 tokens, us before / after: 4096 x 4096 141 / 127, 14336 x 4096
-// 441 / 411, 4096 x 14336 383 / 355; weight gradients 133 / 126, 470 / 443, 467 /
-// 439.  Same bits.
+// request.  8192 tokens, us of both in turn on one part: 4096 x 4096 122 / 114,
+// 14336 x 4096 428 / 414, 4096 x 14336 410 / 398; weight gradients 130 / 124, 477 /
+// 457, 472 / 451 (3-7 %; clocks differ between parts, and with them the times and
+// the gain).  Same bits.
 //
 // TM_ = 1 is the half tile (128 x 256, waves of 32 x 128) that the tiles of a
 // last, at most half-full round are cut into; it keeps the LDS layout of the
@@ -229,8 +230,8 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // Two stages: the operands of k-tile kt + 1 are in flight while kt is
-  // multiplied.  The row scales ride the same global->LDS path (two 4-byte-
-  // per-lane requests per wave and k-tile for the wave's 128 rows): a
+  // multiplied.  The row scales ride the same global->LDS path (one 4-byte-
+  // per-lane request per wave and k-tile for the wave's 64 rows): a
   // compiler-visible load here would make the compiler wait for everything in
   // flight, the prefetched tile included.
   const uint32_t scale_lds0 = lds_base + static_cast<uint32_t>(Cfg::kScaleOffset + wave * Cfg::kScaleSlots * 4);
@@ -358,7 +359,7 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
   auto k_tile = [&](int64_t kt, auto more_tag) {
     constexpr bool more = decltype(more_tag)::value;
     const int stage_off = stage * Cfg::kStageBytes;
-    // The scales are first needed by the fold behind the second block's MFMAs.
+    // The scales are first needed by the first fold, kLag blocks in.
     read_row_scales(s, stage, kt);
     read_column_scales(cs_rows, stage);
     if (kLongK && !kColumnScales && more && (kt & (Cfg::kMaxKTilesInLds - 1)) == Cfg::kMaxKTilesInLds - 1) {

@@ -12,10 +12,10 @@
 // A tall input is its own X^T, so no transpose kernel is needed in either
 // case, and the result lands in the caller's buffer without a copy.
 //
-// GEMM kernels: 256 threads (2x2 wavefronts) on v_mfma_f32_16x16x32_bf16 (the
-// smaller tiles: 32x32x16),
-// operands global -> LDS directly: 256x256x64 tiles for large problems of
-// whole tiles (below), smaller tiles for everything else (gemm_tiles.hpp).
+// GEMM kernels, operands global -> LDS directly: 256x256x64 tiles of 2x2
+// wavefronts on v_mfma_f32_16x16x32_bf16 for large problems (below; those of
+// Newton-Schulz need not be whole tiles), smaller tiles on 32x32x16 for
+// everything else (gemm_tiles.hpp).
 #include "gemm_tiles.hpp"
 #include "muon_groups.hpp"
 
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(DmaGemm::kThreads) void gemm_nt_dma_kernel(const Ge
   // M0 takes the LDS byte address relative to the workgroup's allocation.
   typedef __attribute__((address_space(3))) uint8_t* lds_address;
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_address)lds_bytes));
-  const uint32_t fill_lds = lds_base + static_cast<uint32_t>(wave * 1024);  // + q * 4096 (+ operand, + stage)
+  const uint32_t fill_lds = lds_base + static_cast<uint32_t>(wave * 1024);  // + q * 4096 + the ring slot
   // Operand tile bases of (problem, batch, tile row / column), k-tile 0.
   auto a_base = [&](int which, int64_t batch, int tm) -> const uint8_t* {
     const GemmParams& q = launch.problem[which];

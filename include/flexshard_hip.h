@@ -80,9 +80,11 @@ typedef struct fsh_quant_chunk {
  * scales of tile (tr, tc) at scale_offset + 4*(tr*ceil(in_dim/block) + tc).
  * Bytes [zero0_begin, zero0_end) and [zero1_begin, zero1_end) of the payload
  * are set to zero (the pad between data and scales, and the tail pad).
- * nchunks <= FSH_MAX_QUANT_CHUNKS; block = 128 takes the vectorized path when
- * a chunk's pointers, stride and offsets are 16-byte friendly, any other
- * block size or alignment takes a scalar path with the same results.
+ * nchunks <= FSH_MAX_QUANT_CHUNKS.  block = 128 takes a vectorized path for
+ * chunks whose pointers, stride and offsets are 16-byte friendly, and for all
+ * chunks of a launch of FSH_SRC_BF16 or of FSH_SRC_F32_AS_BF16 alone (unaligned
+ * accesses where they have to be); everything else takes a scalar path.  The
+ * results are the same.
  */
 int fsh_quantize_pack(const fsh_quant_chunk* chunks, int32_t nchunks, void* payload_dev,
                       int64_t payload_nbytes, int64_t zero0_begin, int64_t zero0_end,
