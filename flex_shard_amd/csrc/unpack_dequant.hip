@@ -112,20 +112,21 @@ __device__ __forceinline__ void store_values8(uint8_t* dq, uint32_t idx, const f
 // With a tile's own 128 rows per workgroup, memory lines were written in pieces
 // wherever the width is no multiple of 128, and completed by workgroups on
 // other XCDs.  All loads of a piece go out ahead of its first store and without
-// a branch between them, the FP8 bytes ahead of the scales, whose addresses take
-// a division, and nothing that waits for memory (the ends of a run that are no
-// whole group, the scale's own copy) comes before them.  Us with a tile per
-// workgroup / a branch per load / here, rows from HBM and (just gathered, in the
-// last-level cache):
-//   218 M layer on eight ranks      169 / 163 / 152     (168 / 159 / 150)
-//   67 M of 4096 on one             57 / 56 / 50        (44 / 46 / 44)
-//   33 M of 4104 on three           61 / 36 / 30        (57 / 30 / 25)
-//   16.8 M of 4096 on one           18.1 / 16.7 / 16.1  (15.1 / 16.0 / 15.4)
-//   8.4 M of 4096 on one            10.4 / 11.0 / 10.3  (10.2 / 11.1 / 10.4)
-//   2.1 M of 4096 on one            8.1 / 10.3 / 8.3    (8.9 / 10.1 / 8.9)
-//   59 M of 4096 to fp32            96 / 118 / 86       (110 / 125 / 61)
-// With byte and scale loads in turn the layer took 149 and the others up to 12 %
-// longer.  A tile per workgroup is nowhere ahead by more than 3 %: no second form.
+// a branch between them, and nothing that waits for memory (the ends of a run
+// that are no whole group, the scale's own copy) comes before them.  Four
+// passes' FP8 bytes go ahead of the four scales, whose addresses take a
+// division.  Us with a tile per workgroup / a branch per load / here, rows from
+// HBM and (just gathered, in the last-level cache):
+//   218 M layer on eight ranks      169 / 163 / 149     (168 / 159 / 148)
+//   67 M of 4096 on one             57 / 56 / 49        (44 / 46 / 44)
+//   33 M of 4104 on three           61 / 36 / 29        (57 / 30 / 25)
+//   16.8 M of 4096 on one           18.3 / 16.7 / 15.7  (15.1 / 16.0 / 15.1)
+//   8.4 M of 4096 on one            10.7 / 11.0 / 10.3  (10.2 / 11.1 / 10.3)
+//   2.1 M of 4096 on one            8.2 / 10.3 / 8.3    (8.9 / 10.1 / 8.8)
+//   59 M of 4096 to fp32            100 / 118 / 88      (110 / 125 / 61)
+// Byte and scale loads in turn: up to 10 % longer from 17 M on down, the layer 148;
+// all bytes ahead of all scales: the layer 152.  A tile per workgroup is nowhere
+// ahead by more than the 1 % that runs differ by: no second form.
 template <int DQ, bool kAligned>
 __device__ __forceinline__ void unpack_piece(const uint8_t* src, uint8_t* cq, uint8_t* dq, const uint8_t* scales, int64_t rows,
                                              int64_t in_dim, int64_t tiles_c, int64_t t, int64_t tiles, int64_t lead, int tid) {
@@ -153,14 +154,17 @@ __device__ __forceinline__ void unpack_piece(const uint8_t* src, uint8_t* cq, ui
     // (groups past the piece's end: its last one again)
     const auto group_of = [&](int k) { return min(static_cast<uint32_t>(k * kThreads + tid), count - 1); };
 #pragma unroll
-    for (int k = 0; k < kPasses; ++k) vin[k] = load_group<u32x2, kAligned>(run + 8 * group_of(k));
-    if (dq) {
+    for (int half = 0; half < 2; ++half) {
 #pragma unroll
-      for (int k = 0; k < kPasses; ++k) {
-        const uint32_t c = col0 + 8 * group_of(k);
-        belows[k] = c / width;
-        cols[k] = c - belows[k] * width;
-        scale[k] = scale_at(row0 + belows[k], cols[k]);
+      for (int k = 4 * half; k < 4 * half + 4; ++k) vin[k] = load_group<u32x2, kAligned>(run + 8 * group_of(k));
+      if (dq) {
+#pragma unroll
+        for (int k = 4 * half; k < 4 * half + 4; ++k) {
+          const uint32_t c = col0 + 8 * group_of(k);
+          belows[k] = c / width;
+          cols[k] = c - belows[k] * width;
+          scale[k] = scale_at(row0 + belows[k], cols[k]);
+        }
       }
     }
   }
