@@ -8,49 +8,57 @@ namespace {
 
 using TileLaunch = GemmLaunchOf<8>;
 
-// WM x WN waves, each TM x TN blocks of 32 x 32.  kStages k-tiles of 64 in LDS.
-template <int WM_, int WN_, int TM_, int TN_, int kStages_>
+// WM x WN waves, each TM x TN blocks of 16 x 16.  Operands are requested kDepth
+// k-tiles of 64 ahead: operand A has a slot for each of them and for the k-tile
+// in work, operand B, which is requested later in a k-tile, for one fewer.
+template <int WM_, int WN_, int TM_, int TN_, int kDepth_>
 struct GemmTiles {
-  static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, kStages = kStages_;
-  static constexpr int kWaveM = 32 * TM, kWaveN = 32 * TN, BM = WM * kWaveM, BN = WN * kWaveN, BK = 64, KS = BK / 16;
+  static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, kDepth = kDepth_;
+  static constexpr int kWaveM = 16 * TM, kWaveN = 16 * TN, BM = WM * kWaveM, BN = WN * kWaveN, BK = 64, KS = BK / 32;
   static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves;
   static constexpr int kRowBytes = BK * 2;  // 128
-  static constexpr int kOperandABytes = BM * kRowBytes;
-  static constexpr int kStageBytes = (BM + BN) * kRowBytes;
+  static constexpr int kABytes = BM * kRowBytes, kBBytes = BN * kRowBytes;
+  static constexpr int kARing = (kDepth + 1) * kABytes, kBRing = kDepth * kBBytes;  // B's ring lies behind A's
   // A wave-level request fills 1 KB = 8 tile rows.
   static constexpr int kFillRows = 8 * kWaves;
   static constexpr int kLoadsA = BM / kFillRows, kLoadsB = BN / kFillRows, kLoads = kLoadsA + kLoadsB;
-  // k steps whose fragments are read ahead of their MFMAs: enough MFMAs have
-  // to issue under an LDS read to cover it.
-  static constexpr int kAhead = TM * TN >= 4 ? 1 : 3, kSets = TM * TN >= 4 ? 2 : 4;
-  // Epilogue: one [kWaveM][kWaveN] bf16 image per wave, rows 8 bytes off a
-  // multiple of the bank window.
-  static constexpr int kPitch = kWaveN * 2 + 8;   // [row][col]
-  static constexpr int kPitchT = kWaveM * 2 + 8;  // [col][row]
-  static constexpr int kRegion = max_int(kWaveM * kPitch, kWaveN * kPitchT);
-  static constexpr int kLdsBytes = kStages * kStageBytes;
+  // Epilogue: one [kWaveM][kWaveN] bf16 image per wave.
+  static constexpr int kPitch = kWaveN * 2 + 16, kRegion = kWaveM * kPitch;
+  static constexpr int kLdsBytes = kARing + kBRing;
   static_assert(kWaves * kRegion <= kLdsBytes, "the images fit the loop's LDS");
-  static_assert(BM % kFillRows == 0 && BN % kFillRows == 0, "whole requests");
+  static_assert(BM % kFillRows == 0 && BN % kFillRows == 0 && kFillRows % 16 == 0, "whole requests");
+  static_assert(kDepth >= 2 && kDepth <= 4, "the waits of the k loop's end");
 };
 
+// Four values of one column and four consecutive rows out of a bf16 image with
+// rows in LDS: within 16 lanes, lane 4 j + q passes the address of columns
+// 4 q .. 4 q + 3 of row j, and lane t receives column t of rows 0 .. 3.
+__device__ __forceinline__ u32x2 read_lds_transposed(const uint8_t* at) {
+  typedef short i16x4 __attribute__((__vector_size__(4 * sizeof(short))));
+  typedef __attribute__((address_space(3))) i16x4* lds_i16x4;
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)(const_cast<uint8_t*>(at))));
+}
+
 // Finals bf16(fma(beta, D, alpha * acc) + diagonal term) of a wave's sub-tile
-// at (row0, col0), through its LDS image: D arrives row-wise, C and the
-// transposed (or mirrored) output leave row-wise.  Only the wave itself
-// touches its image, so program order is all the synchronization there is.
+// at (row0, col0), through its LDS image: D arrives row-wise and C leaves
+// row-wise; the transposed (or mirrored) output is read across the image, two
+// transposing reads for eight rows of a column.  (Before, the image was written
+// again as [col][row], 64 two-byte writes per lane of a 64 x 64 sub-tile.)
+// Only the wave itself touches its image, so program order is all the
+// synchronization there is.
 template <typename Cfg>
 __device__ __forceinline__ void store_wave_tile(const GemmParams& p, int64_t batch, int64_t row0, int64_t col0, int lane,
-                                                bool mirror, f32x16 (&acc)[Cfg::TM][Cfg::TN], uint8_t* region) {
+                                                bool mirror, f32x4 (&acc)[Cfg::TM][Cfg::TN], uint8_t* region) {
   constexpr int TM = Cfg::TM, TN = Cfg::TN;
   uint16_t* C = p.C + batch * p.sC;
   uint16_t* Ct = mirror ? C : (p.Ct ? p.Ct + batch * p.sCt : nullptr);
   const int64_t ldct = mirror ? p.ldc : p.ldct;
-  const int r_lane = lane & 31, h = lane >> 5;
-  auto slot = [&](int i, int j, int b) -> u32x2* {  // accumulators 4 b .. 4 b + 3 of block (i, j)
-    return reinterpret_cast<u32x2*>(region + (i * 32 + r_lane) * Cfg::kPitch + (j * 32 + 8 * b + 4 * h) * 2);
+  const int r_lane = lane & 15, c_lane = 4 * (lane >> 4);
+  auto slot = [&](int i, int j) -> u32x2* {  // the four accumulators of block (i, j)
+    return reinterpret_cast<u32x2*>(region + (i * 16 + r_lane) * Cfg::kPitch + (j * 16 + c_lane) * 2);
   };
 
   const bool has_d = p.D != nullptr;
-  u32x2 dv[TM][TN][4];
   if (has_d) {
     constexpr int kLanesPerRow = Cfg::kWaveN / 8, kRowsPerPass = 64 / kLanesPerRow, kPasses = Cfg::kWaveM / kRowsPerPass;
     const uint16_t* D = p.D + batch * p.sD;
@@ -65,89 +73,80 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams& p, int64_t bat
       if (row < p.M && col < p.N) t[pass] = load_row_piece(D + row * p.ldd, col, p.N, vec);
     }
 #pragma unroll
-    for (int pass = 0; pass < kPasses; ++pass) {
-      uint8_t* d = region + (pass * kRowsPerPass + r0) * Cfg::kPitch + chunk * 16;
-      *reinterpret_cast<u32x2*>(d) = u32x2{t[pass].x, t[pass].y};
-      *reinterpret_cast<u32x2*>(d + 8) = u32x2{t[pass].z, t[pass].w};
-    }
+    for (int pass = 0; pass < kPasses; ++pass)
+      *reinterpret_cast<u32x4*>(region + (pass * kRowsPerPass + r0) * Cfg::kPitch + chunk * 16) = t[pass];
     wave_lds_sync();
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) dv[i][j][b] = *slot(i, j, b);
   }
-  u32x2 fin[TM][TN][4];
+  // A lane's finals replace exactly the D values it reads itself.
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < TM; ++i) {
+    u32x2 dv[TN];
+    if (has_d) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+      for (int j = 0; j < TN; ++j) dv[j] = *slot(i, j);
+    }
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        float v[4];
+    for (int j = 0; j < TN; ++j) {
+      float v[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) v[t] = p.alpha * acc[i][j][4 * b + t];  // alpha == 1 is exact
-        if (has_d) {
-          v[0] = __builtin_fmaf(p.beta, u32_as_f32(dv[i][j][b].x << 16), v[0]);
-          v[1] = __builtin_fmaf(p.beta, u32_as_f32(dv[i][j][b].x & 0xFFFF0000u), v[1]);
-          v[2] = __builtin_fmaf(p.beta, u32_as_f32(dv[i][j][b].y << 16), v[2]);
-          v[3] = __builtin_fmaf(p.beta, u32_as_f32(dv[i][j][b].y & 0xFFFF0000u), v[3]);
-        }
-        if (p.diag_add != 0.0f && row0 + 32 * i == col0 + 32 * j) {  // (sub-tiles start at multiples of 32)
-#pragma unroll
-          for (int t = 0; t < 4; ++t) v[t] = r_lane == 8 * b + 4 * h + t ? v[t] + p.diag_add : v[t];
-        }
-        fin[i][j][b] = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      for (int t = 0; t < 4; ++t) v[t] = p.alpha * acc[i][j][t];  // alpha == 1 is exact
+      if (has_d) {
+        v[0] = __builtin_fmaf(p.beta, u32_as_f32(dv[j].x << 16), v[0]);
+        v[1] = __builtin_fmaf(p.beta, u32_as_f32(dv[j].x & 0xFFFF0000u), v[1]);
+        v[2] = __builtin_fmaf(p.beta, u32_as_f32(dv[j].y << 16), v[2]);
+        v[3] = __builtin_fmaf(p.beta, u32_as_f32(dv[j].y & 0xFFFF0000u), v[3]);
       }
+      if (p.diag_add != 0.0f && row0 + 16 * i == col0 + 16 * j) {  // (sub-tiles start at multiples of 16)
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) *slot(i, j, b) = fin[i][j][b];
+        for (int t = 0; t < 4; ++t) v[t] = r_lane == c_lane + t ? v[t] + p.diag_add : v[t];
+      }
+      *slot(i, j) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    }
+  }
   wave_lds_sync();
   store_wave_image<Cfg::kWaveM, Cfg::kWaveN, Cfg::kPitch>(region, C, p.ldc, row0, col0, p.M, p.N, lane);
   if (Ct == nullptr) return;  // uniform over the workgroup
-  wave_lds_sync();  // the row reads are done before the image is written again as [col][row]
+  // Lane t of group g of 16: column t of 16, rows 8 g .. 8 g + 7 of 32.
+  const bool vec = rows_are_16_byte(Ct, ldct);
+  const int t = lane & 15, g = lane >> 4;
+  const uint8_t* from = region + (8 * g + (t >> 2)) * Cfg::kPitch + (t & 3) * 8;
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int cb = 0; cb < TN; ++cb) {
+    const int64_t col = col0 + cb * 16 + t;
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const uint32_t pair = (t >> 1) ? fin[i][j][b].y : fin[i][j][b].x;
-          *reinterpret_cast<uint16_t*>(region + (j * 32 + 8 * b + 4 * h + t) * Cfg::kPitchT + (i * 32 + r_lane) * 2) =
-              static_cast<uint16_t>((t & 1) ? (pair >> 16) : pair);
-        }
-  wave_lds_sync();
-  store_wave_image<Cfg::kWaveN, Cfg::kWaveM, Cfg::kPitchT>(region, Ct, ldct, col0, row0, p.N, p.M, lane);
+    for (int rb = 0; rb < Cfg::kWaveM / 32; ++rb) {
+      const u32x2 lo = read_lds_transposed(from + rb * 32 * Cfg::kPitch + cb * 32);
+      const u32x2 hi = read_lds_transposed(from + (rb * 32 + 4) * Cfg::kPitch + cb * 32);
+      const int64_t row = row0 + rb * 32 + 8 * g;
+      if (col < p.N && row < p.M) store_row_piece(Ct + col * ldct, row, p.M, vec, u32x4{lo.x, lo.y, hi.x, hi.y});
+    }
+  }
 }
 
 // What bounds it: the request path of a compute unit takes a 1 KB request per
 // 16 cycles, so the 32 requests of a 128 x 128 x 64 k-tile last as long as its
-// MFMAs (512 cycles), and a request holds up the wave that issues it; each is
-// therefore issued behind an MFMA, fragments are read a k step ahead (three
-// for 32 x 32 waves), and workgroups that share a compute unit cover each
-// other's barriers.  6592^3 with 128 x 128 tiles: 843 TFLOP/s with the requests
-// in one go at the top of a k-tile and the fragment reads behind the barrier,
-// 988 rotated as below, 1054 with the loop split so that no request sits
-// behind a branch of its own, 1130 with 256 x 128 tiles of eight waves.
-// Against the kernels this one replaced (register-staged 128 x 128 x 32, and
-// 256 x 256 x 64 with predicated accesses for ragged shapes): 6592^3 690 ->
-// 532 us, 768 x 768 x 3072 (batch 4, symmetric) 45 -> 19 us, one 304 x 304 x
-// 704 product 17.7 -> 5.7 us.
+// MFMAs (512 cycles), and a request holds up the wave that issues it.  One
+// 128 x 128 workgroup per compute unit takes 0.22 us per k-tile with its
+// operands in LDS, 0.27 with the fragment reads or the requests and 0.30 with
+// both (64 tiles; 0.40 with every compute unit busy); short contractions spend
+// as long on their start and end.  16 x 16 x 32 MFMAs, a request behind every
+// few of them in both k steps, scalar bases with 32-bit offsets, one orientation
+// in the image, against 32 x 32 x 16 MFMAs, 64-bit addresses per request and the
+// requests of a k-tile in two bunches (same bits), us:
+//   2048 x 2048, k 2048 25.8 -> 20.7 (128 x 128 tiles)   4096 x 4096, k 2048 70.9 -> 58.1
+//   8 x 768 x 768, 4 x 3072 x 768, 4 x 768 x 3072, ...: G 37.4 -> 31.4, P 19.9 -> 17.2, X' 61.6 -> 49.9
+//   20 small matrices, a Muon step 759 -> 669
 //
 // Operands travel global -> LDS directly into swizzled 128-byte rows, as in
 // the 256 x 256 kernel.  Rows past the matrix are read from its last row and
 // the last k-tile's chunks past K from the row's last chunk; what they
 // multiply is never stored, respectively zeroed in the fragments.
-template <typename Cfg, int kBlocksPerUnit>
+// kWide: rows so long that a tile's offsets need 64 bits.
+template <typename Cfg, int kBlocksPerUnit, bool kWide>
 __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) void gemm_nt_tiles_kernel(const TileLaunch launch) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_bytes[];
-  constexpr int TM = Cfg::TM, TN = Cfg::TN, KS = Cfg::KS, kStages = Cfg::kStages, kMfmas = TM * TN, kSets = Cfg::kSets;
+  constexpr int TM = Cfg::TM, TN = Cfg::TN, KS = Cfg::KS, kDepth = Cfg::kDepth, kMfmas = TM * TN;
+  constexpr int kLoadsA = Cfg::kLoadsA, kLoadsB = Cfg::kLoadsB;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -160,7 +159,11 @@ __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) vo
   const GemmParams& p = launch.problem[which];
   int64_t batch;
   int tm, tn;
-  if (!tile_of_workgroup(p, static_cast<int64_t>(blockIdx.x) - launch.first_workgroup[which], &batch, &tm, &tn)) return;  // whole workgroup
+  // An XCD that holds 64 tiles at a time takes patches of 8 x 8 (16 operand panels for 20: 8 x 768 x 768 and
+  // 8 x 768 x 3072, k 768 52.4 -> 49.9 us); eight rows of the few tiles of a small launch cost it (14.7 -> 19.3).
+  const int rows_together = p.items_per_xcd >= 64 ? 2 * kGroupTilesM : kGroupTilesM;
+  if (!tile_of_workgroup(p, static_cast<int64_t>(blockIdx.x) - launch.first_workgroup[which], &batch, &tm, &tn, rows_together))
+    return;  // whole workgroup
   batch = uniform_i64(batch);
   tm = uniform_i32(tm);
   tn = uniform_i32(tn);
@@ -168,160 +171,167 @@ __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) vo
 
   // Load side: wave-level request q of an operand fills tile rows
   // [kFillRows q + 8 wave, +8); lane l fills slot l & 7 of row l >> 3 there.
+  typedef std::conditional_t<kWide, uint64_t, uint32_t> offset_t;
   const int fill_row = 8 * wave + (lane >> 3);
   const int fill_chunk = (lane & 7) ^ ((fill_row >> 1) & 7);
-  const uint8_t* src[Cfg::kLoads];
+  const uint8_t* a_src = uniform_ptr(reinterpret_cast<const uint8_t*>(p.A + batch * p.sA + m0 * p.lda));
+  const uint8_t* b_src = uniform_ptr(reinterpret_cast<const uint8_t*>(p.B + batch * p.sB + n0 * p.ldb));
+  offset_t a_voff[kLoadsA], b_voff[kLoadsB];
+  const int a_last = static_cast<int>(p.M - m0 < Cfg::BM ? p.M - m0 : Cfg::BM) - 1;
+  const int b_last = static_cast<int>(p.N - n0 < Cfg::BN ? p.N - n0 : Cfg::BN) - 1;
 #pragma unroll
-  for (int q = 0; q < Cfg::kLoadsA; ++q) {
-    const int64_t r = m0 + Cfg::kFillRows * q + fill_row;
-    src[q] = reinterpret_cast<const uint8_t*>(p.A + batch * p.sA + (r < p.M ? r : p.M - 1) * p.lda) + fill_chunk * 16;
-  }
+  for (int q = 0; q < kLoadsA; ++q)
+    a_voff[q] = static_cast<offset_t>(min(Cfg::kFillRows * q + fill_row, a_last)) * static_cast<offset_t>(p.lda * 2) + fill_chunk * 16;
 #pragma unroll
-  for (int q = 0; q < Cfg::kLoadsB; ++q) {
-    const int64_t r = n0 + Cfg::kFillRows * q + fill_row;
-    src[Cfg::kLoadsA + q] = reinterpret_cast<const uint8_t*>(p.B + batch * p.sB + (r < p.N ? r : p.N - 1) * p.ldb) + fill_chunk * 16;
-  }
+  for (int q = 0; q < kLoadsB; ++q)
+    b_voff[q] = static_cast<offset_t>(min(Cfg::kFillRows * q + fill_row, b_last)) * static_cast<offset_t>(p.ldb * 2) + fill_chunk * 16;
   typedef __attribute__((address_space(3))) uint8_t* lds_address;
   const uint32_t fill_lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_address)lds_bytes)) + wave * 1024;
   const int ktiles = static_cast<int>((p.K + Cfg::BK - 1) / Cfg::BK);
-  const int tail_chunks = static_cast<int>((p.K / 8) & 7);  // 0: the last k-tile is whole
-  // Byte offset of k-tile kt along the rows; chunks past K read the row's last chunk instead.
-  const int64_t tail_back = tail_chunks != 0 && fill_chunk >= tail_chunks ? (fill_chunk - (tail_chunks - 1)) * 16 : 0;
-  auto k_offset = [&](int kt) -> int64_t {
-    return static_cast<int64_t>(kt) * Cfg::kRowBytes - (kt == ktiles - 1 ? tail_back : 0);
+  const int tail = static_cast<int>(p.K / 8) & 7;  // chunks of the last k-tile, 0 if it is whole
+  // Before the requests of the last k-tile: chunks past K read the row's last chunk instead.
+  auto aim_at_tail = [&]() {
+    const uint32_t back = fill_chunk >= tail ? (fill_chunk - (tail - 1)) * 16 : 0;
+#pragma unroll
+    for (int q = 0; q < kLoadsA; ++q) a_voff[q] -= back;
+#pragma unroll
+    for (int q = 0; q < kLoadsB; ++q) b_voff[q] -= back;
   };
-  auto issue_one = [&](int64_t k_off, uint32_t stage, int idx) {
-    // (operand B's rows follow operand A's in the stage)
-    dma_load_16_at(src[idx] + k_off, fill_lds + stage * Cfg::kStageBytes + idx * (Cfg::kFillRows * Cfg::kRowBytes));
+  auto issue = [&](const uint8_t* src, offset_t voff, uint32_t slot, int q) {
+    if constexpr (kWide) dma_load_16_at(src + voff, fill_lds + slot + q * (Cfg::kFillRows * Cfg::kRowBytes));
+    else dma_load_16(voff, src, fill_lds + slot, q * (Cfg::kFillRows * Cfg::kRowBytes));
   };
 
-  // Fragment side: lane l reads row l & 31 of a 32-row block, chunk 2 ks + (l >> 5).
-  const int frag_row = lane & 31;
-  const uint32_t frag_base = static_cast<uint32_t>(frag_row * Cfg::kRowBytes + (((lane >> 5) ^ ((frag_row >> 1) & 7)) * 16));
-  f32x16 acc[TM][TN];
+  // Fragment side: lane l reads row l & 15 of a 16-row block, chunk 4 ks + (l >> 4).
+  const int frag_row = lane & 15;
+  const uint32_t frag_base = static_cast<uint32_t>(frag_row * Cfg::kRowBytes + (((lane >> 4) ^ ((frag_row >> 1) & 7)) * 16));
+  uint32_t a_frag[KS], b_frag[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    a_frag[ks] = (frag_base ^ (ks * 64)) + wm * Cfg::kWaveM * Cfg::kRowBytes;
+    b_frag[ks] = (frag_base ^ (ks * 64)) + wn * Cfg::kWaveN * Cfg::kRowBytes + Cfg::kARing;
+  }
+  f32x4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-  bf16x8 af[kSets][TM], bf[kSets][TN];
-  // Fragments of k step ks of the k-tile in `stage`; `masked`: the chunks past K as zero.
-  auto read_frags = [&](uint32_t stage, int ks, bool masked) {
-    const uint8_t* base = lds_bytes + stage * Cfg::kStageBytes + (frag_base ^ (ks * 32));
-    const uint8_t* a = base + wm * Cfg::kWaveM * Cfg::kRowBytes;
-    const uint8_t* b = base + Cfg::kOperandABytes + wn * Cfg::kWaveN * Cfg::kRowBytes;
-    const int set = ks % kSets;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) af[set][i] = *reinterpret_cast<const bf16x8*>(a + i * 32 * Cfg::kRowBytes);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) bf[set][j] = *reinterpret_cast<const bf16x8*>(b + j * 32 * Cfg::kRowBytes);
-    if (masked) {
-      const bf16x8 zero = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
-      const bool live = 2 * ks + (lane >> 5) < tail_chunks;
-#pragma unroll
-      for (int i = 0; i < TM; ++i) af[set][i] = live ? af[set][i] : zero;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) bf[set][j] = live ? bf[set][j] : zero;
-    }
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 af[KS][TM], bf[KS][TN];
+  // Fragment g of k step ks: the TM of operand A, then the TN of B.
+  auto read_frag = [&](uint32_t a_slot, uint32_t b_slot, int ks, int g) {
+    if (g < TM) af[ks][g] = *reinterpret_cast<const bf16x8*>(lds_bytes + a_slot + a_frag[ks] + g * 16 * Cfg::kRowBytes);
+    else bf[ks][g - TM] = *reinterpret_cast<const bf16x8*>(lds_bytes + b_slot + b_frag[ks] + (g - TM) * 16 * Cfg::kRowBytes);
   };
-  auto mfma = [&](int ks, int g) {
-    const int i = g / TN, j = g % TN, set = ks % kSets;
-    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[set][j], af[set][i], acc[i][j], 0, 0, 0);
-  };
-  // One k-tile, rotated by a quarter: the barrier that hands over k-tile
-  // kt + 1 sits before the last k step, behind which the first fragments of
-  // kt + 1 are read, and which releases kt's own stage (every wave holds its
-  // last fragments in registers) to the requests for kt + kStages: half of
-  // them behind the MFMAs there, half in the first k step of kt + 1.
-  //   second / first: the second half of the requests for kt + kStages - 1
-  //   and the first half of those for kt + kStages go out
-  constexpr int kFirst = (Cfg::kLoads + 1) / 2, kSecond = Cfg::kLoads - kFirst;
-  uint32_t stage = 0;  // of kt
-  auto k_tile = [&](int kt, auto second_tag, auto first_tag, auto masked_tag, auto last_tag) {
-    constexpr bool second = decltype(second_tag)::value, first = decltype(first_tag)::value;
-    constexpr bool masked = decltype(masked_tag)::value, last = decltype(last_tag)::value;
-    const uint32_t before = stage == 0 ? kStages - 1 : stage - 1, after = stage + 1 == kStages ? 0 : stage + 1;
+  // Past K both operands are zero (the other's last values could be infinite).
+  auto zero_past_k = [&](int ks) {
+    const bool live = 4 * ks + (lane >> 4) < tail;
+    const auto masked = [&](bf16x8& f) {
+      const u32x4 w = __builtin_bit_cast(u32x4, f);
+      f = __builtin_bit_cast(bf16x8, live ? w : u32x4{0, 0, 0, 0});
+    };
 #pragma unroll
-    for (int ks = 0; ks + 1 < KS; ++ks) {
-      if (ks + Cfg::kAhead < KS) read_frags(stage, ks + Cfg::kAhead, masked);
-      __builtin_amdgcn_sched_barrier(0);
-      const int64_t k_off = second && ks == 0 ? k_offset(kt + kStages - 1) : 0;
+    for (int i = 0; i < TM; ++i) masked(af[ks][i]);
 #pragma unroll
-      for (int g = 0; g < kMfmas; ++g) {
-        mfma(ks, g);
-        if (second && ks == 0) {
-#pragma unroll
-          for (int idx = g * kSecond / kMfmas; idx < (g + 1) * kSecond / kMfmas; ++idx) issue_one(k_off, before, kFirst + idx);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (!last) {
-      // k-tile kt + 1 has landed (this wave's part); those behind it stay in flight.
-      const int behind = ktiles - 2 - kt;
-      if (kStages >= 4 && (first || behind >= 2))
-        wait_for_dma_loads_but<2 * Cfg::kLoads>();
-      else if (kStages >= 3 && (first || behind >= 1))
-        wait_for_dma_loads_but<Cfg::kLoads>();
-      else
-        wait_for_dma_loads();
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-      for (int ks = 0; ks < Cfg::kAhead; ++ks) read_frags(after, ks, false);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    const int64_t k_off = first ? k_offset(kt + kStages) : 0;
-#pragma unroll
-    for (int g = 0; g < kMfmas; ++g) {
-      mfma(KS - 1, g);
-      if (first) {
-#pragma unroll
-        for (int idx = g * kFirst / kMfmas; idx < (g + 1) * kFirst / kMfmas; ++idx) issue_one(k_off, stage, idx);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    stage = after;
+    for (int j = 0; j < TN; ++j) masked(bf[ks][j]);
   };
 
-  // Fill the pipeline: the first kStages - 1 k-tiles and half of the next.
+  // One k-tile.  The barrier that hands over k-tile kt + 1 sits before the last
+  // k step: that step's MFMAs cover the first fragment reads of kt + 1, and the
+  // slot of B(kt) is free there (every wave holds its last fragments in registers).
+  //   k step 0:     A(kt + kDepth) into the slot of A(kt - 1)
+  //   wait for k-tile kt + 1, barrier
+  //   k step 1:     B(kt + kDepth) into the slot of B(kt)
+  // Each step reads the next one's fragments.  A request goes out behind every
+  // few MFMAs: several in one go hold up the wave.
+  static_assert(KS == 2, "the sequence above");
+  uint32_t a_slot = 0, b_slot = 0;  // of kt
+  const auto next_of = [](uint32_t slot, uint32_t bytes, uint32_t ring) { return slot + bytes == ring ? 0u : slot + bytes; };
+  constexpr int kReads = TM + TN, kReadSpan = kMfmas >= 2 * kReads ? kMfmas / 2 : kMfmas;
+  // more: k-tile kt + 1 exists; ahead: kt + kDepth does.  a_src and b_src point at the latter.
+  auto k_tile = [&](int kt, auto more_tag, auto ahead_tag) {
+    constexpr bool more = decltype(more_tag)::value, ahead = decltype(ahead_tag)::value;
+    const uint32_t a_next = next_of(a_slot, Cfg::kABytes, Cfg::kARing), b_next = next_of(b_slot, Cfg::kBBytes, Cfg::kBRing);
+    const uint32_t a_before = a_slot == 0 ? Cfg::kARing - Cfg::kABytes : a_slot - Cfg::kABytes;
+    // MFMA g of k step ks with what goes out behind it.
+    auto slice = [&](int ks, int g) {
+      const int i = g / TN, j = g % TN;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[ks][j], af[ks][i], acc[i][j], 0, 0, 0);
+      if (ks == 0 || more) {
 #pragma unroll
-  for (int kt = 0; kt < kStages; ++kt)
-    if (kt < ktiles) {
-      const int64_t k_off = k_offset(kt);
+        for (int r = 0; r < kReads; ++r)
+          if (r * kReadSpan / kReads == g) {
+            if (ks == 0) read_frag(a_slot, b_slot, 1, r);
+            else read_frag(a_next, b_next, 0, r);
+          }
+      }
+      if (ahead) {
 #pragma unroll
-      for (int idx = 0; idx < (kt + 1 < kStages ? Cfg::kLoads : kFirst); ++idx) issue_one(k_off, kt, idx);
+        for (int r = 0; r < (ks == 0 ? kLoadsA : kLoadsB); ++r)
+          if (r * kMfmas / (ks == 0 ? kLoadsA : kLoadsB) == g) {
+            if (ks == 0) issue(a_src, a_voff[r], a_before, r);
+            else issue(b_src, b_voff[r], Cfg::kARing + b_slot, r);
+          }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if (!more && tail) zero_past_k(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < kMfmas; ++g) slice(0, g);
+    if (more) {
+      // k-tile kt + 1 has landed (this wave's part); those behind it stay in flight.
+      if (ahead) {
+        wait_for_dma_loads_but<(kDepth - 1) * kLoadsA + (kDepth - 2) * kLoadsB>();
+      } else {
+        const int behind = ktiles - 2 - kt;
+        if (kDepth >= 4 && behind == 2) wait_for_dma_loads_but<2 * Cfg::kLoads>();
+        else if (kDepth >= 3 && behind == 1) wait_for_dma_loads_but<Cfg::kLoads>();
+        else wait_for_dma_loads();
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    } else if (tail) {
+      zero_past_k(1);
     }
-  if (ktiles >= kStages)
-    wait_for_dma_loads_but<(kStages - 2) * Cfg::kLoads + kFirst>();
-  else if (kStages >= 4 && ktiles == 3)
-    wait_for_dma_loads_but<2 * Cfg::kLoads>();
-  else if (kStages >= 3 && ktiles == 2)
-    wait_for_dma_loads_but<Cfg::kLoads>();
-  else
-    wait_for_dma_loads();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < kMfmas; ++g) slice(1, g);
+    a_slot = a_next;
+    b_slot = b_next;
+    if (ahead) {
+      a_src += Cfg::kRowBytes;
+      b_src += Cfg::kRowBytes;
+    }
+  };
+
+  // Fill the pipeline: the first kDepth k-tiles.
+#pragma unroll
+  for (int kt = 0; kt < kDepth; ++kt)
+    if (kt < ktiles) {
+      if (tail != 0 && kt == ktiles - 1) aim_at_tail();
+#pragma unroll
+      for (int q = 0; q < kLoadsA; ++q) issue(a_src, a_voff[q], kt * Cfg::kABytes, q);
+#pragma unroll
+      for (int q = 0; q < kLoadsB; ++q) issue(b_src, b_voff[q], Cfg::kARing + kt * Cfg::kBBytes, q);
+      a_src += Cfg::kRowBytes;
+      b_src += Cfg::kRowBytes;
+    }
+  if (kDepth >= 4 && ktiles >= 4) wait_for_dma_loads_but<3 * Cfg::kLoads>();
+  else if (kDepth >= 3 && ktiles >= 3) wait_for_dma_loads_but<2 * Cfg::kLoads>();
+  else if (ktiles >= 2) wait_for_dma_loads_but<Cfg::kLoads>();
+  else wait_for_dma_loads();
   asm volatile("s_barrier" ::: "memory");
 #pragma unroll
-  for (int ks = 0; ks < Cfg::kAhead; ++ks) read_frags(0, ks, false);
+  for (int g = 0; g < kReads; ++g) read_frag(0, 0, 0, g);
+  __builtin_amdgcn_sched_barrier(0);
   constexpr std::true_type yes{};
   constexpr std::false_type no{};
   int kt = 0;
-  for (; kt + kStages < ktiles; ++kt) k_tile(kt, yes, yes, no, no);
-  // Drain: nothing more to request but the half that is still due.
-  bool due = ktiles >= kStages;
-  for (; kt + 1 < ktiles; ++kt) {
-    if (due) k_tile(kt, yes, no, no, no);
-    else k_tile(kt, no, no, no, no);
-    due = false;
+  for (; kt + kDepth < ktiles; ++kt) {
+    if (tail != 0 && kt + kDepth == ktiles - 1) aim_at_tail();
+    k_tile(kt, yes, yes);
   }
-  if (tail_chunks != 0) {
-    // the fragments read ahead were read unmasked
-#pragma unroll
-    for (int ks = 0; ks < Cfg::kAhead; ++ks) read_frags(stage, ks, true);
-    k_tile(ktiles - 1, no, no, yes, yes);
-  } else {
-    k_tile(ktiles - 1, no, no, no, yes);
-  }
+  for (; kt + 1 < ktiles; ++kt) k_tile(kt, yes, no);
+  k_tile(ktiles - 1, no, no);
   __syncthreads();  // the images overlay the stages
   store_wave_tile<Cfg>(p, batch, m0 + wm * Cfg::kWaveM, n0 + wn * Cfg::kWaveN, lane, p.symmetric && tn >= p.symmetric * (tm + 1), acc,
                        lds_bytes + wave * Cfg::kRegion);

@@ -69,10 +69,10 @@ constexpr int kXcds = 8;         // accelerator dies, each with its own L2
 constexpr int kGroupTilesM = 4;  // tile rows walked together
 
 // Tile t of a (non-symmetric) matrix in the patch order described below.
-__device__ inline void tile_in_order(const GemmParams& p, int t, int* tm, int* tn) {
-  const int group_span = kGroupTilesM * p.tiles_n;
-  const int first_m = (t / group_span) * kGroupTilesM;
-  const int rows = min(p.tiles_m - first_m, kGroupTilesM);
+__device__ inline void tile_in_order(const GemmParams& p, int t, int* tm, int* tn, int rows_together = kGroupTilesM) {
+  const int group_span = rows_together * p.tiles_n;
+  const int first_m = (t / group_span) * rows_together;
+  const int rows = min(p.tiles_m - first_m, rows_together);
   const int within = t % group_span;
   *tm = first_m + within % rows;
   *tn = within / rows;
@@ -85,7 +85,8 @@ __device__ inline void tile_in_order(const GemmParams& p, int t, int* tm, int* t
 // patch of tiles of one matrix: its L2 then serves 12 distinct operand panels
 // per k-tile instead of 33.  Returns false for the padding ids at the end of
 // an XCD's run.
-__device__ inline bool tile_of_workgroup(const GemmParams& p, int64_t id, int64_t* batch, int* tm, int* tn) {
+__device__ inline bool tile_of_workgroup(const GemmParams& p, int64_t id, int64_t* batch, int* tm, int* tn,
+                                         int rows_together = kGroupTilesM) {
   const int64_t slot = id / kXcds;
   const int64_t item = (id % kXcds) * p.items_per_xcd + slot;
   if (item >= p.work_items) return false;
@@ -106,7 +107,7 @@ __device__ inline bool tile_of_workgroup(const GemmParams& p, int64_t id, int64_
     *tn = p.symmetric * r + t;
     return true;
   }
-  tile_in_order(p, t, tm, tn);
+  tile_in_order(p, t, tm, tn, rows_together);
   return true;
 }
 

@@ -14,8 +14,8 @@
 //
 // GEMM kernels, operands global -> LDS directly: 256x256x64 tiles of 2x2
 // wavefronts on v_mfma_f32_16x16x32_bf16 for large problems (below; those of
-// Newton-Schulz need not be whole tiles), smaller tiles on 32x32x16 for
-// everything else (gemm_tiles.hpp).
+// Newton-Schulz need not be whole tiles), smaller tiles for everything else
+// (gemm_tiles.hpp).
 #include "gemm_tiles.hpp"
 #include "muon_groups.hpp"
 
@@ -490,13 +490,15 @@ struct PlannedGemm {
 //   2048 x 2048    11.5 / 30.6    9.7 / 22.7   11.6 / 28.0   17.2 / 40.6
 //   4096 x 2048    18.8 / 55.6   15.5 / 40.0   14.9 / 36.5   18.8 / 43.4
 //   4096 x 4096    35.9 / 108.5  27.3 / 80.5   28.0 / 74.6   22.4 / 53.3
+// The three smaller kinds have become 5 to 20 % faster since, much alike
+// (4096 x 4096 30.7 / 97.0  22.6 / 60.8  24.8 / 60.4), so the choice among them stands.
 enum TileKind { kTiles64, kTiles128, kTiles128Deep, kTiles256x128, kTiles256 };  // the order of kTileShapes
 constexpr int kTileNames[] = {FSH_TILES_64, FSH_TILES_128, FSH_TILES_128_DEEP, FSH_TILES_256X128, FSH_TILES_256};
 constexpr TileShape kTileShapes[] = {
-    {64, 64, 768.0, 0.17, 0.40, 0.55, 1.7},       // three workgroups per compute unit
+    {64, 64, 768.0, 0.17, 0.40, 0.55, 1.7},       // three workgroups per compute unit (four fit)
     {128, 128, 512.0, 0.37, 0.71, 1.02, 4.2},     // two
-    {128, 128, 256.0, 0.35, 0.43, 0.52, 3.2},     // one, its operands requested three k-tiles ahead
-    {256, 128, 256.0, 0.54, 0.68, 0.91, 5.5},     // one of eight waves
+    {128, 128, 256.0, 0.35, 0.43, 0.52, 3.2},     // one, its operands requested four k-tiles ahead
+    {256, 128, 256.0, 0.54, 0.68, 0.91, 5.5},     // one
     {256, 256, 256.0, 0.94, 1.02, 1.38, 8.5},     // one
 };
 // The products of one launch, as the tiles of every kind see them.
@@ -695,11 +697,12 @@ int launch_large_tiles(const GemmLaunch& launch, bool k_major, hipStream_t strea
   }
 }
 
-template <typename Cfg, int kBlocksPerUnit>
+template <typename Cfg, int kBlocksPerUnit, bool kWide = false>
 int launch_tiles_as(const TileLaunch& launch, hipStream_t stream) {
   static LdsReservation reserved;
-  if (int rc = reserve_lds_once(reserved, &gemm_nt_tiles_kernel<Cfg, kBlocksPerUnit>, Cfg::kLdsBytes)) return rc;
-  hipLaunchKernelGGL((gemm_nt_tiles_kernel<Cfg, kBlocksPerUnit>), dim3(static_cast<uint32_t>(launch.total_workgroups)),
+  constexpr auto* kernel = &gemm_nt_tiles_kernel<Cfg, kBlocksPerUnit, kWide>;
+  if (int rc = reserve_lds_once(reserved, kernel, Cfg::kLdsBytes)) return rc;
+  hipLaunchKernelGGL((gemm_nt_tiles_kernel<Cfg, kBlocksPerUnit, kWide>), dim3(static_cast<uint32_t>(launch.total_workgroups)),
                      dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, launch);
   return check_launch("gemm_nt_tiles_kernel");
 }
@@ -713,15 +716,28 @@ LaunchWork work_of(const PlannedGemm* plans, const int* members, int n) {
   return work;
 }
 
+// Rows so long that the operand offsets of a tile of any kind need 64 bits.
+bool has_wide_rows(const PlannedGemm* plans, const int* members, int n) {
+  for (int k = 0; k < n; ++k) {
+    const GemmParams& p = plans[members[k]].p;
+    if (256 * 2 * (p.lda > p.ldb ? p.lda : p.ldb) >= (1LL << 31)) return true;
+  }
+  return false;
+}
+TileKind small_tile_kind_of(const PlannedGemm* plans, const int* members, int n) {
+  return has_wide_rows(plans, members, n) ? kTiles128 : small_tile_kind(work_of(plans, members, n));
+}
+
 int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stream) {
-  const TileKind kind = small_tile_kind(work_of(plans, members, n));
+  const TileKind kind = small_tile_kind_of(plans, members, n);
   TileLaunch launch;
   if (int rc = fill_launch(plans, members, n, kTileShapes[kind].m, kTileShapes[kind].n, &launch)) return rc;
+  if (has_wide_rows(plans, members, n)) return launch_tiles_as<GemmTiles<2, 2, 4, 4, 2>, 2, true>(launch, stream);
   switch (kind) {
-    case kTiles64: return launch_tiles_as<GemmTiles<2, 2, 1, 1, 3>, 3>(launch, stream);
-    case kTiles128: return launch_tiles_as<GemmTiles<2, 2, 2, 2, 2>, 2>(launch, stream);
-    case kTiles128Deep: return launch_tiles_as<GemmTiles<2, 2, 2, 2, 4>, 1>(launch, stream);
-    default: return launch_tiles_as<GemmTiles<4, 2, 2, 2, 3>, 1>(launch, stream);
+    case kTiles64: return launch_tiles_as<GemmTiles<2, 2, 2, 2, 2>, 4>(launch, stream);
+    case kTiles128: return launch_tiles_as<GemmTiles<2, 2, 4, 4, 2>, 2>(launch, stream);
+    case kTiles128Deep: return launch_tiles_as<GemmTiles<2, 2, 4, 4, 4>, 1>(launch, stream);
+    default: return launch_tiles_as<GemmTiles<2, 2, 8, 4, 2>, 1>(launch, stream);
   }
 }
 
@@ -820,7 +836,7 @@ void report_tiles(const PlannedGemm* plans, int count, int32_t* tiles) {
       if (plans[next].large) tiles[next] = FSH_TILES_256;
       else members[n++] = next;
     }
-    const TileKind kind = small_tile_kind(work_of(plans, members, n));
+    const TileKind kind = small_tile_kind_of(plans, members, n);
     for (int k = 0; k < n; ++k) tiles[members[k]] = kTileNames[kind];
   }
 }
