@@ -30,15 +30,6 @@ struct GemmTiles {
   static_assert(kDepth >= 2 && kDepth <= 4, "the waits of the k loop's end");
 };
 
-// Four values of one column and four consecutive rows out of a bf16 image with
-// rows in LDS: within 16 lanes, lane 4 j + q passes the address of columns
-// 4 q .. 4 q + 3 of row j, and lane t receives column t of rows 0 .. 3.
-__device__ __forceinline__ u32x2 read_lds_transposed(const uint8_t* at) {
-  typedef short i16x4 __attribute__((__vector_size__(4 * sizeof(short))));
-  typedef __attribute__((address_space(3))) i16x4* lds_i16x4;
-  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)(const_cast<uint8_t*>(at))));
-}
-
 // Finals bf16(fma(beta, D, alpha * acc) + diagonal term) of a wave's sub-tile
 // at (row0, col0), through its LDS image: D arrives row-wise and C leaves
 // row-wise; the transposed (or mirrored) output is read across the image, two

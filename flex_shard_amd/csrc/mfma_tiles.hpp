@@ -203,6 +203,15 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Four values of one column and four consecutive rows out of a bf16 image with
+// rows in LDS: within 16 lanes, lane 4 j + q passes the address of columns
+// 4 q .. 4 q + 3 of row j, and lane t receives column t of rows 0 .. 3.
+__device__ __forceinline__ u32x2 read_lds_transposed(const uint8_t* at) {
+  typedef short i16x4 __attribute__((__vector_size__(4 * sizeof(short))));
+  typedef __attribute__((address_space(3))) i16x4* lds_i16x4;
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)(const_cast<uint8_t*>(at))));
+}
+
 // Epilogue of the large-tile kernel, staged through LDS.
 //
 // The accumulate is issued as mfma(B, A), so accumulator r of block (i, j)
@@ -215,8 +224,9 @@ __device__ __forceinline__ void wave_lds_sync() {
 //      written to LDS as [row][col], each over the D value it used;
 //   2. the wave reads its region back row-wise and stores C as 16 bytes per
 //      lane, 256 contiguous bytes per row;
-//   3. for a transposed (or mirrored) output the finals are read back in
-//      accumulator layout, written again as [col][row] and leave the same way.
+//   3. a transposed (or mirrored) output is read across the image: lane t of
+//      group g of 16 takes column t of 16, rows 8 g .. 8 g + 7 of 32, in two
+//      transposing reads, and 64 contiguous bytes of 16 output rows leave per store.
 // The LDS row pitch is the row plus 16 bytes: 8-byte writes of 32 lanes (16
 // rows, two groups of columns) then cover all banks, and rows are read 16 bytes
 // at a time.
@@ -231,9 +241,7 @@ template <typename Cfg>
 struct HalfTileEpilogue {
   static constexpr int kRows = Cfg::kWaveM / 2;                 // 64
   static constexpr int kPitch = Cfg::kWaveN * 2 + 16;           // [row][col] image
-  static constexpr int kPitchT = kRows * 2 + 8;                 // [col][row] image
-  static constexpr int kRegion =
-      (kRows * kPitch > Cfg::kWaveN * kPitchT) ? kRows * kPitch : Cfg::kWaveN * kPitchT;
+  static constexpr int kRegion = kRows * kPitch;
   static constexpr int kLdsBytes = Cfg::WM * Cfg::WN * kRegion;
 };
 
@@ -354,29 +362,21 @@ __device__ __forceinline__ void store_tile_in_halves_as(const GemmParams& p, int
         region, C + (wave_row + hf * Epi::kRows) * p.ldc + wave_col, p.ldc, rows_left - hf * Epi::kRows, cols_left, lane);
     if (hf == 1) FSH_STAMP(10);
     if (Ct != nullptr) {  // uniform over the workgroup
-      // The finals come back in accumulator layout (every read before the
-      // first write: the transposed image reuses the region).
-      u32x2 fin[HM][TN];
+      const int t = lane & 15, g = lane >> 4;
+      const int64_t lane_off = t * ldct * 2 + g * 16;
+      uint8_t* base = uniform_ptr(reinterpret_cast<uint8_t*>(Ct + wave_col * ldct + wave_row + hf * Epi::kRows));
+      const int64_t block_bytes = uniform_i64(32 * ldct);
+      const uint8_t* from = region + (8 * g + (t >> 2)) * Epi::kPitch + (t & 3) * 8;
 #pragma unroll
-      for (int ih = 0; ih < HM; ++ih)
+      for (int j = 0; j < TN; ++j) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-          fin[ih][j] = *reinterpret_cast<const u32x2*>(region + (ih * 16 + r_lane) * Epi::kPitch + (j * 16 + c_lane) * 2);
-      wave_lds_sync();  // these reads and the row reads are done before the region is reused
-#pragma unroll
-      for (int ih = 0; ih < HM; ++ih)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const uint32_t pair = (t >> 1) ? fin[ih][j].y : fin[ih][j].x;
-            *reinterpret_cast<uint16_t*>(region + (j * 16 + c_lane + t) * Epi::kPitchT + (ih * 16 + r_lane) * 2) =
-                static_cast<uint16_t>((t & 1) ? (pair >> 16) : pair);
-          }
-      if (hf == 1) FSH_STAMP(12);
-      wave_lds_sync();
-      store_staged_rows<Cfg::kWaveN, Epi::kRows * 2, Epi::kPitchT>(
-          region, Ct + wave_col * ldct + wave_row + hf * Epi::kRows, ldct, cols_left, rows_left - hf * Epi::kRows, lane);
+        for (int rb = 0; rb < Epi::kRows / 32; ++rb) {
+          const u32x2 lo = read_lds_transposed(from + rb * 32 * Epi::kPitch + j * 32);
+          const u32x2 hi = read_lds_transposed(from + (rb * 32 + 4) * Epi::kPitch + j * 32);
+          if (!kRagged || (j * 16 + t < cols_left && rb * 32 + 8 * g < rows_left - hf * Epi::kRows))
+            *reinterpret_cast<u32x4*>(base + j * block_bytes + rb * 64 + lane_off) = u32x4{lo.x, lo.y, hi.x, hi.y};
+        }
+      }
     }
     if (hf == 0) FSH_STAMP(8);
     if (hf == 0) wave_lds_sync();  // before the lower half overwrites the region
