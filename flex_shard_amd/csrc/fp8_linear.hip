@@ -102,57 +102,60 @@ __global__ __launch_bounds__(kActThreads) void act_quant_1x128_kernel(const ActQ
 // architectural VGPRs, where the vector ALU folds into them, and two waves
 // share a SIMD, so one wave's folds run under the other's MFMAs.  Operand
 // tiles are 128 bytes per row and k-tile and travel global -> LDS directly,
-// 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7), into one of two 64 KB
-// stages.
+// 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7).
 //
-// Bound by the vector ALU and, in the block-scale form, by power (matrix cores
-// 64 % busy at 1.73 GHz; column scales 51 % at 1.93: two vector operations per
-// element and k-block).  A 16x16x128 MFMA is a block's whole product of a
-// k-tile: four registers that a fold can follow four blocks later, where the
-// two 32x32x64 ones before it held sixteen and had to be folded behind the next
-// pair; and the k-tile is a tag's two instantiations instead of a branch per
-// request.  8192 tokens, us of both in turn on one part: 4096 x 4096 122 / 114,
-// 14336 x 4096 428 / 414, 4096 x 14336 410 / 398; weight gradients 130 / 124, 477 /
-// 457, 472 / 451 (3-7 %; clocks differ between parts, and with them the times and
-// the gain).  Same bits.
+// Bound by power, and with column scales by the vector ALU as well (two
+// operations per element and k-block).  What the parts cost, us of 8192 x 14336,
+// k 4096 (404), and of its weight gradient (449): without the requests of the
+// loop 315 and 390, with operands that stay in L2 367 and 422, without the
+// fragment reads 378 and 397, without the folds 367 and 340.
+//
+// A 16x16x128 MFMA is a block's whole product of a k-tile: four registers
+// that a fold can follow four blocks later.  LDS holds two k-tiles and three
+// eighths of a third, in chunks of 64 rows, so that the requests of a k-tile
+// leave one by one behind its MFMAs.  In two 64 KB stages they had to leave in
+// half of it: they then ask for all that the request path can take (64 of 16
+// cycles in 1024), and the last were waited for.  One round of k-tiles on the same
+// card, us before / with the chunks (same bits): forward 4096 x 4096 110 / 110,
+// 14336 x 4096 419 / 403, 4096 x 14336 399 / 370, 1024 x 4096 (half tiles) 39.3 / 34.2;
+// weight gradients 122 / 121, 455 / 441, 449 / 437.  The scales of a k-tile take one 4-byte
+// request of each wave; the block scales had a window of 256 k-tiles of their own
+// and an instantiation that refilled it.
 //
 // TM_ = 1 is the half tile (128 x 256, waves of 32 x 128) that the tiles of a
-// last, at most half-full round are cut into; it keeps the LDS layout of the
-// whole tile and fills the first half of the A area.
+// last, at most half-full round are cut into.
 template <int TM_>
 struct Fp8GemmCfg {
   static constexpr int BM = 128 * TM_, BN = 256, BK = 128, WM = 4, WN = 2;
   static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves, kWaveM = BM / WM, kWaveN = BN / WN;
   static constexpr int TM = kWaveM / 16, TN = kWaveN / 16;  // blocks of 16 x 16 per wave
   static constexpr int kRowBytes = 128;
-  static constexpr int kABytes = 256 * kRowBytes;              // 32 KB (half of it used by the half tile)
-  static constexpr int kStageBytes = (256 + BN) * kRowBytes;   // 64 KB
-  static constexpr int kFillRows = 8 * kWaves;                 // tile rows per wave-level load of all waves
-  static constexpr int kLoadsA = BM / kFillRows, kLoadsB = BN / kFillRows;  // per wave: 4 (2) and 4
+  // A chunk is what one request of every wave fills: 64 rows of an operand.
+  static constexpr int kChunkRows = 8 * kWaves, kChunkBytes = kChunkRows * kRowBytes;       // 8 KB
+  static constexpr int kChunksA = BM / kChunkRows, kChunks = kChunksA + BN / kChunkRows;    // per k-tile: 8 (6)
+  // LDS holds 19: the early chunks of a k-tile, the first of operand A (all of
+  // a half tile's), have three slots each and are requested a k-tile ahead of
+  // the late ones, which have two.
+  static constexpr int kSlots = 19;
+  static constexpr int kEarly = kSlots - 2 * kChunks < kChunks ? kSlots - 2 * kChunks : kChunks, kLate = kChunks - kEarly;
+  static constexpr int kEarlyBytes = kEarly * kChunkBytes, kLateBytes = kLate * kChunkBytes;
+  static constexpr int kLateOffset = 3 * kEarlyBytes;
   static constexpr int kPitch = kWaveN * 2 + 16;               // epilogue staging, bytes
   static constexpr int kRegion = kWaveM * kPitch;              // per wave
-  static constexpr int kStages = 2;
-  static constexpr int kScaleSlots = 64;                        // row scales per wave and stage (one 4-byte request per lane)
-  static constexpr int kScaleStageBytes = kWaves * kScaleSlots * 4;
-  static constexpr int kScaleOffset = kStages * kStageBytes;
-  static constexpr int kWeightScaleOffset = kScaleOffset + kStages * kScaleStageBytes;  // [wave][256] block scales
-  static constexpr int kMaxKTilesInLds = 256;  // window of weight block scales kept in LDS per wave (a power of two)
-  static constexpr int kLdsBytes = max_int(kWeightScaleOffset + kWaves * kMaxKTilesInLds * 4, kWaves * kRegion);
-  static_assert(kWaveM <= kScaleSlots, "one 4-byte scale request per lane covers the wave's rows");
+  // Two stages of scales: 256 row scales, then 256 column scales (or the two
+  // block scales, 64 times each).
+  static constexpr int kScaleOffset = kSlots * kChunkBytes, kScaleStageBytes = 2048;
+  static constexpr int kLdsBytes = kScaleOffset + 2 * kScaleStageBytes;
+  static_assert(kLdsBytes <= 160 * 1024 && kWaves * kRegion <= kLdsBytes, "LDS of a compute unit");
+  static_assert(kEarly > 0 && 3 * kEarly + 2 * kLate <= kSlots, "two k-tiles and a part of the next");
 };
 using Fp8Gemm = Fp8GemmCfg<2>;
-static_assert(Fp8GemmCfg<1>::kLdsBytes <= Fp8Gemm::kLdsBytes, "the half tile lives in the whole tile's LDS");
 
 // One output tile (TM_ = 2) or half tile (TM_ = 1, rows [128 half, +128) of the tile).
-// kLongK: the contraction is longer than one window of weight block scales
-// (kMaxKTilesInLds k-tiles); the block-scale variant then refills the window
-// inside the loop.  A separate instantiation: the refill's few instructions
-// cost the loop 12 % of its rate, which the usual lengths should not pay.
-template <bool kColumnScales, int TM_, bool kLongK>
+template <bool kColumnScales, int TM_>
 __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* lds_bytes, int tm, int tn, int half) {
   using Cfg = Fp8GemmCfg<TM_>;
-  static_assert(Cfg::kStages == 2, "the loop below alternates between two stages");
-  constexpr int TM = Cfg::TM, TN = Cfg::TN;
+  constexpr int TM = Cfg::TM, TN = Cfg::TN, kChunks = Cfg::kChunks, kChunksA = Cfg::kChunksA, kEarly = Cfg::kEarly;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -163,40 +166,65 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
 #ifdef FSH_TRACE
   const uint64_t t_entry = __builtin_amdgcn_s_memrealtime();
 #endif
-  const int64_t ktiles = p.k / Cfg::BK;
+  const int ktiles = static_cast<int>(p.k / Cfg::BK);
 
-  // Load side: wave-level load q of a wave fills tile rows [64 q + 8 wave, +8);
-  // lane l fills slot l & 7 of row l >> 3 there.  Rows past the matrix are
-  // read from its last row (their products are never stored).
+  // Load side: request c of a wave fills rows [64 c + 8 wave, +8) of the tile's
+  // operand A, from c = kChunksA on of operand B; lane l fills slot l & 7 of
+  // row l >> 3 there.  Rows past the matrix are read from its last row (their
+  // products are never stored).
   const int fill_row = lane >> 3;
   const int fill_chunk = (lane & 7) ^ (((8 * wave + fill_row) >> 1) & 7);
-  uint32_t a_voff[Cfg::kLoadsA], b_voff[Cfg::kLoadsB];
+  uint32_t voff[kChunks];
 #pragma unroll
-  for (int q = 0; q < Cfg::kLoadsA; ++q) {
-    int64_t row = m0 + Cfg::kFillRows * q + 8 * wave + fill_row;
-    row = row < p.m ? row : p.m - 1;
-    a_voff[q] = static_cast<uint32_t>((row - m0) * p.ldxq + fill_chunk * 16);
-  }
-#pragma unroll
-  for (int q = 0; q < Cfg::kLoadsB; ++q) {
-    int64_t row = n0 + Cfg::kFillRows * q + 8 * wave + fill_row;
-    row = row < p.n ? row : p.n - 1;
-    b_voff[q] = static_cast<uint32_t>((row - n0) * p.ldwq + fill_chunk * 16);
+  for (int c = 0; c < kChunks; ++c) {
+    const int64_t first = c < kChunksA ? m0 : n0, size = c < kChunksA ? p.m : p.n, ld = c < kChunksA ? p.ldxq : p.ldwq;
+    int64_t row = first + Cfg::kChunkRows * (c < kChunksA ? c : c - kChunksA) + 8 * wave + fill_row;
+    row = row < size ? row : size - 1;
+    voff[c] = static_cast<uint32_t>((row - first) * ld + fill_chunk * 16);
   }
   const uint8_t* Ab = uniform_ptr(p.xq + m0 * p.ldxq);
   const uint8_t* Bb = uniform_ptr(p.wq + n0 * p.ldwq);
   typedef __attribute__((address_space(3))) uint8_t* lds_address;
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_address)lds_bytes));
   const uint32_t fill_lds = lds_base + static_cast<uint32_t>(wave * 1024);
-  auto issue_tile_load = [&](int64_t kt, int stage_off) {
-    const uint8_t* a_src = Ab + kt * Cfg::kRowBytes;
-    const uint8_t* b_src = Bb + kt * Cfg::kRowBytes;
-#pragma unroll
-    for (int q = 0; q < Cfg::kLoadsA; ++q)
-      dma_load_16(a_voff[q], a_src, stage_off + fill_lds, q * Cfg::kFillRows * Cfg::kRowBytes);
-#pragma unroll
-    for (int q = 0; q < Cfg::kLoadsB; ++q)
-      dma_load_16(b_voff[q], b_src, stage_off + fill_lds, Cfg::kABytes + q * Cfg::kFillRows * Cfg::kRowBytes);
+  // Where a k-tile lies: the offsets of its early chunks and of its late ones.
+  struct Place {
+    int early, late;
+  };
+  const auto place_after = [](const Place& at) {
+    return Place{at.early == 2 * Cfg::kEarlyBytes ? 0 : at.early + Cfg::kEarlyBytes,
+                 at.late == Cfg::kLateOffset ? Cfg::kLateOffset + Cfg::kLateBytes : Cfg::kLateOffset};
+  };
+  auto request = [&](int kt, const Place& at, int c) {
+    dma_load_16(voff[c], (c < kChunksA ? Ab : Bb) + static_cast<int64_t>(kt) * Cfg::kRowBytes,
+                fill_lds + (c < kEarly ? at.early : at.late), (c < kEarly ? c : c - kEarly) * Cfg::kChunkBytes);
+  };
+  // The scales of a k-tile ride the same global->LDS path: 64 row scales by
+  // each of the first four waves, 64 column scales by each of the others -- or
+  // by two of them each the block scale of 128 of the tile's columns, 64 times.
+  // (A load that the compiler sees inside the loop makes it wait for all
+  // requests in flight.)
+  const float* scale_src = p.xs;
+  int64_t scale_step = p.m;
+  uint32_t scale_voff = 0, scale_slot = wave % (Cfg::BM / 64);
+  if (wave < 4) {
+    const int64_t row = m0 + scale_slot * 64 + lane;
+    scale_voff = static_cast<uint32_t>((row < p.m ? row : p.m - 1) * 4);
+  } else if (kColumnScales) {
+    const int64_t col = n0 + (wave - 4) * 64 + lane;
+    scale_voff = static_cast<uint32_t>((col < p.n ? col : p.n - 1) * 4);
+    scale_src = p.cs;
+    scale_step = p.n;
+    scale_slot = wave;
+  } else {
+    const int64_t block = n0 / 128 + (wave >> 1 & 1), last = (p.n - 1) / 128;
+    scale_src = p.ws + (block < last ? block : last) * p.ws_cb;
+    scale_step = p.ws_kb;
+    scale_slot = 4 + (wave >> 1 & 1);
+  }
+  const uint32_t scale_lds = lds_base + Cfg::kScaleOffset + scale_slot * 256;
+  auto request_scales = [&](int kt) {
+    dma_touch_4(scale_voff, reinterpret_cast<const uint8_t*>(scale_src + kt * scale_step), scale_lds + (kt & 1) * Cfg::kScaleStageBytes);
   };
 
   // Fragment side: row = lane & 15 of a 16-row block, chunks g and g + 4 of its
@@ -210,18 +238,14 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
 #pragma unroll
   for (int c = 0; c < 2; ++c)
     frag_off[c] = static_cast<uint32_t>(frag_row * Cfg::kRowBytes + (((group + 4 * c) ^ ((frag_row >> 1) & 7)) * 16));
-  auto read_frag = [&](int stage_off, int operand_off, int block) -> v8i32 {
-    const uint8_t* base = lds_bytes + stage_off + operand_off + block * 16 * Cfg::kRowBytes;
+  // `row` of the rows that start at `chunk`
+  auto read_frag = [&](int chunk, int row) -> v8i32 {
+    const uint8_t* base = lds_bytes + chunk + row * Cfg::kRowBytes;
     const u32x4 lo = *reinterpret_cast<const u32x4*>(base + frag_off[0]);
     const u32x4 hi = *reinterpret_cast<const u32x4*>(base + frag_off[1]);
     return v8i32{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z), static_cast<int>(lo.w),
                  static_cast<int>(hi.x), static_cast<int>(hi.y), static_cast<int>(hi.z), static_cast<int>(hi.w)};
   };
-
-  // Scales: a lane owns output row lane & 15 of each of its 16-row blocks, so it
-  // needs xs[kb][row] of those and the one weight scale of the wave's 128 columns.
-  const int64_t wcol = n0 + wn * Cfg::kWaveN;
-  const int64_t wblock = (wcol < p.n ? wcol : p.n - 1) / 128;
 
   f32x4 acc[TM][TN];
 #pragma unroll
@@ -229,78 +253,19 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // Two stages: the operands of k-tile kt + 1 are in flight while kt is
-  // multiplied.  The row scales ride the same global->LDS path (one 4-byte-
-  // per-lane request per wave and k-tile for the wave's 64 rows): a
-  // compiler-visible load here would make the compiler wait for everything in
-  // flight, the prefetched tile included.
-  const uint32_t scale_lds0 = lds_base + static_cast<uint32_t>(Cfg::kScaleOffset + wave * Cfg::kScaleSlots * 4);
-  const int64_t scale_row = m0 + wm * Cfg::kWaveM + (lane & (Cfg::kWaveM - 1));  // lanes past the wave's rows repeat them
-  const uint32_t scale_voff = static_cast<uint32_t>((scale_row < p.m ? scale_row : p.m - 1) * 4);
-  // Per-column scales of the workgroup's 256 columns take the same road, 64
-  // columns per wave (the first four waves), into [stage][256] floats of the
-  // block-scale area.
-  const uint32_t cscale_lds0 = lds_base + static_cast<uint32_t>(Cfg::kWeightScaleOffset + wave * 256);
-  const int64_t cscale_col0 = n0 + wave * 64 + lane;
-  const uint32_t cscale_voff = static_cast<uint32_t>((cscale_col0 < p.n ? cscale_col0 : p.n - 1) * 4);
-  auto issue_scale_loads = [&](int64_t kt, int stage) {
-    const uint8_t* xs_row = reinterpret_cast<const uint8_t*>(p.xs + kt * p.m);
-    dma_touch_4(scale_voff, xs_row, scale_lds0 + stage * Cfg::kScaleStageBytes);
-    if (kColumnScales && wave < 4)
-      dma_touch_4(cscale_voff, reinterpret_cast<const uint8_t*>(p.cs + kt * p.n), cscale_lds0 + stage * 1024);
-  };
-  auto issue_k_tile = [&](int64_t kt, int stage) {
-    issue_tile_load(kt, stage * Cfg::kStageBytes);
-    issue_scale_loads(kt, stage);
-  };
-  // One of the wave's requests for the next k-tile; they are issued a few at
-  // a time behind the MFMAs of the first blocks rather than all at once, which
-  // would hold up the wave's instruction issue while the matrix core runs dry.
-  auto issue_k_tile_part = [&](int64_t kt, int stage, int part) {
-    const int stage_off = stage * Cfg::kStageBytes;
-    if (part >= Cfg::kLoadsA + Cfg::kLoadsB) return;
-    if (part >= Cfg::kLoadsA) {
-      const int q = part - Cfg::kLoadsA;
-      dma_load_16(b_voff[q], Bb + kt * Cfg::kRowBytes,
-                  stage_off + fill_lds, Cfg::kABytes + q * Cfg::kFillRows * Cfg::kRowBytes);
-    } else {
-      dma_load_16(a_voff[part], Ab + kt * Cfg::kRowBytes, stage_off + fill_lds, part * Cfg::kFillRows * Cfg::kRowBytes);
-    }
-    if (part == 0) issue_scale_loads(kt, stage);
-  };
-  // The first k-tile's requests go out before anything else that has to wait
-  // for memory.  The block scales of the wave's 128 columns, one per k-tile,
-  // are copied to LDS once, under those requests (a load from global memory
-  // inside the loop would again wait for the prefetched tile).
-  issue_k_tile(0, 0);
-  float* ws_lds = reinterpret_cast<float*>(lds_bytes + Cfg::kWeightScaleOffset + wave * Cfg::kMaxKTilesInLds * 4);
-  // ws_lds holds the scales of k-tiles [window, window + kMaxKTilesInLds).
-  // For a contraction of at most one window they are copied once, under the
-  // first k-tile's requests.  A longer one (kLongK) refills the window when
-  // the loop reaches its last k-tile, and then the scales travel global -> LDS
-  // like everything else the loop reads (four 4-byte-per-lane requests per
-  // window): a load the compiler sees inside the loop makes it wait for all
-  // memory traffic in flight on every iteration (measured: 20 % slower).
-  const uint32_t ws_lds_addr = lds_base + static_cast<uint32_t>(Cfg::kWeightScaleOffset + wave * Cfg::kMaxKTilesInLds * 4);
-  auto issue_weight_scale_window = [&](int64_t first_kt) {
-    const uint8_t* ws_row = reinterpret_cast<const uint8_t*>(p.ws + wblock * p.ws_cb);
+  // The first k-tile and the early chunks of the second.
+  Place now{0, Cfg::kLateOffset};  // of k-tile kt
+  request_scales(0);
 #pragma unroll
-    for (int q = 0; q < Cfg::kMaxKTilesInLds / 64; ++q) {
-      int64_t kt_of_lane = first_kt + q * 64 + lane;
-      kt_of_lane = kt_of_lane < ktiles ? kt_of_lane : ktiles - 1;  // past the end: any valid entry, never read
-      dma_touch_4(static_cast<uint32_t>(kt_of_lane * p.ws_kb * 4), ws_row, ws_lds_addr + q * 256);
-    }
-  };
-  if (!kColumnScales) {
-    if (kLongK) {
-      issue_weight_scale_window(0);
-    } else {
-      const float* ws_row = p.ws + wblock * p.ws_cb;
-      for (int64_t i = lane; i < ktiles; i += 64) ws_lds[i] = ws_row[i * p.ws_kb];  // ktiles <= kMaxKTilesInLds (host)
-    }
+  for (int c = 0; c < kChunks; ++c) request(0, now, c);
+  if (ktiles > 1) {
+#pragma unroll
+    for (int c = 0; c < kEarly; ++c) request(1, place_after(now), c);
+    wait_for_dma_loads_but<kEarly>();
+  } else {
+    wait_for_dma_loads();
   }
-  wait_for_dma_loads();
-  __syncthreads();
+  asm volatile("s_barrier" ::: "memory");
 
 #ifdef FSH_TRACE
   // Time per phase of the k loop, summed over the k-tiles (10 ns ticks).
@@ -317,58 +282,53 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
   // its MFMAs the wave reads the fragment of kt + 1 that takes the place of the
   // one just used.
   //   carried into a k-tile: afrag, bfrag[0]
+  // Behind that barrier the slots of k-tile kt are free: in k-tile kt + 1 the
+  // late chunks of kt + 2 go out, then the early ones of kt + 3, one request
+  // behind every few MFMAs.
   constexpr int kBlocks = TM * TN;
   v8i32 afrag[TM], bfrag[2];
   constexpr int kScaleRegs = TN / 4;
   float s[TM], cs_rows[kScaleRegs];
-  // Row scales of the wave's rows for the k-tile in `stage`, times the weight
-  // block's scale in the block-scale variant.
-  auto read_row_scales = [&](float (&dst)[TM], int stage, int64_t kt) {
+  // Row scales of the wave's rows for k-tile kt, times the block scale in the
+  // block-scale variant; a lane owns output row lane & 15 of each of its blocks.
+  auto read_scales = [&](int kt) {
+    const float* rows = reinterpret_cast<const float*>(lds_bytes + Cfg::kScaleOffset + (kt & 1) * Cfg::kScaleStageBytes);
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-      dst[i] = *reinterpret_cast<const float*>(lds_bytes + Cfg::kScaleOffset + stage * Cfg::kScaleStageBytes +
-                                               (wave * Cfg::kScaleSlots + i * 16 + frag_row) * 4);
-    if (!kColumnScales) {
-      const float ws_now = ws_lds[kLongK ? (kt & (Cfg::kMaxKTilesInLds - 1)) : kt];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) dst[i] *= ws_now;
-    }
-  };
-  // Per-column scales: register q holds, in every row of 16 lanes, the 16
-  // scales that the lanes of that row fold column blocks 4 q .. 4 q + 3 with:
-  // lane 4 b + r of the row the scale of accumulator r of block 4 q + b.  A fold
-  // takes it through the data-parallel-primitive broadcast of the multiply-add
-  // itself: no scale is read from LDS between a product and its fold.
-  auto read_column_scales = [&](float (&dst)[kScaleRegs], int stage) {
+    for (int i = 0; i < TM; ++i) s[i] = rows[wm * Cfg::kWaveM + i * 16 + frag_row];
     if (kColumnScales) {
-      const uint8_t* cscale_lds = lds_bytes + Cfg::kWeightScaleOffset + stage * 1024 +
-                                  (wn * Cfg::kWaveN + 16 * ((lane & 15) >> 2) + 4 * group + (lane & 3)) * 4;
+      // Register q holds, in every row of 16 lanes, the 16 scales that the lanes
+      // of that row fold column blocks 4 q .. 4 q + 3 with: lane 4 b + r of the
+      // row the scale of accumulator r of block 4 q + b.  A fold takes it through
+      // the data-parallel-primitive broadcast of the multiply-add itself.
 #pragma unroll
-      for (int q = 0; q < kScaleRegs; ++q) dst[q] = *reinterpret_cast<const float*>(cscale_lds + q * 64 * 4);
+      for (int q = 0; q < kScaleRegs; ++q)
+        cs_rows[q] = rows[256 + wn * Cfg::kWaveN + q * 64 + 16 * ((lane & 15) >> 2) + 4 * group + (lane & 3)];
+    } else {
+      const float block_scale = rows[256 + wn * 64];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) s[i] *= block_scale;
     }
   };
-  auto read_a = [&](int stage_off, int i) { afrag[i] = read_frag(stage_off, 0, wm * TM + i); };
-  auto read_b = [&](int stage_off, int j) { bfrag[j & 1] = read_frag(stage_off, Cfg::kABytes, wn * TN + j); };
-  read_b(0, 0);
+  // The chunk of the wave's rows of A (waves of 32 rows share one) and its two of B.
+  const int a_chunk = wm * Cfg::kWaveM / Cfg::kChunkRows, a_row = wm * Cfg::kWaveM % Cfg::kChunkRows;
+  const bool a_early = a_chunk < kEarly;
+  const int a_from = (a_early ? a_chunk : a_chunk - kEarly) * Cfg::kChunkBytes + a_row * Cfg::kRowBytes;
+  constexpr bool kBEarly = kEarly == kChunks;
+  static_assert(kBEarly || kEarly <= kChunksA, "operand B is early or late as a whole");
+  const int b_from = (kChunksA + wn * 2 - (kBEarly ? 0 : kEarly)) * Cfg::kChunkBytes;
+  auto read_a = [&](const Place& at, int i) { afrag[i] = read_frag((a_early ? at.early : at.late) + a_from, i * 16); };
+  auto read_b = [&](const Place& at, int j) { bfrag[j & 1] = read_frag((kBEarly ? at.early : at.late) + b_from, j * 16); };
+  read_b(now, 0);
 #pragma unroll
-  for (int i = 0; i < TM; ++i) read_a(0, i);
+  for (int i = 0; i < TM; ++i) read_a(now, i);
 
-  int stage = 0;
-  // more: k-tile kt + 1 exists (its stage was released by the barrier inside kt - 1).
-  // A tag, so that no request sits behind a branch of its own.
-  auto k_tile = [&](int64_t kt, auto more_tag) {
-    constexpr bool more = decltype(more_tag)::value;
-    const int stage_off = stage * Cfg::kStageBytes;
+  // more: k-tile kt + 1 exists, and its late chunks go out; more2: kt + 2 exists, and its early ones do.
+  // Tags, so that no request sits behind a branch of its own.
+  auto k_tile = [&](int kt, auto more_tag, auto more2_tag) {
+    constexpr bool more = decltype(more_tag)::value, more2 = decltype(more2_tag)::value;
+    const Place next = place_after(now), after = place_after(next);
     // The scales are first needed by the first fold, kLag blocks in.
-    read_row_scales(s, stage, kt);
-    read_column_scales(cs_rows, stage);
-    if (kLongK && !kColumnScales && more && (kt & (Cfg::kMaxKTilesInLds - 1)) == Cfg::kMaxKTilesInLds - 1) {
-      // Last k-tile of the window (once per 32 768 of k): its scale has just
-      // been read; the next window is requested over it and lands before this
-      // k-tile's hand-over barrier, like the operands of k-tile kt + 1.
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      issue_weight_scale_window(kt + 1);
-    }
+    read_scales(kt);
     // The wave's 16x16 blocks, column by column.  One 16x16x128 MFMA gives a
     // block's partial product for this scale block; it is folded into the result
     // (4 fused multiply-adds, or multiply + fused multiply-add with per-column
@@ -394,11 +354,13 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
       const int i = blk % TM, j = blk / TM;
       const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
       if (blk == kBlocks - TM) {
-        // Every fragment of this k-tile is in registers: hand the stage over.
+        // Every fragment of this k-tile is in registers: hand its slots over.
 #ifdef FSH_TRACE
         lap(t_compute);
 #endif
-        if (more) wait_for_dma_loads();  // this wave's part of k-tile kt + 1 has landed
+        // this wave's part of k-tile kt + 1 has landed; the early chunks of kt + 2 stay in flight
+        if (more2) wait_for_dma_loads_but<kEarly>();
+        else if (more) wait_for_dma_loads();
 #ifdef FSH_TRACE
         lap(t_wait);
 #endif
@@ -408,7 +370,7 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
 #endif
       }
       // The next column's B fragment, a column ahead.
-      if (i == 0 && j + 1 < TN) read_b(stage_off, j + 1);
+      if (i == 0 && j + 1 < TN) read_b(now, j + 1);
       // Wave priority falls as the k-tile proceeds: of the two waves of a SIMD
       // the one that is behind wins the issue slot, so both reach the barrier
       // together (with equal priorities the older wave runs ahead and then
@@ -422,25 +384,30 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
           __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bfrag[j & 1], afrag[i], zero, 0, 0, 0, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if (blk >= kBlocks - TM && more) {  // what the next k-tile starts with
-        const int next_off = stage_off ^ Cfg::kStageBytes;
-        if (i == 0) read_b(next_off, 0);
-        read_a(next_off, i);
+        if (i == 0) read_b(next, 0);
+        read_a(next, i);
       }
-      // The next k-tile's requests leave during the first half of this one, so
-      // the data has the second half to arrive (spread over all blocks, the last
-      // requests were still in flight at the hand-over: 0.15-0.35 us of every
-      // 2 us k-tile went to waiting for them).
-      constexpr int kParts = Cfg::kLoadsA + Cfg::kLoadsB, kIssueEvery = kBlocks / 2 / kParts;
-      if (more && blk % kIssueEvery == kIssueEvery - 1 && blk < kBlocks / 2) issue_k_tile_part(kt + 1, stage ^ 1, blk / kIssueEvery);
+      // One request behind every few MFMAs, those of the next k-tile first: the
+      // last of them has the rest of this k-tile to arrive.
+      if (more && blk == 0) request_scales(kt + 1);
+#pragma unroll
+      for (int r = 0; r < kChunks; ++r) {
+        constexpr int kLate = Cfg::kLate;
+        if (r < kLate && more && blk == 3 * r) request(kt + 1, next, kEarly + r);
+        if (r >= kLate && more2 && blk == 3 * kLate + (r - kLate) * TM) request(kt + 2, after, r - kLate);
+      }
       if (blk >= kLag) fold(blk - kLag);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int blk = kBlocks - kLag; blk < kBlocks; ++blk) fold(blk);
-    stage ^= 1;
+    now = next;
   };
-  for (int64_t kt = 0; kt + 1 < ktiles; ++kt) k_tile(kt, std::true_type{});
-  k_tile(ktiles - 1, std::false_type{});
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  for (int kt = 0; kt + 2 < ktiles; ++kt) k_tile(kt, yes, yes);
+  if (ktiles > 1) k_tile(ktiles - 2, yes, no);
+  k_tile(ktiles - 1, no, no);
 #ifdef FSH_TRACE
   if (p.schedule.trace && lane == 0) {
     uint64_t* out = p.schedule.trace + (static_cast<int64_t>(blockIdx.x) * Cfg::kWaves + wave) * 8;
@@ -475,14 +442,14 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
 // kColumnScales = false: the second operand carries one scale per 128 x 128
 // tile (a prequantized weight, either orientation).  true: one scale per
 // output column and k-block (an operand quantized in 128 x 1 runs).
-template <bool kColumnScales, bool kLongK = false>
+template <bool kColumnScales>
 __global__ __launch_bounds__(Fp8Gemm::kThreads) void fp8_gemm_blockwise_kernel(const Fp8GemmParams p) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds_bytes[];
   int64_t unused_batch;
   int tm, tn;
   if (static_cast<int64_t>(blockIdx.x) < p.whole_grid) {
     if (!tile_of_workgroup(p.schedule, blockIdx.x, &unused_batch, &tm, &tn)) return;  // whole workgroup
-    fp8_gemm_tile<kColumnScales, 2, kLongK>(p, lds_bytes, uniform_i32(tm), uniform_i32(tn), 0);
+    fp8_gemm_tile<kColumnScales, 2>(p, lds_bytes, uniform_i32(tm), uniform_i32(tn), 0);
   } else {
     // Same split over the XCDs as the whole tiles: the two halves of a tile are
     // neighbours in an XCD's run and share the tile's second operand in its L2.
@@ -490,8 +457,7 @@ __global__ __launch_bounds__(Fp8Gemm::kThreads) void fp8_gemm_blockwise_kernel(c
     const int64_t item = (id % kXcds) * p.half_items_per_xcd + id / kXcds;
     if (item >= p.half_items) return;
     tile_in_order(p.schedule, static_cast<int>(p.schedule.work_items + item / 2), &tm, &tn);
-    fp8_gemm_tile<kColumnScales, 1, kLongK>(p, lds_bytes, uniform_i32(tm), uniform_i32(tn),
-                                            uniform_i32(static_cast<int>(item & 1)));
+    fp8_gemm_tile<kColumnScales, 1>(p, lds_bytes, uniform_i32(tm), uniform_i32(tn), uniform_i32(static_cast<int>(item & 1)));
   }
 }
 
@@ -591,9 +557,8 @@ Fp8TileKind fp8_tile_kind(int64_t m, int64_t n, int64_t k, bool column_scales, i
   }
   if (best == 0) return best_tiles <= (column_scales ? 2 * units : units) ? kFp8Tiles64Deep : kFp8Tiles64;
   if (best == 1) return best_tiles <= units ? kFp8Tiles128Deep : kFp8Tiles128;
-  // The block-scale variant keeps one window of weight scales in LDS; a longer
-  // contraction takes the instantiation that refills it.
-  return !column_scales && k / 128 > Fp8Gemm::kMaxKTilesInLds ? kFp8Tiles256LongK : kFp8Tiles256;
+  // (One kernel; the name tells contractions of more than 256 k-tiles apart.)
+  return !column_scales && k / 128 > 256 ? kFp8Tiles256LongK : kFp8Tiles256;
 }
 
 template <typename Cfg, int kBlocksPerUnit>
@@ -666,19 +631,13 @@ int launch_fp8_gemm(Fp8GemmParams& p, bool column_scales, const char* who, void*
   p.whole_grid = s.items_per_xcd * kXcds;
   p.half_items = 2 * cut;
   p.half_items_per_xcd = ceil_div(p.half_items, static_cast<int64_t>(kXcds));
-  const bool long_k = kind == kFp8Tiles256LongK;
-  static LdsReservation reserved_block_scales, reserved_block_scales_long, reserved_column_scales;
-  if (int rc = column_scales
-                   ? reserve_lds_once(reserved_column_scales, &fp8_gemm_blockwise_kernel<true>, Fp8Gemm::kLdsBytes)
-               : long_k
-                   ? reserve_lds_once(reserved_block_scales_long, &fp8_gemm_blockwise_kernel<false, true>, Fp8Gemm::kLdsBytes)
-                   : reserve_lds_once(reserved_block_scales, &fp8_gemm_blockwise_kernel<false>, Fp8Gemm::kLdsBytes))
+  static LdsReservation reserved_block_scales, reserved_column_scales;
+  if (int rc = column_scales ? reserve_lds_once(reserved_column_scales, &fp8_gemm_blockwise_kernel<true>, Fp8Gemm::kLdsBytes)
+                             : reserve_lds_once(reserved_block_scales, &fp8_gemm_blockwise_kernel<false>, Fp8Gemm::kLdsBytes))
     return rc;
   const dim3 grid(static_cast<uint32_t>(p.whole_grid + p.half_items_per_xcd * kXcds)), block(Fp8Gemm::kThreads);
   if (column_scales)
     hipLaunchKernelGGL(fp8_gemm_blockwise_kernel<true>, grid, block, Fp8Gemm::kLdsBytes, on, p);
-  else if (long_k)
-    hipLaunchKernelGGL((fp8_gemm_blockwise_kernel<false, true>), grid, block, Fp8Gemm::kLdsBytes, on, p);
   else
     hipLaunchKernelGGL(fp8_gemm_blockwise_kernel<false>, grid, block, Fp8Gemm::kLdsBytes, on, p);
   return check_launch("fp8_gemm_blockwise_kernel");

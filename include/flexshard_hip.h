@@ -313,7 +313,8 @@ int fsh_gemm_bf16_nt_group(const fsh_gemm_desc* descs, int32_t count, void* stre
  * last_step; a problem that iterates on smaller tiles may take the large ones
  * for a product on its own.
  * fsh_fp8_gemm_tiles: the FSH_TILES_* of a product of (8) and (9), negative on
- * bad sizes; column_scales: of fsh_fp8_gemm_1x128_128x1. */
+ * bad sizes; column_scales: of fsh_fp8_gemm_1x128_128x1.  FSH_TILES_256_LONG_K:
+ * the 256 x 256 tiles with block scales over more than 32768 of k. */
 #define FSH_TILES_64 0
 #define FSH_TILES_64_DEEP 1
 #define FSH_TILES_128 2
