@@ -17,10 +17,10 @@ def _integers(shape, device, gen, high):
 
 
 @pytest.mark.parametrize("k", [64, 72, 128, 192, 200, 256, 264, 320, 328, 392])
-@pytest.mark.parametrize("batch,m,n", [(2, 130, 257), (9, 1546, 1288), (1, 1923, 1837), (3, 1433, 1433)])
+@pytest.mark.parametrize("batch,m,n", [(2, 130, 257), (26, 130, 257), (25, 130, 257), (9, 1546, 1288), (1, 1923, 1837), (3, 1433, 1433)])
 def test_pipeline_depths(device, batch, m, n, k):
     tiles = hip_ops.gemm_tiles((batch, m, n, k))
-    assert tiles == ({2: "64", 9: "128", 1: "128 deep", 3: "128"}[batch],)
+    assert tiles == ({2: "64", 25: "64", 26: "64", 9: "128", 1: "128 deep", 3: "128"}[batch],)
     gen = torch.Generator(device=device)
     gen.manual_seed(k)
     a, b, d = (_integers((batch, *s), device, gen, 3) for s in ((m, k), (n, k), (m, n)))
