@@ -122,322 +122,11 @@ __global__ __launch_bounds__(kActThreads) void act_quant_1x128_kernel(const ActQ
 // request of each wave; the block scales had a window of 256 k-tiles of their own
 // and an instantiation that refilled it.
 //
-// TM_ = 1 is the half tile (128 x 256, waves of 32 x 128) that the tiles of a
-// last, at most half-full round are cut into.
-template <int TM_>
-struct Fp8GemmCfg {
-  static constexpr int BM = 128 * TM_, BN = 256, BK = 128, WM = 4, WN = 2;
-  static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves, kWaveM = BM / WM, kWaveN = BN / WN;
-  static constexpr int TM = kWaveM / 16, TN = kWaveN / 16;  // blocks of 16 x 16 per wave
-  static constexpr int kRowBytes = 128;
-  // A chunk is what one request of every wave fills: 64 rows of an operand.
-  static constexpr int kChunkRows = 8 * kWaves, kChunkBytes = kChunkRows * kRowBytes;       // 8 KB
-  static constexpr int kChunksA = BM / kChunkRows, kChunks = kChunksA + BN / kChunkRows;    // per k-tile: 8 (6)
-  // LDS holds 19: the early chunks of a k-tile, the first of operand A (all of
-  // a half tile's), have three slots each and are requested a k-tile ahead of
-  // the late ones, which have two.
-  static constexpr int kSlots = 19;
-  static constexpr int kEarly = kSlots - 2 * kChunks < kChunks ? kSlots - 2 * kChunks : kChunks, kLate = kChunks - kEarly;
-  static constexpr int kEarlyBytes = kEarly * kChunkBytes, kLateBytes = kLate * kChunkBytes;
-  static constexpr int kLateOffset = 3 * kEarlyBytes;
-  static constexpr int kPitch = kWaveN * 2 + 16;               // epilogue staging, bytes
-  static constexpr int kRegion = kWaveM * kPitch;              // per wave
-  // Two stages of scales: 256 row scales, then 256 column scales (or the two
-  // block scales, 64 times each).
-  static constexpr int kScaleOffset = kSlots * kChunkBytes, kScaleStageBytes = 2048;
-  static constexpr int kLdsBytes = kScaleOffset + 2 * kScaleStageBytes;
-  static_assert(kLdsBytes <= 160 * 1024 && kWaves * kRegion <= kLdsBytes, "LDS of a compute unit");
-  static_assert(kEarly > 0 && 3 * kEarly + 2 * kLate <= kSlots, "two k-tiles and a part of the next");
-};
-using Fp8Gemm = Fp8GemmCfg<2>;
-
-// One output tile (TM_ = 2) or half tile (TM_ = 1, rows [128 half, +128) of the tile).
-template <bool kColumnScales, int TM_>
-__device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* lds_bytes, int tm, int tn, int half) {
-  using Cfg = Fp8GemmCfg<TM_>;
-  constexpr int TM = Cfg::TM, TN = Cfg::TN, kChunks = Cfg::kChunks, kChunksA = Cfg::kChunksA, kEarly = Cfg::kEarly;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
-  const int64_t m0 = static_cast<int64_t>(tm) * Fp8Gemm::BM + static_cast<int64_t>(half) * Cfg::BM;
-  const int64_t n0 = static_cast<int64_t>(tn) * Cfg::BN;
-  if (m0 >= p.m) return;  // the second half of a tile that ends in its first (whole workgroup)
-#ifdef FSH_TRACE
-  const uint64_t t_entry = __builtin_amdgcn_s_memrealtime();
-#endif
-  const int ktiles = static_cast<int>(p.k / Cfg::BK);
-
-  // Load side: request c of a wave fills rows [64 c + 8 wave, +8) of the tile's
-  // operand A, from c = kChunksA on of operand B; lane l fills slot l & 7 of
-  // row l >> 3 there.  Rows past the matrix are read from its last row (their
-  // products are never stored).
-  const int fill_row = lane >> 3;
-  const int fill_chunk = (lane & 7) ^ (((8 * wave + fill_row) >> 1) & 7);
-  uint32_t voff[kChunks];
-#pragma unroll
-  for (int c = 0; c < kChunks; ++c) {
-    const int64_t first = c < kChunksA ? m0 : n0, size = c < kChunksA ? p.m : p.n, ld = c < kChunksA ? p.ldxq : p.ldwq;
-    int64_t row = first + Cfg::kChunkRows * (c < kChunksA ? c : c - kChunksA) + 8 * wave + fill_row;
-    row = row < size ? row : size - 1;
-    voff[c] = static_cast<uint32_t>((row - first) * ld + fill_chunk * 16);
-  }
-  const uint8_t* Ab = uniform_ptr(p.xq + m0 * p.ldxq);
-  const uint8_t* Bb = uniform_ptr(p.wq + n0 * p.ldwq);
-  typedef __attribute__((address_space(3))) uint8_t* lds_address;
-  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_address)lds_bytes));
-  const uint32_t fill_lds = lds_base + static_cast<uint32_t>(wave * 1024);
-  // Where a k-tile lies: the offsets of its early chunks and of its late ones.
-  struct Place {
-    int early, late;
-  };
-  const auto place_after = [](const Place& at) {
-    return Place{at.early == 2 * Cfg::kEarlyBytes ? 0 : at.early + Cfg::kEarlyBytes,
-                 at.late == Cfg::kLateOffset ? Cfg::kLateOffset + Cfg::kLateBytes : Cfg::kLateOffset};
-  };
-  auto request = [&](int kt, const Place& at, int c) {
-    dma_load_16(voff[c], (c < kChunksA ? Ab : Bb) + static_cast<int64_t>(kt) * Cfg::kRowBytes,
-                fill_lds + (c < kEarly ? at.early : at.late), (c < kEarly ? c : c - kEarly) * Cfg::kChunkBytes);
-  };
-  // The scales of a k-tile ride the same global->LDS path: 64 row scales by
-  // each of the first four waves, 64 column scales by each of the others -- or
-  // by two of them each the block scale of 128 of the tile's columns, 64 times.
-  // (A load that the compiler sees inside the loop makes it wait for all
-  // requests in flight.)
-  const float* scale_src = p.xs;
-  int64_t scale_step = p.m;
-  uint32_t scale_voff = 0, scale_slot = wave % (Cfg::BM / 64);
-  if (wave < 4) {
-    const int64_t row = m0 + scale_slot * 64 + lane;
-    scale_voff = static_cast<uint32_t>((row < p.m ? row : p.m - 1) * 4);
-  } else if (kColumnScales) {
-    const int64_t col = n0 + (wave - 4) * 64 + lane;
-    scale_voff = static_cast<uint32_t>((col < p.n ? col : p.n - 1) * 4);
-    scale_src = p.cs;
-    scale_step = p.n;
-    scale_slot = wave;
-  } else {
-    const int64_t block = n0 / 128 + (wave >> 1 & 1), last = (p.n - 1) / 128;
-    scale_src = p.ws + (block < last ? block : last) * p.ws_cb;
-    scale_step = p.ws_kb;
-    scale_slot = 4 + (wave >> 1 & 1);
-  }
-  const uint32_t scale_lds = lds_base + Cfg::kScaleOffset + scale_slot * 256;
-  auto request_scales = [&](int kt) {
-    dma_touch_4(scale_voff, reinterpret_cast<const uint8_t*>(scale_src + kt * scale_step), scale_lds + (kt & 1) * Cfg::kScaleStageBytes);
-  };
-
-  // Fragment side: row = lane & 15 of a 16-row block, chunks g and g + 4 of its
-  // eight (g = lane / 16), each in slot chunk ^ ((row >> 1) & 7).  Any split of
-  // the 128 bytes over the four g will do that both operands share; with chunks
-  // 2 g and 2 g + 1 the reads met in the banks (25 % of the kernel's cycles by
-  // the counter: the LDS serves a 16-byte read to lanes of two neighbouring g at
-  // a time, whose slots stay apart if their chunks differ in bit 0).
-  const int frag_row = lane & 15, group = lane >> 4;
-  uint32_t frag_off[2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-    frag_off[c] = static_cast<uint32_t>(frag_row * Cfg::kRowBytes + (((group + 4 * c) ^ ((frag_row >> 1) & 7)) * 16));
-  // `row` of the rows that start at `chunk`
-  auto read_frag = [&](int chunk, int row) -> v8i32 {
-    const uint8_t* base = lds_bytes + chunk + row * Cfg::kRowBytes;
-    const u32x4 lo = *reinterpret_cast<const u32x4*>(base + frag_off[0]);
-    const u32x4 hi = *reinterpret_cast<const u32x4*>(base + frag_off[1]);
-    return v8i32{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z), static_cast<int>(lo.w),
-                 static_cast<int>(hi.x), static_cast<int>(hi.y), static_cast<int>(hi.z), static_cast<int>(hi.w)};
-  };
-
-  f32x4 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // The first k-tile and the early chunks of the second.
-  Place now{0, Cfg::kLateOffset};  // of k-tile kt
-  request_scales(0);
-#pragma unroll
-  for (int c = 0; c < kChunks; ++c) request(0, now, c);
-  if (ktiles > 1) {
-#pragma unroll
-    for (int c = 0; c < kEarly; ++c) request(1, place_after(now), c);
-    wait_for_dma_loads_but<kEarly>();
-  } else {
-    wait_for_dma_loads();
-  }
-  asm volatile("s_barrier" ::: "memory");
-
-#ifdef FSH_TRACE
-  // Time per phase of the k loop, summed over the k-tiles (10 ns ticks).
-  uint64_t t_compute = 0, t_wait = 0, t_barrier = 0, t_mark = __builtin_amdgcn_s_memrealtime();
-  const uint64_t t_begin = t_mark;
-  auto lap = [&](uint64_t& sum) {
-    const uint64_t now = __builtin_amdgcn_s_memrealtime();
-    sum += now - t_mark;
-    t_mark = now;
-  };
-#endif
-  // The k loop is rotated by a column of blocks: the barrier that hands over
-  // k-tile kt + 1 sits before the last column of k-tile kt, and behind each of
-  // its MFMAs the wave reads the fragment of kt + 1 that takes the place of the
-  // one just used.
-  //   carried into a k-tile: afrag, bfrag[0]
-  // Behind that barrier the slots of k-tile kt are free: in k-tile kt + 1 the
-  // late chunks of kt + 2 go out, then the early ones of kt + 3, one request
-  // behind every few MFMAs.
-  constexpr int kBlocks = TM * TN;
-  v8i32 afrag[TM], bfrag[2];
-  constexpr int kScaleRegs = TN / 4;
-  float s[TM], cs_rows[kScaleRegs];
-  // Row scales of the wave's rows for k-tile kt, times the block scale in the
-  // block-scale variant; a lane owns output row lane & 15 of each of its blocks.
-  auto read_scales = [&](int kt) {
-    const float* rows = reinterpret_cast<const float*>(lds_bytes + Cfg::kScaleOffset + (kt & 1) * Cfg::kScaleStageBytes);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) s[i] = rows[wm * Cfg::kWaveM + i * 16 + frag_row];
-    if (kColumnScales) {
-      // Register q holds, in every row of 16 lanes, the 16 scales that the lanes
-      // of that row fold column blocks 4 q .. 4 q + 3 with: lane 4 b + r of the
-      // row the scale of accumulator r of block 4 q + b.  A fold takes it through
-      // the data-parallel-primitive broadcast of the multiply-add itself.
-#pragma unroll
-      for (int q = 0; q < kScaleRegs; ++q)
-        cs_rows[q] = rows[256 + wn * Cfg::kWaveN + q * 64 + 16 * ((lane & 15) >> 2) + 4 * group + (lane & 3)];
-    } else {
-      const float block_scale = rows[256 + wn * 64];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) s[i] *= block_scale;
-    }
-  };
-  // The chunk of the wave's rows of A (waves of 32 rows share one) and its two of B.
-  const int a_chunk = wm * Cfg::kWaveM / Cfg::kChunkRows, a_row = wm * Cfg::kWaveM % Cfg::kChunkRows;
-  const bool a_early = a_chunk < kEarly;
-  const int a_from = (a_early ? a_chunk : a_chunk - kEarly) * Cfg::kChunkBytes + a_row * Cfg::kRowBytes;
-  constexpr bool kBEarly = kEarly == kChunks;
-  static_assert(kBEarly || kEarly <= kChunksA, "operand B is early or late as a whole");
-  const int b_from = (kChunksA + wn * 2 - (kBEarly ? 0 : kEarly)) * Cfg::kChunkBytes;
-  auto read_a = [&](const Place& at, int i) { afrag[i] = read_frag((a_early ? at.early : at.late) + a_from, i * 16); };
-  auto read_b = [&](const Place& at, int j) { bfrag[j & 1] = read_frag((kBEarly ? at.early : at.late) + b_from, j * 16); };
-  read_b(now, 0);
-#pragma unroll
-  for (int i = 0; i < TM; ++i) read_a(now, i);
-
-  // more: k-tile kt + 1 exists, and its late chunks go out; more2: kt + 2 exists, and its early ones do.
-  // Tags, so that no request sits behind a branch of its own.
-  auto k_tile = [&](int kt, auto more_tag, auto more2_tag) {
-    constexpr bool more = decltype(more_tag)::value, more2 = decltype(more2_tag)::value;
-    const Place next = place_after(now), after = place_after(next);
-    // The scales are first needed by the first fold, kLag blocks in.
-    read_scales(kt);
-    // The wave's 16x16 blocks, column by column.  One 16x16x128 MFMA gives a
-    // block's partial product for this scale block; it is folded into the result
-    // (4 fused multiply-adds, or multiply + fused multiply-add with per-column
-    // scales) kLag blocks later: a fold that reads the product of an MFMA issued
-    // just before it waits for the matrix core to drain.
-    constexpr int kLag = 4;
-    f32x4 part[kLag + 1];
-    auto fold = [&](int blk) {
-      const int pi = blk % TM, pj = blk / TM;
-      const f32x4& product = part[blk % (kLag + 1)];
-      if (kColumnScales) {
-        fold_with_row_broadcast(acc[pi][pj], product, s[pi], cs_rows[pj / 4], pj % 4);
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[pi][pj][r] = __builtin_fmaf(product[r], s[pi], acc[pi][pj][r]);
-      }
-      // An empty statement that "uses" the folded block keeps its arithmetic
-      // on this side of the next scheduling barrier.
-      asm volatile("" : "+v"(acc[pi][pj]));
-    };
-#pragma unroll
-    for (int blk = 0; blk < kBlocks; ++blk) {
-      const int i = blk % TM, j = blk / TM;
-      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-      if (blk == kBlocks - TM) {
-        // Every fragment of this k-tile is in registers: hand its slots over.
-#ifdef FSH_TRACE
-        lap(t_compute);
-#endif
-        // this wave's part of k-tile kt + 1 has landed; the early chunks of kt + 2 stay in flight
-        if (more2) wait_for_dma_loads_but<kEarly>();
-        else if (more) wait_for_dma_loads();
-#ifdef FSH_TRACE
-        lap(t_wait);
-#endif
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#ifdef FSH_TRACE
-        lap(t_barrier);
-#endif
-      }
-      // The next column's B fragment, a column ahead.
-      if (i == 0 && j + 1 < TN) read_b(now, j + 1);
-      // Wave priority falls as the k-tile proceeds: of the two waves of a SIMD
-      // the one that is behind wins the issue slot, so both reach the barrier
-      // together (with equal priorities the older wave runs ahead and then
-      // idles at the barrier while the other finishes alone, without a
-      // partner to overlap its folds with).
-      if (blk * 4 == 0 * kBlocks) __builtin_amdgcn_s_setprio(3);
-      if (blk * 4 == 1 * kBlocks) __builtin_amdgcn_s_setprio(2);
-      if (blk * 4 == 2 * kBlocks) __builtin_amdgcn_s_setprio(1);
-      if (blk * 4 == 3 * kBlocks) __builtin_amdgcn_s_setprio(0);
-      part[blk % (kLag + 1)] =
-          __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bfrag[j & 1], afrag[i], zero, 0, 0, 0, 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (blk >= kBlocks - TM && more) {  // what the next k-tile starts with
-        if (i == 0) read_b(next, 0);
-        read_a(next, i);
-      }
-      // One request behind every few MFMAs, those of the next k-tile first: the
-      // last of them has the rest of this k-tile to arrive.
-      if (more && blk == 0) request_scales(kt + 1);
-#pragma unroll
-      for (int r = 0; r < kChunks; ++r) {
-        constexpr int kLate = Cfg::kLate;
-        if (r < kLate && more && blk == 3 * r) request(kt + 1, next, kEarly + r);
-        if (r >= kLate && more2 && blk == 3 * kLate + (r - kLate) * TM) request(kt + 2, after, r - kLate);
-      }
-      if (blk >= kLag) fold(blk - kLag);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int blk = kBlocks - kLag; blk < kBlocks; ++blk) fold(blk);
-    now = next;
-  };
-  constexpr std::true_type yes{};
-  constexpr std::false_type no{};
-  for (int kt = 0; kt + 2 < ktiles; ++kt) k_tile(kt, yes, yes);
-  if (ktiles > 1) k_tile(ktiles - 2, yes, no);
-  k_tile(ktiles - 1, no, no);
-#ifdef FSH_TRACE
-  if (p.schedule.trace && lane == 0) {
-    uint64_t* out = p.schedule.trace + (static_cast<int64_t>(blockIdx.x) * Cfg::kWaves + wave) * 8;
-    out[0] = t_begin; out[1] = t_compute; out[2] = t_wait; out[3] = t_barrier; out[4] = t_mark; out[5] = t_entry;
-  }
-#endif
-
-  // Epilogue: bf16 finals to the wave's staging region as [row][col], then
-  // 16-byte row stores, rows and 8-column groups past the matrix skipped.
-  uint8_t* region = lds_bytes + wave * Cfg::kRegion;
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-      *reinterpret_cast<u32x2*>(region + (i * 16 + frag_row) * Cfg::kPitch + (j * 16 + 4 * group) * 2) =
-          u32x2{pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3])};
-  wave_lds_sync();
-  store_fp8_product<Cfg::kWaveM, Cfg::kWaveN, Cfg::kPitch>(region, p, m0 + wm * Cfg::kWaveM, n0 + wn * Cfg::kWaveN, lane);
-#ifdef FSH_TRACE
-  if (p.schedule.trace && lane == 0) {
-    __builtin_amdgcn_s_waitcnt(0);
-    p.schedule.trace[(static_cast<int64_t>(blockIdx.x) * Cfg::kWaves + wave) * 8 + 6] = __builtin_amdgcn_s_memrealtime();
-    uint32_t hw_id;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_HW_ID)" : "=s"(hw_id));
-    uint32_t xcc_id;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc_id));
-    p.schedule.trace[(static_cast<int64_t>(blockIdx.x) * Cfg::kWaves + wave) * 8 + 7] = (static_cast<uint64_t>(xcc_id) << 32) | hw_id;
-  }
-#endif
-}
+// The half tile (128 x 256, waves of 32 x 128) is what the tiles of a last, at
+// most half-full round are cut into.
+using Fp8Gemm = Fp8Tile<4, 2, 4, 8, 2, 3>;
+using Fp8GemmHalf = Fp8Tile<4, 2, 2, 8, 2, 6>;
+static_assert(Fp8GemmHalf::kLdsBytes <= Fp8Gemm::kLdsBytes, "one launch holds both");
 
 // kColumnScales = false: the second operand carries one scale per 128 x 128
 // tile (a prequantized weight, either orientation).  true: one scale per
@@ -449,7 +138,8 @@ __global__ __launch_bounds__(Fp8Gemm::kThreads) void fp8_gemm_blockwise_kernel(c
   int tm, tn;
   if (static_cast<int64_t>(blockIdx.x) < p.whole_grid) {
     if (!tile_of_workgroup(p.schedule, blockIdx.x, &unused_batch, &tm, &tn)) return;  // whole workgroup
-    fp8_gemm_tile<kColumnScales, 2>(p, lds_bytes, uniform_i32(tm), uniform_i32(tn), 0);
+    fp8_gemm_tile<Fp8Gemm, kColumnScales>(p, lds_bytes, static_cast<int64_t>(uniform_i32(tm)) * Fp8Gemm::BM,
+                                          static_cast<int64_t>(uniform_i32(tn)) * Fp8Gemm::BN);
   } else {
     // Same split over the XCDs as the whole tiles: the two halves of a tile are
     // neighbours in an XCD's run and share the tile's second operand in its L2.
@@ -457,7 +147,9 @@ __global__ __launch_bounds__(Fp8Gemm::kThreads) void fp8_gemm_blockwise_kernel(c
     const int64_t item = (id % kXcds) * p.half_items_per_xcd + id / kXcds;
     if (item >= p.half_items) return;
     tile_in_order(p.schedule, static_cast<int>(p.schedule.work_items + item / 2), &tm, &tn);
-    fp8_gemm_tile<kColumnScales, 1>(p, lds_bytes, uniform_i32(tm), uniform_i32(tn), uniform_i32(static_cast<int>(item & 1)));
+    const int64_t m0 = static_cast<int64_t>(uniform_i32(tm)) * Fp8Gemm::BM + uniform_i32(static_cast<int>(item & 1)) * Fp8GemmHalf::BM;
+    if (m0 >= p.m) return;  // the second half of a tile that ends in its first (whole workgroup)
+    fp8_gemm_tile<Fp8GemmHalf, kColumnScales>(p, lds_bytes, m0, static_cast<int64_t>(uniform_i32(tn)) * Fp8Gemm::BN);
   }
 }
 
@@ -513,21 +205,20 @@ namespace fsh {
 namespace {
 
 // Which tiles a product takes: the ones with the lowest estimated time.
-// Measured (us with 64 x 64 tiles of three stages, 128 x 128 of two, 256 x 256;
-// weights in the last-level cache; block scales, the
-// column-scale variant runs 5-10 % longer on all three):
-//   48 x 14336, k 4096     14.5   24.9   35.5      48 x 4096, k 14336  34.6  69.8  112
-//   256 x 4096, k 4096     13.0   23.4   27.6      1000 x 2048, k 5120 22.1  31.4  46.3
-//   1024 x 4096, k 4096    30.7   26.9   38.3      2048 x 4096, k 4096 55.1  39.4  42.0
-//   1024 x 14336, k 4096   95.6   71.4   54.3      4096 x 4096, k 4096 112   73.0  58.8
+// Measured (us with 64 x 64 tiles, 128 x 128, 256 x 256; weights in the last-level
+// cache; block scales, the column-scale variant runs 5-10 % longer on all three;
+// * fewer tiles than compute units, the deep form below):
+//   48 x 14336, k 4096     10.8*  18.3*  24.2      144 x 3840, k 10240  22.0*  40.7*  55.8
+//   512 x 4096, k 4096     15.3   19.0*  24.7      1000 x 2048, k 5120  19.5   23.1*  31.7
+//   335 x 11136, k 10112   72.5   60.2   55.0      1000 x 5120, k 2048  20.2   16.6   15.7
+//   1400 x 4096, k 4096    39.1   30.2   27.7      2048 x 4096, k 1024  17.8   12.5   12.4
 //
-// A compute unit with one workgroup to run has LDS to spare: more stages,
-// i.e. more operand requests in flight ("deep").  Not where a unit runs several, whose
-// requests cover one another's waits (us, fewer / more stages, weights from memory):
-//   64 x 64, 3 / 4 stages:    48 x 14336, k 4096 18.6 / 16.2   48 x 4096, k 14336 48.2 / 36.1
-//                             512 x 4096, k 4096 17.6 / 18.4 (column scales 20.6 / 19.2)   1024 x 4096, k 4096 32.5 / 32.6
-//   128 x 128, 2 / 4 stages:  1024 x 4096, k 8192 55.9 / 46.9   1000 x 2048, k 5120 30.8 / 29.6   1000 x 5120, k 2048 20.3 / 28.3
-// (eight stages of 64 x 64 tiles: 18.2 and 35.7 us on the first two, 0.4 us more where k is short)
+// A compute unit with one workgroup to run has LDS to spare: more operand
+// requests in flight ("deep").  Not where a unit runs several, whose requests
+// cover one another's waits (us, fewer / more k-tiles in flight):
+//   64 x 64:    48 x 14336, k 4096 12.9 / 10.8   144 x 3840, k 10240 26.9 / 22.0   1000 x 2048, k 5120 19.1 / 19.1
+//               335 x 11136, k 10112 72.5 / 81.2   1000 x 5120, k 2048 20.2 / 21.5
+//   128 x 128:  48 x 14336, k 4096 26.8 / 18.3   1000 x 2048, k 5120 32.5 / 23.1   1000 x 5120, k 2048 16.6 / 22.1
 enum Fp8TileKind {
   kFp8Tiles64 = FSH_TILES_64,
   kFp8Tiles64Deep = FSH_TILES_64_DEEP,
@@ -538,16 +229,18 @@ enum Fp8TileKind {
 };
 Fp8TileKind fp8_tile_kind(int64_t m, int64_t n, int64_t k, bool column_scales, int64_t units) {
   static constexpr TileShape kShapes[] = {
-      {64, 64, 768.0, 0.22, 0.34, 0.61, 2.0},    // three workgroups per compute unit
-      {128, 128, 512.0, 0.56, 0.69, 1.07, 4.0},  // two
-      {256, 256, 256.0, 0.72, 0.99, 1.48, 5.0},  // one; a round of at most half as many is cut into half tiles
+      {64, 64, 768.0, 0.20, 0.31, 0.58, 2.0},    // three workgroups per compute unit
+      {128, 128, 512.0, 0.58, 0.66, 0.92, 4.0},  // two
+      {128, 128, 256.0, 0.36, 0.40, 0.53, 4.0},  // one, deep
+      {256, 256, 256.0, 0.50, 0.68, 1.46, 5.5},  // one; a round of at most half as many is cut into half tiles
   };
   const double ktiles = static_cast<double>(k / 128);
   int best = 0;
   double best_us = 0.0;
   int64_t best_tiles = 0;
-  for (int i = 0; i < 3; ++i) {
+  for (int i = 0; i < 4; ++i) {
     const int64_t tiles = ceil_div(m, kShapes[i].m) * ceil_div(n, kShapes[i].n);
+    if ((i == 1 && tiles <= units) || (i == 2 && tiles > units)) continue;  // 128 x 128 is deep up to a tile per unit
     const double us = rounds_us(kShapes[i], static_cast<double>(tiles), static_cast<double>(tiles) * ktiles, ktiles);
     if (i == 0 || us < best_us) {
       best = i;
@@ -556,7 +249,7 @@ Fp8TileKind fp8_tile_kind(int64_t m, int64_t n, int64_t k, bool column_scales, i
     }
   }
   if (best == 0) return best_tiles <= (column_scales ? 2 * units : units) ? kFp8Tiles64Deep : kFp8Tiles64;
-  if (best == 1) return best_tiles <= units ? kFp8Tiles128Deep : kFp8Tiles128;
+  if (best < 3) return best == 1 ? kFp8Tiles128 : kFp8Tiles128Deep;
   // (One kernel; the name tells contractions of more than 256 k-tiles apart.)
   return !column_scales && k / 128 > 256 ? kFp8Tiles256LongK : kFp8Tiles256;
 }
@@ -571,14 +264,10 @@ int launch_fp8_tiles(Fp8GemmParams& p, bool column_scales, hipStream_t stream) {
   s.work_items = tiles;
   s.items_per_xcd = ceil_div(tiles, static_cast<int64_t>(kXcds));
   const dim3 grid(static_cast<uint32_t>(s.items_per_xcd * kXcds)), block(Cfg::kThreads);
-  static LdsReservation reserved_block_scales, reserved_column_scales;
-  if (column_scales) {
-    if (int rc = reserve_lds_once(reserved_column_scales, &fp8_gemm_tiles_kernel<Cfg, true, kBlocksPerUnit>, Cfg::kLdsBytes)) return rc;
-    hipLaunchKernelGGL((fp8_gemm_tiles_kernel<Cfg, true, kBlocksPerUnit>), grid, block, Cfg::kLdsBytes, stream, p);
-  } else {
-    if (int rc = reserve_lds_once(reserved_block_scales, &fp8_gemm_tiles_kernel<Cfg, false, kBlocksPerUnit>, Cfg::kLdsBytes)) return rc;
-    hipLaunchKernelGGL((fp8_gemm_tiles_kernel<Cfg, false, kBlocksPerUnit>), grid, block, Cfg::kLdsBytes, stream, p);
-  }
+  static LdsReservation reserved[2];
+  const auto kernel = column_scales ? &fp8_gemm_tiles_kernel<Cfg, true, kBlocksPerUnit> : &fp8_gemm_tiles_kernel<Cfg, false, kBlocksPerUnit>;
+  if (int rc = reserve_lds_once(reserved[column_scales], kernel, Cfg::kLdsBytes)) return rc;
+  hipLaunchKernelGGL(kernel, grid, block, Cfg::kLdsBytes, stream, p);
   return check_launch("fp8_gemm_tiles_kernel");
 }
 
@@ -612,12 +301,15 @@ int launch_fp8_gemm(Fp8GemmParams& p, bool column_scales, const char* who, void*
   s.tiles_per_matrix = static_cast<int32_t>(tiles);
   const int64_t units = compute_units();
   const hipStream_t on = static_cast<hipStream_t>(stream);
-  const Fp8TileKind kind = fp8_tile_kind(p.m, p.n, p.k, column_scales, units);
+  Fp8TileKind kind = fp8_tile_kind(p.m, p.n, p.k, column_scales, units);
+#ifdef FORCEKIND
+  if (const char* e = getenv("FSH_KIND")) if (atoi(e) >= 0) kind = static_cast<Fp8TileKind>(atoi(e));
+#endif
   switch (kind) {
-    case kFp8Tiles64: return launch_fp8_tiles<Fp8Tiles<2, 2, 1, 1, 3>, 3>(p, column_scales, on);
-    case kFp8Tiles64Deep: return launch_fp8_tiles<Fp8Tiles<2, 2, 1, 1, 4>, 2>(p, column_scales, on);
-    case kFp8Tiles128: return launch_fp8_tiles<Fp8Tiles<2, 2, 2, 2, 2>, 2>(p, column_scales, on);
-    case kFp8Tiles128Deep: return launch_fp8_tiles<Fp8Tiles<2, 2, 2, 2, 4>, 1>(p, column_scales, on);
+        case kFp8Tiles64: return launch_fp8_tiles<Fp8Tile<2, 2, 2, 2, 3, 0>, 3>(p, column_scales, on);
+    case kFp8Tiles64Deep: return launch_fp8_tiles<Fp8Tile<2, 2, 2, 2, 4, 2>, 2>(p, column_scales, on);
+    case kFp8Tiles128: return launch_fp8_tiles<Fp8Tile<2, 2, 4, 4, 2, 3>, 2>(p, column_scales, on);
+    case kFp8Tiles128Deep: return launch_fp8_tiles<Fp8Tile<2, 2, 4, 4, 4, 4>, 1>(p, column_scales, on);
     default: break;
   }
   // A workgroup holds a CU for a tile, so the tiles go through the chip in

@@ -1,5 +1,6 @@
-// The scaled FP8 product on small tiles: few tokens, few columns, anything
-// that does not fill the chip with the 256 x 256 tiles of fp8_linear.hip.
+// The scaled FP8 product, a tile at a time, and the kernel of the small tiles:
+// few tokens, few columns, anything that does not fill the chip with the
+// 256 x 256 tiles of fp8_linear.hip.
 #pragma once
 #include "mfma_tiles.hpp"
 
@@ -54,26 +55,11 @@ __device__ __forceinline__ void store_fp8_product(const uint8_t* region, const F
     store_wave_image<kRows, kCols, kPitch>(region, p.out, p.ldo, row0, col0, p.m, p.n, lane);
 }
 
-// acc[n] += (product[n] * row_scale) * (column_scales of lane n of this lane's row of 16).
-// The broadcast is the multiply-add's own operand modifier (the compiler keeps
-// a separate move per element when given the builtin).  column_scales comes
-// from LDS, not from the vector ALU, so the modifier's read needs no wait states.
-template <int N = 0>
-__device__ __forceinline__ void fold_with_row_broadcast(f32x16& acc, const f32x16& product, float row_scale,
-                                                        float column_scales) {
-  if constexpr (N < 16) {
-    const float scaled = product[N] * row_scale;
-    float sum = acc[N];
-    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-        : "+v"(sum)
-        : "v"(column_scales), "v"(scaled), "n"(N));
-    acc[N] = sum;
-    fold_with_row_broadcast<N + 1>(acc, product, row_scale, column_scales);
-  }
-}
-
-// The same for a block of 16 x 16: element r takes the scale of lane 4 block + r
-// of its row of 16 lanes (block is a constant after unrolling).
+// acc[r] += (product[r] * row_scale) * (column_scales of lane 4 block + r of this
+// lane's row of 16; block is a constant after unrolling).  The broadcast is the
+// multiply-add's own operand modifier (the compiler keeps a separate move per
+// element when given the builtin).  column_scales comes from LDS, not from the
+// vector ALU, so the modifier's read needs no wait states.
 template <int N>
 __device__ __forceinline__ float fold_one_with_row_broadcast(float sum, float scaled, float column_scales) {
   asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(sum) : "v"(column_scales), "v"(scaled), "n"(N));
@@ -94,267 +80,367 @@ __device__ __forceinline__ void fold_with_row_broadcast(f32x4& acc, const f32x4&
   else fold_block_with_row_broadcast<3>(acc, product, row_scale, column_scales);
 }
 
-// Four waves, WM x WN, each TM x TN blocks of 32 x 32; a k-tile is one scale
-// block (128 bytes of every row) with its row scales and column scales.
-template <int WM_, int WN_, int TM_, int TN_, int kStages_>
-struct Fp8Tiles {
-  static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, kStages = kStages_;
-  static constexpr int kWaveM = 32 * TM, kWaveN = 32 * TN, BM = WM * kWaveM, BN = WN * kWaveN, BK = 128;
-  static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves, kRowBytes = 128;
-  static constexpr int kABytes = BM * kRowBytes, kScaleOffset = (BM + BN) * kRowBytes;
-  static constexpr int kStageBytes = kScaleOffset + (BM + BN) * 4;
-  static constexpr int kFillRows = 8 * kWaves;
-  static constexpr int kLoadsA = BM / kFillRows, kLoadsB = BN / kFillRows;
-  static constexpr int kRequests = kLoadsA + kLoadsB + 1;     // per wave and k-tile; the last one brings 64 scales
-  static constexpr int kScaleRequests = (BM + BN) / 64;       // per workgroup: waves past them repeat
-  static constexpr int kPitch = kWaveN * 2 + 8, kRegion = kWaveM * kPitch;
-  static constexpr int kLdsBytes = kStages * kStageBytes;
-  static_assert(BN <= 128, "a tile's columns share one block scale");
-  static_assert(BM % 64 == 0 && BN % 64 == 0 && kWaves % kScaleRequests == 0, "scale requests of 64");
-  static_assert(kWaves * kRegion <= kLdsBytes, "the images fit the loop's LDS");
+// A tile of WM x WN waves, each TM x TN blocks of 16 x 16; a k-tile is one scale
+// block (128 bytes of every row) with its row and column scales.  A chunk is
+// what one request of every wave fills.  The first kEarly chunks of a k-tile
+// have kDepth + 1 slots in LDS, the others and the scales kDepth.
+template <int WM_, int WN_, int TM_, int TN_, int kDepth_, int kEarly_>
+struct Fp8Tile {
+  static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, kDepth = kDepth_, kEarly = kEarly_;
+  static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves, kWaveM = 16 * TM, kWaveN = 16 * TN;
+  static constexpr int BM = WM * kWaveM, BN = WN * kWaveN, BK = 128, kRowBytes = 128;
+  static constexpr int kChunkRows = 8 * kWaves, kChunkBytes = kChunkRows * kRowBytes;
+  static constexpr int kChunksA = BM / kChunkRows, kChunks = kChunksA + BN / kChunkRows, kLate = kChunks - kEarly;
+  static constexpr int kEarlyBytes = kEarly * kChunkBytes, kLateBytes = kLate * kChunkBytes;
+  static constexpr int kLateOffset = (kDepth + 1) * kEarlyBytes, kScaleOffset = kLateOffset + kDepth * kLateBytes;
+  // Scales of a k-tile: BM row scales, then BN column scales (or the block scale of every 64 columns, 64 times).
+  static constexpr int kScaleRequests = (BM + BN) / 64, kScaleBytes = 256 * kScaleRequests;
+  static constexpr int kLdsBytes = kScaleOffset + kDepth * kScaleBytes;
+  static constexpr int kPitch = kWaveN * 2 + 16, kRegion = kWaveM * kPitch;  // epilogue staging of a wave, bytes
+  static_assert(kLdsBytes <= 160 * 1024 && kWaves * kRegion <= kLdsBytes, "LDS of a compute unit");
+  static_assert(BM % kChunkRows == 0 && BN % kChunkRows == 0 && kWaveN % kChunkRows == 0, "whole chunks");
+  static_assert(kChunkRows % kWaveM == 0 || kWaveM % kChunkRows == 0, "a wave's rows in whole chunks or in one");
+  static_assert(kEarly == kChunks || kEarly <= kChunksA, "operand B is early or late as a whole");
+  static_assert(BM % 64 == 0 && BN % 64 == 0 && kScaleRequests <= kWaves && (TN == 2 || TN % 4 == 0), "scales by 64");
+  static_assert(kDepth >= 2 && kDepth <= 4, "the waits of the k loop's end");
 };
 
-template <typename Cfg, bool kColumnScales, int kBlocksPerUnit>
-__global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) void fp8_gemm_tiles_kernel(const Fp8GemmParams p) {
-  extern __shared__ __attribute__((aligned(1024))) uint8_t lds_bytes[];
-  constexpr int TM = Cfg::TM, TN = Cfg::TN, kStages = Cfg::kStages, kBlocks = TM * TN;
+// One output tile at (m0, n0).
+//
+// The small tiles are bound by the latency of a k-tile where a compute unit has
+// one workgroup (a chain of requests, a barrier, fragment reads), by the request
+// path (one 1 KB request per 16 cycles: the 32 of a 128 x 128 k-tile last as long
+// as its MFMAs) where it has several.  Before, they ran 32 x 32 x 64 MFMAs whose 16
+// registers were folded behind the next one's, and their requests left in one go
+// behind the last block, held up by one another.  us before / now, same bits:
+//   64 x 64:    48 x 14336, k 4096 12.1 / 10.8   144 x 3840, k 10240 23.4 / 22.0   512 x 4096, k 4096 16.1 / 14.6
+//               3000 x 1024 over 1500 tokens, column scales 12.0 / 10.0   1000 x 2048, k 5120 20.1 / 19.1
+//   128 x 128:  1000 x 5120, k 2048 18.9 / 16.6   1024 x 4096, k 8192 45.6 / 38.8
+//               1024 x 4096 over 8192 tokens, column scales 50.9 / 44.7
+template <typename Cfg, bool kColumnScales>
+__device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* lds_bytes, int64_t m0, int64_t n0) {
+  constexpr int TM = Cfg::TM, TN = Cfg::TN, kChunks = Cfg::kChunks, kChunksA = Cfg::kChunksA, kEarly = Cfg::kEarly, kDepth = Cfg::kDepth;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
-  int64_t unused_batch;
-  int tm, tn;
-  if (!tile_of_workgroup(p.schedule, blockIdx.x, &unused_batch, &tm, &tn)) return;  // whole workgroup
-  const int64_t m0 = static_cast<int64_t>(uniform_i32(tm)) * Cfg::BM, n0 = static_cast<int64_t>(uniform_i32(tn)) * Cfg::BN;
+#ifdef FSH_TRACE
+  const uint64_t t_entry = __builtin_amdgcn_s_memrealtime();
+#endif
   const int ktiles = static_cast<int>(p.k / Cfg::BK);
 
-  // Load side, as in the bf16 tile kernel; rows past the matrix are read from
-  // its last row (their products are never stored).
-  const int fill_row = 8 * wave + (lane >> 3);
-  const int fill_chunk = (lane & 7) ^ ((fill_row >> 1) & 7);
-  const uint8_t* src[Cfg::kLoadsA + Cfg::kLoadsB];
+  // Load side: request c of a wave fills rows [kChunkRows c + 8 wave, +8) of
+  // the tile's operand A, from c = kChunksA on of operand B; lane l fills slot l & 7 of
+  // row l >> 3 there.  Rows past the matrix are read from its last row (their
+  // products are never stored).
+  const int fill_row = lane >> 3;
+  const int fill_chunk = (lane & 7) ^ (((8 * wave + fill_row) >> 1) & 7);
+  uint32_t voff[kChunks];
 #pragma unroll
-  for (int q = 0; q < Cfg::kLoadsA; ++q) {
-    const int64_t r = m0 + Cfg::kFillRows * q + fill_row;
-    src[q] = p.xq + (r < p.m ? r : p.m - 1) * p.ldxq + fill_chunk * 16;
+  for (int c = 0; c < kChunks; ++c) {
+    const int64_t first = c < kChunksA ? m0 : n0, size = c < kChunksA ? p.m : p.n, ld = c < kChunksA ? p.ldxq : p.ldwq;
+    int64_t row = first + Cfg::kChunkRows * (c < kChunksA ? c : c - kChunksA) + 8 * wave + fill_row;
+    row = row < size ? row : size - 1;
+    voff[c] = static_cast<uint32_t>((row - first) * ld + fill_chunk * 16);
   }
-#pragma unroll
-  for (int q = 0; q < Cfg::kLoadsB; ++q) {
-    const int64_t r = n0 + Cfg::kFillRows * q + fill_row;
-    src[Cfg::kLoadsA + q] = p.wq + (r < p.n ? r : p.n - 1) * p.ldwq + fill_chunk * 16;
-  }
-  // The wave's scale request: 64 row scales, or 64 column scales -- the block
-  // scale 64 times in the block-scale variant.
-  const int scale_request = wave % Cfg::kScaleRequests;
-  const bool scales_rows = scale_request < Cfg::BM / 64;
-  const int64_t scale_at = (scales_rows ? m0 + 64 * scale_request : n0 + 64 * (scale_request - Cfg::BM / 64)) + lane;
-  const float* scale_src;
-  int64_t scale_step;
-  if (scales_rows) {
-    scale_src = p.xs + (scale_at < p.m ? scale_at : p.m - 1);
-    scale_step = p.m;
-  } else if (kColumnScales) {
-    scale_src = p.cs + (scale_at < p.n ? scale_at : p.n - 1);
-    scale_step = p.n;
-  } else {
-    scale_src = p.ws + n0 / 128 * p.ws_cb;
-    scale_step = p.ws_kb;
-  }
+  const uint8_t* Ab = uniform_ptr(p.xq + m0 * p.ldxq);
+  const uint8_t* Bb = uniform_ptr(p.wq + n0 * p.ldwq);
   typedef __attribute__((address_space(3))) uint8_t* lds_address;
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_address)lds_bytes));
-  auto request = [&](int kt, uint32_t stage, int idx) {
-    const uint32_t at = lds_base + stage * Cfg::kStageBytes;
-    if (idx < Cfg::kLoadsA + Cfg::kLoadsB)  // (operand B's rows follow operand A's in the stage)
-      dma_load_16_at(src[idx] + static_cast<int64_t>(kt) * Cfg::kRowBytes,
-                     at + wave * 1024 + idx * (Cfg::kFillRows * Cfg::kRowBytes));
-    else
-      dma_load_4_at(reinterpret_cast<const uint8_t*>(scale_src + kt * scale_step), at + Cfg::kScaleOffset + scale_request * 256);
+  const uint32_t fill_lds = lds_base + static_cast<uint32_t>(wave * 1024);
+  // Where a k-tile lies: the offsets of its early chunks, of its late ones and of its scales.
+  struct Place {
+    int early, late, scales;
   };
-
-  // Fragment side: row = lane & 31 of a 32-row block; chunks 4 kh + 2 h and
-  // 4 kh + 2 h + 1 of the row (kh = 64-byte half), each in slot chunk ^ ((row >> 1) & 7).
-  const int frag_row = lane & 31, h = lane >> 5;
-  uint32_t frag_off[2][2];
-#pragma unroll
-  for (int kh = 0; kh < 2; ++kh)
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-      frag_off[kh][c] = static_cast<uint32_t>(frag_row * Cfg::kRowBytes + (((4 * kh + 2 * h + c) ^ ((frag_row >> 1) & 7)) * 16));
-  auto read_frag = [&](const uint8_t* block, v8i32 (&frag)[2]) {
-#pragma unroll
-    for (int kh = 0; kh < 2; ++kh) {
-      const u32x4 lo = *reinterpret_cast<const u32x4*>(block + frag_off[kh][0]);
-      const u32x4 hi = *reinterpret_cast<const u32x4*>(block + frag_off[kh][1]);
-      frag[kh] = v8i32{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z), static_cast<int>(lo.w),
-                       static_cast<int>(hi.x), static_cast<int>(hi.y), static_cast<int>(hi.z), static_cast<int>(hi.w)};
-    }
+  constexpr Place kFirst{0, Cfg::kLateOffset, Cfg::kScaleOffset};
+  constexpr Place kLast{kDepth * Cfg::kEarlyBytes, Cfg::kLateOffset + (kDepth - 1) * Cfg::kLateBytes,
+                        Cfg::kScaleOffset + (kDepth - 1) * Cfg::kScaleBytes};
+  const auto place_after = [](const Place& at) {
+    return Place{at.early == kLast.early ? kFirst.early : at.early + Cfg::kEarlyBytes,
+                 at.late == kLast.late ? kFirst.late : at.late + Cfg::kLateBytes,
+                 at.scales == kLast.scales ? kFirst.scales : at.scales + Cfg::kScaleBytes};
   };
-  constexpr int kSets = kBlocks == 1 ? 2 : 1;  // a lone block reads the next k-tile's fragments while it multiplies
-  v8i32 afrag[kSets][TM][2], bfrag[kSets][TN][2];
-  auto read_a = [&](uint32_t stage, int set, int i) {
-    read_frag(lds_bytes + stage * Cfg::kStageBytes + (wm * Cfg::kWaveM + i * 32) * Cfg::kRowBytes, afrag[set][i]);
+  auto request = [&](int kt, const Place& at, int c) {
+    dma_load_16(voff[c], (c < kChunksA ? Ab : Bb) + static_cast<int64_t>(kt) * Cfg::kRowBytes,
+                fill_lds + (c < kEarly ? at.early : at.late), (c < kEarly ? c : c - kEarly) * Cfg::kChunkBytes);
   };
-  auto read_b = [&](uint32_t stage, int set, int j) {
-    read_frag(lds_bytes + stage * Cfg::kStageBytes + Cfg::kABytes + (wn * Cfg::kWaveN + j * 32) * Cfg::kRowBytes, bfrag[set][j]);
-  };
-  // Row scales of the wave's rows, times the block scale in the block-scale
-  // variant; per-column scales arranged for fold_with_row_broadcast: in every
-  // row of 16 lanes, lane n holds the scale of accumulator element n.
-  float row_scale[TM], col_scale[TN];
-  auto read_scales = [&](uint32_t stage) {
-    const float* rows = reinterpret_cast<const float*>(lds_bytes + stage * Cfg::kStageBytes + Cfg::kScaleOffset);
-    const float* cols = rows + Cfg::BM;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) row_scale[i] = rows[wm * Cfg::kWaveM + i * 32 + frag_row];
+  // The scales of a k-tile ride the same global->LDS path, 64 by one request of
+  // each wave: the row scales, then the column scales -- or the block scale of
+  // 64 of the tile's columns, 64 times.  (A load that the compiler sees inside
+  // the loop makes it wait for all requests in flight.)  Waves past the
+  // requests repeat the first ones.
+  const int scale_request = wave % Cfg::kScaleRequests;
+  const float* scale_src = p.xs;
+  int64_t scale_step = p.m;
+  uint32_t scale_voff = 0;
+  if (scale_request < Cfg::BM / 64) {
+    const int64_t row = m0 + scale_request * 64 + lane;
+    scale_voff = static_cast<uint32_t>((row < p.m ? row : p.m - 1) * 4);
+  } else {
+    const int64_t first = n0 + (scale_request - Cfg::BM / 64) * 64;
     if (kColumnScales) {
-#pragma unroll
-      for (int j = 0; j < TN; ++j) col_scale[j] = cols[wn * Cfg::kWaveN + j * 32 + 8 * ((lane & 15) >> 2) + 4 * h + (lane & 3)];
+      scale_voff = static_cast<uint32_t>((first + lane < p.n ? first + lane : p.n - 1) * 4);
+      scale_src = p.cs;
+      scale_step = p.n;
     } else {
-      const float block_scale = cols[0];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) row_scale[i] *= block_scale;
+      const int64_t block = first / 128, last = (p.n - 1) / 128;
+      scale_src = p.ws + (block < last ? block : last) * p.ws_cb;
+      scale_step = p.ws_kb;
     }
+  }
+  const uint32_t scale_lds = lds_base + scale_request * 256;
+  auto request_scales = [&](int kt, const Place& at) {
+    dma_touch_4(scale_voff, reinterpret_cast<const uint8_t*>(scale_src + kt * scale_step), scale_lds + at.scales);
   };
 
-  f32x16 acc[TM][TN];
+  // Fragment side: row = lane & 15 of a 16-row block, chunks g and g + 4 of its
+  // eight (g = lane / 16), each in slot chunk ^ ((row >> 1) & 7).  Any split of
+  // the 128 bytes over the four g will do that both operands share; with chunks
+  // 2 g and 2 g + 1 the reads met in the banks (25 % of the kernel's cycles by
+  // the counter: the LDS serves a 16-byte read to lanes of two neighbouring g at
+  // a time, whose slots stay apart if their chunks differ in bit 0).
+  const int frag_row = lane & 15, group = lane >> 4;
+  uint32_t frag_off[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    frag_off[c] = static_cast<uint32_t>(frag_row * Cfg::kRowBytes + (((group + 4 * c) ^ ((frag_row >> 1) & 7)) * 16));
+  // `row` of the rows that start at `chunk`
+  auto read_frag = [&](int chunk, int row) -> v8i32 {
+    const uint8_t* base = lds_bytes + chunk + row * Cfg::kRowBytes;
+    const u32x4 lo = *reinterpret_cast<const u32x4*>(base + frag_off[0]);
+    const u32x4 hi = *reinterpret_cast<const u32x4*>(base + frag_off[1]);
+    return v8i32{static_cast<int>(lo.x), static_cast<int>(lo.y), static_cast<int>(lo.z), static_cast<int>(lo.w),
+                 static_cast<int>(hi.x), static_cast<int>(hi.y), static_cast<int>(hi.z), static_cast<int>(hi.w)};
+  };
+
+  f32x4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-  auto multiply = [&](int set, int i, int j) -> f32x16 {
-    const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const f32x16 half = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bfrag[set][j][0], afrag[set][i][0], zero, 0, 0, 0, 0, 0, 0);
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bfrag[set][j][1], afrag[set][i][1], half, 0, 0, 0, 0, 0, 0);
-  };
-  auto fold = [&](const f32x16& product, int i, int j) {
-    if (kColumnScales) {
-      fold_with_row_broadcast(acc[i][j], product, row_scale[i], col_scale[j]);
-    } else {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(product[r], row_scale[i], acc[i][j][r]);
-    }
-  };
-  // This wave's part of the k-tile after `kt` has landed (those behind it stay
-  // in flight), everyone's has behind the barrier, and everyone holds in
-  // registers what it still needs of kt's own stage.
-  auto hand_over = [&](int kt) {
-    const int behind = ktiles - 2 - kt;
-    if (kStages >= 4 && behind >= kStages - 2)
-      wait_for_dma_loads_but<(kStages - 2) * Cfg::kRequests>();
-    else if (kStages >= 4 && behind >= (kStages - 2) / 2)
-      wait_for_dma_loads_but<(kStages - 2) / 2 * Cfg::kRequests>();
-    else if (kStages == 3 && behind >= 1)
-      wait_for_dma_loads_but<Cfg::kRequests>();
-    else
-      wait_for_dma_loads();
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  };
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  // The first kDepth - 1 k-tiles and the early chunks of the next.
+  Place now = kFirst, before = kLast;  // of k-tile kt and of the one before it, whose slots are free
+  Place ahead = kFirst;
 #pragma unroll
-  for (int kt = 0; kt < kStages; ++kt)
+  for (int kt = 0; kt < kDepth; ++kt) {
     if (kt < ktiles) {
+      if (kt + 1 < kDepth) request_scales(kt, ahead);
 #pragma unroll
-      for (int idx = 0; idx < Cfg::kRequests; ++idx) request(kt, kt, idx);
+      for (int c = 0; c < kChunks; ++c)
+        if (kt + 1 < kDepth || c < kEarly) request(kt, ahead, c);
     }
-  hand_over(-1);
-  read_a(0, 0, 0);
-  read_b(0, 0, 0);
-  uint32_t stage = 0;
-  // One k-tile; `more`: kt + 1 exists, `ahead`: kt + kStages does.
-  auto k_tile = [&](int kt, auto set_tag, auto more_tag, auto ahead_tag) {
-    constexpr int set = decltype(set_tag)::value;
-    constexpr bool more = decltype(more_tag)::value, ahead = decltype(ahead_tag)::value;
-    const uint32_t after = stage + 1 == kStages ? 0 : stage + 1;
-    read_scales(stage);
-    if constexpr (kBlocks == 1) {
-      if (more) {
-        hand_over(kt);
-        read_a(after, set ^ 1, 0);
-        read_b(after, set ^ 1, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      const f32x16 product = multiply(set, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (ahead) {
+    ahead = place_after(ahead);
+  }
+  constexpr int kRequests = kChunks + 1;  // of a k-tile, per wave
+  if (ktiles >= kDepth) wait_for_dma_loads_but<kEarly + (kDepth - 2) * kRequests>();
+  else if (kDepth >= 4 && ktiles == 3) wait_for_dma_loads_but<2 * kRequests>();
+  else if (kDepth >= 3 && ktiles == 2) wait_for_dma_loads_but<kRequests>();
+  else wait_for_dma_loads();
+  asm volatile("s_barrier" ::: "memory");
+
+#ifdef FSH_TRACE
+  // Time per phase of the k loop, summed over the k-tiles (10 ns ticks).
+  uint64_t t_compute = 0, t_wait = 0, t_barrier = 0, t_mark = __builtin_amdgcn_s_memrealtime();
+  const uint64_t t_begin = t_mark;
+  auto lap = [&](uint64_t& sum) {
+    const uint64_t now = __builtin_amdgcn_s_memrealtime();
+    sum += now - t_mark;
+    t_mark = now;
+  };
+#endif
+  // The k loop is rotated by a column of blocks: the barrier that hands over
+  // k-tile kt + 1 sits before the last column of k-tile kt, and behind each of
+  // its MFMAs the wave reads the fragment of kt + 1 that takes the place of the
+  // one just used.
+  //   carried into a k-tile: afrag, bfrag[0]
+  // Behind that barrier the slots of k-tile kt are free: in k-tile kt + 1 they
+  // take the scales and late chunks of kt + kDepth, then the early ones of
+  // kt + kDepth + 1, one request behind every few MFMAs.
+  constexpr int kBlocks = TM * TN;
+  v8i32 afrag[TM], bfrag[2];
+  constexpr int kScaleRegs = (TN + 3) / 4, kBlocksPerReg = TN < 4 ? TN : 4;
+  float s[TM], cs_rows[kScaleRegs];
+  // Row scales of the wave's rows for k-tile kt, times the block scale in the
+  // block-scale variant; a lane owns output row lane & 15 of each of its blocks.
+  auto read_scales = [&](const Place& at) {
+    const float* rows = reinterpret_cast<const float*>(lds_bytes + at.scales);
 #pragma unroll
-        for (int idx = 0; idx < Cfg::kRequests; ++idx) request(kt + kStages, stage, idx);
-      }
-      fold(product, 0, 0);
+    for (int i = 0; i < TM; ++i) s[i] = rows[wm * Cfg::kWaveM + i * 16 + frag_row];
+    if (kColumnScales) {
+      // Register q holds, in every row of 16 lanes, the 16 scales that the lanes
+      // of that row fold column blocks 4 q .. 4 q + 3 with: lane 4 b + r of the
+      // row the scale of accumulator r of block 4 q + b.  A fold takes it through
+      // the data-parallel-primitive broadcast of the multiply-add itself.
+#pragma unroll
+      for (int q = 0; q < kScaleRegs; ++q)
+        cs_rows[q] = rows[Cfg::BM + wn * Cfg::kWaveN + q * 64 + 16 * (((lane & 15) >> 2) % kBlocksPerReg) + 4 * group + (lane & 3)];
     } else {
-      // The blocks in the order (0,0) (1,0) (0,1) (1,1): the first one's
-      // fragments are free at the last, whose MFMAs cover the read of the next
-      // k-tile's first ones; a block is folded behind the next one's MFMAs.
-      static_assert(kBlocks == 1 || (TM == 2 && TN == 2), "block order");
-      f32x16 part[2];
-      read_a(stage, 0, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      part[0] = multiply(0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      read_b(stage, 0, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      part[1] = multiply(0, 1, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      fold(part[0], 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      part[0] = multiply(0, 0, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      fold(part[1], 1, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (more) {
-        hand_over(kt);
-        read_a(after, 0, 0);
-        read_b(after, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      part[1] = multiply(0, 1, 1);
-      __builtin_amdgcn_sched_barrier(0);
-      if (ahead) {
+      const float block_scale = rows[Cfg::BM + wn * Cfg::kWaveN];
 #pragma unroll
-        for (int idx = 0; idx < Cfg::kRequests; ++idx) request(kt + kStages, stage, idx);
-      }
-      fold(part[0], 0, 1);
-      fold(part[1], 1, 1);
+      for (int i = 0; i < TM; ++i) s[i] *= block_scale;
     }
-    __builtin_amdgcn_sched_barrier(0);
-    stage = after;
+  };
+  // The wave's rows of A lie in whole chunks, or in a part of one; those of B in whole chunks.
+  const int a_chunk = wm * Cfg::kWaveM / Cfg::kChunkRows, a_row = wm * Cfg::kWaveM % Cfg::kChunkRows;
+  const int b_chunk = kChunksA + wn * Cfg::kWaveN / Cfg::kChunkRows;
+  const auto chunk_at = [](const Place& at, int c, bool early) {
+    return (early ? at.early : at.late) + (early ? c : c - kEarly) * Cfg::kChunkBytes;
+  };
+  auto read_a = [&](const Place& at, int i) {
+    const int c = a_chunk + i * 16 / Cfg::kChunkRows;
+    afrag[i] = read_frag(chunk_at(at, c, c < kEarly), a_row + i * 16 % Cfg::kChunkRows);
+  };
+  auto read_b = [&](const Place& at, int j) {
+    bfrag[j & 1] = read_frag(chunk_at(at, b_chunk + j * 16 / Cfg::kChunkRows, kEarly == kChunks), j * 16 % Cfg::kChunkRows);
+  };
+  constexpr bool kWholeAhead = TN == 2;
+  read_b(now, 0);
+  if (kWholeAhead) read_b(now, 1);
+#pragma unroll
+  for (int i = 0; i < TM; ++i) read_a(now, i);
+
+  // The MFMA that request r of a k-tile goes out behind, the late chunks first
+  // and closer together: with kDepth = 2 the last of them has the rest of this
+  // k-tile to arrive.  All go out before the wait for the next k-tile.
+  constexpr auto behind_mfma = [](int r) {
+    if (kBlocks < 2 * kChunks) return r * (kBlocks - TM) / kChunks;
+    const int span = kBlocks / kChunks, late_span = span - 1 > 0 ? span - 1 : 1;
+    return r < Cfg::kLate ? r * late_span : Cfg::kLate * late_span + (r - Cfg::kLate) * span;
+  };
+  static_assert(behind_mfma(kChunks - 1) < kBlocks - TM, "the count that the wait leaves in flight");
+  // more: k-tile kt + 1 exists; late, early: kt + kDepth - 1 and kt + kDepth do, and their late and early
+  // chunks go out.  Tags, so that no request sits behind a branch of its own.
+  auto k_tile = [&](int kt, auto more_tag, auto late_tag, auto early_tag) {
+    constexpr bool more = decltype(more_tag)::value, late = decltype(late_tag)::value, early = decltype(early_tag)::value;
+    const Place next = place_after(now);
+    // The scales are first needed by the first fold, kLag blocks in.
+    read_scales(now);
+    // The wave's 16x16 blocks, column by column.  One 16x16x128 MFMA gives a
+    // block's partial product for this scale block; it is folded into the result
+    // (4 fused multiply-adds, or multiply + fused multiply-add with per-column
+    // scales) kLag blocks later: a fold that reads the product of an MFMA issued
+    // just before it waits for the matrix core to drain.
+    constexpr int kLag = kBlocks > 8 ? 4 : 2;
+    f32x4 part[kLag + 1];
+    auto fold = [&](int blk) {
+      const int pi = blk % TM, pj = blk / TM;
+      const f32x4& product = part[blk % (kLag + 1)];
+      if (kColumnScales) {
+        fold_with_row_broadcast(acc[pi][pj], product, s[pi], cs_rows[pj / 4], pj % 4);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[pi][pj][r] = __builtin_fmaf(product[r], s[pi], acc[pi][pj][r]);
+      }
+      // An empty statement that "uses" the folded block keeps its arithmetic
+      // on this side of the next scheduling barrier.
+      asm volatile("" : "+v"(acc[pi][pj]));
+    };
+#pragma unroll
+    for (int blk = 0; blk < kBlocks; ++blk) {
+      const int i = blk % TM, j = blk / TM;
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+      if (blk == kBlocks - TM) {
+        // Every fragment of this k-tile is in registers: hand its slots over.
+#ifdef FSH_TRACE
+        lap(t_compute);
+#endif
+        // This wave's part of k-tile kt + 1 has landed; what was requested behind it stays in flight.
+        if (early) wait_for_dma_loads_but<kEarly + (kDepth - 2) * kRequests>();
+        else if (kDepth >= 4 && kt + 4 == ktiles) wait_for_dma_loads_but<2 * kRequests>();
+        else if (kDepth >= 3 && kt + 3 == ktiles) wait_for_dma_loads_but<kRequests>();
+        else if (more) wait_for_dma_loads();
+#ifdef FSH_TRACE
+        lap(t_wait);
+#endif
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#ifdef FSH_TRACE
+        lap(t_barrier);
+#endif
+      }
+      // The next column's B fragment, a column ahead (of two columns both come with the k-tile's first ones).
+      if (!kWholeAhead && i == 0 && j + 1 < TN) read_b(now, j + 1);
+      // Wave priority falls as the k-tile proceeds: of the two waves of a SIMD
+      // the one that is behind wins the issue slot, so both reach the barrier
+      // together (with equal priorities the older wave runs ahead and then
+      // idles at the barrier while the other finishes alone, without a
+      // partner to overlap its folds with).
+      if (blk * 4 == 0 * kBlocks) __builtin_amdgcn_s_setprio(3);
+      if (blk * 4 == 1 * kBlocks) __builtin_amdgcn_s_setprio(2);
+      if (blk * 4 == 2 * kBlocks) __builtin_amdgcn_s_setprio(1);
+      if (blk * 4 == 3 * kBlocks) __builtin_amdgcn_s_setprio(0);
+      part[blk % (kLag + 1)] =
+          __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bfrag[j & 1], afrag[i], zero, 0, 0, 0, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (blk >= kBlocks - TM && more) {  // what the next k-tile starts with
+        if (i == 0) read_b(next, 0);
+        read_a(next, i);
+        if (kWholeAhead && blk == kBlocks - 1) read_b(next, 1);
+      }
+      if (late && blk == 0) request_scales(kt + kDepth - 1, before);
+#pragma unroll
+      for (int r = 0; r < kChunks; ++r)
+        if (blk == behind_mfma(r)) {
+          if (r < Cfg::kLate) {
+            if (late) request(kt + kDepth - 1, before, kEarly + r);
+          } else if (early) {
+            request(kt + kDepth, before, r - Cfg::kLate);
+          }
+        }
+      if (blk >= kLag) fold(blk - kLag);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int blk = kBlocks - kLag; blk < kBlocks; ++blk) fold(blk);
+    before = now;
+    now = next;
   };
   constexpr std::true_type yes{};
   constexpr std::false_type no{};
-  constexpr std::integral_constant<int, 0> even{};
-  constexpr std::integral_constant<int, kSets - 1> odd{};
   int kt = 0;
-  for (; kt + 1 + kStages < ktiles; kt += 2) {
-    k_tile(kt, even, yes, yes);
-    k_tile(kt + 1, odd, yes, yes);
+  for (; kt + kDepth < ktiles; ++kt) k_tile(kt, yes, yes, yes);
+  if (kDepth <= ktiles) k_tile(kt++, yes, yes, no);
+  for (; kt + 1 < ktiles; ++kt) k_tile(kt, yes, no, no);
+  k_tile(ktiles - 1, no, no, no);
+#ifdef FSH_TRACE
+  if (p.schedule.trace && lane == 0) {
+    uint64_t* out = p.schedule.trace + (static_cast<int64_t>(blockIdx.x) * Cfg::kWaves + wave) * 8;
+    out[0] = t_begin; out[1] = t_compute; out[2] = t_wait; out[3] = t_barrier; out[4] = t_mark; out[5] = t_entry;
   }
-  for (; kt < ktiles; ++kt) {  // the last few, fragments back in set 0 after each pair
-    const bool more = kt + 1 < ktiles, ahead = kt + kStages < ktiles;
-    if (kSets == 1 || (kt & 1) == 0) {
-      if (ahead) k_tile(kt, even, yes, yes);
-      else if (more) k_tile(kt, even, yes, no);
-      else k_tile(kt, even, no, no);
-    } else {
-      if (ahead) k_tile(kt, odd, yes, yes);
-      else if (more) k_tile(kt, odd, yes, no);
-      else k_tile(kt, odd, no, no);
-    }
-  }
-  __syncthreads();  // the images overlay the stages
+#endif
 
+  // Epilogue: bf16 finals to the wave's staging region as [row][col], then
+  // 16-byte row stores, rows and 8-column groups past the matrix skipped.
   uint8_t* region = lds_bytes + wave * Cfg::kRegion;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        *reinterpret_cast<u32x2*>(region + (i * 32 + frag_row) * Cfg::kPitch + (j * 32 + 8 * b + 4 * h) * 2) =
-            u32x2{pack_bf16x2(acc[i][j][4 * b], acc[i][j][4 * b + 1]),
-                  pack_bf16x2(acc[i][j][4 * b + 2], acc[i][j][4 * b + 3])};
+      *reinterpret_cast<u32x2*>(region + (i * 16 + frag_row) * Cfg::kPitch + (j * 16 + 4 * group) * 2) =
+          u32x2{pack_bf16x2(acc[i][j][0], acc[i][j][1]), pack_bf16x2(acc[i][j][2], acc[i][j][3])};
   wave_lds_sync();
   store_fp8_product<Cfg::kWaveM, Cfg::kWaveN, Cfg::kPitch>(region, p, m0 + wm * Cfg::kWaveM, n0 + wn * Cfg::kWaveN, lane);
+#ifdef FSH_TRACE
+  if (p.schedule.trace && lane == 0) {
+    __builtin_amdgcn_s_waitcnt(0);
+    p.schedule.trace[(static_cast<int64_t>(blockIdx.x) * Cfg::kWaves + wave) * 8 + 6] = __builtin_amdgcn_s_memrealtime();
+    uint32_t hw_id;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_HW_ID)" : "=s"(hw_id));
+    uint32_t xcc_id;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc_id));
+    p.schedule.trace[(static_cast<int64_t>(blockIdx.x) * Cfg::kWaves + wave) * 8 + 7] = (static_cast<uint64_t>(xcc_id) << 32) | hw_id;
+  }
+#endif
+}
+
+template <typename Cfg, bool kColumnScales, int kBlocksPerUnit>
+__global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) void fp8_gemm_tiles_kernel(const Fp8GemmParams p) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds_bytes[];
+  int64_t unused_batch;
+  int tm, tn;
+  if (!tile_of_workgroup(p.schedule, blockIdx.x, &unused_batch, &tm, &tn)) return;  // whole workgroup
+  fp8_gemm_tile<Cfg, kColumnScales>(p, lds_bytes, static_cast<int64_t>(uniform_i32(tm)) * Cfg::BM,
+                                    static_cast<int64_t>(uniform_i32(tn)) * Cfg::BN);
 }
 
 }  // namespace

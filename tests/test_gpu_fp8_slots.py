@@ -1,7 +1,8 @@
-"""The 256 x 256 FP8 tiles over contractions that use every slot of a k-tile's
-chunks (three of the early ones by two of the late ones: six k-tiles), the last
-two k-tiles at every place; 16 of the 272 tiles are cut into halves, whose
-chunks are all early."""
+"""The FP8 tiles over contractions that use every slot of a k-tile's chunks, the
+last k-tiles at every place.  256 x 256: three of the early ones by two of the
+late ones, six k-tiles; 16 of the 272 tiles are cut into halves, whose chunks
+are all early.  Smaller ones: as many slots as k-tiles in flight (two to four)
+and one more of the early ones, twenty k-tiles at the most."""
 
 import pytest
 import torch
@@ -14,9 +15,23 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("ktiles", [2, 3, 6, 7, 8, 9, 10, 11, 13])
 @pytest.mark.parametrize("column_scales", [False, True])
 def test_every_place_of_a_k_tile(device, ktiles, column_scales):
+    _check(device, 4090, 4120, ktiles, column_scales, "256")
+
+
+@pytest.mark.parametrize("column_scales", [False, True])
+@pytest.mark.parametrize(
+    "m,n,tiles,ktiles",
+    [(m, n, tiles, ktiles) for m, n, tiles in ((130, 1000, "64 deep"), (1090, 3080, "128 deep")) for ktiles in (7, 12, 19, 20, 21, 22, 23, 24)]
+    + [(m, n, tiles, ktiles) for m, n, tiles in ((1030, 2050, "64"), (1923, 2180, "128")) for ktiles in (7, 8, 10, 11, 12)],
+)
+def test_every_place_of_a_k_tile_in_small_tiles(device, m, n, tiles, ktiles, column_scales):
+    _check(device, m, n, ktiles, column_scales, tiles)
+
+
+def _check(device, m, n, ktiles, column_scales, tiles):
     """Small integers and powers of two: exact in fp32, one rounding to bf16."""
-    m, n, k = 4090, 4120, 128 * ktiles
-    assert hip_ops.fp8_gemm_tiles(m, n, k, column_scales=column_scales) == "256"
+    k = 128 * ktiles
+    assert hip_ops.fp8_gemm_tiles(m, n, k, column_scales=column_scales) == tiles
     gen = torch.Generator(device=device)
     gen.manual_seed(ktiles)
     a, b = (torch.randint(-3, 4, (rows, k), generator=gen, device=device).float() for rows in (m, n))
