@@ -532,7 +532,12 @@ double launch_us(TileKind kind, const LaunchWork& w) {
 TileKind small_tile_kind(const LaunchWork& w) {
   TileKind best = kTiles64;
   for (const TileKind kind : {kTiles128, kTiles128Deep, kTiles256x128}) {
-    if (kind == kTiles128Deep && w.tiles[kind] > kTileShapes[kind].round) continue;  // one round or none
+    // One round or none; short tiles beside longer ones count by their length there, nine tenths of a round of them:
+    // the hand-out is not that even (Muon steps, us without / with such mixtures: 13 x 3555 x 384 with 2432 x 2432
+    // 790 / 727, 4 x 1024 x 4096 with 8 x 1024 x 1024 690 / 674; a whole round, 2 x 1280 x 1280 with 8 x 832 x 832, 380 / 406).
+    if (kind == kTiles128Deep && w.tiles[kind] > kTileShapes[kind].round &&
+        w.tile_ktiles[kind] > 0.9 * kTileShapes[kind].round * w.max_ktiles)
+      continue;
     if (launch_us(kind, w) < launch_us(best, w)) best = kind;
   }
   return best;
