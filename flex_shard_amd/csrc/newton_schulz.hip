@@ -733,8 +733,6 @@ TileKind small_tile_kind_of(const PlannedGemm* plans, const int* members, int n)
   return has_wide_rows(plans, members, n) ? kTiles128 : small_tile_kind(work_of(plans, members, n));
 }
 
-constexpr double kDeepTiles64 = 384.0;  // one and a half for each of 256 compute units
-
 int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stream) {
   const TileKind kind = small_tile_kind_of(plans, members, n);
   TileLaunch launch;
@@ -743,12 +741,13 @@ int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stre
   switch (kind) {
     case kTiles64: {
       // Tiles that leave a compute unit with one workgroup or two are requested four k-tiles ahead: nothing else
-      // covers their requests.  More of them lose more by the LDS that takes (us, two / four k-tiles ahead; tiles
-      // of a shorter contraction count by their share of the longest):
+      // covers their requests.  More of them, and somewhat fewer of few k-tiles, lose more by the LDS that takes
+      // (us, two / four k-tiles ahead; tiles of a shorter contraction count by their share of the longest):
       //   136 tiles, k 4096 27.9 / 14.7   231, k 1672 9.4 / 9.0   256, k 2048 9.5 / 9.2   300, k 4096 29.0 / 23.7
-      //   384, k 1024 7.7 / 8.2           384, k 2048 15.9 / 13.9   512, k 2048 13.4 / 14.8   624, k 3072 25.7 / 27.7
+      //   384, k 1024 7.7 / 8.2   384, k 2048 15.9 / 13.9   448, k 1280 9.4 / 10.0   406, k 1792 16.3 / 14.7
+      //   484, k 1408 12.3 / 11.3   465, k 3072 23.8 / 23.1   512, k 2048 13.4 / 14.8   624, k 3072 25.7 / 27.7
       const LaunchWork work = work_of(plans, members, n);
-      if (work.tile_ktiles[kTiles64] <= kDeepTiles64 * work.max_ktiles)
+      if (work.tile_ktiles[kTiles64] <= (work.max_ktiles >= 22.0 ? 500.0 : 384.0) * work.max_ktiles)
         return launch_tiles_as<GemmTiles<2, 2, 2, 2, 4>, 2>(launch, stream);
       return launch_tiles_as<GemmTiles<2, 2, 2, 2, 2>, 4>(launch, stream);
     }
