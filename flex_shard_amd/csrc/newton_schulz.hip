@@ -532,11 +532,12 @@ double launch_us(TileKind kind, const LaunchWork& w) {
 TileKind small_tile_kind(const LaunchWork& w) {
   TileKind best = kTiles64;
   for (const TileKind kind : {kTiles128, kTiles128Deep, kTiles256x128}) {
-    // One round or none; short tiles beside longer ones count by their length there, nine tenths of a round of them:
-    // the hand-out is not that even (Muon steps, us without / with such mixtures: 13 x 3555 x 384 with 2432 x 2432
-    // 790 / 727, 4 x 1024 x 4096 with 8 x 1024 x 1024 690 / 674; a whole round, 2 x 1280 x 1280 with 8 x 832 x 832, 380 / 406).
+    // One round or none; short tiles beside longer ones count by their length there, up to 0.86 of a round of them:
+    // the hand-out is not that even.  Muon steps, us without / with such mixtures, by the part of a round: 0.81 (13 of
+    // 3555 x 384, 2432 x 2432) 790 / 727, 0.84 (4 of 1024 x 4096, 8 of 1024 x 1024) 690 / 674, 0.87 (8 of 768 x 768, 4
+    // each of 3072 x 768 and 768 x 3072, four odd ones) 617 / 620, 1.0 (2 of 1280 x 1280, 8 of 832 x 832) 380 / 406.
     if (kind == kTiles128Deep && w.tiles[kind] > kTileShapes[kind].round &&
-        w.tile_ktiles[kind] > 0.9 * kTileShapes[kind].round * w.max_ktiles)
+        w.tile_ktiles[kind] > 0.86 * kTileShapes[kind].round * w.max_ktiles)
       continue;
     if (launch_us(kind, w) < launch_us(best, w)) best = kind;
   }

@@ -30,6 +30,16 @@ def test_problems_of_one_call_share_the_choice():
     assert hip_ops.newton_schulz_large_tiles((24, 7168, 2048), steps=0) == (False,)
 
 
+@pytest.mark.parametrize(
+    "long,short,tiles",
+    [((13, 384, 384, 3560, True), (1, 2432, 2432, 2432, True), "128 deep"), ((4, 1024, 1024, 4096, True), (8, 1024, 1024, 1024, True), "128 deep"),
+     ((8, 768, 768, 3072, True), (10, 768, 768, 768, True), "128"), ((2, 1280, 1280, 1280, True), (8, 832, 832, 832, True), "128")],
+)
+def test_short_tiles_beside_long_ones_count_by_their_length(long, short, tiles):
+    """More than 256 tiles of 128 x 128, by length up to 0.86 of a round of the long ones and more."""
+    assert hip_ops.gemm_tiles(long, short) == (tiles, tiles)
+
+
 def test_third_product_takes_large_tiles_within_one_round_only():
     """Problems that iterate on the small tiles: their third product joins the
     256 x 256 ones up to a round of 256 of them, and only where that is faster."""
