@@ -741,15 +741,17 @@ int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stre
   if (has_wide_rows(plans, members, n)) return launch_tiles_as<GemmTiles<2, 2, 4, 4, 2>, 2, true>(launch, stream);
   switch (kind) {
     case kTiles64: {
-      // Tiles that leave a compute unit with one workgroup or two are requested four k-tiles ahead: nothing else
-      // covers their requests.  More of them, and somewhat fewer of few k-tiles, lose more by the LDS that takes
-      // (us, two / four k-tiles ahead; tiles of a shorter contraction count by their share of the longest):
-      //   136 tiles, k 4096 27.9 / 14.7   231, k 1672 9.4 / 9.0   256, k 2048 9.5 / 9.2   300, k 4096 29.0 / 23.7
-      //   384, k 1024 7.7 / 8.2   384, k 2048 15.9 / 13.9   448, k 1280 9.4 / 10.0   406, k 1792 16.3 / 14.7
-      //   484, k 1408 12.3 / 11.3   465, k 3072 23.8 / 23.1   512, k 2048 13.4 / 14.8   624, k 3072 25.7 / 27.7
+      // Tiles that leave a compute unit with one workgroup or two are requested further ahead: nothing else covers
+      // their requests.  More of them, and somewhat fewer of few k-tiles, lose more by the LDS that takes (us, two /
+      // three / four k-tiles ahead; tiles of a shorter contraction count by their share of the longest):
+      //   136 tiles, k 4096 27.9 / 17.0 / 14.7   256, k 4096 27.6 / - / 14.9   256, k 2048 9.5 / - / 9.2
+      //   231, k 1672 9.4 / - / 9.0   300, k 4096 29.0 / - / 23.7   384, k 2048 15.9 / - / 13.9   406, k 1792 16.3 / - / 14.7
+      //   378, k 2944 22.8 / 21.2 / 21.7   406, k 3072 23.6 / 22.2 / 22.5   435, k 3072 23.7 / 22.3 / 22.6
+      //   484, k 1408 12.3 / - / 11.3   384, k 1024 7.7 / - / 8.2   448, k 1280 9.4 / - / 10.0   512, k 2048 13.4 / - / 14.8
       const LaunchWork work = work_of(plans, members, n);
-      if (work.tile_ktiles[kTiles64] <= (work.max_ktiles >= 22.0 ? 500.0 : 384.0) * work.max_ktiles)
-        return launch_tiles_as<GemmTiles<2, 2, 2, 2, 4>, 2>(launch, stream);
+      const double long_tiles = work.tile_ktiles[kTiles64] / work.max_ktiles;
+      if (long_tiles <= 256.0) return launch_tiles_as<GemmTiles<2, 2, 2, 2, 4>, 2>(launch, stream);
+      if (long_tiles <= (work.max_ktiles >= 22.0 ? 500.0 : 384.0)) return launch_tiles_as<GemmTiles<2, 2, 2, 2, 3>, 2>(launch, stream);
       return launch_tiles_as<GemmTiles<2, 2, 2, 2, 2>, 4>(launch, stream);
     }
     case kTiles128: return launch_tiles_as<GemmTiles<2, 2, 4, 4, 2>, 2>(launch, stream);
