@@ -304,12 +304,8 @@ int launch_fp8_gemm(Fp8GemmParams& p, bool column_scales, const char* who, void*
   s.tiles_per_matrix = static_cast<int32_t>(tiles);
   const int64_t units = compute_units();
   const hipStream_t on = static_cast<hipStream_t>(stream);
-  Fp8TileKind kind = fp8_tile_kind(p.m, p.n, p.k, column_scales, units);
-#ifdef FORCEKIND
-  if (const char* e = getenv("FSH_KIND")) if (atoi(e) >= 0) kind = static_cast<Fp8TileKind>(atoi(e));
-#endif
-  switch (kind) {
-        case kFp8Tiles64: return launch_fp8_tiles<Fp8Tile<2, 2, 2, 2, 3, 0>, 3>(p, column_scales, on);
+  switch (fp8_tile_kind(p.m, p.n, p.k, column_scales, units)) {
+    case kFp8Tiles64: return launch_fp8_tiles<Fp8Tile<2, 2, 2, 2, 3, 0>, 3>(p, column_scales, on);
     case kFp8Tiles64Deep: return launch_fp8_tiles<Fp8Tile<2, 2, 2, 2, 4, 2>, 2>(p, column_scales, on);
     case kFp8Tiles128: return launch_fp8_tiles<Fp8Tile<2, 2, 4, 4, 2, 3>, 2>(p, column_scales, on);
     case kFp8Tiles128Deep: return launch_fp8_tiles<Fp8Tile<2, 2, 4, 4, 4, 4>, 1>(p, column_scales, on);
