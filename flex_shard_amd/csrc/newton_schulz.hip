@@ -498,7 +498,7 @@ constexpr TileShape kTileShapes[] = {
     {64, 64, 768.0, 0.17, 0.40, 0.55, 1.7},       // three workgroups per compute unit (four fit)
     {128, 128, 512.0, 0.37, 0.71, 1.02, 4.2},     // two
     {128, 128, 256.0, 0.35, 0.43, 0.52, 3.2},     // one, its operands requested four k-tiles ahead
-    {256, 128, 256.0, 0.54, 0.68, 0.91, 5.5},     // one
+    {256, 128, 256.0, 0.54, 0.68, 0.91, 5.5},     // one of eight waves
     {256, 256, 256.0, 0.94, 1.02, 1.38, 8.5},     // one
 };
 // The products of one launch, as the tiles of every kind see them.
@@ -756,7 +756,10 @@ int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stre
     }
     case kTiles128: return launch_tiles_as<GemmTiles<2, 2, 4, 4, 2>, 2>(launch, stream);
     case kTiles128Deep: return launch_tiles_as<GemmTiles<2, 2, 4, 4, 4>, 1>(launch, stream);
-    default: return launch_tiles_as<GemmTiles<2, 2, 8, 4, 2>, 1>(launch, stream);
+    // Eight waves: with four of 128 x 64 the start and the staged output of a tile took 2 to 3 us longer (us, four / eight:
+    // 3400 x 3400 symmetric with D, k 3400 59.8 / 56.5   3200 x 3200 symmetric, k 3080 53.1 / 51.1
+    // 8 x 2976 x 992, k 992, two outputs 72.8 / 65.5).
+    default: return launch_tiles_as<GemmTiles<4, 2, 4, 4, 2>, 1>(launch, stream);
   }
 }
 
