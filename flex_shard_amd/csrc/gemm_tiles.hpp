@@ -10,15 +10,17 @@ using TileLaunch = GemmLaunchOf<8>;
 
 // WM x WN waves, each TM x TN blocks of 16 x 16.  Operands are requested kDepth
 // k-tiles of 64 ahead: operand A has a slot for each of them and for the k-tile
-// in work, operand B, which is requested later in a k-tile, for one fewer.
-template <int WM_, int WN_, int TM_, int TN_, int kDepth_>
+// in work, operand B, which is requested later in a k-tile, for one fewer;
+// kLateA: operand A as late as B, with as many slots.
+template <int WM_, int WN_, int TM_, int TN_, int kDepth_, bool kLateA_ = false>
 struct GemmTiles {
   static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, kDepth = kDepth_;
+  static constexpr bool kLateA = kLateA_;
   static constexpr int kWaveM = 16 * TM, kWaveN = 16 * TN, BM = WM * kWaveM, BN = WN * kWaveN, BK = 64, KS = BK / 32;
   static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves;
   static constexpr int kRowBytes = BK * 2;  // 128
   static constexpr int kABytes = BM * kRowBytes, kBBytes = BN * kRowBytes;
-  static constexpr int kARing = (kDepth + 1) * kABytes, kBRing = kDepth * kBBytes;  // B's ring lies behind A's
+  static constexpr int kARing = (kDepth + (kLateA ? 0 : 1)) * kABytes, kBRing = kDepth * kBBytes;  // B's ring lies behind A's
   // A wave-level request fills 1 KB = 8 tile rows.
   static constexpr int kFillRows = 8 * kWaves;
   static constexpr int kLoadsA = BM / kFillRows, kLoadsB = BN / kFillRows, kLoads = kLoadsA + kLoadsB;
@@ -231,7 +233,7 @@ __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) vo
   // slot of B(kt) is free there (every wave holds its last fragments in registers).
   //   k step 0:     A(kt + kDepth) into the slot of A(kt - 1)
   //   wait for k-tile kt + 1, barrier
-  //   k step 1:     B(kt + kDepth) into the slot of B(kt)
+  //   k step 1:     B(kt + kDepth) into the slot of B(kt); kLateA: A(kt + kDepth), too, into the slot of A(kt)
   // Each step reads the next one's fragments.  A request goes out behind every
   // few MFMAs: several in one go hold up the wave.
   static_assert(KS == 2, "the sequence above");
@@ -256,11 +258,13 @@ __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) vo
           }
       }
       if (ahead) {
+        constexpr bool late = Cfg::kLateA;
+        const int first = ks == 0 || late ? 0 : kLoadsA, last = ks == 0 ? (late ? 0 : kLoadsA) : Cfg::kLoads;
 #pragma unroll
-        for (int r = 0; r < (ks == 0 ? kLoadsA : kLoadsB); ++r)
-          if (r * kMfmas / (ks == 0 ? kLoadsA : kLoadsB) == g) {
-            if (ks == 0) issue(a_src, a_voff[r], a_before, r);
-            else issue(b_src, b_voff[r], Cfg::kARing + b_slot, r);
+        for (int r = first; r < last; ++r)
+          if ((r - first) * kMfmas / (last - first) == g) {
+            if (r < kLoadsA) issue(a_src, a_voff[r], late ? a_slot : a_before, r);
+            else issue(b_src, b_voff[r - kLoadsA], Cfg::kARing + b_slot, r - kLoadsA);
           }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -272,7 +276,7 @@ __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) vo
     if (more) {
       // k-tile kt + 1 has landed (this wave's part); those behind it stay in flight.
       if (ahead) {
-        wait_for_dma_loads_but<(kDepth - 1) * kLoadsA + (kDepth - 2) * kLoadsB>();
+        wait_for_dma_loads_but<(kDepth - 2) * Cfg::kLoads + (Cfg::kLateA ? 0 : kLoadsA)>();
       } else {
         const int behind = ktiles - 2 - kt;
         if (kDepth >= 4 && behind == 2) wait_for_dma_loads_but<2 * Cfg::kLoads>();

@@ -730,6 +730,22 @@ bool has_wide_rows(const PlannedGemm* plans, const int* members, int n) {
   }
   return false;
 }
+// Whether most of a launch's work on tiles of a kind reads operand rows that do
+// not start at cache lines: a k-tile's 128 bytes of such a row touch two.
+bool has_split_rows(const PlannedGemm* plans, const int* members, int n, TileKind kind) {
+  double split = 0.0, all = 0.0;
+  for (int k = 0; k < n; ++k) {
+    const GemmParams& p = plans[members[k]].p;
+    LaunchWork work;
+    work.add(p.M, p.N, p.K, p.symmetric != 0, plans[members[k]].batch);
+    all += work.tile_ktiles[kind];
+    const auto at_lines = [&](const uint16_t* rows, int64_t ld, int64_t stride) {
+      return aligned(rows, 128) && ld % 64 == 0 && (plans[members[k]].batch == 1 || stride % 64 == 0);
+    };
+    if (!at_lines(p.A, p.lda, p.sA) || !at_lines(p.B, p.ldb, p.sB)) split += work.tile_ktiles[kind];
+  }
+  return 2.0 * split > all;
+}
 TileKind small_tile_kind_of(const PlannedGemm* plans, const int* members, int n) {
   return has_wide_rows(plans, members, n) ? kTiles128 : small_tile_kind(work_of(plans, members, n));
 }
@@ -754,7 +770,19 @@ int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stre
       if (long_tiles <= (work.max_ktiles >= 22.0 ? 500.0 : 384.0)) return launch_tiles_as<GemmTiles<2, 2, 2, 2, 3>, 2>(launch, stream);
       return launch_tiles_as<GemmTiles<2, 2, 2, 2, 2>, 4>(launch, stream);
     }
-    case kTiles128: return launch_tiles_as<GemmTiles<2, 2, 4, 4, 2>, 2>(launch, stream);
+    case kTiles128: {
+      // Where some compute units have two of these tiles and others one, the ones with two are what a launch waits for.  If
+      // rows straddle cache lines they have twice the lines to fetch, and the more of them in flight the slower (us with
+      // A early / late; up to a round of two per unit):
+      //   276 tiles, k 1032 22.8 / 21.0, k 3080 55.4 / 44.4   300, k 2056 41.8 / 33.2   384 with D, k 504 14.9 / 14.2
+      // From there on all have as much to do, and the early requests are worth more (528, k 2056 63.8 / 70.8; with rows at
+      // cache lines 276, k 2048 27.4 / 27.1 and 288 with D, k 1024 18.0 / 18.8).
+      const LaunchWork work = work_of(plans, members, n);
+      const double long_tiles = work.tile_ktiles[kTiles128] / work.max_ktiles;
+      if (long_tiles > 256.0 && long_tiles <= kTileShapes[kTiles128].round && has_split_rows(plans, members, n, kTiles128))
+        return launch_tiles_as<GemmTiles<2, 2, 4, 4, 2, true>, 2>(launch, stream);
+      return launch_tiles_as<GemmTiles<2, 2, 4, 4, 2>, 2>(launch, stream);
+    }
     case kTiles128Deep: return launch_tiles_as<GemmTiles<2, 2, 4, 4, 4>, 1>(launch, stream);
     // Eight waves: with four of 128 x 64 the start and the staged output of a tile took 2 to 3 us longer (us, four / eight:
     // 3400 x 3400 symmetric with D, k 3400 59.8 / 56.5   3200 x 3200 symmetric, k 3080 53.1 / 51.1

@@ -15,13 +15,14 @@ def _integers(shape, device, gen):
     return torch.randint(-3, 4, shape, generator=gen, device=device, dtype=torch.int8).bfloat16()
 
 
-def _check(device, batch, m, n, k, symmetric, tiles):
-    """alpha a b^T + beta d, with a transposed output where that is allowed, and nothing written beside them."""
+def _check(device, batch, m, n, k, symmetric, tiles, offset=0):
+    """alpha a b^T + beta d, with a transposed output where that is allowed, and nothing written beside them.
+    ``offset``: elements by which the operands lie off a cache line."""
     assert hip_ops.gemm_tiles((batch, m, n, k, symmetric)) == (tiles,)
     gen = torch.Generator(device=device)
     gen.manual_seed(k)
-    a = _integers((batch, m, k), device, gen)
-    b = a if symmetric else _integers((batch, n, k), device, gen)
+    a = _integers((batch * m * k + offset,), device, gen)[offset:].view(batch, m, k)
+    b = a if symmetric else _integers((batch * n * k + offset,), device, gen)[offset:].view(batch, n, k)
     d = _integers((batch, m, n), device, gen)
     if symmetric:
         d = d + d.transpose(1, 2)
@@ -42,3 +43,13 @@ def _check(device, batch, m, n, k, symmetric, tiles):
 )
 def test_256_x_128_tiles(device, batch, m, n, k, symmetric):
     _check(device, batch, m, n, k, symmetric, "256x128")
+
+
+@pytest.mark.parametrize(
+    "batch,m,n,k,symmetric,offset",
+    [(3, 1433, 1433, k, False, offset) for k, offset in ((64, 8), (72, 0), (128, 56), (136, 0), (192, 8), (200, 0), (264, 0), (392, 0))]
+    + [(2, 1968, 1968, k, True, offset) for k, offset in ((392, 0), (448, 8), (1000, 0), (1968, 0))],
+)
+def test_128_x_128_tiles_of_rows_that_straddle_cache_lines(device, batch, m, n, k, symmetric, offset):
+    """432 and 272 tiles: some compute units have two of them, others one."""
+    _check(device, batch, m, n, k, symmetric, "128", offset)
