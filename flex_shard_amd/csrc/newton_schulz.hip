@@ -757,17 +757,29 @@ int launch_tiles(PlannedGemm* plans, const int* members, int n, hipStream_t stre
   if (has_wide_rows(plans, members, n)) return launch_tiles_as<GemmTiles<2, 2, 4, 4, 2>, 2, true>(launch, stream);
   switch (kind) {
     case kTiles64: {
-      // Tiles that leave a compute unit with one workgroup or two are requested further ahead: nothing else covers
-      // their requests.  More of them, and somewhat fewer of few k-tiles, lose more by the LDS that takes (us, two /
-      // three / four k-tiles ahead; tiles of a shorter contraction count by their share of the longest):
-      //   136 tiles, k 4096 27.9 / 17.0 / 14.7   256, k 4096 27.6 / - / 14.9   256, k 2048 9.5 / - / 9.2
-      //   231, k 1672 9.4 / - / 9.0   300, k 4096 29.0 / - / 23.7   384, k 2048 15.9 / - / 13.9   406, k 1792 16.3 / - / 14.7
-      //   378, k 2944 22.8 / 21.2 / 21.7   406, k 3072 23.6 / 22.2 / 22.5   435, k 3072 23.7 / 22.3 / 22.6
-      //   484, k 1408 12.3 / - / 11.3   384, k 1024 7.7 / - / 8.2   448, k 1280 9.4 / - / 10.0   512, k 2048 13.4 / - / 14.8
+      // Tiles that leave a compute unit with one workgroup or two are requested further ahead: nothing else covers their
+      // requests.  Two per unit hold three k-tiles each (A as late as B); more of them, short contractions, whose operands
+      // stay in an XCD's 4 MB of L2, and rows that straddle cache lines, of which a unit can only have so many in flight,
+      // lose by more than two (us, two / three / four k-tiles ahead, symmetric; tiles of a shorter contraction count by
+      // their share of the longest):
+      //   rows at cache lines     k 1024              1152                1408                3072                5376
+      //   253 tiles          6.5 /  6.3 /  6.4    -                   -                  22.2 / 15.5 / 13.0  36.0 / 23.6 / 19.5
+      //   300                7.6 /  7.9 /  8.2    8.3 /  8.5 / -     11.6 /  9.7 / -     22.6 / 19.0 / 19.9  36.4 / 30.8 / 32.2
+      //   351                8.0 /  8.2 /  8.6    9.1 /  8.8 / -     12.6 / 11.1 / -     23.2 / 21.1 / 21.5  37.4 / 33.7 / 35.8
+      //   406                8.5 /  8.7 /  8.9   10.1 /  9.5 / -     13.1 / 11.7 / -     23.5 / 22.0 / 22.0  38.4 / 34.6 / 36.9
+      //   496                9.5 /  9.5 /  9.7   11.6 / 10.6 / -     13.6 / 12.5 / -     24.6 / 23.0 / 23.3  39.9 / 35.4 / 39.1
+      //   528               11.0 / 12.1 / 13.6    -                   -                  24.6 / 30.1 / 30.8  40.1 / 48.8 / 51.1
+      //   rows across them        k 1032              1160                1416                3080                5384
+      //   253                7.4 /  7.3 /  7.4    -                   -                  23.2 / 18.8 / 18.7  37.1 / 29.4 / 29.5
+      //   276                9.0 /  9.9 / -       9.5 / 10.6 / -     11.3 / 12.1 / -     23.5 / 23.1 / -     37.8 / 41.0 / -
+      //   300                9.4 / 10.0 / 10.4   10.0 / 10.8 / -     12.5 / 12.5 / -     24.0 / 25.7 / 27.6  38.5 / 44.4 / 48.4
+      //   406               11.3 / 11.5 / 11.6   12.7 / 13.2 / -     15.2 / 16.3 / -     27.5 / 32.0 / 32.3  47.5 / 53.6 / 53.5
+      //   496               13.2 / 13.0 / 12.9   14.5 / 14.4 / -     17.1 / 17.2 / -     30.2 / 33.7 / 33.8  49.8 / 56.0 / 55.5
       const LaunchWork work = work_of(plans, members, n);
       const double long_tiles = work.tile_ktiles[kTiles64] / work.max_ktiles;
       if (long_tiles <= 256.0) return launch_tiles_as<GemmTiles<2, 2, 2, 2, 4>, 2>(launch, stream);
-      if (long_tiles <= (work.max_ktiles >= 22.0 ? 500.0 : 384.0)) return launch_tiles_as<GemmTiles<2, 2, 2, 2, 3>, 2>(launch, stream);
+      if (long_tiles <= 500.0 && work.max_ktiles >= 18.0 && !has_split_rows(plans, members, n, kTiles64))
+        return launch_tiles_as<GemmTiles<2, 2, 2, 2, 3, true>, 3>(launch, stream);
       return launch_tiles_as<GemmTiles<2, 2, 2, 2, 2>, 4>(launch, stream);
     }
     case kTiles128: {

@@ -3,10 +3,12 @@ requested in a form of their own, at ragged sizes and at contractions around the
 number of k-tiles that are requested ahead.  Sums of products of small integers
 are exact in fp32, so outputs are compared bit for bit."""
 
+import ctypes
+
 import pytest
 import torch
 
-from flex_shard_amd import hip_ops
+from flex_shard_amd import _native, hip_ops
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +55,23 @@ def test_256_x_128_tiles(device, batch, m, n, k, symmetric):
 def test_128_x_128_tiles_of_rows_that_straddle_cache_lines(device, batch, m, n, k, symmetric, offset):
     """432 and 272 tiles: some compute units have two of them, others one."""
     _check(device, batch, m, n, k, symmetric, "128", offset)
+
+
+@pytest.mark.parametrize("k", [64 * 18, 64 * 19, 64 * 20, 64 * 21, 64 * 24])
+@pytest.mark.parametrize("batch,m,n,symmetric,offset", [(26, 130, 257, False, 0), (26, 130, 257, False, 8), (1, 1790, 1790, True, 0)])
+def test_64_x_64_tiles_of_long_contractions(device, batch, m, n, k, symmetric, offset):
+    """390 and 406 tiles of 18 k-tiles and more, rows at cache lines and across them."""
+    _check(device, batch, m, n, k, symmetric, "64", offset)
+
+
+def test_64_x_64_tiles_of_a_contraction_that_ends_in_a_k_tile(device):
+    """Rows of 1152 elements, 1144 of them summed over: whole cache lines, a last k-tile of seven chunks."""
+    gen = torch.Generator(device=device)
+    gen.manual_seed(5)
+    a, b = _integers((26, 130, 1152), device, gen), _integers((26, 257, 1152), device, gen)
+    desc, out = hip_ops._gemm_desc(a, b, None, 1.0, 0.0, None, None, False)
+    desc.k = 1144
+    a[:, :, 1144:], b[:, :, 1144:] = float("nan"), float("inf")  # not part of the product
+    _native.check(_native.lib().fsh_gemm_bf16_nt(ctypes.byref(desc), hip_ops.stream_ptr(device)), "fsh_gemm_bf16_nt")
+    want = torch.bmm(a[:, :, :1144].float(), b[:, :, :1144].float().transpose(1, 2).contiguous()).bfloat16()
+    assert torch.equal(out, want)
