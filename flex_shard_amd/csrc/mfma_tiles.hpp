@@ -12,7 +12,6 @@ namespace fsh {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 struct GemmParams {
   const uint16_t* A;
@@ -134,6 +133,7 @@ __device__ inline void store_staged_rows(const uint8_t* region, uint16_t* dst, i
   constexpr int kLanesPerRow = kRowBytes / 16;
   constexpr int kRowsPerPass = 64 / kLanesPerRow;
   static_assert(kRowBytes % 16 == 0 && 64 % kLanesPerRow == 0 && kRows % kRowsPerPass == 0, "staged store shape");
+  static_assert(kPitch % 16 == 0, "rows are read 16 bytes at a time");
   const int r0 = lane / kLanesPerRow, chunk = lane % kLanesPerRow;
   const uint32_t lane_off = static_cast<uint32_t>(r0) * static_cast<uint32_t>(ld * 2) + chunk * 16;
   uint8_t* base = uniform_ptr(reinterpret_cast<uint8_t*>(dst));
@@ -143,14 +143,7 @@ __device__ inline void store_staged_rows(const uint8_t* region, uint16_t* dst, i
   for (int pass = 0; pass < kRows / kRowsPerPass; ++pass) {
     const int r = pass * kRowsPerPass + r0;
     const uint8_t* src = region + r * kPitch + chunk * 16;
-    u32x4 v;
-    if (kPitch % 16 == 0) {
-      v = *reinterpret_cast<const u32x4*>(src);
-    } else {
-      const u32x2 lo = *reinterpret_cast<const u32x2*>(src);
-      const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8);
-      v = u32x4{lo.x, lo.y, hi.x, hi.y};
-    }
+    const u32x4 v = *reinterpret_cast<const u32x4*>(src);
     if (r < rows) *reinterpret_cast<u32x4*>(base + pass * pass_bytes + lane_off) = v;
   }
 }
@@ -418,19 +411,14 @@ __device__ __forceinline__ void dma_load_16(uint32_t voffset, const uint8_t* bas
 __device__ inline void dma_load_16_at(const uint8_t* src, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory");
 }
-// 4 bytes per lane: lane l writes LDS bytes [M0 + 4 l, M0 + 4 l + 4).
-__device__ inline void dma_load_4_at(const uint8_t* src, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds_addr) : "memory");
-}
 template <int kInFlight>
 __device__ inline void wait_for_dma_loads_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kInFlight) : "memory"); }
 __device__ inline void wait_for_dma_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// 4 bytes per lane from a uniform base plus a 32-bit per-lane offset.
+// 4 bytes per lane from a uniform base plus a 32-bit per-lane offset: lane l
+// writes LDS bytes [M0 + 4 l, M0 + 4 l + 4).
 __device__ inline void dma_touch_4(uint32_t voffset, const uint8_t* base, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voffset), "s"(base), "s"(lds_addr) : "memory");
 }
-
-constexpr int max_int(int a, int b) { return a > b ? a : b; }
 
 // Eight bf16 of a row that ends at column `cols`, starting at column `col`
 // (< cols); 16-byte access when `vec` allows it, columns past the end as zero.

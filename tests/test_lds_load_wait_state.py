@@ -19,4 +19,4 @@ def test_every_load_to_lds_waits_for_m0():
                 if line.startswith(("global_load_lds", "buffer_load")):
                     loads += 1
                     assert i >= 2 and re.match(r"s_\w+ m0,", lines[i - 2]) and lines[i - 1] == "s_nop 0", (name, block)
-    assert loads >= 4
+    assert loads >= 3  # 16 bytes per lane by offset and by address, 4 by offset
