@@ -8,12 +8,11 @@
 //   out[m][n] = bf16( sum over k-blocks kb of
 //                     dot(xq[m][kb], wq[n][kb]) * (xs[kb][m] * ws[n / 128][kb]) )
 //
-// Matrix cores: v_mfma_f32_16x16x128_f8f6f4 here, 32x32x64 in the smaller tiles
-// (twice the rate of the 32x32x16 FP8 form on gfx950).  A k-tile is one scale
-// block (128 bytes of each row), so its partial products are accumulated from
-// zero in a scratch accumulator and folded into the result with one fused
-// multiply-add per element; the folds of one block run on the vector ALU while
-// the matrix core works on the next ones.
+// Matrix cores: v_mfma_f32_16x16x128_f8f6f4 (twice the rate of the 32x32x16 FP8
+// form on gfx950).  A k-tile is one scale block (128 bytes of each row) and one
+// such MFMA per block of 16 x 16: its partial product, from zero, is folded into
+// the result with one fused multiply-add per element; the folds of one block run
+// on the vector ALU while the matrix core works on the next ones.
 #include "fp8_tiles.hpp"
 
 namespace fsh {
@@ -205,13 +204,19 @@ namespace fsh {
 namespace {
 
 // Which tiles a product takes: the ones with the lowest estimated time.
-// Measured (us with 64 x 64 tiles, 128 x 128, 256 x 256; weights in the last-level
-// cache; block scales, the column-scale variant runs 5-10 % longer on all three;
-// * fewer tiles than compute units, the deep form below):
-//   48 x 14336, k 4096     10.8*  18.3*  24.2      144 x 3840, k 10240  22.0*  40.7*  55.8
-//   512 x 4096, k 4096     15.3   19.0*  24.7      1000 x 2048, k 5120  19.5   23.1*  31.7
-//   335 x 11136, k 10112   72.5   60.2   55.0      1000 x 5120, k 2048  20.2   16.6   15.7
-//   1400 x 4096, k 4096    39.1   30.2   27.7      2048 x 4096, k 1024  17.8   12.5   12.4
+// Measured (us with 64 x 64 tiles, 128 x 128, 256 x 256; block scales, the
+// column-scale variant runs 5-10 % longer on all three; * fewer tiles than compute
+// units, the deep form below), launches back to back on the same operands, and
+// with the weight from memory:
+//   48 x 14336, k 4096     11.1*  18.6*  24.2   15.4*  21.3*  32.9
+//   1000 x 2048, k 5120    20.1   23.3*  31.6   25.0   27.6*  39.9
+//   1000 x 5120, k 2048    19.9   16.9   15.5   24.4   21.5   18.5
+//   553 x 12160, k 3456    42.7   29.9   35.2   49.0   33.8   43.9
+//   3192 x 4736, k 1280    35.1   25.4   22.6   37.9   26.6   24.0
+//   2295 x 3072, k 8960    97.2   66.2   60.5   105    76.2   65.2
+// (weight from memory: the order is the same)
+//   144 x 3840, k 10240    22.0*  40.7*  55.8                        512 x 4096, k 4096     15.3   19.0*  24.7
+//   335 x 11136, k 10112   72.5   60.2   55.0                        1400 x 4096, k 4096    39.1   30.2   27.7
 //
 // A compute unit with one workgroup to run has LDS to spare: more operand
 // requests in flight ("deep").  Not where a unit runs several, whose requests
@@ -242,8 +247,10 @@ Fp8TileKind fp8_tile_kind(int64_t m, int64_t n, int64_t k, bool column_scales, i
     const int64_t tiles = ceil_div(m, kShapes[i].m) * ceil_div(n, kShapes[i].n);
     if ((i == 1 && tiles <= units) || (i == 2 && tiles > units)) continue;  // 128 x 128 is deep up to a tile per unit
     TileShape shape = kShapes[i];
-    // (a last round of 129 to 255 is not cut: 1152 x 6784 over 1357 tokens, 135 tiles, column scales 22.3, with 128 x 128 18.8)
-    if (i == 3 && 2 * (tiles % 256) > 256) shape.half = 1.2;
+    // A last round of more than half as many is not cut.  Us with 256 x 256 and 128 x 128 tiles, by the tiles of that round:
+    //   132 33.5 / 29.7   144 35.2 / 29.9   135 22.3 / 18.8 (column scales, k 1408)
+    //   143 38.3 / 48.3 (column scales, k 2944)   147 105 / 143   160 18.9 / 20.6   169 47.0 / 58.9   247 22.6 / 25.4
+    if (i == 3 && units > 0 && 2 * (tiles % units) > units) shape.half = 1.2;
     const double us = rounds_us(shape, static_cast<double>(tiles), static_cast<double>(tiles) * ktiles, ktiles);
     if (i == 0 || us < best_us) {
       best = i;

@@ -152,8 +152,11 @@ __global__ __launch_bounds__(Cfg::kThreads, kBlocksPerUnit * Cfg::kWaves / 4) vo
   const GemmParams& p = launch.problem[which];
   int64_t batch;
   int tm, tn;
-  // An XCD that holds 64 tiles at a time takes patches of 8 x 8 (16 operand panels for 20: 8 x 768 x 768 and
-  // 8 x 768 x 3072, k 768 52.4 -> 49.9 us); eight rows of the few tiles of a small launch cost it (14.7 -> 19.3).
+  // An XCD with 64 tiles or more takes them in patches of eight rows, not four: over 8 x 8 tiles 16 operand panels
+  // serve what takes 20 over 4 x 16.  Us with eight / four: 64 x 64 tiles 1424 x 1424, k 1424 18.5 / 19.6, 2000 x 2000
+  // symmetric 25.1 / 26.5, 3064 x 824, k 824 14.2 / 13.8; 128 x 128 tiles 8 x 768 x 768 with 8 x 768 x 3072, k 768 49.9 /
+  // 52.4, 3 x 4920 x 1032 54.7 / 53.3; 256 x 128 tiles 8 x 2080 x 2080 symmetric 88.3 / 89.5, 8 x 7696 x 1496 369 / 364.
+  // Eight rows of the few tiles of a small launch cost it (14.7 -> 19.3).
   const int rows_together = p.items_per_xcd >= 64 ? 2 * kGroupTilesM : kGroupTilesM;
   if (!tile_of_workgroup(p, static_cast<int64_t>(blockIdx.x) - launch.first_workgroup[which], &batch, &tm, &tn, rows_together))
     return;  // whole workgroup

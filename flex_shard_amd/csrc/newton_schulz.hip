@@ -484,14 +484,22 @@ struct PlannedGemm {
 };
 
 // ---- Which tiles a launch takes.
-// Measured over 13 shapes from 512^2 to 8192 x 6144 at k = 512 and 2048 (us for
-// k = 512 / 2048, tiles of 64 x 64, 128 x 128, 256 x 128, 256 x 256; k-tiles of 64):
-//   1024 x 1024     5.5 / 10.4    8.1 / 17.4   10.2 / 25.4   16.3 / 38.9
-//   2048 x 2048    11.5 / 30.6    9.7 / 22.7   11.6 / 28.0   17.2 / 40.6
-//   4096 x 2048    18.8 / 55.6   15.5 / 40.0   14.9 / 36.5   18.8 / 43.4
-//   4096 x 4096    35.9 / 108.5  27.3 / 80.5   28.0 / 74.6   22.4 / 53.3
-// The three smaller kinds have become 5 to 20 % faster since, much alike
-// (4096 x 4096 30.7 / 97.0  22.6 / 60.8  24.8 / 60.4), so the choice among them stands.
+// Measured at k = 512 / 2048 (us; k-tiles of 64; 128 x 128: where one workgroup
+// per compute unit would do, the deep form in brackets):
+//               64 x 64       128 x 128                   256 x 128      256 x 256
+//   1024 x 1024    5.0 /  9.6    6.9 / 14.8 ( 7.5 / 15.3)    8.9 / 23.8   15.3 / 37.5
+//   2048 x 2048    8.9 / 25.9    8.0 / 21.2 ( 8.5 / 18.4)    9.8 / 24.3   16.0 / 38.6
+//   4096 x 2048   15.4 / 47.3   12.4 / 31.4                 12.2 / 29.9   17.7 / 39.8
+//   4096 x 4096   28.4 / 90.0   21.7 / 58.7                 23.2 / 57.9   19.9 / 49.8
+// The constants below were fitted to earlier kernels of the three smaller sizes
+// (4096 x 4096, k 2048: 108.5, 80.5, 74.6).  Over 50 products of 256 to 8192 a
+// side the estimates are now, as a multiple of the measured time (tenth, middle
+// and ninth of ten), for rows at cache lines 1.06 / 1.23 / 1.36, 1.13 / 1.25 / 1.38,
+// deep 0.96 / 1.07 / 1.19, 1.09 / 1.19 / 1.31 and 0.90 / 0.96 / 1.05, and lower by a
+// tenth for rows that straddle them: beside the others the deep tiles and the
+// 256 x 256 ones look better than they are.  None of 80 products and 50 Muon
+// steps was slower for it than with the earlier kernels; the fastest kind would
+// have been 3 % faster in the mean.
 enum TileKind { kTiles64, kTiles128, kTiles128Deep, kTiles256x128, kTiles256 };  // the order of kTileShapes
 constexpr int kTileNames[] = {FSH_TILES_64, FSH_TILES_128, FSH_TILES_128_DEEP, FSH_TILES_256X128, FSH_TILES_256};
 constexpr TileShape kTileShapes[] = {
@@ -543,7 +551,7 @@ TileKind small_tile_kind(const LaunchWork& w) {
   }
   return best;
 }
-constexpr double kEstimateMargin = 0.95;  // the estimates are off by about 5 %
+constexpr double kEstimateMargin = 0.95;  // for the error of the comparison (see above: it favours the large tiles)
 double small_tiles_us(const LaunchWork& w) { return launch_us(small_tile_kind(w), w); }
 
 // The 256 x 256 kernel has 16-byte accesses in the epilogue and 32-bit tile spans.
