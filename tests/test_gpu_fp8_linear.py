@@ -143,12 +143,10 @@ def test_gemm_rejects_what_the_kernel_cannot_take(device):
         hip_ops.fp8_gemm_1x128_128x128(xq, xs, wq, ws)
 
 
-def test_contraction_longer_than_one_window_of_weight_scales(device):
-    """k = two windows of the 256 x 256 kernel (256 k-tiles of weight scales each)
-    + 3 k-tiles, every weight scale different, against the oracle's product;
-    forward and input-gradient (scale table read across) forms.  So few rows
-    and columns take 64 x 64 tiles, which request the scales of every k-tile
-    with its operands; the next test refills the window."""
+def test_long_contraction_with_every_weight_scale_different(device):
+    """515 k-tiles against the oracle's product, forward and input-gradient
+    (scale table read across) forms.  So few rows and columns take 64 x 64
+    tiles; the next test takes the 256 x 256 ones."""
     gen = torch.Generator().manual_seed(5)
     m, n, k = 96, 384, 2 * 32768 + 384
     x = torch.randn(m, k, generator=gen).bfloat16()
@@ -167,12 +165,13 @@ def test_contraction_longer_than_one_window_of_weight_scales(device):
 
 
 @pytest.mark.parametrize("m,n", [(4096, 4096), (4000, 4100)])
-def test_window_of_weight_scales_refilled_in_the_loop(device, m, n):
-    """The 256 x 256 kernel keeps 256 k-tiles of weight scales in LDS and refills
-    the window when the loop crosses it (here once, three k-tiles before the
-    end).  Operands in -1..1 and power-of-two scales: every sum is a multiple
-    of 2^-2 below 2^18 and so exact in fp32, and the outputs are the one bf16
-    rounding of it; forward and input-gradient (scale table read across) forms."""
+def test_long_contraction_of_the_large_tiles(device, m, n):
+    """259 k-tiles on the 256 x 256 tiles, which request a k-tile's scales with
+    its operands (the rule names contractions of more than 256 of them apart;
+    the kernel is the same).  Operands in -1..1 and power-of-two scales: every
+    sum is a multiple of 2^-2 below 2^18 and so exact in fp32, and the outputs
+    are the one bf16 rounding of it; forward and input-gradient (scale table
+    read across) forms."""
     ktiles = 256 + 3
     k = 128 * ktiles
     assert hip_ops.fp8_gemm_tiles(m, n, k) == "256 long k"

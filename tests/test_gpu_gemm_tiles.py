@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 CASES = [
     # 64 x 64 tiles
     (1, 1, 1, 8), (1, 64, 64, 64), (1, 65, 63, 72), (2, 130, 257, 136), (1, 129, 127, 520), (3, 33, 300, 248),
-    # 128 x 128 tiles, operands requested three k-tiles ahead (240 tiles)
+    # 128 x 128 tiles, operands requested four k-tiles ahead (240 tiles)
     (1, 1920, 1928, 264), (1, 1923, 1837, 392), (1, 1920, 1920, 576),
     # 64 x 64 tiles, more than the chip holds at once (2304 and 2304 tiles)
     (32, 520, 500, 456), (32, 513, 511, 520),
