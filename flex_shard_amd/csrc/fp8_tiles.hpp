@@ -112,7 +112,9 @@ struct Fp8Tile {
 // path (one 1 KB request per 16 cycles: the 32 of a 128 x 128 k-tile last as long
 // as its MFMAs) where it has several.  Before, they ran 32 x 32 x 64 MFMAs whose 16
 // registers were folded behind the next one's, and their requests left in one go
-// behind the last block, held up by one another.  us before / now, same bits:
+// behind the last block, held up by one another.  us before / now; the same bits
+// unless a run's products span more than 24 bits, where up to 4e-5 of the outputs lie on
+// the other side of a bf16 rounding (2-norm from 64-bit sums the same to 1e-6 of it):
 //   64 x 64:    48 x 14336, k 4096 12.1 / 10.8   144 x 3840, k 10240 23.4 / 22.0   512 x 4096, k 4096 16.1 / 14.6
 //               3000 x 1024 over 1500 tokens, column scales 12.0 / 10.0   1000 x 2048, k 5120 20.1 / 19.1
 //   128 x 128:  1000 x 5120, k 2048 18.9 / 16.6   1024 x 4096, k 8192 45.6 / 38.8
@@ -164,6 +166,13 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
     dma_load_16(voff[c], (c < kChunksA ? Ab : Bb) + static_cast<int64_t>(kt) * Cfg::kRowBytes,
                 fill_lds + (c < kEarly ? at.early : at.late), (c < kEarly ? c : c - kEarly) * Cfg::kChunkBytes);
   };
+  // The first k-tile's operands, ahead of everything that has to be worked out
+  // for the scales (behind it, a tile of one k-tile took 0.02 to 0.05 us longer:
+  // us of 6194 x 10880 over 100 tokens, before the chunks / behind / ahead 34.9 /
+  // 35.4 / 35.0; 300 x 2048, k 2048 7.9 / 6.9 / 6.8).
+  Place ahead = kFirst;
+#pragma unroll
+  for (int c = 0; c < kChunks; ++c) request(0, ahead, c);
   // The scales of a k-tile ride the same global->LDS path, 64 by one request of
   // each wave: the row scales, then the column scales -- or the block scale of
   // 64 of the tile's columns, 64 times.  (A load that the compiler sees inside
@@ -193,6 +202,9 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
     dma_touch_4(scale_voff, reinterpret_cast<const uint8_t*>(scale_src + kt * scale_step), scale_lds + at.scales);
   };
 
+  request_scales(0, ahead);
+  ahead = place_after(ahead);
+
   // Fragment side: row = lane & 15 of a 16-row block, chunks g and g + 4 of its
   // eight (g = lane / 16), each in slot chunk ^ ((row >> 1) & 7).  Any split of
   // the 128 bytes over the four g will do that both operands share; with chunks
@@ -219,11 +231,10 @@ __device__ __forceinline__ void fp8_gemm_tile(const Fp8GemmParams& p, uint8_t* l
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // The first kDepth - 1 k-tiles and the early chunks of the next.
+  // The rest of the first kDepth - 1 k-tiles and the early chunks of the next.
   Place now = kFirst, before = kLast;  // of k-tile kt and of the one before it, whose slots are free
-  Place ahead = kFirst;
 #pragma unroll
-  for (int kt = 0; kt < kDepth; ++kt) {
+  for (int kt = 1; kt < kDepth; ++kt) {
     if (kt < ktiles) {
       if (kt + 1 < kDepth) request_scales(kt, ahead);
 #pragma unroll
