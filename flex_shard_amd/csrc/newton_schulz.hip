@@ -738,8 +738,10 @@ bool has_wide_rows(const PlannedGemm* plans, const int* members, int n) {
   }
   return false;
 }
-// Whether most of a launch's work on tiles of a kind reads operand rows that do
-// not start at cache lines: a k-tile's 128 bytes of such a row touch two.
+// Whether three quarters of a launch's work on tiles of a kind read operand rows
+// that do not start at cache lines: a k-tile's 128 bytes of such a row touch two.
+// (With six tenths, 5 of 952 x 1128 beside whole rows, a Muon step takes 438 us as
+// the others and 443 as these; with a half 584 and 587.)
 bool has_split_rows(const PlannedGemm* plans, const int* members, int n, TileKind kind) {
   double split = 0.0, all = 0.0;
   for (int k = 0; k < n; ++k) {
@@ -752,7 +754,7 @@ bool has_split_rows(const PlannedGemm* plans, const int* members, int n, TileKin
     };
     if (!at_lines(p.A, p.lda, p.sA) || !at_lines(p.B, p.ldb, p.sB)) split += work.tile_ktiles[kind];
   }
-  return 2.0 * split > all;
+  return 4.0 * split > 3.0 * all;
 }
 TileKind small_tile_kind_of(const PlannedGemm* plans, const int* members, int n) {
   return has_wide_rows(plans, members, n) ? kTiles128 : small_tile_kind(work_of(plans, members, n));
