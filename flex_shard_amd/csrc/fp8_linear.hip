@@ -214,9 +214,8 @@ namespace {
 //   553 x 12160, k 3456    42.7   29.9   35.2   49.0   33.8   43.9
 //   3192 x 4736, k 1280    35.1   25.4   22.6   37.9   26.6   24.0
 //   2295 x 3072, k 8960    97.2   66.2   60.5   105    76.2   65.2
-// (weight from memory: the order is the same)
-//   144 x 3840, k 10240    22.0*  40.7*  55.8                        512 x 4096, k 4096     15.3   19.0*  24.7
-//   335 x 11136, k 10112   72.5   60.2   55.0                        1400 x 4096, k 4096    39.1   30.2   27.7
+//   144 x 3840, k 10240    22.0*  40.7*  55.8   512 x 4096, k 4096     15.3   19.0*  24.7  (the same operands only)
+//   335 x 11136, k 10112   72.5   60.2   55.0   1400 x 4096, k 4096    39.1   30.2   27.7
 //
 // A compute unit with one workgroup to run has LDS to spare: more operand
 // requests in flight ("deep").  Not where a unit runs several, whose requests
